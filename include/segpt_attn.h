@@ -94,16 +94,14 @@ extern "C" {
 
 /* the four stages segpt_attn_bwd() runs, in this order */
 #define SEGPT_BWD_STAGE_PRE 0    /* bf16: key/value pre-pass (skipped with SEGPT_FLAG_KV_PREPARED): normalised
-                                    Khat (and V' = c1 v + c2 v_first) into kv_workspace;
-                                    fp32: delta = rowsum(dY*Y), dgate and the gate-scaled dO            */
-#define SEGPT_BWD_STAGE_DQ 1     /* dQ and the per-workgroup partials of the scale gradient; on the bf16
-                                    path also delta, dgate and Qhat for stage 2 (a positive gate factor
-                                    is folded into the row statistics; a gate scale <= 0 adds a
-                                    gate-scaled copy of dO)                                              */
-#define SEGPT_BWD_STAGE_DKDV 2   /* dK, dV (, dV_first, partial sums of d vr_coef); bf16: also dg_q, dg_k from
+                                    Khat (and V' = c1 v + c2 v_first) into kv_workspace; fp32: nothing  */
+#define SEGPT_BWD_STAGE_DQ 1     /* dQ, delta, dgate and the per-workgroup partials of the scale gradient; on
+                                    the bf16 path also Qhat for stage 2 (a positive gate factor is folded
+                                    into the row statistics; fp32, or a gate scale <= 0, adds a gate-scaled
+                                    copy of dO)                                                                        */
+#define SEGPT_BWD_STAGE_DKDV 2   /* dK, dV (, dV_first, partial sums of d vr_coef) and dg_q, dg_k from
                                     the partials of stage 1                                              */
-#define SEGPT_BWD_STAGE_REDUCE 3 /* d vr_coef from the partials (fp32: also dg_q, dg_k); launches nothing on
-                                    the bf16 path without a value residual                               */
+#define SEGPT_BWD_STAGE_REDUCE 3 /* d vr_coef from the partials; launches nothing without a value residual */
 
 /* [B, heads, S, D] tensor view; the D axis is contiguous (stride 1). Strides in ELEMENTS.
  * The reference's `(h b) S D` flatten (attention.py:199) is stride_b = S*D, stride_h = B*S*D;

@@ -19,7 +19,9 @@ SOURCES = ["api.hip", "f32_path.hip", "pre_post.hip", "fwd_mfma.hip", "bwd_mfma.
 # The forward is also scheduled with the backend's "max-ilp" strategy (2-4 % faster in same-box A/B runs; no effect
 # on the backward kernels, which keep the default).
 EXTRA_FLAGS = {"fwd_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-sched-strategy=max-ilp"],
-               "decode_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+               "decode_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+               # one workgroup per CU at head_dim 128 as above: dK/dV 49 -> 43 us at B = 2, H = 4, S = 500
+               "f32_path.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 # -packed-fp32-ops is switched off: hipcc -O3 otherwise forms v_pk_*_f32 from ordinary float code.
 HIPCC_FLAGS = [

@@ -11,19 +11,17 @@ static __device__ __align__(256) unsigned char scratch[SEGPT_NOALLOC_SCRATCH_BYT
 
 namespace segpt {
 
-int f32_rows_per_block();
+int f32_dq_grid(const segpt_attn_params& p);
+int f32_finish_grid(const segpt_attn_params& p);
+int f32_dkdv_splits(const segpt_attn_params& p);
 int bf16_dq_grid(const segpt_attn_params& p);
 int bf16_dkdv_grid(const segpt_attn_params& p);
 
 int dq_blocks(const segpt_attn_params& p) {
-  if (p.dtype != SEGPT_DTYPE_FP32) return bf16_dq_grid(p);
-  const int rows = f32_rows_per_block();
-  return ((p.Sq + rows - 1) / rows) * p.H * p.B;
+  return p.dtype == SEGPT_DTYPE_FP32 ? f32_dq_grid(p) : bf16_dq_grid(p);
 }
 int dkdv_blocks(const segpt_attn_params& p) {
-  if (p.dtype != SEGPT_DTYPE_FP32) return bf16_dkdv_grid(p);
-  const int rows = f32_rows_per_block();
-  return ((p.Sk + rows - 1) / rows) * p.Hkv * p.B;
+  return p.dtype == SEGPT_DTYPE_FP32 ? f32_finish_grid(p) : bf16_dkdv_grid(p);
 }
 
 namespace {
@@ -32,7 +30,7 @@ size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 size_t elem_bytes(const segpt_attn_params& p) { return p.dtype == SEGPT_DTYPE_FP32 ? 4 : 2; }
 
 struct WsLayout {
-  size_t delta, nlse2, do_eff, qhat, dg_part, dcoef_part, total;
+  size_t delta, nlse2, do_eff, qhat, dg_part, dcoef_part, f32_dk_part, f32_dv_part, total;
 };
 struct KvLayout {
   size_t khat, vmix, total;
@@ -84,6 +82,12 @@ WsLayout bwd_layout(const segpt_attn_params& p) {
   off += align_up((size_t)dq_blocks(p) * p.D * sizeof(float));
   w.dcoef_part = off;
   off += align_up((size_t)dkdv_blocks(p) * 2 * sizeof(float));
+  w.f32_dk_part = w.f32_dv_part = off;
+  if (p.dtype == SEGPT_DTYPE_FP32) {
+    const size_t part = align_up((size_t)p.B * p.H * f32_dkdv_splits(p) * p.Sk * p.D * sizeof(float));
+    w.f32_dv_part = off + part;
+    off += 2 * part;
+  }
   w.total = off;
   return w;
 }
@@ -326,7 +330,11 @@ static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage
   a.do_eff = gated_do_copy(*p) ? ws + w.do_eff : nullptr;
   a.dg_part = reinterpret_cast<float*>(ws + w.dg_part);
   a.dcoef_part = reinterpret_cast<float*>(ws + w.dcoef_part);
-  if (p->dtype == SEGPT_DTYPE_BF16) {
+  if (p->dtype == SEGPT_DTYPE_FP32) {
+    a.f32_dk_part = reinterpret_cast<float*>(ws + w.f32_dk_part);
+    a.f32_dv_part = reinterpret_cast<float*>(ws + w.f32_dv_part);
+    a.f32_splits = f32_dkdv_splits(*p);
+  } else {
     a.nlse2 = reinterpret_cast<float*>(ws + w.nlse2);
     a.qhat = reinterpret_cast<uint16_t*>(ws + w.qhat);
   }
@@ -338,7 +346,7 @@ static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage
   for (int stage = stage_lo; stage <= stage_hi; ++stage) {
     switch (stage) {
       case SEGPT_BWD_STAGE_PRE:
-        rc = f32 ? launch_bwd_pre(a, st) : ((p->flags & SEGPT_FLAG_KV_PREPARED) ? 0 : launch_kv_prep(a, st));
+        rc = (f32 || (p->flags & SEGPT_FLAG_KV_PREPARED)) ? 0 : launch_kv_prep(a, st);
         break;
       case SEGPT_BWD_STAGE_DKDV: rc = f32 ? launch_bwd_dkdv_f32(a, st) : launch_bwd_dkdv_bf16(a, st); break;
       case SEGPT_BWD_STAGE_DQ: rc = f32 ? launch_bwd_dq_f32(a, st) : launch_bwd_dq_bf16(a, st); break;

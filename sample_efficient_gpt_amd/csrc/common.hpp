@@ -14,7 +14,7 @@ constexpr float kLn2 = 0.6931471805599453f;
 // Everything a kernel needs: the caller's params by value plus the carved-up workspace.
 struct KArgs {
   segpt_attn_params p;
-  float* delta;       // [B,H,Sq] fp32: rowsum(dO_eff * o)  (fp32 path) / its NEGATIVE (bf16 path: MFMA C operand)
+  float* delta;       // [B,H,Sq] fp32: rowsum(dO * o)  (fp32 path) / its NEGATIVE (bf16 path: MFMA C operand)
   float* nlse2;       // [B,H,Sq] fp32: -lse*log2(e)                 (bf16 path only: MFMA C operand)
   void* do_eff;       // [B,H,Sq,D] dtype, contiguous: gate-scaled dO (fp32 path; bf16 path only for a gate scale <= 0), else null
   uint16_t* qhat;     // [B,H,Sq,D]   bf16: sm_scale*log2e * a_i q_i * g_q*g_k   (bf16 path only)
@@ -29,6 +29,10 @@ struct KArgs {
   float* dec_part;
   float* dec_stat;
   int32_t dec_splits, dec_chunk, dec_kend;
+  // fp32 backward: dKhat and dV of one query head and one share of the query tiles, [B*H, f32_splits, Sk, D] each
+  float* f32_dk_part;
+  float* f32_dv_part;
+  int32_t f32_splits;
 };
 
 // Row normaliser 1/sqrt(mean x^2 + eps) from the row's sum of squares ss (inv_d = 1/D); exactly 1 for plain
@@ -189,11 +193,10 @@ int launch_bwd_dq_f32(const KArgs& a, hipStream_t st);
 int launch_fwd_bf16(const KArgs& a, hipStream_t st);
 int launch_bwd_dkdv_bf16(const KArgs& a, hipStream_t st);
 int launch_bwd_dq_bf16(const KArgs& a, hipStream_t st);
-int launch_bwd_pre(const KArgs& a, hipStream_t st);     // fp32 path: delta, dgate, do_eff
 int launch_fwd_decode_bf16(KArgs a, hipStream_t st);    // split-key forward for a few query rows against a long cache
 size_t decode_plan(const segpt_attn_params& p, int* kend, int* splits, int* chunk);  // returns its scratch bytes
 int launch_kv_prep(const KArgs& a, hipStream_t st);     // bf16 path: Khat (and V') into kv_workspace
-int launch_bwd_reduce(const KArgs& a, hipStream_t st);  // fp32: dg_q, dg_k, dvr_coef from the partials; bf16: dvr_coef only
+int launch_bwd_reduce(const KArgs& a, hipStream_t st);  // dvr_coef from the partials (nothing without a value residual)
 
 // block counts shared by the workspace carve-up and the launchers
 int dq_blocks(const segpt_attn_params& p);

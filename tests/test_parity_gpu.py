@@ -83,6 +83,24 @@ def test_fp32_fwd_bwd(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
     _case(gpu_device, F32, B, H, Hkv, Sq, Sk, D, gen_kw=gen_kw, **kw)
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize(
+    "B,H,Hkv,Sq,Sk,kw,gen_kw",
+    [
+        (1, 1, 1, 1, 1, {}, {}),                                  # three of the four waves own no tile
+        (1, 2, 1, 31, 33, {"q_start": 2}, {"extras": True}),      # one row short of / past a 32-row tile
+        (2, 2, 2, 32, 129, {"causal": False}, {}),                # the fifth tile goes to wave 0 again
+        (1, 9, 3, 97, 97, {}, {"extras": True}),                  # every query tile its own split, some splits empty
+        (5, 16, 4, 289, 289, {}, {}),                             # more than 1024 work items: the plain order
+        (1, 2, 1, 5, 300, {"causal": True}, {}),                  # keys that no query sees: zero gradients
+    ],
+)
+def test_fp32_tile_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
+    """The 32-row tiles of the fp32 kernels, the four-way split of the streamed rows and the splits of dK/dV, same
+    1e-5 as above."""
+    _case(gpu_device, F32, B, H, Hkv, Sq, Sk, D, gen_kw=gen_kw, seed=71, **kw)
+
+
 # ------------------------------------------------------------------ bf16 MFMA path
 
 
