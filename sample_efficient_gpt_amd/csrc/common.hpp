@@ -24,7 +24,8 @@ struct KArgs {
   float* dcoef_part;  // [n_dkdv_blocks, 2] fp32 partial sums of (dc1, dc2)
   int32_t n_dq_blocks;
   int32_t n_dkdv_blocks;
-  // decode path (split keys): partial O [B*Hkv, splits, 32, D] and (max, sum) [B*Hkv, splits, 32, 2], both fp32,
+  // decode path (split keys): partial O [B*Hkv, splits, n_rows, D] and (max, sum) [B*Hkv, splits, n_rows, 2], both fp32
+  // (n_rows = H/Hkv * Sq query rows),
   // carved from kv_workspace
   float* dec_part;
   float* dec_stat;

@@ -3,59 +3,101 @@
 // KVCache :15-27 grows K/V, the module masks with k_idx <= q_start + q_idx, :72-78).
 //
 // The training kernel would run B*H workgroups that each walk the whole cache; here the KEYS are split
-// ("flash decoding"): workgroup (b, kv head g, split s) handles one contiguous chunk of the cache for ALL query
+// ("flash decoding"): wave (b, kv head g, split s) handles one contiguous chunk of the cache for ALL query
 // rows of the group (n = hq * Sq + i, at most 32 = one MFMA column block), writes an unnormalised partial
 // (running maximum M, sum L, O) and a second tiny kernel merges the splits.  Memory-bound by design: every
 // K / V row is read exactly once from HBM, so the key normalisation, the rotary embedding and the value
 // residual mix are done on the fly in registers (no pre-pass, no normalised copy).
 //
 // Per wave and 32-key block (orientation as in the training forward: lane = query column):
-//   K rows -> registers in the MFMA A layout (row = key, 16-byte chunks), rotate, b_j = rsqrt(mean k^2 + eps)
-//   across the lane pair that holds a row, scale, pack            S^T = Khat . Qhat^T          (4 or 8 MFMAs)
-//   online softmax per lane, P^T packed to bf16 = B operand
-//   V rows -> wave-private LDS tile (row-major, padded) -> transposing reads    O^T += V'^T . P^T
+//   K rows from LDS in the MFMA A layout (row = key, 16-byte chunks), rotated if asked     S^T = K . Qhat^T  (4 or 8 MFMAs)
+//   scores times b_j = rsqrt(mean k^2 + eps), exp2, P^T packed to bf16 = B operand
+//   V rows by transposing LDS reads                                                        O^T += V'^T . P^T
+#include <algorithm>
+
 #include "mfma_common.hpp"
 
 namespace segpt {
 namespace {
 
-constexpr int kDecThreads = 256;  // 4 waves, 32 keys each per step
-constexpr int kDecKeysPerStep = 4 * 32;
+constexpr int kDecThreads = 256;  // 4 waves
+constexpr int kDecBlock = 32;     // keys per step of a wave
+constexpr int kMaxSplits = 128;
 
-template <int D>
-struct DecTile {
-  static constexpr int kRS = D + 8;  // padded row stride (elements) of the wave-private V tile
-};
-
-// Transposed fragment of a padded row-major tile (see swz_off_tr for the ds_read_b64_tr_b16 semantics):
-// lane's MFMA row = tile column 32*cb + l%32, contraction entries = tile rows 16*s + {4hh.., 8+4hh..}
-template <int D>
-__device__ __forceinline__ bf16x8 dec_frag_tr(const uint16_t* tile, int cb, int s, int lane) {
-  const int r = lane & 15, hh = lane >> 5;
-  const int col = 32 * cb + 16 * ((lane >> 4) & 1) + 4 * (r & 3);
-  const int row = 16 * s + 4 * hh + (r >> 2);
-  const uint16_t* p = tile + row * DecTile<D>::kRS + col;
-  typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
-  s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p));
-  s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p + 8 * DecTile<D>::kRS));
-  typedef short s16x8 __attribute__((ext_vector_type(8)));
-  s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-  return __builtin_bit_cast(bf16x8, v);
+// LDS regions below are private to a wave: program order is enough, the compiler only has to keep it
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
+// acc + lo^2 + hi^2 of a packed bf16 pair (fp32 products and sum)
+__device__ __forceinline__ float sum_sq_bf16_pair(uint32_t w, float acc) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  const bf2 v = __builtin_bit_cast(bf2, w);
+  return __builtin_amdgcn_fdot2_f32_bf16(v, v, acc, false);
+}
+
+// One 32-row tile filled by ONE wave (swizzled like every tile of Swz): lane offsets of its wave-wide loads from the
+// tile's first row; rows past rows_left re-read the last one.
 template <int D>
-__global__ __launch_bounds__(kDecThreads) void decode_split_kernel(KArgs a) {
+struct WaveTile {
+  static constexpr int kLoads = Swz<D, kDecBlock>::kTileBytes / 1024;
+  uint32_t off[kLoads];
+};
+template <int D>
+__device__ __forceinline__ WaveTile<D> wave_tile_offsets(uint32_t step, int rows_left, int lane) {
+  using Z = Swz<D, kDecBlock>;
+  WaveTile<D> o;
+#pragma unroll
+  for (int i = 0; i < WaveTile<D>::kLoads; ++i) {
+    const int row = i * Z::kRowsPerInst + lane / Z::kChunks;
+    o.off[i] = (uint32_t)min(row, rows_left - 1) * step + (((lane % Z::kChunks) ^ Z::f(row)) << 4);
+  }
+  return o;
+}
+template <int D>
+__device__ __forceinline__ void issue_wave_tile(const char* base, const WaveTile<D>& o, uint32_t dst) {
+#pragma unroll
+  for (int i = 0; i < WaveTile<D>::kLoads; ++i) gload_lds16_so(base, o.off[i], dst + i * 1024);
+}
+// this wave's LDS reads have returned (before the tile they came from is requested over)
+__device__ __forceinline__ void wait_lds_reads() {
+  wave_lds_sync();
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0) only
+}
+
+// One wave per (batch, kv head, split).  The four waves of a workgroup take the SAME keys of four consecutive (batch, kv
+// head) pairs, so that with a rotary embedding the table rows of a key block (as long as a K row each: cos and sin
+// together as much as K and V) come in once per workgroup, double-buffered one block ahead.
+//
+// Bound by HBM: every K and V row once.  What the memory system needs for that is whole lines and requests that stay in
+// flight, so K, V, V_first and the tables all travel by direct global->LDS loads into swizzled tiles (see the request
+// order below).  Before, every lane loaded 16-byte pieces of its own row and, with a rotary embedding, of the two
+// table rows, by each wave for itself.  B = 32, 6 kv heads, 8192 keys, head_dim 64 (403 MB): 121.7 -> 79.1 us with a
+// rotary embedding, 83.8 -> 77.8 without; B = 8, 4 kv heads, 5001 keys, head_dim 128 (82 MB): 33.8 -> 22.9 us.  (Sharing
+// the tables alone: 85.8 and 30.6 us.)
+//
+// What else keeps the loop near the memory rate (it has about 200 vector instructions per 32 keys to hide):
+//   * the normaliser b_j multiplies the 16 scores a lane holds, not the 32 K entries: without a rotary embedding the raw
+//     K bits ARE the matrix operand and the row's sum of squares is 16 dot instructions;
+//   * no running maximum where the QK-norm bound on the logits allows none (see logit_bound), else a lazily raised one;
+//   * only the block that holds the last visible key is masked;
+//   * with a value residual c1 P and c2 P are the operands of two products, V and V_first the raw rows of both.
+// Each wave writes its own partial (M, L, O) of its n_rows live query rows: nothing is merged inside the workgroup.
+// workgroups per CU that LDS (tiles and tables) and registers allow
+template <int D, bool ROPE, bool VRES>
+constexpr int kDecOcc = D == 64 ? (VRES ? 2 : 3) : (ROPE || VRES ? 1 : 2);
+
+template <int D, bool ROPE, bool VRES>
+__global__ __launch_bounds__(kDecThreads, (kDecOcc<D, ROPE, VRES>)) void decode_split_kernel(KArgs a) {
   constexpr int KS = D / 16;
   constexpr int MB = D / 32;
-  constexpr int RS = DecTile<D>::kRS;
+  using Z = Swz<D, kDecBlock>;
   const segpt_attn_params& p = a.p;
-  // wave-private V' tiles during the key loop; afterwards the same memory holds the per-wave O^T partials
-  constexpr int kVtBytes = 4 * 32 * RS * 2, kOsmBytes = 4 * D * 32 * 4;
-  __shared__ __attribute__((aligned(16))) char tile_mem[kVtBytes > kOsmBytes ? kVtBytes : kOsmBytes];
-  uint16_t (*vt)[32 * RS] = reinterpret_cast<uint16_t (*)[32 * RS]>(tile_mem);
-  float (*osm)[D][32] = reinterpret_cast<float (*)[D][32]>(tile_mem);
+  __shared__ __attribute__((aligned(1024))) char tab[ROPE ? 2 * 2 * Z::kTileBytes : 16];  // [buffer][cos, sin] of a key block
+  __shared__ __attribute__((aligned(1024))) char tiles[4][VRES ? 3 : 2][Z::kTileBytes];  // wave-private K, V (, V_first) rows
+  __shared__ __attribute__((aligned(16))) float bsm[4][kDecBlock];                  // wave-private b_j
   __shared__ __attribute__((aligned(16))) float gsm[D];
-  __shared__ float msm[4][32], lsm[4][32];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -63,12 +105,54 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(KArgs a) {
   const int rep = p.H / p.Hkv;
   const int n_rows = rep * p.Sq;  // query rows of this kv head, <= 32
   const int split = blockIdx.x % a.dec_splits;
-  const int bg = blockIdx.x / a.dec_splits;
+  const int bg_all = p.B * p.Hkv, bg_raw = 4 * (int)(blockIdx.x / a.dec_splits) + wave;
+  const bool active = bg_raw < bg_all;  // wave-uniform; an idle wave of the last workgroup only keeps the barriers
+  const int bg = active ? bg_raw : bg_all - 1;
   const int g = bg % p.Hkv, b = bg / p.Hkv;
+  const int k_lo = split * a.dec_chunk;
+  const int k_hi = min(k_lo + a.dec_chunk, a.dec_kend);
+
+  const int2 src = swz_src<D>(lane, wave);
+  const uint32_t tab0 = lds_addr_of(tab);
+  auto issue_tables = [&](int jb, int buf) {
+    const int64_t row0 = (int64_t)(p.rope_k_pos0 + jb) * (D / 2);
+    issue_tile_pair<D, kDecBlock>(reinterpret_cast<const char*>(p.rope_cos + row0), reinterpret_cast<const char*>(p.rope_sin + row0),
+                                  tile_lane_offsets<D, kDecBlock>(D * 2, D * 2, p.Sk - jb, src.x, src.y),
+                                  tab0 + buf * 2 * Z::kTileBytes + wave * 1024);
+  };
+  if constexpr (ROPE) issue_tables(k_lo, 0);
+  // Every row travels global -> LDS as part of whole lines (a row-per-lane load covers 32 bytes of each of 32 rows and
+  // leaves the rest of their lines to the L1, which 64 KB in flight overrun).  One buffer per tensor: a tile is requested
+  // again as soon as its last reader has its fragments, so K is in flight during the softmax and the V product, V during
+  // the next block's scores.  Order of the requests: [tables, K, V, V_first] of block 0, then tables, K, V, V_first of
+  // each next block; every wait below leaves exactly the younger ones in flight.
+  constexpr int kTabLoads = ROPE ? 2 * Z::kPasses : 0, kRowLoads = WaveTile<D>::kLoads, kFirstLoads = VRES ? kRowLoads : 0;
+  const char* kbase = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.k, b, g, 0));
+  const char* vbase = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v, b, g, 0));
+  const char* fbase = VRES ? reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v_first, b, g, 0)) : nullptr;
+  const uint32_t kstep = (uint32_t)p.k.stride_s * 2, vstep = (uint32_t)p.v.stride_s * 2, fstep = (uint32_t)p.v_first.stride_s * 2;
+  const uint32_t ktile = lds_addr_of(tiles[wave][0]), vtile = lds_addr_of(tiles[wave][1]), ftile = lds_addr_of(tiles[wave][VRES ? 2 : 1]);
+  const WaveTile<D> koff = wave_tile_offsets<D>(kstep, kDecBlock, lane), voff = wave_tile_offsets<D>(vstep, kDecBlock, lane);
+  auto issue_rows = [&](const char* base, uint32_t step, const WaveTile<D>& full, int jb, uint32_t dst) {
+    const char* src = base + (int64_t)jb * step;
+    if (p.Sk - jb >= kDecBlock) issue_wave_tile<D>(src, full, dst);
+    else issue_wave_tile<D>(src, wave_tile_offsets<D>(step, p.Sk - jb, lane), dst);
+  };
+  auto issue_k = [&](int jb) { issue_rows(kbase, kstep, koff, jb, ktile); };
+  auto issue_v = [&](int jb) { issue_rows(vbase, vstep, voff, jb, vtile); };
+  auto issue_first = [&](int jb) {
+    if constexpr (VRES) issue_wave_tile<D>(fbase + (int64_t)jb * fstep, wave_tile_offsets<D>(fstep, p.Sk - jb, lane), ftile);
+  };
+  if (active) {
+    issue_k(k_lo);
+    issue_v(k_lo);
+    issue_first(k_lo);
+  }
 
   // ---- this lane's query (B operand column n): Qhat = sm_scale*log2e * a q g_q g_k, zero for padding columns
   if (tid < D) gsm[tid] = gprod_at(p, tid) * p.sm_scale * kLog2e;
   __syncthreads();
+  const bool bounded = !(p.flags & (SEGPT_FLAG_RUNNING_MAX | SEGPT_FLAG_NO_NORM)) && logit_bound<D>(gsm, lane) <= kNoMaxBound;  // wave-uniform
   const bool qlive = ln < n_rows;
   const int hq = qlive ? ln / p.Sq : 0, qi = qlive ? ln % p.Sq : 0;
   bf16x8 qreg[KS];
@@ -79,7 +163,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(KArgs a) {
     for (int ks = 0; ks < KS; ++ks) raw[ks] = *reinterpret_cast<const u32x4*>(qp + 16 * ks);
     float x[KS][8];
     unpack_b_layout<KS>(raw, x);
-    if (p.rope_cos) {
+    if constexpr (ROPE) {
       const int64_t pos = (int64_t)(p.rope_q_pos0 + qi) * (D / 2);
       rope_b_layout<KS>(x, p.rope_cos + pos, p.rope_sin + pos, hh);
     }
@@ -102,124 +186,151 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(KArgs a) {
       qreg[ks] = as_bf16x8(w);
     }
   }
-  // last visible key of this lane's query
+  // last visible key of this lane's query, and the last one every query row sees
   const int qlim = p.causal ? min(qi + p.q_start, p.Sk - 1) : p.Sk - 1;
+  const int all_see = p.causal ? min(p.q_start, p.Sk - 1) : p.Sk - 1;
 
   float c1 = 1.f, c2 = 0.f;
-  if (p.vr_coef) { c1 = p.vr_coef[0]; c2 = p.vr_coef[1]; }
+  if constexpr (VRES) { c1 = p.vr_coef[0]; c2 = p.vr_coef[1]; }
 
   f32x16 oacc[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) oacc[mb] = splat16(0.f);
-  float m_run = -INFINITY, l_run[2] = {0.f, 0.f};  // l_run: this lane's half of the keys, as two partial sums
+  float m_ref = bounded ? 0.f : -INFINITY, l_run[2] = {0.f, 0.f};  // l_run: this lane's half of the keys, as two partial sums
 
-  // keys [k_lo, k_hi) of this split; wave w takes the 32-key blocks w, w+4, ...
-  const int k_lo = split * a.dec_chunk;
-  const int k_hi = min(k_lo + a.dec_chunk, a.dec_kend);
-  uint16_t* my_vt = vt[wave];
-  for (int jb = k_lo + 32 * wave; jb < k_hi; jb += kDecKeysPerStep) {
-    // ---- K rows of the block in the A layout: lane (row ln, chunk hh)
-    const int krow = min(jb + ln, p.Sk - 1);
-    const uint16_t* kp = row_ptr<uint16_t>(p.k, b, g, krow) + 8 * hh;
-    const uint16_t* vp = row_ptr<uint16_t>(p.v, b, g, krow) + 8 * hh;
-    u32x4 kraw[KS], vraw[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      kraw[ks] = *reinterpret_cast<const u32x4*>(kp + 16 * ks);
-      vraw[ks] = *reinterpret_cast<const u32x4*>(vp + 16 * ks);
+  const uint32_t row16 = tab0 + swz_off_row16<D>(lane);
+  const uint32_t krm = ktile + swz_off_rm<D>(lane), vtr = vtile + swz_off_tr<D>(lane), ftr = ftile + swz_off_tr<D>(lane);
+  int buf = 0;
+  wait_vmcnt<0>();  // nothing but tile requests may be in flight in the loop, whose waits count them
+  wave_lds_sync();
+  for (int jb = k_lo; jb < k_hi; jb += kDecBlock) {
+    const bool more = jb + kDecBlock < k_hi;
+    if (active) wait_vmcnt<kRowLoads + kFirstLoads>();  // this block's tables and K
+    else wait_vmcnt<0>();
+    if constexpr (ROPE) {
+      __syncthreads();  // every wave's pieces of the tables are there, and nobody reads the other buffer any more
+      if (more) issue_tables(jb + kDecBlock, buf ^ 1);
     }
-    if (p.v_first.ptr) {
-      const uint16_t* fp = row_ptr<uint16_t>(p.v_first, b, g, krow) + 8 * hh;
+    if (active) {
+      wave_lds_sync();
+      u32x4 kraw[KS];
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const u32x4 f = *reinterpret_cast<const u32x4*>(fp + 16 * ks);
+      for (int ks = 0; ks < KS; ++ks) kraw[ks] = __builtin_bit_cast(u32x4, swz_frag_rm<D>(krm, 0, ks));
+      float ss = 0.f;
+      if constexpr (ROPE) {
+        // one pair of 16-byte chunks (elements e and e + D/2) at a time: few registers beside the loads in flight
+        const uint32_t cos16 = row16 + buf * 2 * Z::kTileBytes, sin16 = cos16 + Z::kTileBytes;
+        float s4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          vraw[ks][i] = pack_bf16x2(c1 * bf16lo(vraw[ks][i]) + c2 * bf16lo(f[i]), c1 * bf16hi(vraw[ks][i]) + c2 * bf16hi(f[i]));
+        for (int ks = 0; ks < KS / 2; ++ks)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const uint32_t off = (uint32_t)((4 * ks + 2 * hh + i) << 4);  // floats 16 ks + 8 hh + 4 i ..
+            const f32x4 c = lds_read_f4(cos16 ^ off), sn = lds_read_f4(sin16 ^ off);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+              const uint32_t wa = kraw[ks][2 * i + t], wb = kraw[ks + KS / 2][2 * i + t];
+              float a0 = bf16lo(wa), a1 = bf16hi(wa), b0 = bf16lo(wb), b1 = bf16hi(wb);
+              rope_pair(a0, b0, c[2 * t], sn[2 * t]);
+              rope_pair(a1, b1, c[2 * t + 1], sn[2 * t + 1]);
+              s4[0] += a0 * a0; s4[1] += a1 * a1; s4[2] += b0 * b0; s4[3] += b1 * b1;
+              kraw[ks][2 * i + t] = pack_bf16x2(a0, a1);
+              kraw[ks + KS / 2][2 * i + t] = pack_bf16x2(b0, b1);
+            }
+          }
+        ss = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+      } else {
+        float s2[2] = {0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s2[i & 1] = sum_sq_bf16_pair(kraw[ks][i], s2[i & 1]);
+        ss = s2[0] + s2[1];
+      }
+      ss = half_sum(ss);
+      if (hh == 0) bsm[wave][ln] = row_normaliser_fast(p, ss, 1.0f / D);
+      f32x16 s = splat16(0.f);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) s = mfma32(as_bf16x8(kraw[ks]), qreg[ks], s);
+      wait_lds_reads();
+      if (more) issue_k(jb + kDecBlock);
+      // register r holds key jb + 4hh + c_r, c_r = 8(r/4) + r%4
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 bj = *reinterpret_cast<const float4*>(&bsm[wave][8 * q + 4 * hh]);
+        s[4 * q + 0] *= bj.x; s[4 * q + 1] *= bj.y; s[4 * q + 2] *= bj.z; s[4 * q + 3] *= bj.w;
+      }
+      if (jb + kDecBlock - 1 > min(all_see, k_hi - 1)) {  // visible iff <= qlim and < k_hi
+        const int t = min(qlim, k_hi - 1) - jb - 4 * hh;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (8 * (r >> 2) + (r & 3) > t) s[r] = -INFINITY;
+      }
+      if (!bounded) {
+        float mx = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+        mx = half_max(mx);
+        const bool need = mx > m_ref + kLazyThresh;
+        if (__builtin_amdgcn_ballot_w64(need) != 0) {
+          const float m_new = need ? mx : m_ref;
+          const float corr = need ? fast_exp2(m_ref - m_new) : 1.0f;
+          m_ref = m_new;
+          l_run[0] *= corr;
+          l_run[1] *= corr;
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[mb][r] *= corr;
+        }
+        const float mu = m_ref == -INFINITY ? 0.f : m_ref;  // nothing visible yet: keep exp2 away from inf - inf
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] -= mu;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r]);
+      auto add_product = [&](uint32_t tr, bf16x8 p0, bf16x8 p1) {
+        wave_lds_sync();
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          oacc[mb] = mfma32(swz_frag_tr<D>(tr, mb, 0), p0, oacc[mb]);
+          oacc[mb] = mfma32(swz_frag_tr<D>(tr, mb, 1), p1, oacc[mb]);
+        }
+        wait_lds_reads();
+      };
+      if (more) wait_vmcnt<kFirstLoads + kTabLoads + kRowLoads>(); else wait_vmcnt<kFirstLoads>();  // this block's V
+      if constexpr (!VRES) {
+        const bf16x8 p0 = pack_c_half_sum(s, 0, l_run), p1 = pack_c_half_sum(s, 1, l_run);
+        add_product(vtr, p0, p1);
+        if (more) issue_v(jb + kDecBlock);
+      } else {
+        f32x16 s1, s2;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          l_run[r & 1] += s[r];
+          s1[r] = c1 * s[r];
+          s2[r] = c2 * s[r];
+        }
+        add_product(vtr, pack_c_half(s1, 0), pack_c_half(s1, 1));
+        if (more) { issue_v(jb + kDecBlock); wait_vmcnt<kTabLoads + 2 * kRowLoads>(); } else wait_vmcnt<0>();  // V_first
+        add_product(ftr, pack_c_half(s2, 0), pack_c_half(s2, 1));
+        if (more) issue_first(jb + kDecBlock);
       }
     }
-    float kx[KS][8];
-    unpack_b_layout<KS>(kraw, kx);
-    if (p.rope_cos) {
-      const int64_t pos = (int64_t)(p.rope_k_pos0 + krow) * (D / 2);
-      rope_b_layout<KS>(kx, p.rope_cos + pos, p.rope_sin + pos, hh);
-    }
-    float ss = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int t = 0; t < 8; ++t) ss += kx[ks][t] * kx[ks][t];
-    ss = half_sum(ss);
-    const float beta = row_normaliser_fast(p, ss, 1.0f / D);
-    f32x16 s = splat16(0.f);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      u32x4 w;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(kx[ks][2 * i] * beta, kx[ks][2 * i + 1] * beta);
-      s = mfma32(as_bf16x8(w), qreg[ks], s);
-    }
-    // ---- V' rows into the wave's LDS tile (row-major); read back transposed after the softmax
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) *reinterpret_cast<u32x4*>(my_vt + ln * RS + 16 * ks + 8 * hh) = vraw[ks];
-
-    // ---- mask: register r holds key jb + 4hh + c_r, c_r = 8(r/4) + r%4; visible iff <= qlim and < k_hi
-    {
-      const int t = min(qlim, k_hi - 1) - jb - 4 * hh;
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (8 * (r >> 2) + (r & 3) > t) s[r] = -INFINITY;
-    }
-    // ---- online softmax (per lane = per query; the two lane halves hold different keys)
-    float mx = s[0];
-#pragma unroll
-    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
-    mx = half_max(mx);
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;  // nothing visible yet: keep exp2 away from inf - inf
-    const float corr = fast_exp2(m_run - m_use);           // m_run = -inf gives 0
-    m_run = m_new;
-    l_run[0] *= corr;
-    l_run[1] *= corr;
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) oacc[mb][r] *= corr;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r] - m_use);
-    bf16x8 pb[2];
-    pb[0] = pack_c_half_sum(s, 0, l_run);
-    pb[1] = pack_c_half_sum(s, 1, l_run);
-    __builtin_amdgcn_wave_barrier();  // the tile was written by this wave only; keep the reads below the writes
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) oacc[mb] = mfma32(dec_frag_tr<D>(my_vt, mb, s2, lane), pb[s2], oacc[mb]);
-    __builtin_amdgcn_wave_barrier();  // next iteration overwrites the tile
+    buf ^= 1;
   }
 
-  // ---- merge the four waves (different keys, same queries) and write this split's partial
-  __syncthreads();  // every wave is done with its V' tile: the memory is reused for the partials
+  // ---- this wave's partial: rows n of [bg, split][n_rows][D]
   const float l_tot = half_sum(l_run[0] + l_run[1]);
-  if (hh == 0) { msm[wave][ln] = m_run; lsm[wave][ln] = l_tot; }
+  if (active && qlive) {
+    const int64_t at = ((int64_t)bg * a.dec_splits + split) * n_rows + ln;
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) osm[wave][32 * mb + 8 * (r >> 2) + 4 * hh + (r & 3)][ln] = oacc[mb][r];
-  __syncthreads();
-  float* part_o = a.dec_part + ((int64_t)bg * a.dec_splits + split) * 32 * D;
-  float* part_s = a.dec_stat + ((int64_t)bg * a.dec_splits + split) * 32 * 2;
-  for (int e = tid; e < 32 * D; e += kDecThreads) {
-    const int n = e % 32, d = e / 32;
-    const float m0 = msm[0][n], m1 = msm[1][n], m2 = msm[2][n], m3 = msm[3][n];
-    const float M = fmaxf(fmaxf(m0, m1), fmaxf(m2, m3));
-    const float Mu = M == -INFINITY ? 0.f : M;
-    const float w0 = fast_exp2(m0 - Mu), w1 = fast_exp2(m1 - Mu), w2 = fast_exp2(m2 - Mu), w3 = fast_exp2(m3 - Mu);
-    part_o[n * D + d] = (osm[0][d][n] * w0 + osm[1][d][n] * w1) + (osm[2][d][n] * w2 + osm[3][d][n] * w3);
-    if (d == 0) {
-      part_s[n * 2] = M;
-      part_s[n * 2 + 1] = (lsm[0][n] * w0 + lsm[1][n] * w1) + (lsm[2][n] * w2 + lsm[3][n] * w3);
-    }
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<float4*>(a.dec_part + at * D + 32 * mb + 8 * q + 4 * hh) =
+            make_float4(oacc[mb][4 * q], oacc[mb][4 * q + 1], oacc[mb][4 * q + 2], oacc[mb][4 * q + 3]);
+    if (hh == 0) *reinterpret_cast<float2*>(a.dec_stat + at * 2) = make_float2(m_ref, l_tot);
   }
 }
 
@@ -228,7 +339,6 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(KArgs a) {
 // its first partial values are requested before the split statistics are reduced, so that the kernel is about
 // two memory round trips long whatever the number of splits.  Every sum has a fixed order: deterministic.
 constexpr int kMergeThreads = 256;
-constexpr int kMaxSplits = 512;
 constexpr int kMergeEarly = 16;  // partial values per thread requested up front
 
 __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(KArgs a) {
@@ -243,16 +353,17 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(KArgs a) {
   const int g = bg % p.Hkv, b = bg / p.Hkv;
   const int S = a.dec_splits;
   const int G = kMergeThreads / D, gi = tid / D, d = tid - gi * D;
-  const float* col = a.dec_part + (int64_t)bg * S * 32 * D + (int64_t)n * D + d;
-  const float* ss = a.dec_stat + (int64_t)bg * S * 32 * 2;
+  const float* col = a.dec_part + ((int64_t)bg * S * n_rows + n) * D + d;  // split sp: + sp * n_rows * D
+  const float* ss = a.dec_stat + ((int64_t)bg * S * n_rows + n) * 2;
+  const int64_t part_step = (int64_t)n_rows * D;
   float pv[kMergeEarly];
 #pragma unroll
   for (int u = 0; u < kMergeEarly; ++u) {
     const int sp = gi + G * u;
-    pv[u] = sp < S ? col[(int64_t)sp * 32 * D] : 0.f;
+    pv[u] = sp < S ? col[sp * part_step] : 0.f;
   }
   float m = -INFINITY;
-  for (int sp = tid; sp < S; sp += kMergeThreads) m = fmaxf(m, ss[(sp * 32 + n) * 2]);
+  for (int sp = tid; sp < S; sp += kMergeThreads) m = fmaxf(m, ss[sp * n_rows * 2]);
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
   if (lane == 0) redm[wave] = m;
@@ -260,9 +371,9 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(KArgs a) {
   const float M = fmaxf(fmaxf(redm[0], redm[1]), fmaxf(redm[2], redm[3]));
   float l = 0.f;
   for (int sp = tid; sp < S; sp += kMergeThreads) {
-    const float w = exp2f(ss[(sp * 32 + n) * 2] - M);  // a split with nothing visible has (-inf, 0): weight 0
+    const float w = exp2f(ss[sp * n_rows * 2] - M);  // a split with nothing visible has (-inf, 0): weight 0
     wsm[sp] = w;
-    l += ss[(sp * 32 + n) * 2 + 1] * w;
+    l += ss[sp * n_rows * 2 + 1] * w;
   }
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) l += __shfl_xor(l, o, 64);
@@ -275,7 +386,7 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(KArgs a) {
     const int sp = gi + G * u;
     if (sp < S) acc += pv[u] * wsm[sp];
   }
-  for (int sp = gi + G * kMergeEarly; sp < S; sp += G) acc += col[(int64_t)sp * 32 * D] * wsm[sp];
+  for (int sp = gi + G * kMergeEarly; sp < S; sp += G) acc += col[sp * part_step] * wsm[sp];
   part[tid] = acc;
   __syncthreads();
   const int hq = n / p.Sq, qi = n % p.Sq;
@@ -295,25 +406,51 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(KArgs a) {
 
 }  // namespace
 
-// Split plan of a decode-shaped call: keys [0, kend) in `splits` chunks of `chunk` keys (a multiple of 128):
-// enough workgroups for one resident round, no empty split: three per CU at head_dim 64 (what the kernel's
-// registers allow; measured 17 % faster than two per CU, four is slower again), one per CU at head_dim 128
-// (15 % faster than two).  Returns the scratch bytes the partials need.
+// Split plan of a decode-shaped call: keys [0, kend) in `splits` chunks of `chunk` keys (whole 32-key blocks), no empty
+// split.  One workgroup (four (batch, kv head) pairs) per CU already keeps 32 KB (head_dim 128: 64 KB) of rows in
+// flight, and more of them only shorten the chunks: 8 x 4 pairs, 5001 keys, head_dim 128: 256 workgroups 22.9 us, 424
+// 31.6, 632 38.5; 24 x 6 pairs, 1332 keys, head_dim 64: 252 workgroups 19.8 us, 756 23.1.  So the split count is the one
+// that leaves the fewest blocks on the fullest CU with one workgroup on each; a second or third round only where it evens
+// the load out by more than 3 % each (32 x 6 pairs, 8192 keys: 768 workgroups of 16 blocks 79.6 us, 288 of 48 89.6).
+// At least two blocks per split, and at most 128 (head_dim 128: 64) splits, bound what the merge has to read (one
+// sequence, 4096 keys: two blocks each 10.8 us, one each 13.6; head_dim 128, 2 x 4 pairs, 8192 keys: 64 splits 16.6 us,
+// 128 23.7).  Returns the scratch bytes the partials need.
 size_t decode_plan(const segpt_attn_params& p, int* kend_out, int* splits_out, int* chunk_out) {
   int kend = p.Sk;
   if (p.causal && p.Sq + p.q_start < kend) kend = p.Sq + p.q_start;
-  const int groups = p.B * p.Hkv;
-  const int target = p.D == 64 ? 768 : 256;
-  int s = (target + groups - 1) / groups;
-  const int max_s = (kend + kDecKeysPerStep - 1) / kDecKeysPerStep;
-  if (s > max_s) s = max_s;
-  if (s > kMaxSplits) s = kMaxSplits;
-  if (s < 1) s = 1;
-  const int per = (kend + s - 1) / s;
-  const int chunk = (per + kDecKeysPerStep - 1) / kDecKeysPerStep * kDecKeysPerStep;
-  s = (kend + chunk - 1) / chunk;
-  *kend_out = kend; *splits_out = s; *chunk_out = chunk;
-  return (size_t)p.B * p.Hkv * s * 32 * ((size_t)p.D + 2) * sizeof(float);
+  constexpr int kCUs = 256;
+  const int groups = (p.B * p.Hkv + 3) / 4;
+  const int blocks = (kend + kDecBlock - 1) / kDecBlock;
+  // (the last bound keeps the partials of many query rows within what 24576 / 8192 rows take)
+  const int64_t rows = (int64_t)p.B * p.H * p.Sq, most_rows = p.D == 64 ? 24576 : 8192;
+  const int most = (int)std::min<int64_t>(p.D == 64 ? kMaxSplits : kMaxSplits / 2, std::max<int64_t>(1, most_rows / rows));
+  int best_per = 0;
+  double best = 0;
+  for (int round = 1; round <= 3; ++round) {
+    int s = kCUs * round / groups;
+    s = s < 1 ? 1 : (s > most ? most : s);
+    int per = (blocks + s - 1) / s;
+    if (per < 2) per = 2;
+    const int64_t wgs = (int64_t)groups * ((blocks + per - 1) / per);
+    const double load = (double)((wgs + kCUs - 1) / kCUs) * per * (1.0 + 0.03 * (round - 1));
+    if (!best_per || load < best) { best = load; best_per = per; }
+  }
+  *kend_out = kend;
+  *splits_out = (blocks + best_per - 1) / best_per;
+  *chunk_out = best_per * kDecBlock;
+  return (size_t)p.B * p.Hkv * *splits_out * (p.H / p.Hkv * p.Sq) * ((size_t)p.D + 2) * sizeof(float);
+}
+
+template <int D>
+void launch_split(const KArgs& a, dim3 grid, hipStream_t st) {
+  const bool vres = a.p.v_first.ptr != nullptr;
+  if (a.p.rope_cos) {
+    if (vres) hipLaunchKernelGGL((decode_split_kernel<D, true, true>), grid, dim3(kDecThreads), 0, st, a);
+    else hipLaunchKernelGGL((decode_split_kernel<D, true, false>), grid, dim3(kDecThreads), 0, st, a);
+  } else {
+    if (vres) hipLaunchKernelGGL((decode_split_kernel<D, false, true>), grid, dim3(kDecThreads), 0, st, a);
+    else hipLaunchKernelGGL((decode_split_kernel<D, false, false>), grid, dim3(kDecThreads), 0, st, a);
+  }
 }
 
 int launch_fwd_decode_bf16(KArgs a, hipStream_t st) {
@@ -321,10 +458,10 @@ int launch_fwd_decode_bf16(KArgs a, hipStream_t st) {
   decode_plan(p, &a.dec_kend, &a.dec_splits, &a.dec_chunk);
   char* ws = reinterpret_cast<char*>(p.kv_workspace);
   a.dec_part = reinterpret_cast<float*>(ws);
-  a.dec_stat = a.dec_part + (size_t)p.B * p.Hkv * a.dec_splits * 32 * p.D;
-  const dim3 grid((unsigned)(p.B * p.Hkv * a.dec_splits));
-  if (p.D == 64) hipLaunchKernelGGL(decode_split_kernel<64>, grid, dim3(kDecThreads), 0, st, a);
-  else if (p.D == 128) hipLaunchKernelGGL(decode_split_kernel<128>, grid, dim3(kDecThreads), 0, st, a);
+  a.dec_stat = a.dec_part + (size_t)p.B * p.H * p.Sq * a.dec_splits * p.D;
+  const dim3 grid((unsigned)((p.B * p.Hkv + 3) / 4 * a.dec_splits));
+  if (p.D == 64) launch_split<64>(a, grid, st);
+  else if (p.D == 128) launch_split<128>(a, grid, st);
   else return (int)hipErrorInvalidValue;
   int rc = (int)hipGetLastError();
   if (rc) return rc;

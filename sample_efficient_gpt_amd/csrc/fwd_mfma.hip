@@ -15,36 +15,6 @@
 namespace segpt {
 namespace {
 
-// Largest |log2-unit logit| the normalised operands can produce: |Qhat.Khat| <= |Qhat| |Khat| with
-// |Khat| <= sqrt(D) and |Qhat| <= sm_scale*log2e*sqrt(D)*max|g_q g_k|.  When it is small the softmax needs
-// no running maximum at all (softmax is shift invariant and exp2 cannot overflow): P = exp2(S2) directly.
-// Read from the scale vector already in LDS (gsm[d] = sm_scale * log2e * g_q[d] * g_k[d]); 2 % of slack for the
-// bf16 rounding of the operands.
-template <int D>
-__device__ __forceinline__ float logit_bound(const float* gsm, int lane) {
-  float gm = 0.f;
-#pragma unroll
-  for (int d = lane; d < D; d += 64) gm = fmaxf(gm, fabsf(gsm[d]));
-  // wave-wide maximum by six DPP steps (shifts by 1, 2, 4, 8 inside the rows of 16 lanes, then the row maxima
-  // passed on to the next row and the next half): lane 63 ends up with it.  A lane whose source does not exist
-  // keeps its own value.
-  auto step = [](float v, auto ctrl, auto rows) {
-    const int t = __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
-    return fmaxf(v, __int_as_float(t));
-  };
-  gm = step(gm, IC<0x111>{}, IC<0xf>{});
-  gm = step(gm, IC<0x112>{}, IC<0xf>{});
-  gm = step(gm, IC<0x114>{}, IC<0xf>{});
-  gm = step(gm, IC<0x118>{}, IC<0xf>{});
-  gm = step(gm, IC<0x142>{}, IC<0xa>{});
-  gm = step(gm, IC<0x143>{}, IC<0xc>{});
-  gm = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gm), 63));
-  return (float)D * gm * 1.02f;
-}
-
-constexpr float kNoMaxBound = 64.f;   // |S2| below this: P in [2^-64, 2^64], sums stay far inside fp32 range
-constexpr float kLazyThresh = 16.f;   // general path: the subtracted reference is raised only when exceeded by 2^16
-
 // Khat / V' come from the key/value pre-pass (bf16, contiguous [B,Hkv,Sk,D]) and travel global->LDS
 // directly into a swizzled ring of stages, so the loop holds no staging registers and no normalisation
 // work.  Software pipeline over 32-key blocks n (two per staged tile), one barrier per tile:

@@ -622,6 +622,27 @@ def test_decode_path_matches_oracle_and_training_kernel(gpu_device, B, H, Hkv, S
     assert torch.allclose(dec["lse"], trn["lse"], atol=2e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("extras,use_rope,qk_norm", [(False, True, True), (True, True, True), (True, False, False)])
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk", [
+    (1, 2, 1, 1, 31),      # one partial block; three waves of the workgroup idle
+    (1, 10, 5, 2, 65),     # the second workgroup has one live wave; two blocks and a third of one key
+    (3, 3, 1, 1, 448),     # 14 blocks over 2-block splits, whole tiles only
+    (2, 32, 4, 4, 2085),   # 32 query rows, 66 blocks, last split shorter
+    (30, 4, 4, 1, 1001),   # 30 workgroups in three rounds at most: unequal blocks per split
+])
+def test_decode_split_edges(gpu_device, B, H, Hkv, Sq, Sk, D, extras, use_rope, qk_norm):
+    """Tile and split edges of the decode kernels (32-key blocks, four (batch, kv head) pairs per workgroup); values
+    scaled per head without QK-norm so that the running maximum moves."""
+    x = gen(B, H, Hkv, Sq, Sk, D, BF16, seed=43, extras=extras, head_scales=not qk_norm)
+    kw = {"q_start": Sk - Sq, "qk_norm": qk_norm}
+    if use_rope:
+        kw["rope"] = orc.rope_tables(Sk, 10000.0, D)
+    ref = run_oracle(x, backward=False, **kw)
+    with torch.no_grad():
+        compare(run_gpu(x, gpu_device, backward=False, **kw), ref, BF16)
+
+
 # ------------------------------------------------------------------ attention without QK-norm (SEGPT_FLAG_NO_NORM)
 
 
