@@ -76,7 +76,9 @@ extern "C" {
                                     32 query rows per kv head (H/Hkv * Sq, the reference's generation step,
                                     attention.py:191-198) may run the split-key decode kernels, which read k / v /
                                     v_first once, normalise and rotate on the fly and use kv_workspace for partial
-                                    results instead of normalised keys */
+                                    results instead of normalised keys; any other bf16 call may share out the keys of
+                                    its query tiles over several workgroups, with the partial results behind the
+                                    normalised keys (skipped when kv_workspace holds the keys only) */
 
 #define SEGPT_FLAG_NO_NORM 8     /* plain attention: both RMS normalisers are exactly 1 (eps is ignored), so
                                     s_ij = sm_scale * (q_i o g_q) . (k_j o g_k); with g_q = 1 and no g_k this is the
@@ -181,7 +183,8 @@ const char* segpt_strerror(int code);
 /* Bytes of device scratch of kind `which` (SEGPT_WS_*) these params need (0 is possible). Validates
  * nothing but sizes; returns 0 for invalid params (the launch call will report the error).
  * SEGPT_WS_KV follows p->flags: a decode-shaped forward with SEGPT_FLAG_DECODE needs only the split-key partial
- * results (a small fraction of the cache), every other call the normalised keys (and mixed values).
+ * results (a small fraction of the cache), every other call the normalised keys (and mixed values), with the flag
+ * plus the partial results where splitting the keys pays.
  * Replaces the in-op allocations of triton_flash_attn_qknorm.py:286-287 / :320-323: the caller
  * allocates. */
 size_t segpt_attn_workspace_bytes(const segpt_attn_params* p, int which);

@@ -34,6 +34,7 @@ struct WsLayout {
 };
 struct KvLayout {
   size_t khat, vmix, total;
+  size_t fwd_part, total_split;  // a forward-only call whose keys may be split uses more of the workspace if it is there
 };
 
 // A forward-only bf16 call with at most 32 query rows per kv head takes the split-key decode kernels when the
@@ -45,18 +46,21 @@ bool decode_shape(const segpt_attn_params& p) {
 // bf16 only: normalised keys and (with a value residual) mixed values, contiguous [B,Hkv,Sk,D]; for a decode-shaped
 // call the per-split partial results instead (a small fraction of the cache)
 KvLayout kv_layout(const segpt_attn_params& p) {
-  KvLayout w{0, 0, 0};
+  KvLayout w{0, 0, 0, 0, 0};
   if (p.dtype != SEGPT_DTYPE_BF16) return w;
   if (decode_shape(p)) {
     int kend, splits, chunk;
-    w.total = align_up(decode_plan(p, &kend, &splits, &chunk));
+    w.total = w.total_split = align_up(decode_plan(p, &kend, &splits, &chunk));
     return w;
   }
   const size_t kvrows = (size_t)p.B * p.Hkv * p.Sk;
   size_t off = align_up(kvrows * p.D * 2);
   w.vmix = off;
   if (p.v_first.ptr) off += align_up(kvrows * p.D * 2);
-  w.total = off;
+  w.total = w.fwd_part = off;
+  int splits, chunk;
+  if (p.flags & SEGPT_FLAG_DECODE) off += align_up(fwd_split_plan(p, &splits, &chunk));
+  w.total_split = off;
   return w;
 }
 
@@ -228,7 +232,7 @@ size_t segpt_attn_workspace_bytes(const segpt_attn_params* p, int which) {
   if (!p || p->struct_bytes != sizeof(segpt_attn_params)) return 0;
   if (p->B <= 0 || p->H <= 0 || p->Hkv <= 0 || p->Sq <= 0 || p->Sk <= 0 || p->D <= 0) return 0;
   if (p->dtype == SEGPT_DTYPE_BF16 && p->D != 64 && p->D != 128) return 0;
-  if (which == SEGPT_WS_KV) return kv_layout(*p).total;
+  if (which == SEGPT_WS_KV) return kv_layout(*p).total_split;
   if (which == SEGPT_WS_BWD) return bwd_layout(*p).total;
   return 0;
 }
@@ -242,6 +246,15 @@ static int fwd_stage_impl(const segpt_attn_params* p, int stage_lo, int stage_hi
   KArgs a{};
   a.p = *p;
   bind_kv(a);
+  a.fwd_splits = 1;
+  if (p->dtype == SEGPT_DTYPE_BF16) {
+    const KvLayout kv = kv_layout(*p);
+    if (kv.total_split > kv.total && p->kv_workspace_bytes >= kv.total_split) {
+      fwd_split_plan(*p, &a.fwd_splits, &a.fwd_chunk);
+      a.fwd_part = reinterpret_cast<float*>(reinterpret_cast<char*>(p->kv_workspace) + kv.fwd_part);
+      a.fwd_stat = a.fwd_part + (size_t)p->B * p->H * a.fwd_splits * p->Sq * p->D;
+    }
+  }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool f32 = p->dtype == SEGPT_DTYPE_FP32;
   const bool decode = use_decode(p);
@@ -295,7 +308,9 @@ int segpt_attn_fwd_noalloc(const segpt_attn_params* p, void* stream) {
   q.kv_workspace_bytes = 0;
   q.flags &= ~SEGPT_FLAG_KV_PREPARED;  // the scratch is shared by every call on this GPU: never assume its contents
   if (q.dtype == SEGPT_DTYPE_BF16) {
-    if (segpt_attn_workspace_bytes(&q, SEGPT_WS_KV) > (size_t)SEGPT_NOALLOC_SCRATCH_BYTES) return SEGPT_E_SCRATCH_LIMIT;
+    if (q.B > 0 && q.H > 0 && q.Hkv > 0 && q.Sq > 0 && q.Sk > 0 && (q.D == 64 || q.D == 128) &&
+        kv_layout(q).total > (size_t)SEGPT_NOALLOC_SCRATCH_BYTES)
+      return SEGPT_E_SCRATCH_LIMIT;
     // argument errors first (they need no device): validate against a stand-in address, then look the real one up
     q.kv_workspace = reinterpret_cast<void*>(uintptr_t{256});
     q.kv_workspace_bytes = SEGPT_NOALLOC_SCRATCH_BYTES;

@@ -30,6 +30,11 @@ struct KArgs {
   float* dec_part;
   float* dec_stat;
   int32_t dec_splits, dec_chunk, dec_kend;
+  // bf16 forward with its keys split: partial O [B,H,fwd_splits,Sq,D] and (reference, sum) [B,H,fwd_splits,Sq,2], fp32,
+  // carved from kv_workspace behind the keys; shares of fwd_chunk key tiles
+  float* fwd_part;
+  float* fwd_stat;
+  int32_t fwd_splits, fwd_chunk;
   // fp32 backward: dKhat and dV of one query head and one share of the query tiles, [B*H, f32_splits, Sk, D] each
   float* f32_dk_part;
   float* f32_dv_part;
@@ -196,6 +201,7 @@ int launch_bwd_dkdv_bf16(const KArgs& a, hipStream_t st);
 int launch_bwd_dq_bf16(const KArgs& a, hipStream_t st);
 int launch_fwd_decode_bf16(KArgs a, hipStream_t st);    // split-key forward for a few query rows against a long cache
 size_t decode_plan(const segpt_attn_params& p, int* kend, int* splits, int* chunk);  // returns its scratch bytes
+size_t fwd_split_plan(const segpt_attn_params& p, int* splits, int* chunk);  // returns its scratch bytes (0: not split)
 int launch_kv_prep(const KArgs& a, hipStream_t st);     // bf16 path: Khat (and V') into kv_workspace
 int launch_bwd_reduce(const KArgs& a, hipStream_t st);  // dvr_coef from the partials (nothing without a value residual)
 

@@ -9,6 +9,8 @@
 //   O^T[d][query] += V'^T[d][key] . P^T[key][query]          (A = transposing LDS read of the V' tile).
 // Qhat = sm_scale*log2(e) * a_i * q_i * g_q * g_k  (both scale vectors live on the query side) is formed in
 // the prologue; Khat = b_j * k_j and V' = c1 v + c2 v_first are read as written by the pre-pass.
+#include <algorithm>
+
 #include "mfma_common.hpp"
 #include "ring_protocol.hpp"
 
@@ -39,11 +41,16 @@ struct FwdShape {
   static constexpr int kStages = D == 64 ? (WIDE ? 4 : 3) : 4;
   static constexpr int kOcc = D == 64 ? (WIDE ? 2 : 3) : 2;
   static constexpr int kBQ = 4 * 32 * kNQB;
+  static constexpr int kStoreUnits = D / 64;              // partial results of a split launch, in 32 KB
 };
 
 // ROPE (rope tables given) is a compile-time switch so that the table rows are ordinary, unconditional loads that
 // travel with the start-up tiles instead of costing a memory round trip of their own behind a branch.
-template <int D, bool WIDE, bool ROPE>
+//
+// SPLIT: workgroup (tile, head, batch; y = share s) takes only the key tiles [s, s + 1) * fwd_chunk of its query tile
+// and, unless that is all of them, leaves an unnormalised partial (reference m, sum l, O in fp32) for
+// fwd_merge_kernel; see fwd_split_plan() for when.
+template <int D, bool WIDE, bool ROPE, bool SPLIT>
 __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16_kernel(KArgs a) {
   using F = FwdShape<D, WIDE>;
   constexpr int NQB = F::kNQB, BQ = F::kBQ, NS = F::kStages, BK = F::kBK;
@@ -70,10 +77,16 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
 
   int kend = p.Sk;
   if (p.causal) kend = min(p.Sk, q0 + BQ + p.q_start);
+  const int all_kt = (kend + BK - 1) / BK;
+  // this workgroup's keys: k0 .. kend - 1; everything below counts keys from k0
+  const int share = SPLIT ? (int)blockIdx.y : 0, k0 = SPLIT ? share * a.fwd_chunk * BK : 0;
+  if (SPLIT && k0 >= kend) return;
+  const int Sk = p.Sk - k0, q_start = p.q_start - k0;
+  kend = SPLIT ? min(kend - k0, a.fwd_chunk * BK) : kend;
   const int n_kt = (kend + BK - 1) / BK;
-  const char* kbase = reinterpret_cast<const char*>(a.khat + ((int64_t)b * p.Hkv + g) * p.Sk * D);
-  const char* vbase = a.vmix ? reinterpret_cast<const char*>(a.vmix + ((int64_t)b * p.Hkv + g) * p.Sk * D)
-                             : reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v, b, g, 0));
+  const char* kbase = reinterpret_cast<const char*>(a.khat + (((int64_t)b * p.Hkv + g) * p.Sk + k0) * D);
+  const char* vbase = a.vmix ? reinterpret_cast<const char*>(a.vmix + (((int64_t)b * p.Hkv + g) * p.Sk + k0) * D)
+                             : reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v, b, g, k0));
   const uint32_t kstep = D * 2, vstep = a.vmix ? (uint32_t)D * 2 : (uint32_t)p.v.stride_s * 2;
 
   const uint32_t lds0 = lds_addr_of(lds);
@@ -84,7 +97,7 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
     const char* ksrc = kbase + (int64_t)jt * BK * kstep;
     const char* vsrc = vbase + (int64_t)jt * BK * vstep;
     const uint32_t dst = wave_dst + (jt % NS) * kStageBytes;
-    const int left = p.Sk - jt * BK;
+    const int left = Sk - jt * BK;
     if (left >= BK) issue_tile_pair<D, BK>(ksrc, vsrc, full_tile, dst);
     else issue_tile_pair<D, BK>(ksrc, vsrc, tile_lane_offsets<D, BK>(kstep, vstep, left, src.x, src.y), dst);
   };
@@ -171,12 +184,13 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
   for (int nb = 0; nb < NQB; ++nb) {
     m_ref[nb] = bounded ? 0.f : -INFINITY;
     l_run[nb][0] = l_run[nb][1] = 0.f;
-    qlim[nb] = p.causal ? min(qw0 + 32 * nb + ln + p.q_start, p.Sk - 1) : p.Sk - 1;
+    qlim[nb] = p.causal ? min(qw0 + 32 * nb + ln + q_start, Sk - 1) : Sk - 1;
   }
 
   // 32-key blocks this wave has to visit (causal: up to the block holding its last query's diagonal)
   int n_act = (kend + 31) / 32;
-  if (p.causal) n_act = min(n_act, (qw0 + 32 * NQB - 1 + p.q_start) / 32 + 1);
+  if (p.causal) n_act = min(n_act, (qw0 + 32 * NQB - 1 + q_start) / 32 + 1);
+  if (SPLIT && p.causal && qw0 + 32 * NQB - 1 + q_start < 0) n_act = 0;
 
   const uint32_t rm_lane = lds0 + swz_off_rm<D>(lane);
   const uint32_t tr_lane = lds0 + swz_off_tr<D>(lane) + Z::kTileBytes;  // V' tile of a stage
@@ -226,7 +240,7 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
         const bool need = mx > m_ref[nb] + kLazyThresh;
         if (__builtin_amdgcn_ballot_w64(need) != 0) {
           const float m_new = need ? mx : m_ref[nb];
-          const float corr = fast_exp2(m_ref[nb] - m_new);
+          const float corr = SPLIT && !need ? 1.f : fast_exp2(m_ref[nb] - m_new);
           m_ref[nb] = m_new;
           l_run[nb][0] *= corr;
           l_run[nb][1] *= corr;
@@ -235,8 +249,9 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
 #pragma unroll
             for (int r = 0; r < 16; ++r) oacc[mb][nb][r] *= corr;
         }
+        const float mu = SPLIT && m_ref[nb] == -INFINITY ? 0.f : m_ref[nb];  // a share may hold no visible key of a row
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[nb][r] -= m_ref[nb];
+        for (int r = 0; r < 16; ++r) s[nb][r] -= mu;
       }
     }
     bf16x8 pb[2][NQB];
@@ -258,8 +273,9 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
 
   // leading blocks of this wave that need no mask: every key of the block is visible to every query of the
   // wave and lies inside the key range
-  int n_full = p.Sk / 32;
-  if (p.causal) n_full = min(n_full, (qw0 + p.q_start + 1) / 32);
+  int n_full = Sk / 32;
+  if (p.causal) n_full = min(n_full, (qw0 + q_start + 1) / 32);
+  if (SPLIT) n_full = max(0, min(n_full, kend / 32));
 
   // ---- pipeline.  The tile loads that stay in flight across iterations must be the youngest vector-memory
   // operations of the wave (waits are in-order): the prologue's wait left nothing else behind.
@@ -318,6 +334,19 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
     const int row = qw0 + 32 * nb + ln;
     const bool live = row < p.Sq;
     const float l = half_sum(l_run[nb][0] + l_run[nb][1]);
+    if (SPLIT && all_kt > a.fwd_chunk) {
+      if (live) {
+        const int64_t at = (((int64_t)b * p.H + h) * a.fwd_splits + share) * p.Sq + row;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<float4*>(a.fwd_part + at * D + 32 * mb + 8 * q + 4 * hh) =
+                make_float4(oacc[mb][nb][4 * q], oacc[mb][nb][4 * q + 1], oacc[mb][nb][4 * q + 2], oacc[mb][nb][4 * q + 3]);
+        if (hh == 0) *reinterpret_cast<float2*>(a.fwd_stat + at * 2) = make_float2(m_ref[nb], l);
+      }
+      continue;
+    }
     float f = fast_rcp(l);
     if (p.gate.ptr) {
       const int rc = live ? row : p.Sq - 1;
@@ -336,21 +365,153 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
   }
 }
 
+// Adds up the shares of the query tiles that were split: D/4 lanes across a row, G groups of them across the shares.
+// Few rows want the shares side by side (4608 rows, 16 shares: 8.9 us with G = 1, 6.4 with a wave per row), many rows are
+// better off with more rows per wave (73728 rows, 2 shares: 5.2 and 11.4 us).  Fixed order: deterministic.
+constexpr int kMergeThreads = 256, kMergeFewRows = 8192;
+template <int D, int G>
+__global__ __launch_bounds__(kMergeThreads) void fwd_merge_kernel(KArgs a) {
+  const segpt_attn_params& p = a.p;
+  using F = FwdShape<D, D != 64>;
+  constexpr int LPR = D / 4, RPW = 64 / (LPR * G), kRows = kMergeThreads / 64 * RPW;
+  const int lane = threadIdx.x & 63, part = lane % LPR, gi = lane / (LPR * RPW);
+  const int i = blockIdx.x * kRows + (threadIdx.x >> 6) * RPW + lane / LPR % RPW;
+  const int h = blockIdx.y, b = blockIdx.z;
+  if (i >= p.Sq) return;
+  int kend = p.Sk;
+  if (p.causal) kend = min(p.Sk, i / F::kBQ * F::kBQ + F::kBQ + p.q_start);
+  const int n_kt = (kend + F::kBK - 1) / F::kBK, n = (n_kt + a.fwd_chunk - 1) / a.fwd_chunk;
+  if (n <= 1) return;  // written by its only share
+  const int64_t at = ((int64_t)b * p.H + h) * a.fwd_splits * p.Sq + i;
+  const float2* stat = reinterpret_cast<const float2*>(a.fwd_stat) + at;
+  const float* o = a.fwd_part + at * D + 4 * part;
+  float m = -INFINITY;
+  for (int s = gi; s < n; s += G) m = fmaxf(m, stat[(int64_t)s * p.Sq].x);
+#pragma unroll
+  for (int x = LPR * RPW; x < 64; x <<= 1) m = fmaxf(m, __shfl_xor(m, x, 64));
+  float l = 0.f, y[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = gi; s < n; s += G) {
+    const float2 ml = stat[(int64_t)s * p.Sq];
+    const float4 t = *reinterpret_cast<const float4*>(o + (int64_t)s * p.Sq * D);
+    const float w = fast_exp2(ml.x - m);  // a share without a visible key has (-inf, 0): weight 0
+    l += w * ml.y;
+    y[0] += w * t.x; y[1] += w * t.y; y[2] += w * t.z; y[3] += w * t.w;
+  }
+#pragma unroll
+  for (int x = LPR * RPW; x < 64; x <<= 1) {
+    l += __shfl_xor(l, x, 64);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] += __shfl_xor(y[e], x, 64);
+  }
+  float f = 1.0f / l;
+  if (p.gate.ptr) {
+    const float z = bf16_to_f32(reinterpret_cast<const uint16_t*>(p.gate.ptr)[(int64_t)b * p.gate.stride_b + (int64_t)i * p.gate.stride_s + (int64_t)h * p.gate.stride_h]);
+    f *= p.gate_scale / (1.0f + __expf(-z));
+  }
+  if (gi == 0) {
+    if (part == 0) p.lse[((int64_t)b * p.H + h) * p.Sq + i] = (m + __log2f(l)) * kLn2;
+    const u32x2 w = {pack_bf16x2(y[0] * f, y[1] * f), pack_bf16x2(y[2] * f, y[3] * f)};
+    *reinterpret_cast<u32x2*>(row_ptr_mut<uint16_t>(p.o, b, h, i) + 4 * part) = w;
+  }
+}
+
 template <int D, bool WIDE>
 int launch_fwd_t(const KArgs& a, hipStream_t st) {
   const segpt_attn_params& p = a.p;
   const int n_qt = (p.Sq + FwdShape<D, WIDE>::kBQ - 1) / FwdShape<D, WIDE>::kBQ;
   const dim3 grid((unsigned)wg_grid(n_qt, p.B, p.Hkv, p.H / p.Hkv, wg_pinned_pairs(p.B, p.Hkv, false)));
-  if (p.rope_cos) hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, true>), grid, dim3(kThreadsM), 0, st, a);
-  else hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, false>), grid, dim3(kThreadsM), 0, st, a);
+  if (p.rope_cos) hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, true, false>), grid, dim3(kThreadsM), 0, st, a);
+  else hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, false, false>), grid, dim3(kThreadsM), 0, st, a);
   return (int)hipGetLastError();
 }
 
+template <int D>
+int launch_fwd_split(const KArgs& a, hipStream_t st) {
+  constexpr bool WIDE = D != 64;
+  using F = FwdShape<D, WIDE>;
+  const segpt_attn_params& p = a.p;
+  const int n_qt = (p.Sq + F::kBQ - 1) / F::kBQ;
+  const dim3 grid((unsigned)wg_grid(n_qt, p.B, p.Hkv, p.H / p.Hkv, wg_pinned_pairs(p.B, p.Hkv, false)), (unsigned)a.fwd_splits);
+  if (p.rope_cos) hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, true, true>), grid, dim3(kThreadsM), 0, st, a);
+  else hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, false, true>), grid, dim3(kThreadsM), 0, st, a);
+  const int rc = (int)hipGetLastError();
+  if (rc) return rc;
+  const bool few = (int64_t)p.B * p.H * p.Sq <= kMergeFewRows;
+  constexpr int LPR = D / 4, G = 64 / LPR;
+  const int rows = few ? kMergeThreads / 64 : kMergeThreads / LPR;
+  const dim3 mgrid((unsigned)((p.Sq + rows - 1) / rows), (unsigned)p.H, (unsigned)p.B);
+  if (few) hipLaunchKernelGGL((fwd_merge_kernel<D, G>), mgrid, dim3(kMergeThreads), 0, st, a);
+  else hipLaunchKernelGGL((fwd_merge_kernel<D, 1>), mgrid, dim3(kMergeThreads), 0, st, a);
+  return (int)hipGetLastError();
+}
+
+// Number of key tiles of all query tiles of one head, and of its longest one
+template <typename F>
+void count_tiles(const segpt_attn_params& p, int64_t* total, int* most) {
+  const int n_qt = (p.Sq + F::kBQ - 1) / F::kBQ;
+  *total = 0; *most = 0;
+  for (int t = 0; t < n_qt; ++t) {
+    int64_t kend = p.Sk;
+    if (p.causal && (int64_t)(t + 1) * F::kBQ + p.q_start < kend) kend = (int64_t)(t + 1) * F::kBQ + p.q_start;
+    const int n = (int)((kend + F::kBK - 1) / F::kBK);
+    *total += n;
+    *most = n > *most ? n : *most;
+  }
+}
+
+// Splits the keys of a query tile over several workgroups where the query tiles alone leave CUs idle.  A CU computes
+// one key tile (128 rows x 64 keys at head_dim 64, 128 x 32 at 128: 2.1 MFLOP) per 0.59 us whether one workgroup
+// is resident or two, and everything here counts in that unit.  Cost of a launch: its longest workgroup, or where there
+// are more of them than CUs the average load plus a fifth of the longest; storing a partial result adds kStore, the
+// second kernel kMerge and its reading time (94 measured launches: 9 % mean deviation).  A call is split when the model says
+// 10 % faster: chunks of a long prompt (18 / 6 heads, 256 queries against 8192 keys: 7 shares, 124 -> 33 us; 1024 queries:
+// 120 -> 62), small batches of few queries (10 x 8 heads, 45 queries, 5783 keys: 99 -> 48).
+template <typename S, typename N>  // S: shape of a split launch, N: of an unsplit one; n_unit: what a tile of N costs
+size_t split_plan(const segpt_attn_params& p, double n_unit, int* splits, int* chunk) {
+  constexpr double kCUs = 256, kStore = S::kStoreUnits, kMerge = 7.3, kReadPerUnit = 4.4e6;
+  const int64_t heads = (int64_t)p.B * p.H;
+  const int n_whole = (p.Sq + N::kBQ - 1) / N::kBQ, n_qt = (p.Sq + S::kBQ - 1) / S::kBQ;
+  *splits = 1; *chunk = 0;
+  if (heads * n_whole >= 2 * kCUs) return 0;
+  auto launch = [&](double items, double total, double longest) {
+    return items <= kCUs ? longest : std::max(longest, total / kCUs + 0.2 * longest);
+  };
+  int64_t total;
+  int most;
+  count_tiles<N>(p, &total, &most);
+  const double whole = n_unit * launch((double)(heads * n_whole), (double)(heads * total), most);
+  count_tiles<S>(p, &total, &most);
+  double best = 0.9 * whole;
+  for (int s = 2; s <= 64; ++s) {
+    const int c = (most + s - 1) / s;
+    if (c < 4) break;
+    if ((most + c - 1) / c != s) continue;
+    const double items = (double)heads * std::min((double)n_qt * s, (double)total / c + 0.5 * n_qt);  // shorter tiles: fewer shares
+    const double read = (double)heads * s * p.Sq * p.D * sizeof(float) / kReadPerUnit;
+    const double cost = launch(items, (double)(heads * total) + 2 * kStore * items, c + kStore) + kMerge + read;
+    if (cost < best) { best = cost; *splits = s; *chunk = c; }
+  }
+  return *splits > 1 ? (size_t)heads * *splits * p.Sq * (p.D + 2) * sizeof(float) : 0;
+}
+
+bool wide_fwd(const segpt_attn_params& p) { return p.D != 64 || p.Sk > 2048; }
+
 }  // namespace
 
+// Forward-only calls: bytes of the partials when the keys are to be split, 0 when not.
+size_t fwd_split_plan(const segpt_attn_params& p, int* splits, int* chunk) {
+  if (p.D == 128) return split_plan<FwdShape<128, true>, FwdShape<128, true>>(p, 1.0, splits, chunk);
+  if (wide_fwd(p)) return split_plan<FwdShape<64, false>, FwdShape<64, true>>(p, 1.5, splits, chunk);
+  return split_plan<FwdShape<64, false>, FwdShape<64, false>>(p, 1.0, splits, chunk);
+}
+
 int launch_fwd_bf16(const KArgs& a, hipStream_t st) {
-  if (a.p.D == 64) return a.p.Sk > 2048 ? launch_fwd_t<64, true>(a, st) : launch_fwd_t<64, false>(a, st);
-  if (a.p.D == 128) return launch_fwd_t<128, true>(a, st);
+  if (a.p.D == 64) {
+    if (a.fwd_splits > 1) return launch_fwd_split<64>(a, st);
+    return wide_fwd(a.p) ? launch_fwd_t<64, true>(a, st) : launch_fwd_t<64, false>(a, st);
+  }
+  if (a.p.D == 128) return a.fwd_splits > 1 ? launch_fwd_split<128>(a, st) : launch_fwd_t<128, true>(a, st);
   return (int)hipErrorInvalidValue;
 }
 

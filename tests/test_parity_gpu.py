@@ -643,6 +643,31 @@ def test_decode_split_edges(gpu_device, B, H, Hkv, Sq, Sk, D, extras, use_rope, 
         compare(run_gpu(x, gpu_device, backward=False, **kw), ref, BF16)
 
 
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,kw,gen_kw,use_rope", [
+    (1, 2, 1, 70, 2500, 64, {"q_start": 2430}, {"extras": True}, True),                       # one ragged query tile, last share ragged
+    (2, 3, 3, 130, 1100, 128, {"q_start": 970}, {}, False),                                   # two query tiles, the second of 2 rows
+    (1, 2, 1, 1500, 1500, 64, {}, {"extras": True}, False),                                   # early tiles fit one share, later ones do not
+    (1, 2, 1, 1500, 1500, 128, {"qk_norm": False}, {"head_scales": True}, True),              # shares whose keys some rows do not see
+    (1, 8, 2, 257, 2113, 64, {"q_start": 1856, "qk_norm": False}, {"head_scales": True}, False),
+    (1, 4, 2, 200, 1900, 64, {"causal": False}, {}, False),
+])
+def test_forward_only_split_keys(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw, use_rope):
+    """Forward-only calls with few query tiles share out the keys of a tile (partials in the kv workspace, merged by a
+    second kernel): against the oracle, and against the unsplit kernel that a call with gradients runs."""
+    x = gen(B, H, Hkv, Sq, Sk, D, BF16, seed=47, **gen_kw)
+    if use_rope:
+        kw = dict(kw, rope=orc.rope_tables(Sk, 10000.0, D))
+    ref = run_oracle(x, backward=False, **kw)
+    with torch.no_grad():
+        split = run_gpu(x, gpu_device, backward=False, **kw)
+    compare(split, ref, BF16)
+    whole = run_gpu(x, gpu_device, backward=True, **kw)
+    # the same scores; with a running maximum the probabilities are rounded to bf16 against another reference, each by at
+    # most 2^-9 of itself on either side, so the logarithms of their sums differ by at most 2^-8
+    assert torch.allclose(split["lse"], whole["lse"], atol=2.0**-8 if kw.get("qk_norm") is False else 1e-4, rtol=0)
+    assert not torch.equal(split["y"], whole["y"]), "the two launches agree bit for bit: the call was not split"
+
+
 # ------------------------------------------------------------------ attention without QK-norm (SEGPT_FLAG_NO_NORM)
 
 
