@@ -1,4 +1,4 @@
-"""Builds libsegpt_attn.so (gfx950) in-tree with hipcc.  `python -m sample_efficient_gpt_amd.build`."""
+"""Builds libsegpt_attn.so (gfx950, hipcc) and the torch binding (_segpt_torch.so, g++) in-tree.  `python -m sample_efficient_gpt_amd.build`."""
 
 from __future__ import annotations
 
@@ -12,6 +12,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libsegpt_attn.so")
+BINDING_PATH = os.path.join(PKG_DIR, "_segpt_torch.so")  # native host side for PyTorch callers, linked against LIB_PATH
 SOURCES = ["api.hip", "f32_path.hip", "pre_post.hip", "fwd_mfma.hip", "bwd_mfma.hip", "decode_mfma.hip"]
 # Per-source flags.  The forward never needs more than 256 registers, but at head_dim 128 it runs one
 # workgroup per CU and the compiler would then move every MFMA result into the accumulation registers
@@ -48,6 +49,26 @@ def _run(cmd):
     return out
 
 
+def build_binding(verbose: bool = False) -> str:
+    """Compile csrc/torch_binding.cpp (host code only) against this interpreter and its torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    tmp = BINDING_PATH + ".tmp"
+    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w",
+          "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          "-DTORCH_EXTENSION_NAME=_segpt_torch", f"-I{INCLUDE}", *(a for d in include_paths() for a in ("-isystem", d)),
+          "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"],
+          os.path.join(CSRC, "torch_binding.cpp"), "-o", tmp, f"-L{PKG_DIR}", "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN",
+          *(f"-L{d}" for d in library_paths()), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
+    os.replace(tmp, BINDING_PATH)
+    if verbose:
+        print("built", BINDING_PATH)
+    return BINDING_PATH
+
+
 def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
     """Compile every HIP source and link the shared library; returns its path."""
     hipcc = _hipcc()
@@ -69,6 +90,7 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
     os.replace(tmp, LIB_PATH)
     if verbose:
         print("built", LIB_PATH)
+    build_binding(verbose)
     # stand-alone measurement programs (not part of the library): one executable per source under csrc/microbench
     mb_dir = os.path.join(CSRC, "microbench")
     for src in sorted(f for f in os.listdir(mb_dir) if f.endswith(".hip")):

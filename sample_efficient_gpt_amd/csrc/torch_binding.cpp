@@ -1,0 +1,329 @@
+// Host side of the op for PyTorch callers: argument checks, output / workspace allocation, the launch through the C ABI
+// and the autograd node, in native code.
+//
+// Why native: the same steps in Python (ctypes struct, autograd.Function) cost 40 us per direction, and the backward's
+// part runs on the autograd engine's thread, where taking the interpreter over from the calling thread doubles the cost of
+// every Python instruction on either side when the two threads sit on different core complexes.  A forward + backward of
+// 512 tokens (58 us of kernels) took 130 to 240 us, depending on that placement alone; a node in C++ runs its backward
+// without the interpreter.
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/DeviceGuard.h>
+
+#include <cmath>
+#include <optional>
+#include <string>
+
+#include "segpt_attn.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+
+// What a Python caller is to see as AssertionError / TypeError / the package's SegptError
+struct CheckFailed : std::runtime_error { using std::runtime_error::runtime_error; };
+struct BadType : std::runtime_error { using std::runtime_error::runtime_error; };
+struct LibraryError : std::runtime_error {
+  int code;
+  std::string where;
+  LibraryError(int c, const char* w)
+      : std::runtime_error(std::string(w) + " failed with code " + std::to_string(c) + ": " + segpt_strerror(c)), code(c), where(w) {}
+};
+void check(bool ok, const char* what) { if (!ok) throw CheckFailed(what); }
+
+Tensor defined_or_none(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+
+// Everything of a call that is not a differentiable operand.  heads > 0: the flattened [(h b), S, d] layout of the
+// positional drop-ins, head-major (attention.py:199), with `heads` / `kv_heads` heads; 0: canonical [B, heads, S, D].
+struct Call : torch::CustomClassHolder {
+  double gate_scale = 2.0, eps = 1e-6, sm_scale = 0.0;
+  bool causal = true;
+  int64_t q_start = 0, q_pos0 = 0, k_pos0 = 0;
+  int64_t heads = 0, kv_heads = 0;
+  int flags = 0;
+  Tensor cos, sin;
+};
+
+struct Operands {
+  Tensor q, k, v, g_q, g_k, v_first, coef, gate;
+};
+
+Tensor f32_vector(const Tensor& t, const at::Device& dev) {
+  if (!t.defined()) return t;
+  if (t.scalar_type() == at::kFloat && t.device() == dev && t.is_contiguous()) return t;
+  return t.detach().to(dev, at::kFloat).reshape({-1}).contiguous();
+}
+Tensor last_dim_contiguous(const Tensor& t) { return !t.defined() || t.stride(-1) == 1 ? t : t.contiguous(); }
+
+struct Sizes {
+  int64_t B, H, S, D;
+};
+Sizes sizes_of(const Tensor& t, int64_t heads) {
+  if (heads) return {t.size(0) / heads, heads, t.size(1), t.size(2)};
+  return {t.size(0), t.size(1), t.size(2), t.size(3)};
+}
+segpt_tensor4 view4(const Tensor& t, int64_t heads) {
+  if (!t.defined()) return {nullptr, 0, 0, 0};
+  if (heads) return {t.data_ptr(), t.stride(0), t.size(0) / heads * t.stride(0), t.stride(1)};
+  return {t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)};
+}
+segpt_tensor3 view3(const Tensor& t) {
+  if (!t.defined()) return {nullptr, 0, 0, 0};
+  return {t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)};
+}
+template <typename T>
+T* ptr_of(const Tensor& t) { return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr; }
+
+void check_operands(const Operands& x, const Call& c) {
+  const auto dt = x.q.scalar_type();
+  if (dt != at::kBFloat16 && dt != at::kFloat)
+    throw BadType(std::string("qknorm attention supports bfloat16 and float32 tensors, got ") + c10::toString(dt));
+  auto same_type = [&](const Tensor& t, const char* name) {
+    if (t.defined() && t.scalar_type() != dt)
+      throw BadType(std::string(name) + " has dtype " + c10::toString(t.scalar_type()) + ", expected " + c10::toString(dt));
+  };
+  same_type(x.k, "k"); same_type(x.v, "v"); same_type(x.v_first, "v_first"); same_type(x.gate, "gate_logits");
+  check(x.q.is_cuda() && x.k.is_cuda() && x.v.is_cuda(), "q, k, v must be device tensors");
+  const int64_t dims = c.heads ? 3 : 4;
+  check(x.q.dim() == dims && x.k.dim() == dims && x.v.sizes() == x.k.sizes(), "k/v shape mismatch");
+  const Sizes q = sizes_of(x.q, c.heads), k = sizes_of(x.k, c.kv_heads);
+  check(k.B == q.B && k.D == q.D, "k/v shape mismatch");
+  check(k.H > 0 && q.H % k.H == 0, "number of query heads must be a multiple of the kv heads");
+  check(x.g_q.numel() == 1 || x.g_q.numel() == q.D, "gain must have 1 or head_dim elements");
+  check(!x.g_k.defined() || x.g_k.numel() == 1 || x.g_k.numel() == q.D, "k_gain must have 1 or head_dim elements");
+  check(x.v_first.defined() == x.coef.defined(), "v_first and vr_coef go together");
+  if (x.v_first.defined()) check(x.v_first.sizes() == x.v.sizes() && x.coef.numel() == 2, "v_first must have v's shape, vr_coef two elements");
+  if (x.gate.defined())
+    check(x.gate.dim() == 3 && x.gate.size(0) == q.B && x.gate.size(1) == q.S && x.gate.size(2) == q.H, "gate_logits must be [B, Sq, H]");
+}
+
+void fill(segpt_attn_params& p, const Operands& x, const Call& c, const Tensor& y, const Tensor& lse) {
+  const Sizes q = sizes_of(x.q, c.heads), k = sizes_of(x.k, c.kv_heads);
+  p.struct_bytes = sizeof(p);
+  p.dtype = x.q.scalar_type() == at::kFloat ? SEGPT_DTYPE_FP32 : SEGPT_DTYPE_BF16;
+  p.B = (int32_t)q.B; p.H = (int32_t)q.H; p.Hkv = (int32_t)k.H; p.Sq = (int32_t)q.S; p.Sk = (int32_t)k.S; p.D = (int32_t)q.D;
+  p.causal = c.causal;
+  p.q_start = (int32_t)c.q_start;
+  p.gq_numel = (int32_t)x.g_q.numel();
+  p.gk_numel = x.g_k.defined() ? (int32_t)x.g_k.numel() : 0;
+  p.eps = (float)c.eps; p.sm_scale = (float)c.sm_scale; p.gate_scale = (float)c.gate_scale;
+  p.flags = c.flags;
+  p.q = view4(x.q, c.heads); p.k = view4(x.k, c.kv_heads); p.v = view4(x.v, c.kv_heads); p.v_first = view4(x.v_first, c.kv_heads);
+  p.o = view4(y, c.heads);
+  p.gate = view3(x.gate);
+  p.lse = ptr_of<float>(lse);
+  p.g_q = ptr_of<float>(x.g_q); p.g_k = ptr_of<float>(x.g_k); p.vr_coef = ptr_of<float>(x.coef);
+  if (c.cos.defined()) {
+    p.rope_cos = ptr_of<float>(c.cos); p.rope_sin = ptr_of<float>(c.sin);
+    p.rope_len = (int32_t)c.cos.size(0);
+    p.rope_q_pos0 = (int32_t)c.q_pos0; p.rope_k_pos0 = (int32_t)c.k_pos0;
+  }
+}
+
+Tensor scratch(const segpt_attn_params& p, int which, const at::Device& dev) {
+  const size_t n = segpt_attn_workspace_bytes(&p, which);
+  return at::empty({(int64_t)(n < 256 ? 256 : n)}, at::TensorOptions().dtype(at::kByte).device(dev));
+}
+void* current_stream(const at::Device& dev) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream(); }
+
+// operands as the kernels take them: fp32 scale vectors, contiguous last dimensions; checked
+Operands prepared(const Operands& x, const Call& c) {
+  const auto dev = x.q.device();
+  Operands r{x.q, x.k, x.v, f32_vector(x.g_q, dev), f32_vector(x.g_k, dev), x.v_first, f32_vector(x.coef, dev), x.gate};
+  check_operands(r, c);
+  r.q = last_dim_contiguous(r.q); r.k = last_dim_contiguous(r.k); r.v = last_dim_contiguous(r.v);
+  r.v_first = last_dim_contiguous(r.v_first);
+  return r;
+}
+
+struct Forward {
+  Tensor lse, kv_ws;
+};
+// x: prepared(); y is written
+Forward run_forward(const Operands& x, const Call& c, const Tensor& y) {
+  const auto dev = x.q.device();
+  const Sizes q = sizes_of(x.q, c.heads);
+  Forward r;
+  r.lse = at::empty({q.B, q.H, q.S}, x.q.options().dtype(at::kFloat));
+  if (x.q.numel() == 0) {  // empty batch / no query rows: nothing to launch (the C ABI rejects zero sizes)
+    r.kv_ws = at::empty({0}, x.q.options().dtype(at::kByte));
+    return r;
+  }
+  segpt_attn_params p{};
+  fill(p, x, c, y, r.lse);
+  r.kv_ws = scratch(p, SEGPT_WS_KV, dev);
+  p.kv_workspace = r.kv_ws.data_ptr();
+  p.kv_workspace_bytes = (size_t)r.kv_ws.numel();
+  const c10::DeviceGuard guard(dev);  // the launch goes to the tensors' device, whatever the current one is
+  const int rc = segpt_attn_fwd(&p, current_stream(dev));
+  if (rc) throw LibraryError(rc, "segpt_attn_fwd");
+  return r;
+}
+
+struct Grads {
+  Tensor q, k, v, g_q, g_k, v_first, coef, gate;
+};
+Tensor as_param_grad(const Tensor& g32, const Tensor& param) {
+  return param.scalar_type() == at::kFloat ? g32 : g32.to(param.scalar_type());
+}
+// x: the operands as the caller passed them; kv_ws: the forward's (its key/value pre-pass is not repeated)
+Grads run_backward(const Operands& raw, const Call& c, const Tensor& y, const Tensor& lse, const Tensor& kv_ws, Tensor dy) {
+  const Operands x = prepared(raw, c);
+  const auto dev = x.q.device();
+  if (dy.scalar_type() != x.q.scalar_type()) dy = dy.to(x.q.scalar_type());
+  dy = c.heads ? dy.contiguous() : last_dim_contiguous(dy);
+  const auto f32 = x.q.options().dtype(at::kFloat);
+  auto vector_grad = [&](const Tensor& t) { return t.defined() ? at::empty(t.sizes(), f32) : Tensor(); };
+  auto like = [](const Tensor& t) { return t.defined() ? at::empty_like(t) : Tensor(); };
+  Grads g{like(x.q), like(x.k), like(x.v), vector_grad(raw.g_q), vector_grad(raw.g_k), like(x.v_first), vector_grad(raw.coef), like(x.gate)};
+  if (x.q.numel() == 0) {  // no query rows: every gradient is zero
+    for (Tensor* t : {&g.q, &g.k, &g.v, &g.g_q, &g.g_k, &g.v_first, &g.coef, &g.gate})
+      if (t->defined()) t->zero_();
+  } else {
+    segpt_attn_params p{};
+    fill(p, x, c, y, lse);
+    p.flags = (c.flags & ~SEGPT_FLAG_DECODE) | SEGPT_FLAG_KV_PREPARED;
+    p.d_o = view4(dy, c.heads);
+    p.dq = view4(g.q, c.heads); p.dk = view4(g.k, c.kv_heads); p.dv = view4(g.v, c.kv_heads); p.dv_first = view4(g.v_first, c.kv_heads);
+    p.dgate = view3(g.gate);
+    p.dg_q = ptr_of<float>(g.g_q); p.dg_k = ptr_of<float>(g.g_k); p.dvr_coef = ptr_of<float>(g.coef);
+    const Tensor ws = scratch(p, SEGPT_WS_BWD, dev);
+    p.workspace = ws.data_ptr(); p.workspace_bytes = (size_t)ws.numel();
+    p.kv_workspace = kv_ws.data_ptr(); p.kv_workspace_bytes = (size_t)kv_ws.numel();
+    const c10::DeviceGuard guard(dev);
+    const int rc = segpt_attn_bwd(&p, current_stream(dev));
+    if (rc) throw LibraryError(rc, "segpt_attn_bwd");
+  }
+  g.g_q = as_param_grad(g.g_q, raw.g_q);
+  if (raw.g_k.defined()) g.g_k = as_param_grad(g.g_k, raw.g_k);
+  if (raw.coef.defined()) g.coef = as_param_grad(g.coef, raw.coef);
+  return g;
+}
+
+// y of the op: q's layout, or (bshd) a [B,H,Sq,D] view of a [B,Sq,H,D] buffer, the layout the output projection consumes
+Tensor output_like(const Tensor& q, bool bshd) {
+  if (bshd) return at::empty({q.size(0), q.size(2), q.size(1), q.size(3)}, q.options()).permute({0, 2, 1, 3});
+  Tensor y = at::empty_like(q);
+  return y.stride(-1) == 1 ? y : at::empty(q.sizes(), q.options());
+}
+
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+struct AttentionNode : torch::autograd::Function<AttentionNode> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g_q, const OptTensor& og_k,
+                               const OptTensor& ov_first, const OptTensor& ocoef, const OptTensor& ogate, c10::intrusive_ptr<Call> call, bool bshd,
+                               bool with_lse) {
+    const Tensor g_k = defined_or_none(og_k), coef = defined_or_none(ocoef), gate = defined_or_none(ogate);
+    const Operands x = prepared({q, k, v, g_q, g_k, defined_or_none(ov_first), coef, gate}, *call);
+    const Tensor y = output_like(x.q, bshd);
+    const Forward f = run_forward(x, *call, y);
+    // the normalised keys (bf16 path) are kept for the backward: 1/rep of q's size
+    ctx->save_for_backward({x.q, x.k, x.v, g_q, g_k, x.v_first, coef, gate, y, f.lse, f.kv_ws});
+    ctx->saved_data["call"] = c10::IValue::make_capsule(call);
+    ctx->set_materialize_grads(false);
+    if (!with_lse) return {y};
+    ctx->mark_non_differentiable({f.lse});
+    return {y, f.lse};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    variable_list out(11);
+    if (!grads[0].defined()) return out;
+    const variable_list s = ctx->get_saved_variables();
+    const auto call = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
+    const Grads g = run_backward({s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7]}, *call, s[8], s[9], s[10], grads[0]);
+    out[0] = g.q; out[1] = g.k; out[2] = g.v; out[3] = g.g_q; out[4] = g.g_k; out[5] = g.v_first; out[6] = g.coef; out[7] = g.gate;
+    return out;
+  }
+};
+
+c10::intrusive_ptr<Call> make_call(const Tensor& q, double gate_scale, double eps, std::optional<double> sm_scale, bool causal, int64_t q_start,
+                                   const OptTensor& rope_cos, const OptTensor& rope_sin, std::optional<int64_t> rope_q_pos0, int64_t rope_k_pos0,
+                                   int64_t flags, int64_t heads, int64_t kv_heads) {
+  auto c = c10::make_intrusive<Call>();
+  c->gate_scale = gate_scale; c->eps = eps;
+  c->sm_scale = sm_scale.has_value() ? *sm_scale : 1.0 / std::sqrt((double)q.size(-1));
+  c->causal = causal; c->q_start = q_start; c->flags = (int)flags;
+  c->heads = heads; c->kv_heads = kv_heads;
+  check(rope_cos.has_value() == rope_sin.has_value(), "rope_cos and rope_sin go together");
+  if (rope_cos.has_value()) {
+    // fp32 contiguous tables of shape [len, head_dim / 2]; query row i sits at position q_pos0 + i (default q_start, as
+    // in the reference's caller, attention.py:191-204), key row j at k_pos0 + j
+    auto table = [&](const Tensor& t) { return t.detach().to(q.device(), at::kFloat).contiguous(); };
+    c->cos = table(*rope_cos); c->sin = table(*rope_sin);
+    check(c->cos.dim() == 2 && c->cos.sizes() == c->sin.sizes() && c->cos.size(1) == q.size(-1) / 2, "rope tables must be [len, head_dim // 2]");
+    c->q_pos0 = rope_q_pos0.has_value() ? *rope_q_pos0 : q_start;
+    c->k_pos0 = rope_k_pos0;
+  }
+  return c;
+}
+
+// The differentiable op.  Nothing is recorded when no gradient can be asked for.
+std::pair<Tensor, Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g_q, const OptTensor& g_k, const OptTensor& v_first,
+                                    const OptTensor& coef, const OptTensor& gate, double gate_scale, double eps, std::optional<double> sm_scale,
+                                    bool causal, int64_t q_start, const OptTensor& rope_cos, const OptTensor& rope_sin,
+                                    std::optional<int64_t> rope_q_pos0, int64_t rope_k_pos0, int64_t flags, int64_t heads, int64_t kv_heads, bool bshd,
+                                    bool with_lse) {
+  const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin, rope_q_pos0, rope_k_pos0, flags, heads, kv_heads);
+  const Operands x{q, k, v, g_q, defined_or_none(g_k), defined_or_none(v_first), defined_or_none(coef), defined_or_none(gate)};
+  bool record = false;
+  if (at::GradMode::is_enabled())
+    for (const Tensor* t : {&x.q, &x.k, &x.v, &x.g_q, &x.g_k, &x.v_first, &x.coef, &x.gate}) record |= t->defined() && t->requires_grad();
+  if (record) {
+    const variable_list r = AttentionNode::apply(x.q, x.k, x.v, x.g_q, g_k, v_first, coef, gate, call, bshd, with_lse);
+    return {r[0], with_lse ? r[1] : Tensor()};
+  }
+  const at::NoGradGuard no_grad;
+  const Operands px = prepared(x, *call);
+  const Tensor y = output_like(px.q, bshd);
+  const Forward f = run_forward(px, *call, y);
+  return {y, with_lse ? f.lse : Tensor()};
+}
+
+// The two halves for the registered op (its autograd formula is torch.library's): y in a fixed layout, workspace returned
+std::tuple<Tensor, Tensor, Tensor> op_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g_q, const OptTensor& g_k,
+                                              const OptTensor& v_first, const OptTensor& coef, const OptTensor& gate, double gate_scale, double eps,
+                                              double sm_scale, bool causal, int64_t q_start, const OptTensor& rope_cos, const OptTensor& rope_sin,
+                                              std::optional<int64_t> rope_q_pos0, int64_t rope_k_pos0, int64_t flags, const Tensor& y) {
+  const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin, rope_q_pos0, rope_k_pos0, flags, 0, 0);
+  const Operands x = prepared({q, k, v, g_q, defined_or_none(g_k), defined_or_none(v_first), defined_or_none(coef), defined_or_none(gate)}, *call);
+  const Forward f = run_forward(x, *call, y);
+  return {y, f.lse, f.kv_ws};
+}
+std::vector<OptTensor> op_backward(const Tensor& dy, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g_q, const OptTensor& g_k,
+                                   const OptTensor& v_first, const OptTensor& coef, const OptTensor& gate, const Tensor& y, const Tensor& lse,
+                                   const Tensor& kv_ws, double gate_scale, double eps, double sm_scale, bool causal, int64_t q_start,
+                                   const OptTensor& rope_cos, const OptTensor& rope_sin, std::optional<int64_t> rope_q_pos0, int64_t rope_k_pos0,
+                                   int64_t flags) {
+  const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin, rope_q_pos0, rope_k_pos0, flags, 0, 0);
+  const Grads g = run_backward({q, k, v, g_q, defined_or_none(g_k), defined_or_none(v_first), defined_or_none(coef), defined_or_none(gate)}, *call, y,
+                               lse, kv_ws, dy);
+  auto opt = [](const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); };
+  return {g.q, g.k, g.v, g.g_q, opt(g.g_k), opt(g.v_first), opt(g.coef), opt(g.gate)};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_segpt_torch, m) {
+  static auto* segpt_error = new py::object();  // set by the package: its exception class for the library's return codes
+  m.def("set_error_class", [](py::object cls) { *segpt_error = std::move(cls); });
+  py::register_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const CheckFailed& e) {
+      PyErr_SetString(PyExc_AssertionError, e.what());
+    } catch (const BadType& e) {
+      PyErr_SetString(PyExc_TypeError, e.what());
+    } catch (const LibraryError& e) {
+      const py::object err = (*segpt_error)(e.code, e.where);
+      PyErr_SetObject((PyObject*)Py_TYPE(err.ptr()), err.ptr());
+    }
+  });
+  m.def("attention", &attention);
+  m.def("op_forward", &op_forward);
+  m.def("op_backward", &op_backward);
+}

@@ -1,4 +1,5 @@
-"""Autograd front end of the fused QK-norm flash attention (HIP kernels behind a C ABI).
+"""Front end of the fused QK-norm flash attention (HIP kernels behind a C ABI; checks, allocation, launch and the
+autograd node are native code, csrc/torch_binding.cpp).
 
 Two entry points share one implementation:
 
@@ -19,22 +20,16 @@ own formula (triton_flash_attn_qknorm.py:67-91).
 
 from __future__ import annotations
 
-import math
 import threading
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 
 _DTYPES = {torch.bfloat16: _lib.SEGPT_DTYPE_BF16, torch.float32: _lib.SEGPT_DTYPE_FP32}
 
 
-def _scale_arg(g, device):
-    """Scale parameter -> contiguous fp32 device vector (or None)."""
-    if g is None:
-        return None
-    return g.detach().to(device=device, dtype=torch.float32).reshape(-1).contiguous()
-
+# ---- filling the C ABI's struct from Python, for callers that hold on to one (plan.py)
 
 def _rope_arg(rope_cos, rope_sin, rope_q_pos0, rope_k_pos0, q_start, device, head_dim):
     """Normalise the rotary-embedding arguments to `(cos, sin, q_pos0, k_pos0)` (fp32 contiguous device tables
@@ -70,87 +65,6 @@ def _fill_common(p, q, k, v, y, lse, g_q, g_k, v_first, vr_coef, gate, gate_scal
         p.rope_q_pos0, p.rope_k_pos0 = q_pos0, k_pos0
 
 
-def _check_inputs(q, k, v, g_q, g_k, v_first, vr_coef, gate):
-    if q.dtype not in _DTYPES:
-        raise TypeError(f"qknorm attention supports bfloat16 and float32 tensors, got {q.dtype}")
-    for name, t in (("k", k), ("v", v), ("v_first", v_first), ("gate_logits", gate)):
-        if t is not None and t.dtype != q.dtype:
-            raise TypeError(f"{name} has dtype {t.dtype}, expected {q.dtype}")
-    assert q.is_cuda and k.is_cuda and v.is_cuda, "q, k, v must be device tensors"
-    B, H, Sq, D = q.shape
-    assert k.dim() == 4 and v.shape == k.shape and k.shape[0] == B and k.shape[3] == D, "k/v shape mismatch"
-    assert H % k.shape[1] == 0, "number of query heads must be a multiple of the kv heads"
-    assert g_q.numel() in (1, D), "gain must have 1 or head_dim elements"
-    assert g_k is None or g_k.numel() in (1, D), "k_gain must have 1 or head_dim elements"
-    assert (v_first is None) == (vr_coef is None), "v_first and vr_coef go together"
-    if v_first is not None:
-        assert v_first.shape == v.shape and vr_coef.numel() == 2
-    if gate is not None:
-        assert gate.shape == (B, Sq, H), "gate_logits must be [B, Sq, H]"
-
-
-def _forward(q, k, v, g_q, g_k, v_first, vr_coef, gate, gate_scale, eps, sm_scale, causal, q_start, y, rope=None,
-             inference=False, flags=0):
-    """Launch the forward on canonical 4-D views; returns (lse [B,H,Sq] fp32, kv workspace).  `y` is written.
-    The kv workspace holds the normalised keys (and mixed values) the backward can reuse.  `inference`: no
-    backward will follow, so a decode-shaped call (few query rows, long cache) may take the split-key kernels.
-    `flags`: SEGPT_FLAG_* bits of the call itself (SEGPT_FLAG_NO_NORM for attention without QK-norm)."""
-    lib = _lib.load()
-    B, H, Sq, _ = q.shape
-    lse = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)
-    if q.numel() == 0:  # empty batch / no query rows: nothing to launch (the C ABI rejects zero sizes)
-        return lse, torch.empty(0, dtype=torch.uint8, device=q.device)
-    p = _lib.new_params()
-    _fill_common(p, q, k, v, y, lse, g_q, g_k, v_first, vr_coef, gate, gate_scale, eps, sm_scale, causal, q_start, rope)
-    p.flags = flags | (_lib.SEGPT_FLAG_DECODE if inference else 0)  # before sizing: a decode-shaped call needs less
-    kv_ws = _lib.alloc_workspace(lib, p, _lib.SEGPT_WS_KV, q.device)
-    p.kv_workspace, p.kv_workspace_bytes = kv_ws.data_ptr(), kv_ws.numel()
-    with torch.cuda.device(q.device):  # the launch goes to the tensors' device, whatever the current one is
-        rc = lib.segpt_attn_fwd(p, torch.cuda.current_stream(q.device).cuda_stream)
-    if rc != 0:
-        raise _lib.SegptError(rc, "segpt_attn_fwd")
-    return lse, kv_ws
-
-
-def _backward(q, k, v, g_q, g_k, v_first, vr_coef, gate, gate_scale, eps, sm_scale, causal, q_start, y, lse, dy,
-              dq, dk, dv, dv_first, dgate, kv_ws=None, rope=None, flags=0):
-    """Launch the backward; dq/dk/dv(/dv_first/dgate) are written; returns (dg_q, dg_k, dvr_coef) fp32.
-    `kv_ws`: the forward's kv workspace (skips the key/value pre-pass); None allocates a fresh one."""
-    lib = _lib.load()
-    dev = q.device
-    dg_q = torch.empty_like(g_q)
-    dg_k = None if g_k is None else torch.empty_like(g_k)
-    dcoef = None if vr_coef is None else torch.empty(2, dtype=torch.float32, device=dev)
-    if q.numel() == 0:  # no query rows: every gradient is zero
-        for t in (dq, dk, dv, dv_first, dgate, dg_q, dg_k, dcoef):
-            if t is not None:
-                t.zero_()
-        return dg_q, dg_k, dcoef
-    p = _lib.new_params()
-    _fill_common(p, q, k, v, y, lse, g_q, g_k, v_first, vr_coef, gate, gate_scale, eps, sm_scale, causal, q_start, rope)
-    p.d_o, p.dq, p.dk, p.dv = _lib.t4(dy), _lib.t4(dq), _lib.t4(dk), _lib.t4(dv)
-    p.dv_first = _lib.t4(dv_first)
-    p.dgate = _lib.t3(dgate)
-    p.dg_q, p.dg_k, p.dvr_coef = _lib.ptr(dg_q), _lib.ptr(dg_k), _lib.ptr(dcoef)
-    ws = _lib.alloc_workspace(lib, p, _lib.SEGPT_WS_BWD, dev)
-    p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
-    p.flags = flags
-    if kv_ws is None:
-        kv_ws = _lib.alloc_workspace(lib, p, _lib.SEGPT_WS_KV, dev)
-    else:
-        p.flags |= _lib.SEGPT_FLAG_KV_PREPARED
-    p.kv_workspace, p.kv_workspace_bytes = kv_ws.data_ptr(), kv_ws.numel()
-    with torch.cuda.device(dev):
-        rc = lib.segpt_attn_bwd(p, torch.cuda.current_stream(dev).cuda_stream)
-    if rc != 0:
-        raise _lib.SegptError(rc, "segpt_attn_bwd")
-    return dg_q, dg_k, dcoef
-
-
-def _lastdim_contig(x):
-    return x if x.stride(-1) == 1 else x.contiguous()
-
-
 def _no_backward_will_follow(*tensors):
     """True when nothing can ask for a gradient of this call: grad mode is off (torch.no_grad / inference_mode,
     as in the reference's generate loop, transformer.py:160) or no tensor input requires one.  Must be evaluated
@@ -160,74 +74,24 @@ def _no_backward_will_follow(*tensors):
 
 
 class _GradModeAtApply:
-    """Mix-in for the positional drop-in Functions: records, in ``apply`` (the caller's context), whether a
-    backward can follow, for ``forward`` to read."""
+    """Mix-in for the positional drop-in Functions: ``apply`` runs ``forward`` in the caller's grad mode (the autograd
+    node is the native op's) and records there, for ``forward`` to read, whether a backward can follow."""
 
     _tls = threading.local()
 
     @classmethod
-    @torch.compiler.disable  # Python-side bookkeeping the compiler cannot trace: a compiled caller breaks the graph here
-    def apply(cls, *args, **kwargs):
+    @torch.compiler.disable  # native call and Python-side bookkeeping the compiler cannot trace: a compiled caller breaks the graph here
+    def apply(cls, *args):
         outer = getattr(cls._tls, "inference", False)  # a nested apply must leave the outer call's decision in place
         cls._tls.inference = _no_backward_will_follow(*(a for a in args if isinstance(a, torch.Tensor)))
         try:
-            return super().apply(*args, **kwargs)
+            return cls.forward(None, *args)
         finally:
             cls._tls.inference = outer
 
     @classmethod
     def _inference(cls):
         return bool(getattr(cls._tls, "inference", False))
-
-
-class _CoreFunc(torch.autograd.Function):
-    """Canonical-layout op: q [B,H,Sq,D], k/v/v_first [B,Hkv,Sk,D], gate [B,Sq,H]."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, g_q, g_k, v_first, vr_coef, gate, gate_scale, eps, sm_scale, causal, q_start, rope=None,
-                flags=0, out_bshd=False, inference=False):
-        gq32, gk32 = _scale_arg(g_q, q.device), _scale_arg(g_k, q.device)
-        coef32 = None if vr_coef is None else vr_coef.detach().to(device=q.device, dtype=torch.float32).reshape(-1).contiguous()
-        _check_inputs(q, k, v, gq32, gk32, v_first, coef32, gate)
-        q, k, v = _lastdim_contig(q), _lastdim_contig(k), _lastdim_contig(v)
-        v_first = None if v_first is None else _lastdim_contig(v_first)
-        if sm_scale is None:
-            sm_scale = 1.0 / math.sqrt(q.shape[-1])
-        if out_bshd:  # [B,H,Sq,D] view of a [B,Sq,H,D] buffer: the layout the output projection consumes
-            B, H, Sq, D = q.shape
-            y = torch.empty((B, Sq, H, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
-        else:
-            y = torch.empty_like(q)
-            if y.stride(-1) != 1:
-                y = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        lse, kv_ws = _forward(q, k, v, gq32, gk32, v_first, coef32, gate, gate_scale, eps, sm_scale, causal, q_start, y, rope,
-                              inference=inference, flags=flags)
-        # the normalised keys (bf16 path) are kept for the backward: 1/rep of q's size
-        ctx.save_for_backward(q, k, v, g_q, g_k, v_first, vr_coef, gate, y, lse, kv_ws)
-        ctx.cfg = (gate_scale, eps, sm_scale, causal, q_start, rope, flags)
-        ctx.mark_non_differentiable(lse)
-        return y, lse
-
-    @staticmethod
-    def backward(ctx, dy, _dlse):
-        q, k, v, g_q, g_k, v_first, vr_coef, gate, y, lse, kv_ws = ctx.saved_tensors
-        gate_scale, eps, sm_scale, causal, q_start, rope, flags = ctx.cfg
-        gq32, gk32 = _scale_arg(g_q, q.device), _scale_arg(g_k, q.device)
-        coef32 = None if vr_coef is None else vr_coef.detach().to(device=q.device, dtype=torch.float32).reshape(-1).contiguous()
-        dy = _lastdim_contig(dy)
-        if dy.dtype != q.dtype:
-            dy = dy.to(q.dtype)
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        dv_first = None if v_first is None else torch.empty_like(v_first)
-        dgate = None if gate is None else torch.empty_like(gate)
-        dg_q, dg_k, dcoef = _backward(q, k, v, gq32, gk32, v_first, coef32, gate, gate_scale, eps, sm_scale, causal,
-                                      q_start, y, lse, dy, dq, dk, dv, dv_first, dgate, kv_ws, rope, flags)
-        dg_q = dg_q.reshape(g_q.shape).to(g_q.dtype)
-        if g_k is not None:
-            dg_k = dg_k.reshape(g_k.shape).to(g_k.dtype)
-        if vr_coef is not None:
-            dcoef = dcoef.reshape(vr_coef.shape).to(vr_coef.dtype)
-        return dq, dk, dv, dg_q, dg_k, dv_first, dcoef, dgate, None, None, None, None, None, None, None, None, None
 
 
 def qknorm_attention(q, k, v, g_q, g_k=None, *, v_first=None, vr_coef=None, gate_logits=None, gate_scale=2.0,
@@ -246,17 +110,43 @@ def qknorm_attention(q, k, v, g_q, g_k=None, *, v_first=None, vr_coef=None, gate
     ``out_bshd=True``: the returned ``[B,H,Sq,D]`` tensor is a view of a ``[B,Sq,H,D]`` buffer, so that
     ``y.permute(0, 2, 1, 3).reshape(B, Sq, H*D)`` is the ``b seq (h head_d)`` tensor of attention.py:243 without a copy.
     """
-    rope = _rope_arg(rope_cos, rope_sin, rope_q_pos0, rope_k_pos0, q_start, q.device, q.shape[-1])
-    inference = _no_backward_will_follow(q, k, v, g_q, g_k, v_first, vr_coef, gate_logits)
-    y, lse = _CoreFunc.apply(q, k, v, g_q, g_k, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale, causal, q_start,
-                             rope, 0 if qk_norm else _lib.SEGPT_FLAG_NO_NORM, out_bshd, inference)
+    y, lse = _native.load().attention(
+        q, k, v, g_q, g_k, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin,
+        rope_q_pos0, rope_k_pos0, _call_flags(qk_norm, _no_backward_will_follow(q, k, v, g_q, g_k, v_first, vr_coef, gate_logits)),
+        0, 0, out_bshd, return_lse)
     return (y, lse) if return_lse else y
+
+
+def _call_flags(qk_norm, inference):
+    """SEGPT_FLAG_* bits of a call; `inference`: no backward will follow, so a forward with few query rows or few query
+    tiles may split the keys."""
+    return (0 if qk_norm else _lib.SEGPT_FLAG_NO_NORM) | (_lib.SEGPT_FLAG_DECODE if inference else 0)
 
 
 def _canon(x, n_heads):
     """[(h b), S, d] -> [B, H, S, d] view (no copy): head-major flatten of attention.py:199."""
     n, S, d = x.shape
     return x.view(n_heads, n // n_heads, S, d).permute(1, 0, 2, 3)
+
+
+def _flat_operands(Q, K, V, n_kv_heads, gate_logits):
+    """The reference's checks on the flattened operands (triton_flash_attn_qknorm.py:273-281) and the head counts:
+    ``(Q, K, V, H, Hkv)`` with 2-D tensors promoted to 3-D."""
+    assert Q.is_cuda and Q.is_contiguous()
+    assert K.is_cuda and K.is_contiguous()
+    assert V.is_cuda and V.is_contiguous()
+    if Q.ndim == 2:
+        Q, K, V = Q.unsqueeze(0), K.unsqueeze(0), V.unsqueeze(0)
+    nq, nk = Q.shape[0], K.shape[0]
+    if n_kv_heads is None:
+        assert nk == nq, "n_kv_heads is required for un-expanded GQA K/V"
+        # without a gate every flattened row is its own (batch, head): plain MHA layout of the reference
+        H = Hkv = 1 if gate_logits is None else gate_logits.shape[-1]
+    else:
+        Hkv = int(n_kv_heads)
+        assert nq % nk == 0 and nk % Hkv == 0, "K/V rows must be n_kv_heads * batch"
+        H = Hkv * (nq // nk)
+    return Q, K, V, H, Hkv
 
 
 class QKNormFlashAttnFunc(_GradModeAtApply, torch.autograd.Function):
@@ -276,66 +166,15 @@ class QKNormFlashAttnFunc(_GradModeAtApply, torch.autograd.Function):
     def forward(ctx, Q, K, V, gain, is_causal=True, q_start=0, k_gain=None, v_first=None, vr_coef=None,
                 gate_logits=None, gate_scale=2.0, n_kv_heads=None, eps=1e-6, sm_scale=None, rope_cos=None,
                 rope_sin=None):
-        assert Q.is_cuda and Q.is_contiguous()
-        assert K.is_cuda and K.is_contiguous()
-        assert V.is_cuda and V.is_contiguous()
+        Q, K, V, H, Hkv = _flat_operands(Q, K, V, n_kv_heads, gate_logits)
         assert gain.is_cuda
-        if Q.ndim == 2:
-            Q, K, V = Q.unsqueeze(0), K.unsqueeze(0), V.unsqueeze(0)
-            if v_first is not None and v_first.ndim == 2:
-                v_first = v_first.unsqueeze(0)
-        nq, nk = Q.shape[0], K.shape[0]
-        if nk != nq or n_kv_heads is not None or gate_logits is not None:
-            if n_kv_heads is None:
-                assert gate_logits is not None and nk == nq, "n_kv_heads is required for un-expanded GQA K/V"
-                H = Hkv = gate_logits.shape[-1]
-            else:
-                Hkv = int(n_kv_heads)
-                assert nq % nk == 0 and nk % Hkv == 0, "K/V rows must be n_kv_heads * batch"
-                H = Hkv * (nq // nk)
-        else:
-            H = Hkv = 1  # every flattened row is its own (batch, head): plain MHA layout of the reference
         if v_first is not None:
             assert v_first.is_cuda and v_first.is_contiguous()
-        q4, k4, v4 = _canon(Q, H), _canon(K, Hkv), _canon(V, Hkv)
-        vf4 = None if v_first is None else _canon(v_first, Hkv)
-        gq32, gk32 = _scale_arg(gain, Q.device), _scale_arg(k_gain, Q.device)
-        coef32 = None if vr_coef is None else vr_coef.detach().to(device=Q.device, dtype=torch.float32).reshape(-1).contiguous()
-        _check_inputs(q4, k4, v4, gq32, gk32, vf4, coef32, gate_logits)
-        if sm_scale is None:
-            sm_scale = 1.0 / math.sqrt(Q.shape[-1])
-        O = torch.empty_like(Q)
-        rope = _rope_arg(rope_cos, rope_sin, None, 0, q_start, Q.device, Q.shape[-1])
-        lse, kv_ws = _forward(q4, k4, v4, gq32, gk32, vf4, coef32, gate_logits, gate_scale, eps, sm_scale, is_causal,
-                              q_start, _canon(O, H), rope, inference=QKNormFlashAttnFunc._inference())
-        ctx.save_for_backward(lse, Q, K, V, gain, O, k_gain, v_first, vr_coef, gate_logits, kv_ws)
-        ctx.cfg = (H, Hkv, gate_scale, eps, sm_scale, bool(is_causal), int(q_start), rope)
-        return O
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        lse, Q, K, V, gain, O, k_gain, v_first, vr_coef, gate, kv_ws = ctx.saved_tensors
-        H, Hkv, gate_scale, eps, sm_scale, causal, q_start, rope = ctx.cfg
-        grad_output = grad_output.contiguous()
-        if grad_output.dtype != Q.dtype:
-            grad_output = grad_output.to(Q.dtype)
-        if grad_output.ndim == 2:
-            grad_output = grad_output.unsqueeze(0)
-        dQ, dK, dV = torch.empty_like(Q), torch.empty_like(K), torch.empty_like(V)
-        dVf = None if v_first is None else torch.empty_like(v_first)
-        dgate = None if gate is None else torch.empty_like(gate)
-        gq32, gk32 = _scale_arg(gain, Q.device), _scale_arg(k_gain, Q.device)
-        coef32 = None if vr_coef is None else vr_coef.detach().to(device=Q.device, dtype=torch.float32).reshape(-1).contiguous()
-        dg_q, dg_k, dcoef = _backward(
-            _canon(Q, H), _canon(K, Hkv), _canon(V, Hkv), gq32, gk32,
-            None if v_first is None else _canon(v_first, Hkv), coef32, gate, gate_scale, eps, sm_scale, causal, q_start,
-            _canon(O, H), lse, _canon(grad_output, H), _canon(dQ, H), _canon(dK, Hkv), _canon(dV, Hkv),
-            None if dVf is None else _canon(dVf, Hkv), dgate, kv_ws, rope)
-        dgain = dg_q.reshape(gain.shape).to(gain.dtype)
-        dk_gain = None if k_gain is None else dg_k.reshape(k_gain.shape).to(k_gain.dtype)
-        dcoef = None if vr_coef is None else dcoef.reshape(vr_coef.shape).to(vr_coef.dtype)
-        #      Q   K   V   gain   causal q_start k_gain  v_first vr_coef gate  gate_scale n_kv eps sm_scale rope tables
-        return dQ, dK, dV, dgain, None, None, dk_gain, dVf, dcoef, dgate, None, None, None, None, None, None
+            if v_first.ndim == 2:
+                v_first = v_first.unsqueeze(0)
+        return _native.load().attention(Q, K, V, gain, k_gain, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale,
+                                        is_causal, q_start, rope_cos, rope_sin, None, 0, _call_flags(True, QKNormFlashAttnFunc._inference()),
+                                        H, Hkv, False, False)[0]
 
 
 class TritonFlashAttnQKNormFunc(QKNormFlashAttnFunc):
@@ -366,41 +205,7 @@ class FlashAttnFunc(_GradModeAtApply, torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, Q, K, V, q_start=0, is_causal=True, n_kv_heads=None):
-        assert Q.is_cuda and Q.is_contiguous()
-        assert K.is_cuda and K.is_contiguous()
-        assert V.is_cuda and V.is_contiguous()
-        if Q.ndim == 2:
-            Q, K, V = Q.unsqueeze(0), K.unsqueeze(0), V.unsqueeze(0)
-        nq, nk = Q.shape[0], K.shape[0]
-        if n_kv_heads is None:
-            assert nk == nq, "n_kv_heads is required for un-expanded GQA K/V"
-            H = Hkv = 1
-        else:
-            Hkv = int(n_kv_heads)
-            assert nq % nk == 0 and nk % Hkv == 0, "K/V rows must be n_kv_heads * batch"
-            H = Hkv * (nq // nk)
-        q4, k4, v4 = _canon(Q, H), _canon(K, Hkv), _canon(V, Hkv)
+        Q, K, V, H, Hkv = _flat_operands(Q, K, V, n_kv_heads, None)
         one = torch.ones(1, dtype=torch.float32, device=Q.device)
-        _check_inputs(q4, k4, v4, one, None, None, None, None)
-        sm_scale = 1.0 / math.sqrt(Q.shape[-1])
-        O = torch.empty_like(Q)
-        lse, kv_ws = _forward(q4, k4, v4, one, None, None, None, None, 1.0, 0.0, sm_scale, is_causal, q_start, _canon(O, H),
-                              None, inference=FlashAttnFunc._inference(), flags=_lib.SEGPT_FLAG_NO_NORM)
-        ctx.save_for_backward(lse, Q, K, V, O, one, kv_ws)
-        ctx.cfg = (H, Hkv, sm_scale, bool(is_causal), int(q_start))
-        return O
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        lse, Q, K, V, O, one, kv_ws = ctx.saved_tensors
-        H, Hkv, sm_scale, causal, q_start = ctx.cfg
-        grad_output = grad_output.contiguous()
-        if grad_output.dtype != Q.dtype:
-            grad_output = grad_output.to(Q.dtype)
-        if grad_output.ndim == 2:
-            grad_output = grad_output.unsqueeze(0)
-        dQ, dK, dV = torch.empty_like(Q), torch.empty_like(K), torch.empty_like(V)
-        _backward(_canon(Q, H), _canon(K, Hkv), _canon(V, Hkv), one, None, None, None, None, 1.0, 0.0, sm_scale, causal,
-                  q_start, _canon(O, H), lse, _canon(grad_output, H), _canon(dQ, H), _canon(dK, Hkv), _canon(dV, Hkv),
-                  None, None, kv_ws, None, _lib.SEGPT_FLAG_NO_NORM)
-        return dQ, dK, dV, None, None, None
+        return _native.load().attention(Q, K, V, one, None, None, None, None, 1.0, 0.0, None, is_causal, q_start, None, None, None, 0,
+                                        _call_flags(False, FlashAttnFunc._inference()), H, Hkv, False, False)[0]

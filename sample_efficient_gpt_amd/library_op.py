@@ -23,9 +23,8 @@ from typing import List, Optional
 import torch
 from torch import Tensor
 
-from . import _lib
-from .function import (_backward, _check_inputs, _forward, _lastdim_contig, _no_backward_will_follow, _rope_arg,
-                       _scale_arg)
+from . import _native
+from .function import _call_flags, _no_backward_will_follow, qknorm_attention
 
 __all__ = ["qknorm_attention_op"]
 
@@ -39,23 +38,14 @@ def _empty_out(q, out_bshd):
     return q.new_empty((B, H, Sq, D))
 
 
-def _coef32(vr_coef, device):
-    return None if vr_coef is None else vr_coef.detach().to(device=device, dtype=torch.float32).reshape(-1).contiguous()
-
-
 @torch.library.custom_op("segpt::qknorm_attention", mutates_args=())
 def _fwd_op(q: Tensor, k: Tensor, v: Tensor, g_q: Tensor, g_k: Optional[Tensor], v_first: Optional[Tensor],
             vr_coef: Optional[Tensor], gate_logits: Optional[Tensor], gate_scale: float, eps: float, sm_scale: float,
             causal: bool, q_start: int, rope_cos: Optional[Tensor], rope_sin: Optional[Tensor],
             rope_q_pos0: int, rope_k_pos0: int, qk_norm: bool, out_bshd: bool, inference: bool) -> List[Tensor]:
-    rope = _rope_arg(rope_cos, rope_sin, None if rope_q_pos0 < 0 else rope_q_pos0, rope_k_pos0, q_start, q.device, q.shape[-1])
-    gq32, gk32, c32 = _scale_arg(g_q, q.device), _scale_arg(g_k, q.device), _coef32(vr_coef, q.device)
-    _check_inputs(q, k, v, gq32, gk32, v_first, c32, gate_logits)
-    q, k, v = _lastdim_contig(q), _lastdim_contig(k), _lastdim_contig(v)
-    v_first = None if v_first is None else _lastdim_contig(v_first)
-    y = _empty_out(q, out_bshd)
-    lse, kv_ws = _forward(q, k, v, gq32, gk32, v_first, c32, gate_logits, gate_scale, eps, sm_scale, causal, q_start, y, rope,
-                          inference=inference, flags=0 if qk_norm else _lib.SEGPT_FLAG_NO_NORM)
+    y, lse, kv_ws = _native.load().op_forward(
+        q, k, v, g_q, g_k, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin,
+        None if rope_q_pos0 < 0 else rope_q_pos0, rope_k_pos0, _call_flags(qk_norm, inference), _empty_out(q, out_bshd))
     if inference:  # no backward will read it (and after the decode kernels it holds no keys)
         kv_ws = q.new_empty((0,), dtype=torch.uint8)
     return [y, lse, kv_ws]
@@ -84,26 +74,11 @@ def _bwd_op(dy: Tensor, q: Tensor, k: Tensor, v: Tensor, g_q: Tensor, g_k: Optio
             rope_cos: Optional[Tensor], rope_sin: Optional[Tensor], rope_q_pos0: int, rope_k_pos0: int,
             qk_norm: bool) -> List[Tensor]:
     """Returns [dq, dk, dv, dg_q, dg_k, dv_first, dvr_coef, dgate]; absent ones are empty tensors."""
-    dev = q.device
-    rope = _rope_arg(rope_cos, rope_sin, None if rope_q_pos0 < 0 else rope_q_pos0, rope_k_pos0, q_start, dev, q.shape[-1])
-    gq32, gk32, c32 = _scale_arg(g_q, dev), _scale_arg(g_k, dev), _coef32(vr_coef, dev)
-    q, k, v = _lastdim_contig(q), _lastdim_contig(k), _lastdim_contig(v)
-    v_first = None if v_first is None else _lastdim_contig(v_first)
-    dy = _lastdim_contig(dy)
-    if dy.dtype != q.dtype:
-        dy = dy.to(q.dtype)
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    dvf = None if v_first is None else torch.empty_like(v_first)
-    dgate = None if gate_logits is None else torch.empty_like(gate_logits)
-    dg_q, dg_k, dcoef = _backward(q, k, v, gq32, gk32, v_first, c32, gate_logits, gate_scale, eps, sm_scale, causal, q_start,
-                                  y, lse, dy, dq, dk, dv, dvf, dgate, kv_ws, rope,
-                                  0 if qk_norm else _lib.SEGPT_FLAG_NO_NORM)
-    none = lambda: q.new_empty((0,))  # a fresh tensor each: returns of a custom op must not alias one another
-    return [dq, dk, dv, dg_q.reshape(g_q.shape).to(g_q.dtype),
-            none() if g_k is None else dg_k.reshape(g_k.shape).to(g_k.dtype),
-            none() if dvf is None else dvf,
-            none() if vr_coef is None else dcoef.reshape(vr_coef.shape).to(vr_coef.dtype),
-            none() if dgate is None else dgate]
+    grads = _native.load().op_backward(
+        dy, q, k, v, g_q, g_k, v_first, vr_coef, gate_logits, y, lse, kv_ws, gate_scale, eps, sm_scale, causal, q_start,
+        rope_cos, rope_sin, None if rope_q_pos0 < 0 else rope_q_pos0, rope_k_pos0, _call_flags(qk_norm, False))
+    # an absent operand's place is a fresh tensor each: returns of a custom op must not alias one another
+    return [q.new_empty((0,)) if g is None else g for g in grads]
 
 
 @_bwd_op.register_fake
@@ -144,6 +119,12 @@ def qknorm_attention_op(q, k, v, g_q, g_k=None, *, v_first=None, vr_coef=None, g
                         eps=1e-6, sm_scale=None, causal=True, q_start=0, return_lse=False,
                         rope_cos=None, rope_sin=None, rope_q_pos0=None, rope_k_pos0=0, qk_norm=True, out_bshd=False):
     """Keyword front end of ``torch.ops.segpt.qknorm_attention`` (same arguments as ``qknorm_attention``)."""
+    if q.is_cuda and not torch.compiler.is_compiling() and not torch._C._len_torch_dispatch_stack():
+        # nobody is looking at the call as an operator (no compiler, no dispatch mode such as a selective-checkpoint
+        # policy or fake tensors): the same kernels without the registered op's 45 us of Python dispatch
+        return qknorm_attention(q, k, v, g_q, g_k, v_first=v_first, vr_coef=vr_coef, gate_logits=gate_logits, gate_scale=gate_scale,
+                                eps=eps, sm_scale=sm_scale, causal=causal, q_start=q_start, return_lse=return_lse, rope_cos=rope_cos,
+                                rope_sin=rope_sin, rope_q_pos0=rope_q_pos0, rope_k_pos0=rope_k_pos0, qk_norm=qk_norm, out_bshd=out_bshd)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(q.shape[-1])
     # decided here, in the caller's grad mode: a forward-only call (the reference's generate loop runs under

@@ -230,6 +230,15 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
         _lib.load()
 
 
+def test_missing_binding_fails_loudly(monkeypatch, tmp_path):
+    from sample_efficient_gpt_amd import _native
+
+    monkeypatch.setattr(_native, "_module", None)
+    monkeypatch.setattr(_native, "MODULE_PATH", str(tmp_path / "_segpt_torch.so"))
+    with pytest.raises(RuntimeError, match="no fallback"):
+        _native.load()
+
+
 def test_input_generators_are_seeded_and_shaped():
     c = CONFIGS[1]
     a, b = make_inputs(c), make_inputs(c)

@@ -509,6 +509,46 @@ def test_positional_dropin_functions_under_torch_compile(gpu_device):
         QKNormFlashAttnFunc._tls.inference = False
 
 
+def test_native_node_on_other_threads_and_streams(gpu_device):
+    """The op and its native autograd node from two Python threads, each on a stream of its own, with the backward run
+    after a retained graph's first one: every result equals the default stream's bit for bit; an undefined output
+    gradient gives no gradients and a library error in the forward is the package's exception class."""
+    import threading
+
+    from sample_efficient_gpt_amd import _lib
+
+    x = gen(2, 6, 2, 160, 160, 64, BF16, extras=True, seed=51)
+    names = ["q", "k", "v", "g_q", "g_k", "v_first", "vr_coef", "gate_logits"]
+
+    def run(out, stream):
+        with torch.cuda.stream(stream):
+            t = {n: x[n].to(gpu_device).requires_grad_(True) for n in names}
+            y = qknorm_attention(t["q"], t["k"], t["v"], t["g_q"], t["g_k"], v_first=t["v_first"], vr_coef=t["vr_coef"], gate_logits=t["gate_logits"])
+            d_o = x["d_o"].to(gpu_device)
+            first = torch.autograd.grad(y, [t[n] for n in names], d_o, retain_graph=True)
+            again = torch.autograd.grad(y, [t[n] for n in names], d_o)
+            out.extend([y.detach(), *first, *again])
+        stream.synchronize()
+
+    ref, a, b = [], [], []
+    run(ref, torch.cuda.default_stream())
+    threads = [threading.Thread(target=run, args=(o, torch.cuda.Stream())) for o in (a, b)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(a) == len(b) == len(ref) == 1 + 2 * len(names)
+    for got in (a, b):
+        for i, (r, g) in enumerate(zip(ref, got)):
+            assert torch.equal(r, g), i
+    q = x["q"].to(gpu_device).requires_grad_(True)
+    k, v, g = (x[n].to(gpu_device) for n in ("k", "v", "g_q"))
+    y, lse = qknorm_attention(q, k, v, g, return_lse=True)
+    assert not lse.requires_grad and torch.autograd.grad((y * 0.0).sum() + q.sum() * 0.0, q)[0].abs().max() == 0
+    with pytest.raises(_lib.SegptError):
+        qknorm_attention(q[..., :32], k[..., :32], v[..., :32], torch.ones(1, device=gpu_device))
+
+
 # ------------------------------------------------------------------ rotary embedding fused into the loads
 
 
