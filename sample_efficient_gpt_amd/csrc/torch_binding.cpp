@@ -6,10 +6,12 @@
 // every Python instruction on either side when the two threads sit on different core complexes.  A forward + backward of
 // 512 tokens (58 us of kernels) took 130 to 240 us, depending on that placement alone; a node in C++ runs its backward
 // without the interpreter.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/ATen.h>
+#include <ATen/FuncTorchTLS.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 
@@ -34,6 +36,12 @@ struct LibraryError : std::runtime_error {
       : std::runtime_error(std::string(w) + " failed with code " + std::to_string(c) + ": " + segpt_strerror(c)), code(c), where(w) {}
 };
 void check(bool ok, const char* what) { if (!ok) throw CheckFailed(what); }
+
+PyObject* segpt_error = nullptr;  // the package's exception class for the library's return codes, set by it
+void set_python_error(const LibraryError& e) {
+  const py::object err = py::handle(segpt_error)(e.code, e.where);
+  PyErr_SetObject((PyObject*)Py_TYPE(err.ptr()), err.ptr());
+}
 
 Tensor defined_or_none(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 
@@ -90,7 +98,9 @@ void check_operands(const Operands& x, const Call& c) {
   check(x.q.is_cuda() && x.k.is_cuda() && x.v.is_cuda(), "q, k, v must be device tensors");
   const int64_t dims = c.heads ? 3 : 4;
   check(x.q.dim() == dims && x.k.dim() == dims && x.v.sizes() == x.k.sizes(), "k/v shape mismatch");
+  if (c.heads) check(x.q.size(0) % c.heads == 0 && x.k.size(0) % c.kv_heads == 0, "Q rows must be heads * batch");
   const Sizes q = sizes_of(x.q, c.heads), k = sizes_of(x.k, c.kv_heads);
+  check(q.D > 0, "head_dim must not be zero");
   check(k.B == q.B && k.D == q.D, "k/v shape mismatch");
   check(k.H > 0 && q.H % k.H == 0, "number of query heads must be a multiple of the kv heads");
   check(x.g_q.numel() == 1 || x.g_q.numel() == q.D, "gain must have 1 or head_dim elements");
@@ -232,10 +242,19 @@ struct AttentionNode : torch::autograd::Function<AttentionNode> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     variable_list out(11);
-    if (!grads[0].defined()) return out;
     const variable_list s = ctx->get_saved_variables();
     const auto call = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
-    const Grads g = run_backward({s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7]}, *call, s[8], s[9], s[10], grads[0]);
+    const Tensor dy = grads[0].defined() ? grads[0] : at::zeros_like(s[8]);
+    Grads g;
+    try {
+      g = run_backward({s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7]}, *call, s[8], s[9], s[10], dy);
+    } catch (const LibraryError& e) {  // on the engine's thread: carried to the caller's as the Python exception it is there
+      const py::gil_scoped_acquire gil;
+      set_python_error(e);
+      python_error err;
+      err.persist();
+      throw err;
+    }
     out[0] = g.q; out[1] = g.k; out[2] = g.v; out[3] = g.g_q; out[4] = g.g_k; out[5] = g.v_first; out[6] = g.coef; out[7] = g.gate;
     return out;
   }
@@ -262,7 +281,8 @@ c10::intrusive_ptr<Call> make_call(const Tensor& q, double gate_scale, double ep
   return c;
 }
 
-// The differentiable op.  Nothing is recorded when no gradient can be asked for.
+// The differentiable op.  Nothing is recorded when no gradient can be asked for.  Function transforms and forward-mode
+// tangents are refused, as by an autograd function that defines neither: the short way around the node must not drop them.
 std::pair<Tensor, Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g_q, const OptTensor& g_k, const OptTensor& v_first,
                                     const OptTensor& coef, const OptTensor& gate, double gate_scale, double eps, std::optional<double> sm_scale,
                                     bool causal, int64_t q_start, const OptTensor& rope_cos, const OptTensor& rope_sin,
@@ -270,9 +290,11 @@ std::pair<Tensor, Tensor> attention(const Tensor& q, const Tensor& k, const Tens
                                     bool with_lse) {
   const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin, rope_q_pos0, rope_k_pos0, flags, heads, kv_heads);
   const Operands x{q, k, v, g_q, defined_or_none(g_k), defined_or_none(v_first), defined_or_none(coef), defined_or_none(gate)};
+  if (const auto& transforms = at::functorch::functorchTLSAccessor()) transforms->checkSupportsCppAutogradFunction();
+  const bool grad_mode = at::GradMode::is_enabled();
   bool record = false;
-  if (at::GradMode::is_enabled())
-    for (const Tensor* t : {&x.q, &x.k, &x.v, &x.g_q, &x.g_k, &x.v_first, &x.coef, &x.gate}) record |= t->defined() && t->requires_grad();
+  for (const Tensor* t : {&x.q, &x.k, &x.v, &x.g_q, &x.g_k, &x.v_first, &x.coef, &x.gate})
+    record |= t->defined() && ((grad_mode && t->requires_grad()) || t->_fw_grad(0).defined());
   if (record) {
     const variable_list r = AttentionNode::apply(x.q, x.k, x.v, x.g_q, g_k, v_first, coef, gate, call, bshd, with_lse);
     return {r[0], with_lse ? r[1] : Tensor()};
@@ -306,11 +328,29 @@ std::vector<OptTensor> op_backward(const Tensor& dy, const Tensor& q, const Tens
   return {g.q, g.k, g.v, g.g_q, opt(g.g_k), opt(g.v_first), opt(g.coef), opt(g.gate)};
 }
 
+// What torch raises (out of memory, an error from a saved-tensor hook) keeps its Python type across the binding
+template <typename R, typename... A>
+auto bound(R (*f)(A...)) {
+  return [f](A... a) -> R {
+    try {
+      return f(std::forward<A>(a)...);
+    } catch (const CheckFailed&) {
+      throw;
+    } catch (const BadType&) {
+      throw;
+    } catch (const LibraryError&) {
+      throw;
+    } catch (...) {
+      torch::translate_exception_to_python(std::current_exception());
+      throw py::error_already_set();
+    }
+  };
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_segpt_torch, m) {
-  static auto* segpt_error = new py::object();  // set by the package: its exception class for the library's return codes
-  m.def("set_error_class", [](py::object cls) { *segpt_error = std::move(cls); });
+  m.def("set_error_class", [](py::object cls) { segpt_error = cls.release().ptr(); });
   py::register_exception_translator([](std::exception_ptr p) {
     try {
       if (p) std::rethrow_exception(p);
@@ -319,11 +359,10 @@ PYBIND11_MODULE(_segpt_torch, m) {
     } catch (const BadType& e) {
       PyErr_SetString(PyExc_TypeError, e.what());
     } catch (const LibraryError& e) {
-      const py::object err = (*segpt_error)(e.code, e.where);
-      PyErr_SetObject((PyObject*)Py_TYPE(err.ptr()), err.ptr());
+      set_python_error(e);
     }
   });
-  m.def("attention", &attention);
-  m.def("op_forward", &op_forward);
-  m.def("op_backward", &op_backward);
+  m.def("attention", bound(&attention));
+  m.def("op_forward", bound(&op_forward));
+  m.def("op_backward", bound(&op_backward));
 }

@@ -166,11 +166,12 @@ class QKNormFlashAttnFunc(_GradModeAtApply, torch.autograd.Function):
     def forward(ctx, Q, K, V, gain, is_causal=True, q_start=0, k_gain=None, v_first=None, vr_coef=None,
                 gate_logits=None, gate_scale=2.0, n_kv_heads=None, eps=1e-6, sm_scale=None, rope_cos=None,
                 rope_sin=None):
+        promoted = Q.ndim == 2
         Q, K, V, H, Hkv = _flat_operands(Q, K, V, n_kv_heads, gate_logits)
         assert gain.is_cuda
         if v_first is not None:
             assert v_first.is_cuda and v_first.is_contiguous()
-            if v_first.ndim == 2:
+            if promoted and v_first.ndim == 2:
                 v_first = v_first.unsqueeze(0)
         return _native.load().attention(Q, K, V, gain, k_gain, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale,
                                         is_causal, q_start, rope_cos, rope_sin, None, 0, _call_flags(True, QKNormFlashAttnFunc._inference()),

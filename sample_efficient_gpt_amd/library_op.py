@@ -115,13 +115,20 @@ def _autograd_backward(ctx, grads):
 _fwd_op.register_autograd(_autograd_backward, setup_context=_setup_context)
 
 
+def _seen_as_operator(*operands):
+    """Somebody looks at the call as an operator: a compiler, a dispatch or function mode (a selective-checkpoint policy,
+    fake tensors), a function transform (vmap, torch.func.grad) or an operand of a tensor subclass."""
+    return (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._are_functorch_transforms_active()
+            or any(t is not None and type(t) not in (Tensor, torch.nn.Parameter) for t in operands))
+
+
 def qknorm_attention_op(q, k, v, g_q, g_k=None, *, v_first=None, vr_coef=None, gate_logits=None, gate_scale=2.0,
                         eps=1e-6, sm_scale=None, causal=True, q_start=0, return_lse=False,
                         rope_cos=None, rope_sin=None, rope_q_pos0=None, rope_k_pos0=0, qk_norm=True, out_bshd=False):
     """Keyword front end of ``torch.ops.segpt.qknorm_attention`` (same arguments as ``qknorm_attention``)."""
-    if q.is_cuda and not torch.compiler.is_compiling() and not torch._C._len_torch_dispatch_stack():
-        # nobody is looking at the call as an operator (no compiler, no dispatch mode such as a selective-checkpoint
-        # policy or fake tensors): the same kernels without the registered op's 45 us of Python dispatch
+    if q.is_cuda and not _seen_as_operator(q, k, v, g_q, g_k, v_first, vr_coef, gate_logits, rope_cos, rope_sin):
+        # the same kernels without the registered op's 45 us of Python dispatch
         return qknorm_attention(q, k, v, g_q, g_k, v_first=v_first, vr_coef=vr_coef, gate_logits=gate_logits, gate_scale=gate_scale,
                                 eps=eps, sm_scale=sm_scale, causal=causal, q_start=q_start, return_lse=return_lse, rope_cos=rope_cos,
                                 rope_sin=rope_sin, rope_q_pos0=rope_q_pos0, rope_k_pos0=rope_k_pos0, qk_norm=qk_norm, out_bshd=out_bshd)

@@ -511,8 +511,8 @@ def test_positional_dropin_functions_under_torch_compile(gpu_device):
 
 def test_native_node_on_other_threads_and_streams(gpu_device):
     """The op and its native autograd node from two Python threads, each on a stream of its own, with the backward run
-    after a retained graph's first one: every result equals the default stream's bit for bit; an undefined output
-    gradient gives no gradients and a library error in the forward is the package's exception class."""
+    after a retained graph's first one: every result equals the default stream's bit for bit; lse takes no gradient and
+    a library error in the forward is the package's exception class."""
     import threading
 
     from sample_efficient_gpt_amd import _lib
@@ -547,6 +547,80 @@ def test_native_node_on_other_threads_and_streams(gpu_device):
     assert not lse.requires_grad and torch.autograd.grad((y * 0.0).sum() + q.sum() * 0.0, q)[0].abs().max() == 0
     with pytest.raises(_lib.SegptError):
         qknorm_attention(q[..., :32], k[..., :32], v[..., :32], torch.ones(1, device=gpu_device))
+
+
+def test_native_node_keeps_what_python_callers_see(gpu_device):
+    """What an autograd function in Python gives its callers holds for the native node: an undefined output gradient counts
+    as zero, torch's exceptions and the package's own keep their types in both directions, what a saved-tensor hook
+    raises reaches the caller, forward-mode tangents and function transforms are refused whether or not a gradient is
+    recorded, and operand combinations that do not add up are refused before any launch."""
+    import torch.autograd.forward_ad as fwAD
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from sample_efficient_gpt_amd import _lib
+
+    x = gen(1, 6, 2, 96, 96, 64, BF16, seed=52)
+    dev = {n: x[n].to(gpu_device) for n in ("q", "k", "v", "g_q", "d_o")}
+    call = lambda **kw: qknorm_attention(*(kw.get(n, dev[n]) for n in ("q", "k", "v", "g_q")))
+
+    class Drops(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            return t.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    q = dev["q"].clone().requires_grad_(True)
+    g = torch.autograd.grad(Drops.apply(call(q=q)), q, dev["d_o"])[0]
+    assert g.shape == q.shape and g.abs().max() == 0
+
+    odd = torch.empty(q.numel() + 1, dtype=BF16, device=gpu_device)[1:].view(q.shape)  # rows that are not 16-byte aligned
+    with pytest.raises(_lib.SegptError, match="segpt_attn_bwd"):
+        torch.autograd.grad(call(q=q), q, odd)
+
+    class Stop(Exception):
+        pass
+
+    def refuse(t):
+        raise Stop("hook")
+
+    with pytest.raises(Stop), torch.autograd.graph.saved_tensors_hooks(refuse, lambda t: t):
+        call(q=q)
+
+    for qq in (q, dev["q"]):
+        with fwAD.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+            call(q=fwAD.make_dual(qq, torch.ones_like(qq)))
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda t: call(q=t))(dev["q"][None])
+
+    seen = []
+
+    class Look(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad(), Look():
+        y = qknorm_attention_op(dev["q"], dev["k"], dev["v"], dev["g_q"])
+    assert torch.ops.segpt.qknorm_attention.default in seen and torch.equal(y, call())
+
+    Q, K = (t.transpose(0, 1).reshape(-1, 96, 64).contiguous() for t in (dev["q"], dev["k"]))
+    gate = torch.zeros(1, 96, 4, dtype=BF16, device=gpu_device)  # six rows are not a multiple of its four heads
+    with pytest.raises((AssertionError, RuntimeError)):
+        QKNormFlashAttnFunc.apply(Q, Q, Q, dev["g_q"], True, 0, None, None, None, gate)
+    with pytest.raises((AssertionError, RuntimeError, ValueError, IndexError)):
+        QKNormFlashAttnFunc.apply(Q[:2], K, K, dev["g_q"], True, 0, None, K[0], torch.ones(2, device=gpu_device), None, 2.0, 2)
+
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(1e-4)
+    try:
+        with pytest.raises(torch.OutOfMemoryError), torch.no_grad():
+            big = dev["q"].expand(400, -1, -1, -1)
+            qknorm_attention(big, dev["k"].expand(400, -1, -1, -1), dev["v"].expand(400, -1, -1, -1), dev["g_q"])
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
 
 
 # ------------------------------------------------------------------ rotary embedding fused into the loads
