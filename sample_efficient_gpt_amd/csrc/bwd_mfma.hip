@@ -24,6 +24,9 @@
 #include "ring_protocol.hpp"
 
 namespace segpt {
+
+int bf16_dkdv_grid(const segpt_attn_params& p);
+
 namespace {
 
 constexpr int kBwdRows = 4 * 32;  // rows (queries for dQ, keys for dK/dV) owned by a workgroup
@@ -31,6 +34,23 @@ constexpr int kBwdRows = 4 * 32;  // rows (queries for dQ, keys for dK/dV) owned
 // The dK/dV launch pins (batch, kv head) pairs to XCDs only when ALL of them can be pinned: with a spread remainder it
 // was measured 13 % slower at B*Hkv = 12, S = 8192 (where forward and dQ gain 2-4 % from pinning 8 of the 12).
 __host__ __device__ inline int dkdv_pinned(const segpt_attn_params& p) { return wg_pinned_pairs(p.B, p.Hkv, true); }
+
+// How the four waves of a dK/dV workgroup share a launch's work.  1: four key blocks (128 keys), every wave computes both
+// 32-query blocks of a streamed tile.  2: two key blocks (64 keys) times the two query blocks of the tile: twice as many
+// workgroups, each half as long, for twice the tile loads and barriers per matrix instruction.  What decides is whether
+// the launch is as long as its longest workgroup (the early key tiles stream every query of every head of the group) or
+// as its total work, i.e. how many 128-key workgroups there are for the 512 (head_dim 64, two per CU) or 256 (head_dim
+// 128) resident ones.  Measured, 1 against 2, us: head_dim 64, 18 / 6 heads, 1 x 2048 (96 workgroups) 100 / 63, 8 x 999 (384)
+// 71 / 57, 1 x 8192 (384) 430 / 318, 6 x 2048 (576) 132 / 126, 8 x 2048 (768) 156 / 160; head_dim 128, 16 / 4 heads,
+// 4 x 2048 (256) 226 / 151, 6 x 2048 (384) 235 / 237, 8 x 2048 (512) 272 / 302.  Between half full and full, short
+// workgroups (8 / 8 heads, 12 x 512, 8 tiles each: 17.1 / 17.6) have too little to halve: kLongTiles and more do (16 x 512,
+// 18 / 6 heads, 24 tiles: 34.8 / 32.2).
+inline int dkdv_parts(const segpt_attn_params& p) {
+  constexpr int kLongTiles = 24;
+  const int64_t wgs = (int64_t)p.B * p.Hkv * ((p.Sk + kBwdRows - 1) / kBwdRows);
+  const int64_t tiles = (int64_t)(p.H / p.Hkv) * ((p.Sq + kBK - 1) / kBK);
+  return wgs <= 256 || (p.D == 64 && wgs <= 512 && tiles >= kLongTiles) ? 2 : 1;
+}
 
 constexpr float kGateFactorFloor = 1e-30f;  // a smaller gate factor switches its row off in the dK/dV kernel
 
@@ -456,11 +476,14 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
 // ============================================================================================ dK, dV
 // Same pipeline with the roles swapped: the streamed tiles are Qhat / dO (64 queries of one head), the
 // blocks are 32 queries, and B(n) starts from the two row statistics of the block, read from LDS
-// straight into the accumulators of S and dP.
-template <int D, bool ROPE>
+// straight into the accumulators of S and dP.  PARTS: see dkdv_parts(); with 2 a wave computes one block of every tile
+// and the two waves of a key block add up their accumulators through LDS behind the loop.
+template <int D, bool ROPE, int PARTS>
 __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kernel(KArgs a) {
   using Z = Swz<D>;
-  constexpr int BKV = kBwdRows;
+  static_assert(PARTS == 1 || PARTS == 2, "a tile has two 32-query blocks");
+  constexpr int BKV = kBwdRows / PARTS;
+  constexpr int kKeyWaves = 4 / PARTS;  // waves side by side along the keys
   constexpr int KS = D / 16;
   constexpr int MB = D / 32;
   constexpr int kStageBytes = 2 * Z::kTileBytes;
@@ -494,7 +517,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   wg.tile = n_kvt - 1 - wg.tile;  // early key tiles see the most queries: issue them first
   const int b = wg.b, g = wg.g;
   const int k0 = wg.tile * BKV;
-  const int kw0 = k0 + wave * 32;
+  const int key_wave = wave % kKeyWaves, part = wave / kKeyWaves;
+  const int kw0 = k0 + key_wave * 32;
   const int key = kw0 + ln;
   const int key_c = min(key, p.Sk - 1);
 
@@ -562,26 +586,31 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
     if (t < n_it) issue_next();
   constexpr int kRowStage = R.row_stage_first;  // Khat block in stage kRowStage, V' block in the next
   {
-    const int rows_left = p.Sk - k0;
+    const int rows_left = min(p.Sk - k0, BKV);
     const int64_t krow = ((int64_t)b * p.Hkv + g) * p.Sk + k0;
     const char* kb = reinterpret_cast<const char*>(a.khat + krow * D);
     const char* vb = a.vmix ? reinterpret_cast<const char*>(a.vmix + krow * D) : reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v, b, g, k0));
     const uint32_t vstep = a.vmix ? (uint32_t)D * 2 : (uint32_t)p.v.stride_s * 2;
     const uint32_t wave_dst = lds0 + wave * 1024;
-    issue_tile_pair<D>(kb, kb, rowblock_lane_offsets<D>(D * 2, 0, rows_left, src.x, src.y), wave_dst + kRowStage * kStageBytes);
-    issue_tile_pair<D>(vb, vb, rowblock_lane_offsets<D>(vstep, 0, rows_left, src.x, src.y), wave_dst + (kRowStage + 1) * kStageBytes);
+    if constexpr (PARTS == 1) {
+      issue_tile_pair<D>(kb, kb, rowblock_lane_offsets<D>(D * 2, 0, rows_left, src.x, src.y), wave_dst + kRowStage * kStageBytes);
+      issue_tile_pair<D>(vb, vb, rowblock_lane_offsets<D>(vstep, 0, rows_left, src.x, src.y), wave_dst + (kRowStage + 1) * kStageBytes);
+    } else {  // 64 rows each: the two tiles of one stage
+      issue_tile_pair<D>(kb, vb, tile_lane_offsets<D>(D * 2, vstep, rows_left, src.x, src.y), wave_dst + kRowStage * kStageBytes);
+    }
   }
   wait_vmcnt<0>();
   __syncthreads();
-  // stationary B operands: Khat and V' rows of this lane's key (rows 32*wave .. +31 of the block)
+  // stationary B operands: Khat and V' rows of this lane's key (rows 32*key_wave .. +31 of the block)
   bf16x8 kreg[KS], vreg[KS];
   {
-    const uint32_t rm = lds0 + (wave >> 1) * Z::kTileBytes + swz_off_rm<D>(lane);
-    const int rb = wave & 1;
+    const uint32_t rm = lds0 + kRowStage * kStageBytes + (key_wave >> 1) * Z::kTileBytes + swz_off_rm<D>(lane);
+    const int rb = key_wave & 1;
+    constexpr int kVRows = PARTS == 1 ? kStageBytes : Z::kTileBytes;  // where the V' rows lie behind the Khat rows
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      kreg[ks] = swz_frag_rm<D>(rm + kRowStage * kStageBytes, rb, ks);
-      vreg[ks] = swz_frag_rm<D>(rm + (kRowStage + 1) * kStageBytes, rb, ks);
+      kreg[ks] = swz_frag_rm<D>(rm, rb, ks);
+      vreg[ks] = swz_frag_rm<D>(rm + kVRows, rb, ks);
     }
   }
   __syncthreads();  // the borrowed stages are free again
@@ -592,9 +621,10 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) { dvacc[mb] = splat16(0.f); dkacc[mb] = splat16(0.f); }
 
-  const uint32_t rm_lane = lds0 + swz_off_rm<D>(lane);
-  const uint32_t tr_lane = lds0 + swz_off_tr<D>(lane);
-  const uint32_t st_lane = ldl0 + 16 * hh;
+  // PARTS == 2: this wave's block of every tile is number `part` (a multiple of 4 KB further: the XOR terms stay below)
+  const uint32_t rm_lane = lds0 + swz_off_rm<D>(lane) + part * 32 * Z::kRB;
+  const uint32_t tr_lane = lds0 + swz_off_tr<D>(lane) + part * 32 * Z::kRB;
+  const uint32_t st_lane = ldl0 + 16 * hh + part * 32 * 4;
 
   bf16x8 qf[KS], df[KS];
   auto request_rowmajor = [&](uint32_t rm, int qb) {  // qb is a compile-time constant at every call site
@@ -685,9 +715,15 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
       const uint32_t st = st_lane + stage * 512;
       // on the diagonal a block whose last query still lies before this wave's first key is masked entirely:
       // it only passes the fragment request on (wave-uniform, so the barrier below is reached all the same)
-      if (MASK == 1 && kw0 > i0 + 31 + p.q_start) request_rowmajor(rm, 1); else step(masked_c, tr, st, 0, i0, rm, 1);
-      if (MASK == 1 && kw0 > i0 + 63 + p.q_start) request_rowmajor(rm_lane + nstage * kStageBytes, 0);
-      else step(masked_c, tr, st, 1, i0 + 32, rm_lane + nstage * kStageBytes, 0);
+      if constexpr (PARTS == 1) {
+        if (MASK == 1 && kw0 > i0 + 31 + p.q_start) request_rowmajor(rm, 1); else step(masked_c, tr, st, 0, i0, rm, 1);
+        if (MASK == 1 && kw0 > i0 + 63 + p.q_start) request_rowmajor(rm_lane + nstage * kStageBytes, 0);
+        else step(masked_c, tr, st, 1, i0 + 32, rm_lane + nstage * kStageBytes, 0);
+      } else {
+        const int ib = i0 + 32 * part;
+        if (MASK == 1 && kw0 > ib + 31 + p.q_start) request_rowmajor(rm_lane + nstage * kStageBytes, 0);
+        else step(masked_c, tr, st, 0, ib, rm_lane + nstage * kStageBytes, 0);
+      }
       if (it + R.issue_ahead < n_it) { issue_next(); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
       __syncthreads();
       stage = nstage;
@@ -712,20 +748,51 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   if (p.vr_coef) { c1 = p.vr_coef[0]; c2 = p.vr_coef[1]; }
   u32x2 kraw[MB][4], vraw[MB][4], fraw[MB][4];
   {
-    const int rows_left = p.Sk - k0;
+    const int rows_left = min(p.Sk - k0, BKV);
     const uint32_t wave_dst = lds0 + wave * 1024;
     const char* kb = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.k, b, g, k0));
-    issue_tile_pair<D>(kb, kb, rowblock_lane_offsets<D>((uint32_t)p.k.stride_s * 2, 0, rows_left, src.x, src.y), wave_dst);
-    if (p.vr_coef) {
-      const char* vb = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v, b, g, k0));
-      const char* fb = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v_first, b, g, k0));
-      issue_tile_pair<D>(vb, vb, rowblock_lane_offsets<D>((uint32_t)p.v.stride_s * 2, 0, rows_left, src.x, src.y), wave_dst + kStageBytes);
-      issue_tile_pair<D>(fb, fb, rowblock_lane_offsets<D>((uint32_t)p.v_first.stride_s * 2, 0, rows_left, src.x, src.y), wave_dst + 2 * kStageBytes);
+    const char* vb = p.vr_coef ? reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v, b, g, k0)) : kb;
+    const char* fb = p.vr_coef ? reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v_first, b, g, k0)) : kb;
+    const uint32_t kst = (uint32_t)p.k.stride_s * 2, vst = p.vr_coef ? (uint32_t)p.v.stride_s * 2 : kst, fst = (uint32_t)p.v_first.stride_s * 2;
+    if constexpr (PARTS == 1) {
+      issue_tile_pair<D>(kb, kb, rowblock_lane_offsets<D>(kst, 0, rows_left, src.x, src.y), wave_dst);
+      if (p.vr_coef) {
+        issue_tile_pair<D>(vb, vb, rowblock_lane_offsets<D>(vst, 0, rows_left, src.x, src.y), wave_dst + kStageBytes);
+        issue_tile_pair<D>(fb, fb, rowblock_lane_offsets<D>(fst, 0, rows_left, src.x, src.y), wave_dst + 2 * kStageBytes);
+      }
+    } else {  // 64 rows each: the two tiles of stage 0 and the first of stage 1
+      issue_tile_pair<D>(kb, vb, tile_lane_offsets<D>(kst, vst, rows_left, src.x, src.y), wave_dst);
+      if (p.vr_coef) issue_tile_pair<D>(fb, fb, tile_lane_offsets<D>(fst, fst, rows_left, src.x, src.y), wave_dst + kStageBytes);
+      // The two parts of a key block meet here: part 0 finishes dK, part 1 dV, so each hands the other's half over
+      // through the idle stages 2 and 3 (one slot per wave, 16 bytes per lane and access: conflict-free).
+      static_assert(4 * MB * 4096 <= 2 * kStageBytes, "one accumulator per wave in two stages");
+      char* const slot = lds + 2 * kStageBytes + lane * 16;
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          f32x4 t;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) t[i] = part == 0 ? dvacc[mb][4 * c + i] : dkacc[mb][4 * c + i];
+          *reinterpret_cast<f32x4*>(slot + wave * (MB * 4096) + (4 * mb + c) * 1024) = t;
+        }
     }
     wait_vmcnt<0>();
     __syncthreads();
-    // rows 32*wave .. +31 of a block: half (wave >> 1) of its stage, row block (wave & 1) of that tile
-    const uint32_t ct = lds0 + (wave >> 1) * Z::kTileBytes + swz_off_ct<D>(lane) + (wave & 1) * 32 * Z::kRB;
+    if constexpr (PARTS == 2) {
+      const char* const other = lds + 2 * kStageBytes + lane * 16 + (wave ^ kKeyWaves) * (MB * 4096);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const f32x4 t = *reinterpret_cast<const f32x4*>(other + (4 * mb + c) * 1024);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) { dvacc[mb][4 * c + i] += t[i]; dkacc[mb][4 * c + i] += t[i]; }  // each uses its own one only
+        }
+    }
+    // rows 32*key_wave .. +31 of a block: half (key_wave >> 1) of its stage, row block (key_wave & 1) of that tile
+    constexpr int kVRows = PARTS == 1 ? kStageBytes : Z::kTileBytes, kFRows = PARTS == 1 ? 2 * kStageBytes : kStageBytes;
+    const uint32_t ct = lds0 + (key_wave >> 1) * Z::kTileBytes + swz_off_ct<D>(lane) + (key_wave & 1) * 32 * Z::kRB;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -733,8 +800,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
         const uint32_t off = (uint32_t)((4 * mb + c) << 4);
         kraw[mb][c] = lds_read8(ct ^ off);
         if (p.vr_coef) {
-          vraw[mb][c] = lds_read8((ct + kStageBytes) ^ off);
-          fraw[mb][c] = lds_read8((ct + 2 * kStageBytes) ^ off);
+          vraw[mb][c] = lds_read8((ct + kVRows) ^ off);
+          fraw[mb][c] = lds_read8((ct + kFRows) ^ off);
         }
       }
   }
@@ -743,7 +810,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
     const int64_t pos = (int64_t)(p.rope_k_pos0 + key_c) * (D / 2);
     rope_ct = rope_ct_load<MB>(p.rope_cos + pos, p.rope_sin + pos, hh);
   }
-  {
+  const bool own_dk = PARTS == 1 || part == 0, own_dv = PARTS == 1 || part == 1;
+  if (own_dv) {
     uint16_t* ovp = row_ptr_mut<uint16_t>(p.dv, b, g, key_c);
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
@@ -755,18 +823,20 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   }
   if (p.vr_coef) {
     float s1 = 0.f, s2 = 0.f;
-    uint16_t* ofp = row_ptr_mut<uint16_t>(p.dv_first, b, g, key_c);
+    if (own_dv) {
+      uint16_t* ofp = row_ptr_mut<uint16_t>(p.dv_first, b, g, key_c);
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      float val[16], vv[16], ff[16];
+      for (int mb = 0; mb < MB; ++mb) {
+        float val[16], vv[16], ff[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) val[r] = c2 * dvacc[mb][r];
-      store_ct_block(ofp, mb, hh, live, val);
-      unpack_ct_block(vraw[mb], vv);
-      unpack_ct_block(fraw[mb], ff);
+        for (int r = 0; r < 16; ++r) val[r] = c2 * dvacc[mb][r];
+        store_ct_block(ofp, mb, hh, live, val);
+        unpack_ct_block(vraw[mb], vv);
+        unpack_ct_block(fraw[mb], ff);
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (live) { s1 += dvacc[mb][r] * vv[r]; s2 += dvacc[mb][r] * ff[r]; }
+        for (int r = 0; r < 16; ++r)
+          if (live) { s1 += dvacc[mb][r] * vv[r]; s2 += dvacc[mb][r] * ff[r]; }
+      }
     }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) { s1 += __shfl_xor(s1, o, 64); s2 += __shfl_xor(s2, o, 64); }
@@ -775,7 +845,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
     if (tid < 2) a.dcoef_part[(int64_t)bid * 2 + tid] = red[tid] + red[2 + tid] + red[4 + tid] + red[6 + tid];
   }
   // dk through the normaliser: W = ln2 * dkacc = dL/dKhat (natural units), dk = b W - (b^3/D)(W.k) k
-  {
+  if (own_dk) {
     float kv[MB][16];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) unpack_ct_block(kraw[mb], kv[mb]);
@@ -805,10 +875,14 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
 template <int D>
 int launch_dkdv_t(const KArgs& a, hipStream_t st) {
   const segpt_attn_params& p = a.p;
-  const int n_kvt = (p.Sk + kBwdRows - 1) / kBwdRows;
-  const dim3 grid((unsigned)(wg_grid(n_kvt, p.B, p.Hkv, 1, dkdv_pinned(p)) + 1));
-  if (p.rope_cos) hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, true>), grid, dim3(kThreadsM), 0, st, a);
-  else hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, false>), grid, dim3(kThreadsM), 0, st, a);
+  const dim3 grid((unsigned)(bf16_dkdv_grid(p) + 1));
+  if (dkdv_parts(p) == 1) {
+    if (p.rope_cos) hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, true, 1>), grid, dim3(kThreadsM), 0, st, a);
+    else hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, false, 1>), grid, dim3(kThreadsM), 0, st, a);
+  } else {
+    if (p.rope_cos) hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, true, 2>), grid, dim3(kThreadsM), 0, st, a);
+    else hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, false, 2>), grid, dim3(kThreadsM), 0, st, a);
+  }
   return (int)hipGetLastError();
 }
 
@@ -827,7 +901,10 @@ int launch_dq_t(const KArgs& a, hipStream_t st) {
 // workgroups of the two launches (the dK/dV launch has one more, its extra reducing workgroup): the workspace holds one
 // row of partial sums per workgroup, idle padding workgroups included
 int bf16_dq_grid(const segpt_attn_params& p) { return wg_grid((p.Sq + kBwdRows - 1) / kBwdRows, p.B, p.Hkv, p.H / p.Hkv, wg_pinned_pairs(p.B, p.Hkv, false)); }
-int bf16_dkdv_grid(const segpt_attn_params& p) { return wg_grid((p.Sk + kBwdRows - 1) / kBwdRows, p.B, p.Hkv, 1, dkdv_pinned(p)); }
+int bf16_dkdv_grid(const segpt_attn_params& p) {
+  const int rows = kBwdRows / dkdv_parts(p);
+  return wg_grid((p.Sk + rows - 1) / rows, p.B, p.Hkv, 1, dkdv_pinned(p));
+}
 
 int launch_bwd_dkdv_bf16(const KArgs& a, hipStream_t st) {
   if (a.p.D == 64) return launch_dkdv_t<64>(a, st);

@@ -163,6 +163,20 @@ def test_bf16_gate_factor_through_the_row_statistics(gpu_device, D):
         assert torch.isfinite(t.float()).all(), n
 
 
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,kw", [
+    (1, 3, 1, 33, 65, 64, {"q_start": 32}),                # one key in the last workgroup, second key wave beyond the end
+    (2, 3, 1, 161, 97, 64, {"causal": False}),             # three key blocks: the last workgroup holds one
+    (2, 2, 1, 64, 290, 128, {"q_start": 226}),             # the last 64-key tile is 34 rows
+    (4, 64, 64, 96, 200, 64, {"q_start": 104}),            # 512 128-key workgroups, short: not split
+    (3, 86, 86, 70, 190, 64, {"causal": False}),           # more than 512
+    (2, 65, 65, 130, 250, 128, {"q_start": 120}),          # head_dim 128, just more than 256: not split
+])
+def test_bf16_dkdv_workgroup_shapes(gpu_device, B, H, Hkv, Sq, Sk, D, kw):
+    """dK/dV with 64-key workgroups whose waves split the queries (launches that do not fill the card) and with 128-key
+    ones, at the ragged ends of both, with gate, value residual and rotary embedding."""
+    _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, D, seed=61, gen_kw={"extras": True}, rope=orc.rope_tables(max(Sq, Sk), 10000.0, D), **kw)
+
+
 def test_bf16_gate_scale_not_positive_takes_the_gated_copy(gpu_device):
     """A gate scale <= 0 has no logarithm: the dQ kernel then leaves a gate-scaled copy of dO for the dK/dV kernel
     (the workspace grows by that tensor)."""
