@@ -25,6 +25,7 @@
 
 namespace segpt {
 
+int bf16_dq_grid(const segpt_attn_params& p);
 int bf16_dkdv_grid(const segpt_attn_params& p);
 
 namespace {
@@ -52,6 +53,17 @@ inline int dkdv_parts(const segpt_attn_params& p) {
   return wgs <= 256 || (p.D == 64 && wgs <= 512 && tiles >= kLongTiles) ? 2 : 1;
 }
 
+// The same for the query rows of a dQ workgroup: 1: 128 rows, 2: 64 rows times the two 32-key blocks of a tile.  Both waves of
+// a pair compute the row prologue (normaliser, Qhat, delta), so 2 costs more here and ends earlier.  Measured, 1 against 2,
+// us: head_dim 64, 18 / 6 heads, 2 x 512 (144 workgroups) 12.1 / 10.3, 4 x 512 (288) 13.9 / 16.2, 1 x 2048 (288) 32.3 / 25.1;
+// 16 / 4 heads, 4 x 512 (256) 13.2 / 11.5, 3 x 1024 (384) 21.9 / 21.9, 1 x 4096 (512) 67 / 66; head_dim 128, 2 x 512 (128) 19.6 /
+// 16.4, 3 x 512 (192) 21.0 / 23.1, 2 x 1024 (256) 31.4 / 32.3.
+inline int dq_parts(const segpt_attn_params& p) {
+  constexpr int kLongTiles = 16;
+  const int64_t wgs = (int64_t)p.B * p.H * ((p.Sq + kBwdRows - 1) / kBwdRows), tiles = (p.Sk + kBK - 1) / kBK;
+  return wgs <= (p.D == 128 ? 128 : tiles >= kLongTiles ? 384 : 256) ? 2 : 1;
+}
+
 constexpr float kGateFactorFloor = 1e-30f;  // a smaller gate factor switches its row off in the dK/dV kernel
 
 constexpr int kStages = 4;  // LDS ring of streamed stages (two tiles each): tile t lives in stage t % 4
@@ -70,10 +82,15 @@ constexpr int kStages = 4;  // LDS ring of streamed stages (two tiles each): til
 // ROPE (rope tables given) is a compile-time switch so that the table rows are ordinary, unconditional loads which
 // travel with the start-up tiles (prologue) and with the first stores (epilogue) instead of costing a memory round
 // trip of their own behind a branch.
-template <int D, bool ROPE>
+//
+// PARTS: see dq_parts(); with 2 the workgroup owns 64 query rows, two waves each take one of the two 32-key blocks of
+// every tile for the same rows, and the pair adds up T^T through LDS behind the loop.
+template <int D, bool ROPE, int PARTS>
 __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel(KArgs a) {
   using Z = Swz<D>;
-  constexpr int BQ = kBwdRows;
+  static_assert(PARTS == 1 || PARTS == 2, "a tile has two 32-key blocks");
+  constexpr int BQ = kBwdRows / PARTS;
+  constexpr int kRowWaves = 4 / PARTS;  // waves side by side along the query rows
   constexpr int KS = D / 16;
   constexpr int MB = D / 32;
   constexpr int kStageBytes = 2 * Z::kTileBytes;
@@ -104,7 +121,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   }
   const int b = wg.b, g = wg.g, h = wg.g * rep + wg.hh;
   const int q0 = wg.tile * BQ;
-  const int qw0 = q0 + wave * 32;
+  const int row_wave = PARTS == 1 ? wave : wave % kRowWaves, part = PARTS == 1 ? 0 : wave / kRowWaves;
+  const int qw0 = q0 + row_wave * 32;
   const int row = qw0 + ln;
   const bool live = row < p.Sq;
   const int row_c = live ? row : p.Sq - 1;  // padding lanes recompute the last row and store nothing
@@ -149,30 +167,46 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   constexpr int kQStage = ROPE ? 0 : kRowStage, kCosStage = 1, kSinStage = 2;
   constexpr int kDoStage = ROPE ? 3 : kRowStage + 1, kOStage = ROPE ? kRowStage : kRowStage + 2;
   static_assert(!ROPE || kOStage == 3, "first phase: q, cos, sin, dO; second phase: tiles 0..2, o");
-  const int rows_left = p.Sq - q0;
+  // where the row blocks lie.  PARTS == 2: blocks of 64 rows, two of them are the two tiles of one stage
+  constexpr uint32_t kPair = Z::kTileBytes;
+  constexpr uint32_t kQRows = kQStage * kStageBytes, kDoRows = PARTS == 1 ? kDoStage * kStageBytes : kQRows + kPair;
+  constexpr uint32_t kCosRows = kCosStage * kStageBytes, kSinRows = PARTS == 1 ? kSinStage * kStageBytes : kCosRows + kPair;
+  constexpr uint32_t kORows = kOStage * kStageBytes;
+  const int rows_left = min(p.Sq - q0, BQ);
   const char* qb = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.q, b, h, q0));
   const char* db = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.d_o, b, h, q0));
   const char* yb = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.o, b, h, q0));
   const int64_t rope_row0 = ROPE ? (int64_t)(p.rope_q_pos0 + q0) * (D / 2) : 0;  // the tables' row of query q0
-  auto issue_rope_rows = [&](int cos_stage, int sin_stage) {  // 128 table rows each, laid out like tensor rows
-    const TileLaneOff<D> o = rowblock_lane_offsets<D>(D * 2, 0, rows_left, src.x, src.y);
+  const uint32_t qst = (uint32_t)p.q.stride_s * 2, dst = (uint32_t)p.d_o.stride_s * 2, yst = (uint32_t)p.o.stride_s * 2;
+  auto issue_rope_rows = [&](uint32_t cos_at, uint32_t sin_at) {  // BQ table rows each, laid out like tensor rows
     const char* cb = reinterpret_cast<const char*>(p.rope_cos + rope_row0);
     const char* sb = reinterpret_cast<const char*>(p.rope_sin + rope_row0);
-    issue_tile_pair<D>(cb, cb, o, wave_dst + cos_stage * kStageBytes);
-    issue_tile_pair<D>(sb, sb, o, wave_dst + sin_stage * kStageBytes);
+    if constexpr (PARTS == 1) {
+      const TileLaneOff<D> o = rowblock_lane_offsets<D>(D * 2, 0, rows_left, src.x, src.y);
+      issue_tile_pair<D>(cb, cb, o, wave_dst + cos_at);
+      issue_tile_pair<D>(sb, sb, o, wave_dst + sin_at);
+    } else {
+      issue_tile_pair<D>(cb, sb, tile_lane_offsets<D>(D * 2, D * 2, rows_left, src.x, src.y), wave_dst + cos_at);
+    }
   };
-  if constexpr (ROPE) {
-    issue_tile_pair<D>(qb, qb, rowblock_lane_offsets<D>((uint32_t)p.q.stride_s * 2, 0, rows_left, src.x, src.y), wave_dst + kQStage * kStageBytes);
-    issue_rope_rows(kCosStage, kSinStage);
-    issue_tile_pair<D>(db, db, rowblock_lane_offsets<D>((uint32_t)p.d_o.stride_s * 2, 0, rows_left, src.x, src.y), wave_dst + kDoStage * kStageBytes);
-  } else {
+  auto issue_o_rows = [&]() {
+    if constexpr (PARTS == 1) issue_tile_pair<D>(yb, yb, rowblock_lane_offsets<D>(yst, 0, rows_left, src.x, src.y), wave_dst + kORows);
+    else issue_tile_pair<D>(yb, yb, tile_lane_offsets<D>(yst, yst, rows_left, src.x, src.y), wave_dst + kORows);
+  };
+  if constexpr (!ROPE) {
 #pragma unroll
     for (int t = 0; t < R.early_tiles; ++t)
       if (t < n_kt) issue_tile(t);
-    issue_tile_pair<D>(qb, qb, rowblock_lane_offsets<D>((uint32_t)p.q.stride_s * 2, 0, rows_left, src.x, src.y), wave_dst + kQStage * kStageBytes);
-    issue_tile_pair<D>(db, db, rowblock_lane_offsets<D>((uint32_t)p.d_o.stride_s * 2, 0, rows_left, src.x, src.y), wave_dst + kDoStage * kStageBytes);
-    issue_tile_pair<D>(yb, yb, rowblock_lane_offsets<D>((uint32_t)p.o.stride_s * 2, 0, rows_left, src.x, src.y), wave_dst + kOStage * kStageBytes);
   }
+  if constexpr (PARTS == 1) {
+    issue_tile_pair<D>(qb, qb, rowblock_lane_offsets<D>(qst, 0, rows_left, src.x, src.y), wave_dst + kQRows);
+    if constexpr (ROPE) issue_rope_rows(kCosRows, kSinRows);
+    issue_tile_pair<D>(db, db, rowblock_lane_offsets<D>(dst, 0, rows_left, src.x, src.y), wave_dst + kDoRows);
+  } else {
+    issue_tile_pair<D>(qb, db, tile_lane_offsets<D>(qst, dst, rows_left, src.x, src.y), wave_dst + kQRows);
+    if constexpr (ROPE) issue_rope_rows(kCosRows, kSinRows);
+  }
+  if constexpr (!ROPE) issue_o_rows();
   const float lse_row = p.lse[ridx];
   // the conditional reads last: the compiler waits for every outstanding load where their branches join
   float gate_z = 0.f;
@@ -183,30 +217,30 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   if (tid < D) gsm[tid] = gval;
   wait_vmcnt<0>();
   __syncthreads();
-  // rows 32*wave .. 32*wave+31 of the block: half (wave >> 1) of each stage, row block (wave & 1) of that tile
+  // rows 32*row_wave .. +31 of a block: half (row_wave >> 1) of it, row block (row_wave & 1) of that tile
   u32x4 qraw[KS], dyraw[KS], yraw[KS];
   u32x2 qct[MB][4];  // the query row once more, in the layout of the epilogue's C tiles (packed pairs)
   RopeB<KS> rope_b;
-  const uint32_t row_half = (wave >> 1) * Z::kTileBytes, row_rb = wave & 1;
+  const uint32_t row_half = (row_wave >> 1) * Z::kTileBytes, row_rb = row_wave & 1;
   const uint32_t row_rm = lds0 + row_half + swz_off_rm<D>(lane);
   const uint32_t row16 = lds0 + row_half + swz_off_row16<D>(lane) + row_rb * 32 * Z::kRB;  // chunk 0 of the lane's row
   {
-    const uint32_t ct = lds0 + kQStage * kStageBytes + row_half + swz_off_ct<D>(lane) + row_rb * 32 * Z::kRB;
+    const uint32_t ct = lds0 + kQRows + row_half + swz_off_ct<D>(lane) + row_rb * 32 * Z::kRB;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      qraw[ks] = __builtin_bit_cast(u32x4, swz_frag_rm<D>(row_rm + kQStage * kStageBytes, row_rb, ks));
-      dyraw[ks] = __builtin_bit_cast(u32x4, swz_frag_rm<D>(row_rm + kDoStage * kStageBytes, row_rb, ks));
-      if constexpr (!ROPE) yraw[ks] = __builtin_bit_cast(u32x4, swz_frag_rm<D>(row_rm + kOStage * kStageBytes, row_rb, ks));
+      qraw[ks] = __builtin_bit_cast(u32x4, swz_frag_rm<D>(row_rm + kQRows, row_rb, ks));
+      dyraw[ks] = __builtin_bit_cast(u32x4, swz_frag_rm<D>(row_rm + kDoRows, row_rb, ks));
+      if constexpr (!ROPE) yraw[ks] = __builtin_bit_cast(u32x4, swz_frag_rm<D>(row_rm + kORows, row_rb, ks));
     }
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int c = 0; c < 4; ++c) qct[mb][c] = lds_read8(ct ^ (uint32_t)((4 * mb + c) << 4));
-    if constexpr (ROPE) rope_b = rope_b_from_lds<KS>(row16 + kCosStage * kStageBytes, row16 + kSinStage * kStageBytes, hh);
+    if constexpr (ROPE) rope_b = rope_b_from_lds<KS>(row16 + kCosRows, row16 + kSinRows, hh);
   }
   __syncthreads();  // the borrowed stages are free again
   if constexpr (ROPE) {
-    issue_tile_pair<D>(yb, yb, rowblock_lane_offsets<D>((uint32_t)p.o.stride_s * 2, 0, rows_left, src.x, src.y), wave_dst + kOStage * kStageBytes);
+    issue_o_rows();
 #pragma unroll
     for (int t = 0; t < R.early_tiles; ++t)
       if (t < n_kt) issue_tile(t);
@@ -264,7 +298,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     wait_vmcnt<0>();
     __syncthreads();
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) yraw[ks] = __builtin_bit_cast(u32x4, swz_frag_rm<D>(row_rm + kOStage * kStageBytes, row_rb, ks));
+    for (int ks = 0; ks < KS; ++ks) yraw[ks] = __builtin_bit_cast(u32x4, swz_frag_rm<D>(row_rm + kORows, row_rb, ks));
     row_dot();
     __syncthreads();
   }
@@ -283,8 +317,9 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   if (p.causal) n_act = min(n_act, (qw0 + 31 + p.q_start) / 32 + 1);
   const int qlim = p.causal ? min(row + p.q_start, p.Sk - 1) : p.Sk - 1;  // last visible key of this lane's query
 
-  const uint32_t rm_lane = lds0 + swz_off_rm<D>(lane);
-  const uint32_t tr_lane = lds0 + swz_off_tr<D>(lane);
+  // PARTS == 2: this wave's block of every tile is number `part` (a multiple of 4 KB further: the XOR terms stay below)
+  const uint32_t rm_lane = lds0 + swz_off_rm<D>(lane) + part * 32 * Z::kRB;
+  const uint32_t tr_lane = lds0 + swz_off_tr<D>(lane) + part * 32 * Z::kRB;
   bf16x8 kf[KS], vf[KS];
   auto request_rowmajor = [&](uint32_t rm, int kb) {  // kb compile-time at every call site
 #pragma unroll
@@ -354,13 +389,17 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   if (p.causal) n_full = min(n_full, (qw0 + p.q_start + 1) / 32);
   // Loop A: tiles whose two blocks need no mask; loop B: the rest (masking a fully visible block is a no-op).
   // Two loops, so that each body holds one variant of the block and the accumulators never meet at a join.
-  const int n_a = n_full / 2;  // n_full <= n_act
+  const int n_a = PARTS == 1 ? n_full / 2 : (n_full + 1 - part) / 2;  // n_full <= n_act
   int stage = 0, jt = 0;
   for (; jt < n_a; ++jt) {
     const int nstage = stage == kStages - 1 ? 0 : stage + 1;
     const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
-    step(IC<0>{}, tr, 0, 64 * jt, rm, 1);
-    step(IC<0>{}, tr, 1, 64 * jt + 32, rm_lane + nstage * kStageBytes, 0);
+    if constexpr (PARTS == 1) {
+      step(IC<0>{}, tr, 0, 64 * jt, rm, 1);
+      step(IC<0>{}, tr, 1, 64 * jt + 32, rm_lane + nstage * kStageBytes, 0);
+    } else {
+      step(IC<0>{}, tr, 0, 64 * jt + 32 * part, rm_lane + nstage * kStageBytes, 0);
+    }
     // stage (jt+3) % 4 == (jt-1) % 4 was last read in the previous iteration: refill it, then make sure
     // this wave's part of tile jt+2 (needed from the next iteration's prefetch on) has landed
     if (jt + R.issue_ahead < n_kt) { issue_tile(jt + R.issue_ahead); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
@@ -370,8 +409,12 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   for (; jt < n_kt; ++jt) {
     const int nstage = stage == kStages - 1 ? 0 : stage + 1;
     const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
-    if (2 * jt < n_act) step(IC<1>{}, tr, 0, 64 * jt, rm, 1);
-    if (2 * jt + 1 < n_act) step(IC<1>{}, tr, 1, 64 * jt + 32, rm_lane + nstage * kStageBytes, 0);
+    if constexpr (PARTS == 1) {
+      if (2 * jt < n_act) step(IC<1>{}, tr, 0, 64 * jt, rm, 1);
+      if (2 * jt + 1 < n_act) step(IC<1>{}, tr, 1, 64 * jt + 32, rm_lane + nstage * kStageBytes, 0);
+    } else {
+      if (2 * jt + part < n_act) step(IC<1>{}, tr, 0, 64 * jt + 32 * part, rm_lane + nstage * kStageBytes, 0);
+    }
     if (jt + R.issue_ahead < n_kt) { issue_tile(jt + R.issue_ahead); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
     __syncthreads();
     stage = nstage;
@@ -384,74 +427,101 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   // With a rotary embedding the table rows come in once more, into the idle ring (every wave has passed the last
   // iteration's barrier), now for the accumulators' layout; the second barrier keeps the scale-gradient staging
   // below, which reuses the ring, behind every wave's reads.
+  // PARTS == 2: part 1 leaves its T^T in the idle stage 2 (one slot per wave, 16 bytes per lane and access: conflict-free)
+  // and is done but for the column sums; part 0 adds it to its own.
+  char* const slot = lds + 2 * kStageBytes + row_wave * (MB * 4096) + lane * 16;
+  static_assert(PARTS == 1 || (kRowWaves * MB * 4096 <= 2 * kStageBytes && BQ * kRedStride * 4 <= 2 * kStageBytes), "slots behind the dg staging area");
+  if constexpr (PARTS == 2) {
+    if (part == 1) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          *reinterpret_cast<f32x4*>(slot + (4 * mb + c) * 1024) = f32x4{acc[mb][4 * c], acc[mb][4 * c + 1], acc[mb][4 * c + 2], acc[mb][4 * c + 3]};
+    }
+    if constexpr (!ROPE) __syncthreads();
+  }
   RopeCt<MB> rope_ct;
   if constexpr (ROPE) {
-    issue_rope_rows(0, 1);
+    constexpr uint32_t kSinAt = PARTS == 1 ? kStageBytes : kPair;
+    issue_rope_rows(0, kSinAt);
     wait_vmcnt<0>();
     __syncthreads();
-    rope_ct = rope_ct_from_lds<MB>(row16, row16 + kStageBytes, hh);
+    rope_ct = rope_ct_from_lds<MB>(row16, row16 + kSinAt, hh);
     __syncthreads();
   }
-  if (live) {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      *reinterpret_cast<bf16x8*>(a.qhat + ridx * D + 16 * ks + 8 * hh) = qreg[ks];
-      if (a.do_eff) *reinterpret_cast<bf16x8*>(reinterpret_cast<uint16_t*>(a.do_eff) + ridx * D + 16 * ks + 8 * hh) = doreg[ks];
-    }
-    if (hh == 0) {
-      float stat_d = -delta, stat_l = nlse2;
-      if (p.gate.ptr && !a.do_eff) {
-        const bool on = gfac > kGateFactorFloor;
-        stat_l = on ? nlse2 + __log2f(gfac) : -INFINITY;
-        stat_d = on ? -delta / gfac : 0.f;
-      }
-      a.delta[ridx] = stat_d;
-      a.nlse2[ridx] = stat_l;
-      if (p.gate.ptr)
-        reinterpret_cast<uint16_t*>(p.dgate.ptr)[(int64_t)b * p.dgate.stride_b + (int64_t)row * p.dgate.stride_s + (int64_t)h * p.dgate.stride_h] = f32_to_bf16(dgate_row);
-    }
-  }
-  // acc = T^T: lane = query, registers = head-dim entries.
-  float dot = 0.f;
   float* red = reinterpret_cast<float*>(lds);
-  // q in the C-tile layout (rotated like the operand was), then dq = a (u - (a^2/D)(u.q) q) in the rotated frame
-  // and back through the transpose of the rotation
-  float qv[MB][16];
+  if (PARTS == 1 || part == 0) {
+    if constexpr (PARTS == 2) {
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) unpack_ct_block(qct[mb], qv[mb]);
-  const float aq = live ? alpha : 0.f;  // padding rows add nothing to the scale gradient
-  if (ROPE) rope_ct_apply<MB, false>(qv, rope_ct);
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
+        for (int c = 0; c < 4; ++c) {
+          const f32x4 t = *reinterpret_cast<const f32x4*>(slot + (4 * mb + c) * 1024);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int d0 = 32 * mb + 8 * c + 4 * hh;
-      const float4 g4 = *reinterpret_cast<const float4*>(gsm + d0);
-      const float gv[4] = {g4.x, g4.y, g4.z, g4.w};
-      float dgc[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 4 * c + i;
-        const float t = acc[mb][r] * p.sm_scale;                 // sm_scale * T
-        dgc[i] = t * aq * qv[mb][r];                             // dg contribution of this row
-        acc[mb][r] = t * gv[i];                                  // u = dL/d(a q)
-        dot += acc[mb][r] * qv[mb][r];
-      }
-      *reinterpret_cast<float4*>(red + (wave * 32 + ln) * kRedStride + d0) = make_float4(dgc[0], dgc[1], dgc[2], dgc[3]);
+          for (int i = 0; i < 4; ++i) acc[mb][4 * c + i] += t[i];
+        }
     }
+    if (live) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        *reinterpret_cast<bf16x8*>(a.qhat + ridx * D + 16 * ks + 8 * hh) = qreg[ks];
+        if (a.do_eff) *reinterpret_cast<bf16x8*>(reinterpret_cast<uint16_t*>(a.do_eff) + ridx * D + 16 * ks + 8 * hh) = doreg[ks];
+      }
+      if (hh == 0) {
+        float stat_d = -delta, stat_l = nlse2;
+        if (p.gate.ptr && !a.do_eff) {
+          const bool on = gfac > kGateFactorFloor;
+          stat_l = on ? nlse2 + __log2f(gfac) : -INFINITY;
+          stat_d = on ? -delta / gfac : 0.f;
+        }
+        a.delta[ridx] = stat_d;
+        a.nlse2[ridx] = stat_l;
+        if (p.gate.ptr)
+          reinterpret_cast<uint16_t*>(p.dgate.ptr)[(int64_t)b * p.dgate.stride_b + (int64_t)row * p.dgate.stride_s + (int64_t)h * p.dgate.stride_h] = f32_to_bf16(dgate_row);
+      }
+    }
+    // acc = T^T: lane = query, registers = head-dim entries.
+    float dot = 0.f;
+    // q in the C-tile layout (rotated like the operand was), then dq = a (u - (a^2/D)(u.q) q) in the rotated frame
+    // and back through the transpose of the rotation
+    float qv[MB][16];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) unpack_ct_block(qct[mb], qv[mb]);
+    const float aq = live ? alpha : 0.f;  // padding rows add nothing to the scale gradient
+    if (ROPE) rope_ct_apply<MB, false>(qv, rope_ct);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int d0 = 32 * mb + 8 * c + 4 * hh;
+        const float4 g4 = *reinterpret_cast<const float4*>(gsm + d0);
+        const float gv[4] = {g4.x, g4.y, g4.z, g4.w};
+        float dgc[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 4 * c + i;
+          const float t = acc[mb][r] * p.sm_scale;                 // sm_scale * T
+          dgc[i] = t * aq * qv[mb][r];                             // dg contribution of this row
+          acc[mb][r] = t * gv[i];                                  // u = dL/d(a q)
+          dot += acc[mb][r] * qv[mb][r];
+        }
+        *reinterpret_cast<float4*>(red + (row_wave * 32 + ln) * kRedStride + d0) = make_float4(dgc[0], dgc[1], dgc[2], dgc[3]);
+      }
+    }
+    dot = half_sum(dot);
+    const float a3 = norm_grad_coef(p, alpha, 1.0f / D) * dot;
+    uint16_t* op = row_ptr_mut<uint16_t>(p.dq, b, h, row_c);
+    float val[MB][16];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) val[mb][r] = alpha * acc[mb][r] - a3 * qv[mb][r];
+    if (ROPE) rope_ct_apply<MB, true>(val, rope_ct);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) store_ct_block(op, mb, hh, live, val[mb]);
   }
-  dot = half_sum(dot);
-  const float a3 = norm_grad_coef(p, alpha, 1.0f / D) * dot;
-  uint16_t* op = row_ptr_mut<uint16_t>(p.dq, b, h, row_c);
-  float val[MB][16];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) val[mb][r] = alpha * acc[mb][r] - a3 * qv[mb][r];
-  if (ROPE) rope_ct_apply<MB, true>(val, rope_ct);
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) store_ct_block(op, mb, hh, live, val[mb]);
-  // workgroup partial of dg: column sums over the 128 (wave, lane%32) rows, in two levels so that all
+  // workgroup partial of dg: column sums over the BQ (wave, lane%32) rows, in two levels so that all
   // 256 threads share the LDS reads (fixed order: deterministic)
   __syncthreads();
   {
@@ -517,7 +587,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   wg.tile = n_kvt - 1 - wg.tile;  // early key tiles see the most queries: issue them first
   const int b = wg.b, g = wg.g;
   const int k0 = wg.tile * BKV;
-  const int key_wave = wave % kKeyWaves, part = wave / kKeyWaves;
+  const int key_wave = PARTS == 1 ? wave : wave % kKeyWaves, part = PARTS == 1 ? 0 : wave / kKeyWaves;
   const int kw0 = k0 + key_wave * 32;
   const int key = kw0 + ln;
   const int key_c = min(key, p.Sk - 1);
@@ -889,10 +959,14 @@ int launch_dkdv_t(const KArgs& a, hipStream_t st) {
 template <int D>
 int launch_dq_t(const KArgs& a, hipStream_t st) {
   const segpt_attn_params& p = a.p;
-  const int n_qt = (p.Sq + kBwdRows - 1) / kBwdRows;
-  const dim3 grid((unsigned)wg_grid(n_qt, p.B, p.Hkv, p.H / p.Hkv, wg_pinned_pairs(p.B, p.Hkv, false)));
-  if (p.rope_cos) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, true>), grid, dim3(kThreadsM), 0, st, a);
-  else hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false>), grid, dim3(kThreadsM), 0, st, a);
+  const dim3 grid((unsigned)bf16_dq_grid(p));
+  if (dq_parts(p) == 1) {
+    if (p.rope_cos) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, true, 1>), grid, dim3(kThreadsM), 0, st, a);
+    else hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 1>), grid, dim3(kThreadsM), 0, st, a);
+  } else {
+    if (p.rope_cos) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, true, 2>), grid, dim3(kThreadsM), 0, st, a);
+    else hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 2>), grid, dim3(kThreadsM), 0, st, a);
+  }
   return (int)hipGetLastError();
 }
 
@@ -900,7 +974,10 @@ int launch_dq_t(const KArgs& a, hipStream_t st) {
 
 // workgroups of the two launches (the dK/dV launch has one more, its extra reducing workgroup): the workspace holds one
 // row of partial sums per workgroup, idle padding workgroups included
-int bf16_dq_grid(const segpt_attn_params& p) { return wg_grid((p.Sq + kBwdRows - 1) / kBwdRows, p.B, p.Hkv, p.H / p.Hkv, wg_pinned_pairs(p.B, p.Hkv, false)); }
+int bf16_dq_grid(const segpt_attn_params& p) {
+  const int rows = kBwdRows / dq_parts(p);
+  return wg_grid((p.Sq + rows - 1) / rows, p.B, p.Hkv, p.H / p.Hkv, wg_pinned_pairs(p.B, p.Hkv, false));
+}
 int bf16_dkdv_grid(const segpt_attn_params& p) {
   const int rows = kBwdRows / dkdv_parts(p);
   return wg_grid((p.Sk + rows - 1) / rows, p.B, p.Hkv, 1, dkdv_pinned(p));
