@@ -34,13 +34,16 @@ namespace {
 // tile carries twice the MFMAs, so one block per tile keeps the ratio of barriers and tile loads to MFMAs), four stages
 // = 64 KB, two workgroups per CU.  With 64-key tiles the ring alone is 96 KB and a CU holds one workgroup, i.e. one
 // wave per SIMD with nothing to overlap its softmax phase with.
-template <int D, bool WIDE>
+// PARTS == 2 (see fwd_parts()): the workgroup owns 64 query rows, two waves each take one of the two 32-key blocks of
+// every 64-key tile for the same rows, and the pair merges its softmax states through LDS behind the loop.
+template <int D, bool WIDE, int PARTS = 1>
 struct FwdShape {
-  static constexpr int kNQB = (D == 64 && WIDE) ? 2 : 1;  // 32-query blocks per wave
-  static constexpr int kBK = D == 64 ? 64 : 32;           // keys per streamed tile
-  static constexpr int kStages = D == 64 ? (WIDE ? 4 : 3) : 4;
-  static constexpr int kOcc = D == 64 ? (WIDE ? 2 : 3) : 2;
-  static constexpr int kBQ = 4 * 32 * kNQB;
+  static constexpr int kNQB = (D == 64 && WIDE && PARTS == 1) ? 2 : 1;  // 32-query blocks per wave
+  static constexpr int kBK = D == 64 || PARTS == 2 ? 64 : 32;           // keys per streamed tile
+  static constexpr int kStages = PARTS == 2 ? 3 : (D == 64 ? (WIDE ? 4 : 3) : 4);
+  static constexpr int kOcc = PARTS == 2 ? (D == 64 ? 3 : 1) : (D == 64 ? (WIDE ? 2 : 3) : 2);
+  static constexpr int kRowWaves = 4 / PARTS;             // waves side by side along the query rows
+  static constexpr int kBQ = kRowWaves * 32 * kNQB;
   static constexpr int kStoreUnits = D / 64;              // partial results of a split launch, in 32 KB
 };
 
@@ -50,9 +53,11 @@ struct FwdShape {
 // SPLIT: workgroup (tile, head, batch; y = share s) takes only the key tiles [s, s + 1) * fwd_chunk of its query tile
 // and, unless that is all of them, leaves an unnormalised partial (reference m, sum l, O in fp32) for
 // fwd_merge_kernel; see fwd_split_plan() for when.
-template <int D, bool WIDE, bool ROPE, bool SPLIT>
-__global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16_kernel(KArgs a) {
-  using F = FwdShape<D, WIDE>;
+template <int D, bool WIDE, bool ROPE, bool SPLIT, int PARTS>
+__global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE, PARTS>::kOcc)) void fwd_bf16_kernel(KArgs a) {
+  using F = FwdShape<D, WIDE, PARTS>;
+  static_assert(PARTS == 1 || (PARTS == 2 && !SPLIT && F::kNQB == 1 && F::kBK == 64), "a tile has two 32-key blocks");
+  constexpr bool kMayMissKeys = SPLIT || PARTS == 2;  // a row may have no visible key among those a wave sees
   constexpr int NQB = F::kNQB, BQ = F::kBQ, NS = F::kStages, BK = F::kBK;
   constexpr int kBlocksPerTile = BK / 32;
   using Z = Swz<D, BK>;
@@ -73,7 +78,8 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
   if (!wg.valid) return;  // idle padding workgroup (whole workgroup, before any barrier)
   const int b = wg.b, g = wg.g, h = wg.g * rep + wg.hh;
   const int q0 = wg.tile * BQ;
-  const int qw0 = q0 + wave * 32 * NQB;  // first query of this wave
+  const int row_wave = PARTS == 1 ? wave : wave % F::kRowWaves, part = PARTS == 1 ? 0 : wave / F::kRowWaves;
+  const int qw0 = q0 + row_wave * 32 * NQB;  // first query of this wave
 
   int kend = p.Sk;
   if (p.causal) kend = min(p.Sk, q0 + BQ + p.q_start);
@@ -108,7 +114,7 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
   // kQStages stages of the ring, the first kEarlyTiles key tiles (those that fit before them) are requested at the
   // same time, the scale vector behind them: one memory round trip.  The remaining start-up tiles follow once the
   // query rows sit in registers (run() below).
-  constexpr int kQStages = BQ / (2 * BK);       // a stage holds two tiles of BK rows
+  constexpr int kQStages = (BQ + 2 * BK - 1) / (2 * BK);  // a stage holds two tiles of BK rows
   constexpr ring::Protocol R = ring::forward(NS, kQStages, Z::kPasses);  // the pipeline's numbers: ring_protocol.hpp
   static_assert(ring::well_formed(R) && R.loads_per_tile == kLoadsPerTile && !R.wait_before_loop && R.issue_at_top, "tile pipeline");
   static_assert(R.early_tiles >= ring::kTilesNeededAtLoopStart, "the loop is entered without a further wait");
@@ -119,7 +125,7 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
     const char* qb = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.q, b, h, q0));
 #pragma unroll
     for (int i = 0; i < kQStages; ++i)
-      issue_tile_pair<D, BK>(qb, qb, rowblock_lane_offsets<D, BK>((uint32_t)p.q.stride_s * 2, 2 * BK * i, p.Sq - q0, src.x, src.y),
+      issue_tile_pair<D, BK>(qb, qb, rowblock_lane_offsets<D, BK>((uint32_t)p.q.stride_s * 2, 2 * BK * i, min(p.Sq - q0, BQ), src.x, src.y),
                          wave_dst + (R.row_stage_first + i) * kStageBytes);
   }
 
@@ -142,8 +148,8 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
 #pragma unroll
   for (int nb = 0; nb < NQB; ++nb) {
     const int row = min(qw0 + 32 * nb + ln, p.Sq - 1);
-    // rows 32*(NQB*wave + nb) .. +31 of the block: which BK-row tile of the staged block, and which 32-row block of it
-    const int blk = NQB * wave + nb, tile = blk / kBlocksPerTile, rb = blk % kBlocksPerTile;
+    // rows 32*(NQB*row_wave + nb) .. +31 of the block: which BK-row tile of the staged block, and which 32-row block of it
+    const int blk = NQB * row_wave + nb, tile = blk / kBlocksPerTile, rb = blk % kBlocksPerTile;
     const uint32_t rm = lds0 + (R.row_stage_first + (tile >> 1)) * kStageBytes + (tile & 1) * Z::kTileBytes + swz_off_rm<D>(lane);
     u32x4 raw[KS];
 #pragma unroll
@@ -192,8 +198,9 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
   if (p.causal) n_act = min(n_act, (qw0 + 32 * NQB - 1 + q_start) / 32 + 1);
   if (SPLIT && p.causal && qw0 + 32 * NQB - 1 + q_start < 0) n_act = 0;
 
-  const uint32_t rm_lane = lds0 + swz_off_rm<D>(lane);
-  const uint32_t tr_lane = lds0 + swz_off_tr<D>(lane) + Z::kTileBytes;  // V' tile of a stage
+  // PARTS == 2: this wave's block of every tile is number `part` (a multiple of 4 KB further: the XOR terms stay below)
+  const uint32_t rm_lane = lds0 + swz_off_rm<D>(lane) + part * 32 * Z::kRB;
+  const uint32_t tr_lane = lds0 + swz_off_tr<D>(lane) + part * 32 * Z::kRB + Z::kTileBytes;  // V' tile of a stage
   bf16x8 kf[KS];
   auto request_rowmajor = [&](uint32_t rm, int kb) {  // kb compile-time at every call site
 #pragma unroll
@@ -240,7 +247,7 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
         const bool need = mx > m_ref[nb] + kLazyThresh;
         if (__builtin_amdgcn_ballot_w64(need) != 0) {
           const float m_new = need ? mx : m_ref[nb];
-          const float corr = SPLIT && !need ? 1.f : fast_exp2(m_ref[nb] - m_new);
+          const float corr = kMayMissKeys && !need ? 1.f : fast_exp2(m_ref[nb] - m_new);
           m_ref[nb] = m_new;
           l_run[nb][0] *= corr;
           l_run[nb][1] *= corr;
@@ -249,7 +256,7 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
 #pragma unroll
             for (int r = 0; r < 16; ++r) oacc[mb][nb][r] *= corr;
         }
-        const float mu = SPLIT && m_ref[nb] == -INFINITY ? 0.f : m_ref[nb];  // a share may hold no visible key of a row
+        const float mu = kMayMissKeys && m_ref[nb] == -INFINITY ? 0.f : m_ref[nb];
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[nb][r] -= mu;
       }
@@ -293,14 +300,16 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
     // Two loops instead of a per-block choice inside one: each body is then a single straight-line region
     // with one variant of the block (a join of the two variants costs a copy of every accumulator).
     // Loop A: tiles whose two blocks need no mask.  Loop B: the rest (masking a fully visible block is a no-op).
-    const int n_a = n_full / kBlocksPerTile;  // n_full <= n_act, so these tiles are all active
+    const int n_a = PARTS == 1 ? n_full / kBlocksPerTile : (n_full + 1 - part) / 2;  // n_full <= n_act, so these tiles are all active
     int jt = 0;
     for (; jt < n_a; ++jt) {
       const int nstage = stage == NS - 1 ? 0 : stage + 1;
       const bool issued = jt + R.issue_ahead < n_kt;
       if (issued) issue_tile(jt + R.issue_ahead);
       const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
-      if constexpr (kBlocksPerTile == 2) {
+      if constexpr (PARTS == 2) {
+        step(IC<0>{}, bounded_c, tr, 0, BK * jt + 32 * part, rm_lane + nstage * kStageBytes, 0);
+      } else if constexpr (kBlocksPerTile == 2) {
         step(IC<0>{}, bounded_c, tr, 0, BK * jt, rm, 1);
         step(IC<0>{}, bounded_c, tr, 1, BK * jt + 32, rm_lane + nstage * kStageBytes, 0);
       } else {
@@ -315,7 +324,9 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
       const bool issued = jt + R.issue_ahead < n_kt;
       if (issued) issue_tile(jt + R.issue_ahead);
       const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
-      if constexpr (kBlocksPerTile == 2) {
+      if constexpr (PARTS == 2) {
+        if (2 * jt + part < n_act) step(IC<1>{}, bounded_c, tr, 0, BK * jt + 32 * part, rm_lane + nstage * kStageBytes, 0);
+      } else if constexpr (kBlocksPerTile == 2) {
         if (2 * jt < n_act) step(IC<1>{}, bounded_c, tr, 0, BK * jt, rm, 1);
         if (2 * jt + 1 < n_act) step(IC<1>{}, bounded_c, tr, 1, BK * jt + 32, rm_lane + nstage * kStageBytes, 0);
       } else {
@@ -327,6 +338,40 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE>::kOcc)) void fwd_bf16
     }
   };
   if (bounded) run(IC<1>{}); else run(IC<0>{});
+
+  if constexpr (PARTS == 2) {
+    // The ring is idle (every wave has passed the last iteration's barrier): part 1 leaves its state there, 16 (8) bytes
+    // per lane and access, one slot per wave, and part 0 takes it over.
+    constexpr int kSlot = MB * 4096;
+    static_assert(2 * kSlot + 2 * 512 <= NS * kStageBytes, "two slots in the ring");
+    char* const slot = lds + row_wave * kSlot + lane * 16;
+    float2* const stat = reinterpret_cast<float2*>(lds + 2 * kSlot + row_wave * 512) + lane;
+    if (part == 1) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          *reinterpret_cast<f32x4*>(slot + (4 * mb + c) * 1024) = f32x4{oacc[mb][0][4 * c], oacc[mb][0][4 * c + 1], oacc[mb][0][4 * c + 2], oacc[mb][0][4 * c + 3]};
+      *stat = make_float2(m_ref[0], l_run[0][0] + l_run[0][1]);
+    }
+    __syncthreads();
+    if (part == 1) return;
+    const float2 ml = *stat;
+    const float m = fmaxf(m_ref[0], ml.x);
+    // both references are 0 on the bounded path; a part without a visible key of the row has (-inf, 0): weight 0
+    const float w0 = bounded ? 1.f : fast_exp2(m_ref[0] - m), w1 = bounded ? 1.f : fast_exp2(ml.x - m);
+    m_ref[0] = m;
+    l_run[0][0] = w0 * (l_run[0][0] + l_run[0][1]) + w1 * ml.y;
+    l_run[0][1] = 0.f;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const f32x4 t = *reinterpret_cast<const f32x4*>(slot + (4 * mb + c) * 1024);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) oacc[mb][0][4 * c + i] = w0 * oacc[mb][0][4 * c + i] + w1 * t[i];
+      }
+  }
 
   // ---- epilogue: normalise, gate, store y (bf16) and lse (fp32, natural log)
 #pragma unroll
@@ -416,13 +461,13 @@ __global__ __launch_bounds__(kMergeThreads) void fwd_merge_kernel(KArgs a) {
   }
 }
 
-template <int D, bool WIDE>
+template <int D, bool WIDE, int PARTS = 1>
 int launch_fwd_t(const KArgs& a, hipStream_t st) {
   const segpt_attn_params& p = a.p;
-  const int n_qt = (p.Sq + FwdShape<D, WIDE>::kBQ - 1) / FwdShape<D, WIDE>::kBQ;
-  const dim3 grid((unsigned)wg_grid(n_qt, p.B, p.Hkv, p.H / p.Hkv, wg_pinned_pairs(p.B, p.Hkv, false)));
-  if (p.rope_cos) hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, true, false>), grid, dim3(kThreadsM), 0, st, a);
-  else hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, false, false>), grid, dim3(kThreadsM), 0, st, a);
+  constexpr int BQ = FwdShape<D, WIDE, PARTS>::kBQ;
+  const dim3 grid((unsigned)wg_grid((p.Sq + BQ - 1) / BQ, p.B, p.Hkv, p.H / p.Hkv, wg_pinned_pairs(p.B, p.Hkv, false)));
+  if (p.rope_cos) hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, true, false, PARTS>), grid, dim3(kThreadsM), 0, st, a);
+  else hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, false, false, PARTS>), grid, dim3(kThreadsM), 0, st, a);
   return (int)hipGetLastError();
 }
 
@@ -433,8 +478,8 @@ int launch_fwd_split(const KArgs& a, hipStream_t st) {
   const segpt_attn_params& p = a.p;
   const int n_qt = (p.Sq + F::kBQ - 1) / F::kBQ;
   const dim3 grid((unsigned)wg_grid(n_qt, p.B, p.Hkv, p.H / p.Hkv, wg_pinned_pairs(p.B, p.Hkv, false)), (unsigned)a.fwd_splits);
-  if (p.rope_cos) hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, true, true>), grid, dim3(kThreadsM), 0, st, a);
-  else hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, false, true>), grid, dim3(kThreadsM), 0, st, a);
+  if (p.rope_cos) hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, true, true, 1>), grid, dim3(kThreadsM), 0, st, a);
+  else hipLaunchKernelGGL((fwd_bf16_kernel<D, WIDE, false, true, 1>), grid, dim3(kThreadsM), 0, st, a);
   const int rc = (int)hipGetLastError();
   if (rc) return rc;
   const bool few = (int64_t)p.B * p.H * p.Sq <= kMergeFewRows;
@@ -497,6 +542,23 @@ size_t split_plan(const segpt_attn_params& p, double n_unit, int* splits, int* c
 
 bool wide_fwd(const segpt_attn_params& p) { return p.D != 64 || p.Sk > 2048; }
 
+// Waves of a workgroup that share its query rows (launches whose keys are not split over workgroups).  1: four or eight
+// 32-row blocks per workgroup, every wave computes all blocks of a key tile.  2: 64 rows, the two 32-key blocks of a tile go
+// to two waves: twice as many workgroups, each half as long, for twice the tile loads and barriers per matrix
+// instruction.  2 wins while the launch is as long as its longest workgroup, i.e. while the 128-row workgroups leave resident slots
+// empty; the more key tiles a row has, the later that ends.  Measured, 1 against 2, us: head_dim 64, 18 / 6 heads, 1 x
+// 512 (72 workgroups) 9.8 / 8.2, 4 x 512 (288) 10.7 / 9.3, 6 x 512 (432) 11.7 / 12.9, 2 x 2048 (576) 34.7 / 28.2, 3 x 2048 (864) 39.8 /
+// 40.9, 1 x 4096 (576) 66.7 / 50.6; 8 / 8 heads, 1 x 4096 (256) 61.2 / 34.1; head_dim 128 (one workgroup per CU with 64-key
+// tiles), 16 / 4 heads, 2 x 512 (128) 13.9 / 10.9, 4 x 512 (256) 14.9 / 16.1, 1 x 2048 (256) 36.7 / 31.2, 2 x 2048 (512) 47 / 60.
+// Without QK-norm (or on request) the softmax keeps a running reference; a row's probabilities are then rounded against
+// ONE reference, whatever the launch, so those calls stay with 1.
+int fwd_parts(const segpt_attn_params& p) {
+  if (p.flags & (SEGPT_FLAG_RUNNING_MAX | SEGPT_FLAG_NO_NORM)) return 1;
+  const int64_t wgs = (int64_t)p.B * p.H * ((p.Sq + 127) / 128), tiles = (p.Sk + kBK - 1) / kBK;
+  if (p.D == 64) return wgs <= (tiles >= 32 ? 640 : 384) ? 2 : 1;
+  return wgs <= (tiles >= 16 ? 256 : 128) ? 2 : 1;
+}
+
 }  // namespace
 
 // Forward-only calls: bytes of the partials when the keys are to be split, 0 when not.
@@ -509,9 +571,13 @@ size_t fwd_split_plan(const segpt_attn_params& p, int* splits, int* chunk) {
 int launch_fwd_bf16(const KArgs& a, hipStream_t st) {
   if (a.p.D == 64) {
     if (a.fwd_splits > 1) return launch_fwd_split<64>(a, st);
+    if (fwd_parts(a.p) == 2) return launch_fwd_t<64, false, 2>(a, st);
     return wide_fwd(a.p) ? launch_fwd_t<64, true>(a, st) : launch_fwd_t<64, false>(a, st);
   }
-  if (a.p.D == 128) return a.fwd_splits > 1 ? launch_fwd_split<128>(a, st) : launch_fwd_t<128, true>(a, st);
+  if (a.p.D == 128) {
+    if (a.fwd_splits > 1) return launch_fwd_split<128>(a, st);
+    return fwd_parts(a.p) == 2 ? launch_fwd_t<128, true, 2>(a, st) : launch_fwd_t<128, true>(a, st);
+  }
   return (int)hipErrorInvalidValue;
 }
 

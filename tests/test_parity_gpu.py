@@ -177,6 +177,42 @@ def test_bf16_dkdv_workgroup_shapes(gpu_device, B, H, Hkv, Sq, Sk, D, kw):
     _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, D, seed=61, gen_kw={"extras": True}, rope=orc.rope_tables(max(Sq, Sk), 10000.0, D), **kw)
 
 
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,kw,gen_kw,use_rope", [
+    (1, 2, 1, 65, 65, 64, {}, {"extras": True}, True),                         # one row in the last workgroup, its second wave beyond the end
+    (1, 2, 2, 31, 130, 64, {"q_start": 99}, {"extras": True}, False),          # fewer rows than one wave owns
+    (2, 2, 1, 97, 33, 64, {"causal": False}, {}, True),                        # the second wave of a pair has one key
+    (1, 1, 1, 70, 20, 128, {"causal": False}, {"extras": True}, True),         # ... or none
+    (2, 3, 1, 129, 229, 128, {"q_start": 100}, {"extras": True}, False),
+    # the launches with thousands of rows at head_dim 128 go without a gate: its gradient (1 - sigma) sum_d y dy sees the
+    # bf16 rounding of y, rms 2^-9 / sqrt(3) sqrt(128) |y| |dy| = 0.013 for a row of one key, and 16128 such rows reach 4 rms
+    (3, 42, 42, 128, 130, 128, {"q_start": 2}, {}, True),                      # 126 workgroups of 128 rows: the last shape below the line
+    (3, 43, 43, 130, 100, 128, {"causal": False}, {}, True),                   # 258: above it
+    (4, 97, 97, 65, 70, 64, {"q_start": 5}, {"extras": True}, True),           # 388: forward and dQ above it
+])
+def test_bf16_forward_and_dq_workgroup_shapes(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw, use_rope):
+    """Forward and dQ with 64-row workgroups whose waves split the key blocks of a tile (launches that do not fill the
+    card) and with 128-row ones, at the ragged ends of both."""
+    if use_rope:
+        kw = dict(kw, rope=orc.rope_tables(max(Sq, Sk), 10000.0, D))
+    _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, D, seed=62, gen_kw=gen_kw, **kw)
+
+
+def test_bf16_forward_parts_with_scales_beyond_the_bound(gpu_device):
+    """Scale vectors too large for the fixed softmax reference (known on the device only): the two waves of a pair then
+    keep a running one each, and the early rows' second wave sees no key at all."""
+    x = gen(1, 2, 1, 150, 150, 64, BF16, seed=63)
+    x["g_q"] = x["g_q"] * 7.0
+    print("scales beyond the bound", flush=True)
+    ref = run_oracle(x, backward=False)
+    got = run_gpu(x, gpu_device, backward=False)
+    full = run_gpu(dict(x, g_q=x["g_q"].clone()), gpu_device)  # the training forward: never split over workgroups
+    # |logit| <= sqrt(64) * 7 * max g: exp2 arguments carry a relative 2^-8 of two bf16 operands' rounding, 0.25 in the worst
+    # row; the oracle comparison takes the operands' rounding out by tolerance, the two launches have it in common
+    assert torch.isfinite(full["y"].float()).all()
+    assert (full["lse"].double().cpu() - ref["lse"].double().reshape(full["lse"].shape)).abs().max() < 0.25
+    assert (got["lse"].double() - full["lse"].double()).abs().max() < 2.0**-8
+
+
 def test_bf16_gate_scale_not_positive_takes_the_gated_copy(gpu_device):
     """A gate scale <= 0 has no logarithm: the dQ kernel then leaves a gate-scaled copy of dO for the dK/dV kernel
     (the workspace grows by that tensor)."""
@@ -782,6 +818,9 @@ def test_decode_split_edges(gpu_device, B, H, Hkv, Sq, Sk, D, extras, use_rope, 
 def test_forward_only_split_keys(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw, use_rope):
     """Forward-only calls with few query tiles share out the keys of a tile (partials in the kv workspace, merged by a
     second kernel): against the oracle, and against the unsplit kernel that a call with gradients runs."""
+    from sample_efficient_gpt_amd import _lib
+    from sample_efficient_gpt_amd.plan import AttnPlan
+
     x = gen(B, H, Hkv, Sq, Sk, D, BF16, seed=47, **gen_kw)
     if use_rope:
         kw = dict(kw, rope=orc.rope_tables(Sk, 10000.0, D))
@@ -793,7 +832,14 @@ def test_forward_only_split_keys(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw, u
     # the same scores; with a running maximum the probabilities are rounded to bf16 against another reference, each by at
     # most 2^-9 of itself on either side, so the logarithms of their sums differ by at most 2^-8
     assert torch.allclose(split["lse"], whole["lse"], atol=2.0**-8 if kw.get("qk_norm") is False else 1e-4, rtol=0)
-    assert not torch.equal(split["y"], whole["y"]), "the two launches agree bit for bit: the call was not split"
+    plan = AttnPlan({n: None if t is None else t.to(gpu_device) for n, t in x.items() if n != "gate_logits"}, causal=kw.get("causal", True),
+                    q_start=kw.get("q_start", 0), backward=False)
+
+    def kv_bytes(flags):
+        plan.p.flags = flags
+        return plan.lib.segpt_attn_workspace_bytes(plan.p, _lib.SEGPT_WS_KV)
+
+    assert kv_bytes(_lib.SEGPT_FLAG_DECODE) > kv_bytes(0), "no room for partials is asked for: the call is not split"
 
 
 # ------------------------------------------------------------------ attention without QK-norm (SEGPT_FLAG_NO_NORM)
