@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   const int ln = lane & 31, hh = lane >> 5;
   const int rep = p.H / p.Hkv;
   const int n_qt = (p.Sq + BQ - 1) / BQ;
-  const WgCoord wg = decode_wg(blockIdx.x, n_qt, p.B, p.Hkv, rep, wg_pinned_pairs(p.B, p.Hkv, false));
+  const WgCoord wg = decode_wg(D == 64 ? balanced_id(blockIdx.x, gridDim.x) : (int)blockIdx.x, n_qt, p.B, p.Hkv, rep, wg_pinned_pairs(p.B, p.Hkv, false));
   if (!wg.valid) {  // idle padding workgroup: its row of the scale-gradient partials must still read as zero
     if (tid < D) a.dg_part[(int64_t)blockIdx.x * D + tid] = 0.f;
     return;

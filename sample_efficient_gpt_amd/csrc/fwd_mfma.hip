@@ -74,7 +74,7 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE, PARTS>::kOcc)) void f
   const int ln = lane & 31, hh = lane >> 5;
   const int rep = p.H / p.Hkv;
   const int n_qt = (p.Sq + BQ - 1) / BQ;
-  const WgCoord wg = decode_wg(blockIdx.x, n_qt, p.B, p.Hkv, rep, wg_pinned_pairs(p.B, p.Hkv, false));
+  const WgCoord wg = decode_wg(!SPLIT && F::kOcc >= 2 ? balanced_id(blockIdx.x, gridDim.x) : (int)blockIdx.x, n_qt, p.B, p.Hkv, rep, wg_pinned_pairs(p.B, p.Hkv, false));
   if (!wg.valid) return;  // idle padding workgroup (whole workgroup, before any barrier)
   const int b = wg.b, g = wg.g, h = wg.g * rep + wg.hh;
   const int q0 = wg.tile * BQ;

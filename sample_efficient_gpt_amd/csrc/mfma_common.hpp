@@ -490,6 +490,19 @@ __host__ __device__ inline int wg_grid(int n_tiles, int B, int Hkv, int rep, int
   const int rem_wgs = (B * Hkv - pinned) * per_pair;
   return (pinned ? ((rem_wgs + 7) & ~7) : rem_wgs) + pinned * per_pair;
 }
+// Workgroup ids with every second round of 256 (one workgroup per CU) reversed within its XCD.  A launch that is resident as
+// a whole, or nearly so, keeps the neighbours the dispatcher gave it: in plain heaviest-first order the heaviest
+// workgroups share their CUs with the next heaviest, reversed with the lightest.  Measured, plain against reversed, us:
+// forward, 18 / 6 heads, 8 x 512 (576 workgroups, three per CU) 13.9 / 12.8, 3 x 2048 (864) 39.0 / 36.1, 1 x 8192 (576, two per CU)
+// 163 / 150, head_dim 128 3 x 2048 (768, two per CU) 63.7 / 57.6 (12 x 512: 26.5 / 27.0); dQ 8 / 8 heads 1 x 8192 (512) 115.8 / 109.6.  Several rounds balance by
+// themselves and want their lightest workgroups last (forward, 1024 workgroups: 42.2 / 45.0), as do launches with one
+// workgroup per CU (head_dim 128 dQ 2 x 2048: 65 / 77), and dK/dV does not gain (159.3 / 160.4): those keep the plain order.
+__device__ __forceinline__ int balanced_id(int id, int n) {
+  constexpr int kMaxWgs = 896;
+  const int slot = id >> 3, slots = n >> 3, first = slot & ~31;
+  if (n > kMaxWgs || !(slot & 32) || slot >= slots) return id;
+  return ((first + min(first + 31, slots - 1) - slot) << 3) | (id & 7);
+}
 __device__ __forceinline__ WgCoord decode_wg(int bid, int n_tiles, int B, int Hkv, int rep, int pinned) {
   const int rem = B * Hkv - pinned, pp = pinned >> 3;
   const int rem_wgs = rem * n_tiles * rep;
