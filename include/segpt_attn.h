@@ -225,6 +225,13 @@ int segpt_attn_fwd_stage(const segpt_attn_params* p, int stage, void* stream);
  * occupies its SEGPT_NOALLOC_SCRATCH_BYTES on every GPU the library is loaded on, used or not. */
 int segpt_attn_fwd_noalloc(const segpt_attn_params* p, void* stream);
 
+/* Copies S rows of every (batch, kv head) of k and v, [B, Hkv, S, D], behind the rows a key/value cache holds, in one launch:
+ * k_to / v_to point at the first free row of the two buffers (strides of the buffers).  Any strides of rows that are
+ * whole 16-byte pieces at 16-byte aligned addresses (SEGPT_E_ALIGN / SEGPT_E_STRIDE otherwise, nothing launched); source and
+ * destination must not overlap.  Replaces the two concatenations per step of the reference's cache, attention.py:20-27. */
+int segpt_kv_append(int dtype, int B, int Hkv, int S, int D, const segpt_tensor4* k, const segpt_tensor4* v,
+                    const segpt_tensor4* k_to, const segpt_tensor4* v_to, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -35,6 +35,7 @@ EXPORTED_SYMBOLS = (
     "segpt_attn_bwd_stage",
     "segpt_attn_fwd_stage",
     "segpt_attn_fwd_noalloc",
+    "segpt_kv_append",
 )
 
 
@@ -114,6 +115,8 @@ def load():
         lib.segpt_attn_fwd_stage.argtypes = [C.POINTER(AttnParams), C.c_int, C.c_void_p]
         lib.segpt_attn_fwd_noalloc.restype = C.c_int
         lib.segpt_attn_fwd_noalloc.argtypes = [C.POINTER(AttnParams), C.c_void_p]
+        lib.segpt_kv_append.restype = C.c_int
+        lib.segpt_kv_append.argtypes = [C.c_int] * 5 + [C.POINTER(Tensor4)] * 4 + [C.c_void_p]
         ver = lib.segpt_abi_version()
         if ver != SEGPT_ABI_VERSION:
             raise RuntimeError(f"libsegpt_attn.so ABI version {ver}, binding expects {SEGPT_ABI_VERSION}")

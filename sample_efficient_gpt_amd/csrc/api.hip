@@ -329,6 +329,32 @@ int segpt_attn_fwd_stage(const segpt_attn_params* p, int stage, void* stream) {
   return fwd_stage_impl(p, stage, stage, stream);
 }
 
+int segpt_kv_append(int dtype, int B, int Hkv, int S, int D, const segpt_tensor4* k, const segpt_tensor4* v, const segpt_tensor4* k_to,
+                    const segpt_tensor4* v_to, void* stream) {
+  if (!k || !v || !k_to || !v_to) return SEGPT_E_NULL;
+  if (dtype != SEGPT_DTYPE_BF16 && dtype != SEGPT_DTYPE_FP32) return SEGPT_E_DTYPE;
+  if (B <= 0 || Hkv <= 0 || S <= 0 || D <= 0 || B > 65535 || Hkv > 32767) return SEGPT_E_SHAPE;
+  const int64_t elem = dtype == SEGPT_DTYPE_FP32 ? 4 : 2;
+  if (D * elem % 16) return SEGPT_E_STRIDE;
+  if ((int64_t)S * (D * elem / 16) > INT32_MAX - 64) return SEGPT_E_SHAPE;
+  segpt_attn_params shape{};  // what the stride checks look at
+  shape.dtype = dtype; shape.B = B; shape.D = D;
+  const segpt_tensor4* t[4] = {k, v, k_to, v_to};
+  for (int i = 0; i < 4; ++i) {
+    const int rc = i < 2 ? check_t4(*t[i], shape) : check_t4_out(*t[i], shape, Hkv, S);
+    if (rc) return rc;
+  }
+  KvAppendArgs a{};
+  for (int i = 0; i < 2; ++i) {
+    a.src[i] = reinterpret_cast<const char*>(t[i]->ptr);
+    a.dst[i] = reinterpret_cast<char*>(t[2 + i]->ptr);
+    a.src_b[i] = t[i]->stride_b * elem; a.src_h[i] = t[i]->stride_h * elem; a.src_s[i] = t[i]->stride_s * elem;
+    a.dst_b[i] = t[2 + i]->stride_b * elem; a.dst_h[i] = t[2 + i]->stride_h * elem; a.dst_s[i] = t[2 + i]->stride_s * elem;
+  }
+  a.B = B; a.Hkv = Hkv; a.S = S; a.chunks = (int)(D * elem / 16);
+  return launch_kv_append(a, reinterpret_cast<hipStream_t>(stream));
+}
+
 static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage_hi, void* stream) {
   if (!p_in) return SEGPT_E_NULL;
   segpt_attn_params p_copy = *p_in;

@@ -192,6 +192,15 @@ __device__ __forceinline__ void reduce_scale_grad(const KArgs& a, int tid, float
   }
 }
 
+// segpt_kv_append: byte addresses and strides of k (index 0) and v (1)
+struct KvAppendArgs {
+  const char* src[2];
+  char* dst[2];
+  int64_t src_b[2], src_h[2], src_s[2], dst_b[2], dst_h[2], dst_s[2];
+  int32_t B, Hkv, S, chunks;  // chunks: 16-byte pieces per row
+};
+int launch_kv_append(const KvAppendArgs& a, hipStream_t st);
+
 // host-side launchers (one per translation unit); each returns a hipError_t as int
 int launch_fwd_f32(const KArgs& a, hipStream_t st);
 int launch_bwd_dkdv_f32(const KArgs& a, hipStream_t st);

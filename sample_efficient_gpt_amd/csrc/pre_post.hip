@@ -84,6 +84,19 @@ __global__ __launch_bounds__(256) void kv_prep_kernel(KArgs a) {
   }
 }
 
+// One step's rows of k and v behind the rows of a cache.  A generation step appends a kilobyte: what counts is that both
+// tensors are ONE launch (two copies of 2.3 us each and their dispatch before, 2.3 us now); a prompt is bound by HBM.
+constexpr int kAppendThreads = 64;
+__global__ __launch_bounds__(kAppendThreads) void kv_append_kernel(KvAppendArgs a) {
+  const int i = blockIdx.x * kAppendThreads + threadIdx.x;
+  if (i >= a.S * a.chunks) return;
+  const int s = i / a.chunks, c = i - s * a.chunks;
+  const int t = blockIdx.y & 1, g = blockIdx.y >> 1, b = blockIdx.z;
+  const char* src = a.src[t] + b * a.src_b[t] + g * a.src_h[t] + s * a.src_s[t] + 16 * c;
+  char* dst = a.dst[t] + b * a.dst_b[t] + g * a.dst_h[t] + s * a.dst_s[t] + 16 * c;
+  *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
+}
+
 constexpr int kReduceThreads = 1024;
 
 __global__ __launch_bounds__(kReduceThreads) void bwd_reduce_kernel(KArgs a) {
@@ -126,6 +139,12 @@ static void launch_kv_prep_t(const KArgs& a, hipStream_t st) {
 int launch_kv_prep(const KArgs& a, hipStream_t st) {
   if (a.p.D == 64) launch_kv_prep_t<64>(a, st);
   else launch_kv_prep_t<128>(a, st);
+  return (int)hipGetLastError();
+}
+
+int launch_kv_append(const KvAppendArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)((a.S * a.chunks + kAppendThreads - 1) / kAppendThreads), (unsigned)(2 * a.Hkv), (unsigned)a.B);
+  hipLaunchKernelGGL(kv_append_kernel, grid, dim3(kAppendThreads), 0, st, a);
   return (int)hipGetLastError();
 }
 

@@ -328,6 +328,33 @@ std::vector<OptTensor> op_backward(const Tensor& dy, const Tensor& q, const Tens
   return {g.q, g.k, g.v, g.g_q, opt(g.g_k), opt(g.v_first), opt(g.coef), opt(g.gate)};
 }
 
+// KVCache.append in one launch: k and v, [B, Hkv, S, D], become rows length .. length + S - 1 of the two buffers; returns the
+// filled prefixes.  None (nothing done, the caller copies) for what plain copies treat otherwise: recorded gradients or
+// tangents, sizes or types that differ, rows that are not whole 16-byte pieces.
+std::optional<std::pair<Tensor, Tensor>> kv_append(const Tensor& kbuf, const Tensor& vbuf, const Tensor& k, const Tensor& v, int64_t length) {
+  const auto dt = k.scalar_type();
+  const auto dev = k.device();
+  if ((dt != at::kBFloat16 && dt != at::kFloat) || !k.is_cuda() || k.dim() != 4 || k.numel() == 0 || v.sizes() != k.sizes()) return std::nullopt;
+  const int64_t need = length + k.size(2);
+  for (const Tensor* t : {&kbuf, &vbuf, &k, &v}) {
+    if (t->scalar_type() != dt || t->device() != dev || t->dim() != 4 || t->stride(3) != 1) return std::nullopt;
+    if ((at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(0).defined()) return std::nullopt;
+  }
+  for (const Tensor* t : {&kbuf, &vbuf})
+    if (t->size(0) != k.size(0) || t->size(1) != k.size(1) || t->size(2) < need || t->size(3) != k.size(3) ||
+        (t->is_inference() && !c10::InferenceMode::is_enabled()))
+      return std::nullopt;
+  segpt_tensor4 from[2] = {view4(k, 0), view4(v, 0)}, to[2] = {view4(kbuf, 0), view4(vbuf, 0)};
+  for (auto& t : to) t.ptr = static_cast<char*>(t.ptr) + length * t.stride_s * k.element_size();
+  const c10::DeviceGuard guard(dev);
+  const int rc = segpt_kv_append(dt == at::kFloat ? SEGPT_DTYPE_FP32 : SEGPT_DTYPE_BF16, (int)k.size(0), (int)k.size(1), (int)k.size(2),
+                                 (int)k.size(3), &from[0], &from[1], &to[0], &to[1], current_stream(dev));
+  if (rc < 0) return std::nullopt;
+  if (rc) throw LibraryError(rc, "segpt_kv_append");
+  for (const Tensor* t : {&kbuf, &vbuf}) torch::autograd::impl::bump_version(*t);
+  return std::make_pair(kbuf.narrow(2, 0, need), vbuf.narrow(2, 0, need));
+}
+
 // What torch raises (out of memory, an error from a saved-tensor hook) keeps its Python type across the binding
 template <typename R, typename... A>
 auto bound(R (*f)(A...)) {
@@ -365,4 +392,5 @@ PYBIND11_MODULE(_segpt_torch, m) {
   m.def("attention", bound(&attention));
   m.def("op_forward", bound(&op_forward));
   m.def("op_backward", bound(&op_backward));
+  m.def("kv_append", bound(&kv_append));
 }

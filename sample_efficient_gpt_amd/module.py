@@ -5,7 +5,9 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from . import _native
 from .function import QKNormFlashAttnFunc
+from .library_op import _seen_as_operator
 
 
 class SelfDotProductAttnQKNorm(nn.Module):
@@ -59,11 +61,16 @@ class KVCache:
                 kb[:, :, : self.length].copy_(self._kbuf[:, :, : self.length])
                 vb[:, :, : self.length].copy_(self._vbuf[:, :, : self.length])
             self._kbuf, self._vbuf = kb, vb
-        self._kbuf[:, :, self.length : need].copy_(k)
-        self._vbuf[:, :, self.length : need].copy_(v)
+        views = None
+        if k.is_cuda and not _seen_as_operator(k, v, self._kbuf, self._vbuf):
+            views = _native.load().kv_append(self._kbuf, self._vbuf, k, v, self.length)  # both in one launch
+        if views is None:
+            self._kbuf[:, :, self.length : need].copy_(k)
+            self._vbuf[:, :, self.length : need].copy_(v)
+            views = self._kbuf[:, :, :need], self._vbuf[:, :, :need]
         self.length = need
-        self.keys, self.values = self._kbuf[:, :, :need], self._vbuf[:, :, :need]
-        return self.keys, self.values
+        self.keys, self.values = views
+        return views
 
     @property
     def mixed_length(self):

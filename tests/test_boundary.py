@@ -223,6 +223,19 @@ def test_module_interface():
     assert list(sig.parameters) == ["Q", "K", "V", "is_causal", "q_start"]
 
 
+def test_kv_append_rejects_bad_arguments_before_any_launch(lib):
+    """segpt_kv_append returns its error codes without a device."""
+    t = lambda ptr=256, sb=4096, sh=1024, ss=64: _lib.Tensor4(ptr, sb, sh, ss)
+    call = lambda dtype=_lib.SEGPT_DTYPE_BF16, B=2, Hkv=4, S=8, D=64, k=t(), v=t(), kt=t(), vt=t(): lib.segpt_kv_append(dtype, B, Hkv, S, D, k, v, kt, vt, None)
+    codes = dict(re.findall(r"#define\s+(SEGPT_E_\w+)\s+\(?(-?\d+)", open(HEADER).read()))
+    want = lambda name: int(codes["SEGPT_E_" + name])
+    assert call(k=t(ptr=0)) == want("NULL") and call(vt=t(ptr=0)) == want("NULL")
+    assert call(dtype=7) == want("DTYPE") and call(S=0) == want("SHAPE") and call(Hkv=40000) == want("SHAPE")
+    assert call(S=1 << 29) == want("SHAPE")                      # more 16-byte pieces than an int counts
+    assert call(D=60) == want("STRIDE") and call(v=t(ss=66)) == want("STRIDE") and call(kt=t(ptr=264)) == want("ALIGN")
+    assert call(kt=t(sh=64, ss=64)) == want("STRIDE")            # a destination whose rows overlap
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libsegpt_attn.so"))

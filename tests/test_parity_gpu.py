@@ -1319,6 +1319,30 @@ def test_mhsa_module_generation_with_cache(gpu_device):
     assert torch.allclose(steps.cpu().double(), ref, atol=2e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("dtype,D", [(BF16, 64), (BF16, 128), (F32, 32), (F32, 64)])
+def test_kv_cache_append_is_the_two_copies(gpu_device, dtype, D):
+    """KVCache.append in one launch: a prompt, single rows, a run that makes the buffers grow and an odd run, from strided views
+    of a projection, hold exactly what was appended; what the launch does not take (rows off 16 bytes, a tensor that records
+    gradients) goes the old way; the views of earlier steps notice that their buffer was written."""
+    B, Hkv = 3, 5
+    cache, want_k, want_v = KVCache(capacity=70), [], []
+    for i, S in enumerate((37, 1, 1, 64, 129, 1)):
+        proj = torch.randn(B, S, 3 * Hkv * D + 8, device=gpu_device, dtype=dtype)
+        lo = 1 if i == 4 else 0  # the fifth run: rows that start at an odd element
+        k, v = (proj[..., lo + j * Hkv * D : lo + (j + 1) * Hkv * D].unflatten(-1, (Hkv, D)).permute(0, 2, 1, 3) for j in (1, 2))
+        before = cache._kbuf._version if cache._kbuf is not None else None
+        grown = cache.length + S > (0 if cache._kbuf is None else cache._kbuf.shape[2])
+        with torch.no_grad():
+            keys, values = cache.append(k, v)
+        want_k.append(k); want_v.append(v)
+        assert torch.equal(keys, torch.cat(want_k, dim=2)) and torch.equal(values, torch.cat(want_v, dim=2)), i
+        assert keys.data_ptr() == cache._kbuf.data_ptr() and cache.length == keys.shape[2]
+        assert grown or cache._kbuf._version > before
+    k = torch.randn(B, Hkv, 2, D, device=gpu_device, dtype=dtype, requires_grad=True)
+    keys, _ = cache.append(k, k.detach())
+    assert keys.requires_grad and torch.equal(keys[:, :, -2:], k)
+
+
 def test_mhsa_module_prefill_with_grad_then_cached_steps_without(gpu_device):
     """A prefill that runs with gradients enabled (its mixed values are not kept in the cache) followed by
     generation steps under no_grad: the first cached step mixes every row the cache is still missing, and the value
