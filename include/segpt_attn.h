@@ -43,7 +43,7 @@ extern "C" {
 
 /* element type of q/k/v/o/gate and their gradients */
 #define SEGPT_DTYPE_BF16 0 /* MFMA path: D in {64, 128}                       */
-#define SEGPT_DTYPE_FP32 1 /* fp32 FMA path (1e-5 parity): D in {32, 64, 128} */
+#define SEGPT_DTYPE_FP32 1 /* fp32 MFMA path (1e-5 parity): D in {32, 64, 128} */
 
 /* error codes (negative); segpt_strerror() gives the text */
 #define SEGPT_OK 0
