@@ -24,9 +24,8 @@ struct KArgs {
   float* dcoef_part;  // [n_dkdv_blocks, 2] fp32 partial sums of (dc1, dc2)
   int32_t n_dq_blocks;
   int32_t n_dkdv_blocks;
-  // decode path (split keys): partial O [B*Hkv, splits, n_rows, D] and (max, sum) [B*Hkv, splits, n_rows, 2], both fp32
-  // (n_rows = H/Hkv * Sq query rows),
-  // carved from kv_workspace
+  // decode path (split keys): partial O [B*Hkv, partials, n_rows, D] and (max, sum) [B*Hkv, partials, n_rows, 2], both fp32
+  // (n_rows = H/Hkv * Sq query rows; one partial per split or per stream of one), carved from kv_workspace
   float* dec_part;
   float* dec_stat;
   int32_t dec_splits, dec_chunk, dec_kend;

@@ -180,3 +180,40 @@ def kernel_rounding_model(Q, K, V, g, dO, *, eps, sm_scale, causal, q_start):
     W = ln2 * dKhat                                           # dL/dkhat
     dk = b * W - (b ** 3 / D) * (W * K).sum(-1, keepdim=True) * K
     return {"y": y, "dq": dq, "dk": dk, "dv": dv, "dg": dg}
+
+
+def decode_rounding_model(x, *, q_start, chunk, streams, rope=None, eps=1e-6):
+    """The split-key forward (csrc/decode_mfma.hip) in float64 with a bf16 rounding where it holds a bf16 value: Qhat, Khat,
+    V' = c1 v + c2 v_first, the probabilities, y.  A probability is rounded relative to the running maximum of its stream:
+    the keys come in chunks, the 32-key blocks of a chunk go round robin to `streams` streams."""
+    q, k, v = (x[n].double() for n in ("q", "k", "v"))
+    B, H, Sq, D = q.shape
+    Hkv, Sk = k.shape[1], k.shape[2]
+    if rope is not None:
+        q, k = orc.apply_rope(q, *rope, q_start), orc.apply_rope(k, *rope, 0)
+    norm = lambda t: t * torch.rsqrt((t * t).mean(-1, keepdim=True) + eps)
+    g = x["g_q"].double() * (1.0 if x["g_k"] is None else x["g_k"].double())
+    qhat = bf16_round(norm(q) * g * (1.4426950408889634 / D**0.5)).reshape(B, Hkv, -1, D)
+    khat = bf16_round(norm(k))
+    if x.get("v_first") is not None:
+        v = bf16_round(float(x["vr_coef"][0]) * v + float(x["vr_coef"][1]) * x["v_first"].double())
+    seen = torch.arange(Sk) <= (torch.arange(Sq) + q_start).unsqueeze(1)
+    s = (qhat @ khat.transpose(2, 3)).masked_fill(~seen.repeat(H // Hkv, 1), float("-inf"))
+    parts = []
+    for lo in range(0, Sk, chunk):
+        for w in range(streams):
+            m, l, o = torch.full(s.shape[:3] + (1,), float("-inf"), dtype=torch.float64), 0.0, 0.0
+            for j in range(lo + 32 * w, min(lo + chunk, Sk), 32 * streams):
+                hi = min(j + 32, Sk)
+                new = torch.maximum(m, s[..., j:hi].amax(-1, keepdim=True))
+                p = bf16_round(torch.exp2(s[..., j:hi] - new.clamp_min(-1e30)))
+                corr = torch.exp2(m - new.clamp_min(-1e30))
+                m, l, o = new, l * corr + p.sum(-1, keepdim=True), o * corr + p @ v[:, :, j:hi]
+                if j + 32 * streams >= min(lo + chunk, Sk):
+                    parts.append((m, l, o))
+    M = torch.stack([m for m, _, _ in parts]).amax(0)
+    y = sum(o * torch.exp2(m - M) for m, _, o in parts) / sum(l * torch.exp2(m - M) for m, l, _ in parts)
+    y = y.reshape(B, H, Sq, D)
+    if x.get("gate_logits") is not None:
+        y = y * 2.0 * torch.sigmoid(x["gate_logits"].double()).permute(0, 2, 1).unsqueeze(-1)
+    return bf16_round(y)

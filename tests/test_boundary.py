@@ -236,6 +236,25 @@ def test_kv_append_rejects_bad_arguments_before_any_launch(lib):
     assert call(kt=t(sh=64, ss=64)) == want("STRIDE")            # a destination whose rows overlap
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_decode_partials_fit_the_scratch_of_a_split(lib, D):
+    """The split-key forward asks for at most 32 rows of partials per 128 keys and (batch, kv head) pair and per pair of one
+    resident round: a workspace sized without SEGPT_FLAG_DECODE (the normalised keys) holds them from 256 keys on, and the
+    entry point without a workspace takes every call it could take."""
+    round_ = 768 if D == 64 else 256
+    for B, H, Hkv, Sq in ((1, 1, 1, 1), (1, 18, 6, 1), (3, 12, 4, 2), (1, 8, 8, 9), (2, 8, 4, 16), (5, 32, 1, 1), (64, 18, 6, 1), (1, 32, 32, 32), (300, 16, 4, 8)):
+        for Sk in (1, 31, 128, 129, 1000, 4096, 70000):
+            p = _lib.new_params()
+            p.dtype, p.B, p.H, p.Hkv, p.Sq, p.Sk, p.D, p.causal, p.q_start = _lib.SEGPT_DTYPE_BF16, B, H, Hkv, Sq, Sk, D, 1, max(0, Sk - Sq)
+            keys = lib.segpt_attn_workspace_bytes(p, _lib.SEGPT_WS_KV)
+            p.flags = _lib.SEGPT_FLAG_DECODE
+            part = lib.segpt_attn_workspace_bytes(p, _lib.SEGPT_WS_KV)
+            pairs = B * Hkv
+            splits = min(-(-round_ // pairs), -(-Sk // 128), 512)
+            assert 0 < part <= -(-pairs * splits * 32 * (D + 2) * 4 // 256) * 256, (B, H, Hkv, Sq, Sk)
+            assert Sk < 256 or part <= keys, (B, H, Hkv, Sq, Sk)
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libsegpt_attn.so"))

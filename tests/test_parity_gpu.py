@@ -11,7 +11,7 @@ import torch
 from oracle import qknorm_attn_oracle as orc
 from sample_efficient_gpt_amd import (CONFIGS, FlashAttnFunc, KVCache, MultiHeadSelfAttention, QKNormFlashAttnFunc,
                                       SelfDotProductAttnQKNorm, make_inputs, qknorm_attention, qknorm_attention_op)
-from tests.parity_util import compare, gen, run_gpu, run_oracle, scalar_gain_scale, value_residual_scale
+from tests.parity_util import compare, decode_rounding_model, gen, run_gpu, run_oracle, scalar_gain_scale, value_residual_scale
 
 pytestmark = pytest.mark.gpu
 BF16, F32 = torch.bfloat16, torch.float32
@@ -819,6 +819,36 @@ def test_decode_split_edges(gpu_device, B, H, Hkv, Sq, Sk, D, extras, use_rope, 
     ref = run_oracle(x, backward=False, **kw)
     with torch.no_grad():
         compare(run_gpu(x, gpu_device, backward=False, **kw), ref, BF16)
+
+
+def _decode_distance(device, x, use_rope):
+    """Norm-wise distance of a decode-shaped call to the model of its roundings (chunks as decode_plan() cuts them)."""
+    (B, H, Sq, D), (Hkv, Sk) = x["q"].shape, x["k"].shape[1:3]
+    splits = min(-(-(768 if D == 64 else 256) // (B * Hkv)), -(-Sk // 128))
+    chunk = -(-(-(-Sk // splits)) // 128) * 128
+    rope = orc.rope_tables(Sk, 10000.0, D) if use_rope else None
+    model = decode_rounding_model(x, q_start=Sk - Sq, chunk=chunk, streams=4, rope=rope)
+    with torch.no_grad():
+        y = run_gpu(x, device, backward=False, q_start=Sk - Sq, **({"rope": rope} if use_rope else {}))["y"].double()
+    return float((y - model).norm() / model.norm())
+
+
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,use_rope", [
+    (2, 6, 2, 1, 700, 64, True),       # one block per stream, the last streams empty
+    (70, 18, 6, 1, 900, 64, False),    # three or four blocks per stream
+    (20, 16, 4, 1, 1333, 128, True),
+    (3, 8, 4, 2, 2100, 128, False),
+    (2, 8, 8, 32, 1500, 64, True),     # 9 to 32 query rows per kv head: streams merged inside a workgroup
+    (100, 4, 2, 5, 700, 64, False),
+    (2, 12, 4, 3, 1000, 128, True),
+    (40, 10, 5, 8, 1100, 128, False),
+])
+def test_decode_rounds_keys_and_probabilities_like_the_training_kernels(gpu_device, B, H, Hkv, Sq, Sk, D, use_rope):
+    """Normalised keys as bf16, probabilities against the running maximum of their stream.  Bound: what is left is fp32 against
+    float64 in front of a rounding.  A score off by 2^-20 flips the rounding of one probability in 2^12 by 2^-8, 6e-5 in
+    norm; y off by 1e-5 flips one value in 400 by 2^-8, 2e-4 (seen 0 to 2.6e-4; another reference or raw keys 3.7e-3)."""
+    print(f"decode rounding B={B} H={H} Hkv={Hkv} Sq={Sq} Sk={Sk} D={D} rope={use_rope}", flush=True)
+    assert _decode_distance(gpu_device, gen(B, H, Hkv, Sq, Sk, D, BF16, seed=81), use_rope) < 1e-3
 
 
 @pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,kw,gen_kw,use_rope", [
