@@ -56,6 +56,14 @@ __device__ __forceinline__ void issue_wave_tile(const char* base, const WaveTile
 #pragma unroll
   for (int i = 0; i < WaveTile<D>::kLoads; ++i) gload_lds16_so(base, o.off[i], dst + i * 1024);
 }
+// c1 v + c2 f of eight elements, in fp32, rounded once
+__device__ __forceinline__ bf16x8 mix8(bf16x8 v, bf16x8 f, float c1, float c2) {
+  const u32x4 a = __builtin_bit_cast(u32x4, v), b = __builtin_bit_cast(u32x4, f);
+  u32x4 w;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(c1 * bf16lo(a[i]) + c2 * bf16lo(b[i]), c1 * bf16hi(a[i]) + c2 * bf16hi(b[i]));
+  return as_bf16x8(w);
+}
 // (maximum, sum) of a split from those of its streams, at(w), and the streams' weights; a stream with nothing visible has
 // (-inf, 0): weight 0
 template <typename At>
@@ -93,6 +101,9 @@ __device__ __forceinline__ void wait_lds_reads() {
 // against the exact running maximum of the wave's keys, so that the largest is 1.  Cheaper forms (the normaliser on the 16
 // scores a lane holds and the raw key bits as operand; a fixed softmax reference where the QK-norm bound allows one)
 // cost 3 to 5 % of accuracy (3.2e-3 -> 3.3e-3 from float64, in norm) and moved every output by 4e-3.
+// A value residual is mixed in fp32 and rounded once, on the transposed fragments of V and V_first (elementwise, so the
+// layout does not matter).  Two products with c1 P and c2 P are a little faster (32 x 6 pairs, 8192 keys: 110 us against 112),
+// but their roundings do not cancel where the two parts do: v_first = v, coefficients (0.9, -0.85): 4e-2 from the exact mix.
 // Only the block that holds the last visible key is masked, and the accumulators are rescaled only where a maximum moved.
 // workgroups per CU that LDS (tiles and tables) and registers allow
 template <int D, bool ROPE, bool VRES>
@@ -287,32 +298,21 @@ __global__ __launch_bounds__(kDecThreads, (kDecOcc<D, ROPE, VRES>)) void decode_
       m_run = m_new;
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r] - mu);
-      auto add_product = [&](uint32_t tr, bf16x8 p0, bf16x8 p1) {
-        wave_lds_sync();
+      if (more) wait_vmcnt<kTabLoads + kRowLoads>(); else wait_vmcnt<0>();  // this block's V (and V_first)
+      const bf16x8 pb[2] = {pack_c_half_sum(s, 0, l_run), pack_c_half_sum(s, 1, l_run)};
+      wave_lds_sync();
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          oacc[mb] = mfma32(swz_frag_tr<D>(tr, mb, 0), p0, oacc[mb]);
-          oacc[mb] = mfma32(swz_frag_tr<D>(tr, mb, 1), p1, oacc[mb]);
-        }
-        wait_lds_reads();
-      };
-      if (more) wait_vmcnt<kFirstLoads + kTabLoads + kRowLoads>(); else wait_vmcnt<kFirstLoads>();  // this block's V
-      if constexpr (!VRES) {
-        const bf16x8 p0 = pack_c_half_sum(s, 0, l_run), p1 = pack_c_half_sum(s, 1, l_run);
-        add_product(vtr, p0, p1);
-        if (more) issue_v(jb + kStep);
-      } else {
-        f32x16 s1, s2;
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          l_run[r & 1] += s[r];
-          s1[r] = c1 * s[r];
-          s2[r] = c2 * s[r];
+        for (int s2 = 0; s2 < 2; ++s2) {
+          bf16x8 vT = swz_frag_tr<D>(vtr, mb, s2);
+          if constexpr (VRES) vT = mix8(vT, swz_frag_tr<D>(ftr, mb, s2), c1, c2);
+          oacc[mb] = mfma32(vT, pb[s2], oacc[mb]);
         }
-        add_product(vtr, pack_c_half(s1, 0), pack_c_half(s1, 1));
-        if (more) { issue_v(jb + kStep); wait_vmcnt<kTabLoads + 2 * kRowLoads>(); } else wait_vmcnt<0>();  // V_first
-        add_product(ftr, pack_c_half(s2, 0), pack_c_half(s2, 1));
-        if (more) issue_first(jb + kStep);
+      wait_lds_reads();
+      if (more) {
+        issue_v(jb + kStep);
+        issue_first(jb + kStep);
       }
     }
     buf ^= 1;

@@ -851,6 +851,18 @@ def test_decode_rounds_keys_and_probabilities_like_the_training_kernels(gpu_devi
     assert _decode_distance(gpu_device, gen(B, H, Hkv, Sq, Sk, D, BF16, seed=81), use_rope) < 1e-3
 
 
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,use_rope", [(2, 6, 2, 1, 700, 64, True), (70, 18, 6, 1, 900, 64, False), (20, 16, 4, 1, 1333, 128, True),
+                                                      (2, 12, 4, 3, 1000, 64, True), (40, 10, 5, 8, 1100, 128, False)])
+def test_decode_mixes_a_value_residual_before_it_rounds(gpu_device, B, H, Hkv, Sq, Sk, D, use_rope):
+    """Coefficients of opposite sign on nearly equal values (a first layer's v_first is its own v; the coefficients are learned):
+    V' = c1 v + c2 v_first is a small difference, and its rounding error has to be relative to it.  Bound as above (seen
+    0 to 2.2e-4; the two parts rounded one by one 4e-2)."""
+    x = gen(B, H, Hkv, Sq, Sk, D, BF16, seed=82, extras=True)
+    x["vr_coef"], x["v_first"] = torch.tensor([0.9, -0.85]), x["v"].clone()
+    print(f"decode value residual B={B} H={H} Hkv={Hkv} Sq={Sq} Sk={Sk} D={D} rope={use_rope}", flush=True)
+    assert _decode_distance(gpu_device, x, use_rope) < 1e-3
+
+
 @pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,kw,gen_kw,use_rope", [
     (1, 2, 1, 70, 2500, 64, {"q_start": 2430}, {"extras": True}, True),                       # one ragged query tile, last share ragged
     (2, 3, 3, 130, 1100, 128, {"q_start": 970}, {}, False),                                   # two query tiles, the second of 2 rows
