@@ -20,6 +20,7 @@ own formula (triton_flash_attn_qknorm.py:67-91).
 
 from __future__ import annotations
 
+import math
 import threading
 
 import torch
@@ -110,11 +111,28 @@ def qknorm_attention(q, k, v, g_q, g_k=None, *, v_first=None, vr_coef=None, gate
     ``out_bshd=True``: the returned ``[B,H,Sq,D]`` tensor is a view of a ``[B,Sq,H,D]`` buffer, so that
     ``y.permute(0, 2, 1, 3).reshape(B, Sq, H*D)`` is the ``b seq (h head_d)`` tensor of attention.py:243 without a copy.
     """
-    y, lse = _native.load().attention(
-        q, k, v, g_q, g_k, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin,
-        rope_q_pos0, rope_k_pos0, _call_flags(qk_norm, _no_backward_will_follow(q, k, v, g_q, g_k, v_first, vr_coef, gate_logits)),
-        0, 0, out_bshd, return_lse)
+    inference = _no_backward_will_follow(q, k, v, g_q, g_k, v_first, vr_coef, gate_logits)
+    y, lse = _attend(q, k, v, g_q, g_k, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin,
+                     rope_q_pos0, rope_k_pos0, qk_norm, inference, 0, 0, out_bshd, return_lse)
     return (y, lse) if return_lse else y
+
+
+def _attend(q, k, v, g_q, g_k, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin,
+            rope_q_pos0, rope_k_pos0, qk_norm, inference, heads, kv_heads, out_bshd, with_lse):
+    """The native call behind every function here: ``(y, lse)``; heads > 0: flattened ``[(h b), S, d]`` operands."""
+    if torch.jit.is_tracing():
+        # a tracer records operators only: the native call would leave the allocation of y in the graph and nothing that
+        # fills it, so a traced caller gets the registered operator
+        from . import library_op  # noqa: F401  (registers it)
+
+        canon = (lambda t, n: None if t is None else _canon(t, n)) if heads else (lambda t, n: t)
+        y, lse, _ = torch.ops.segpt.qknorm_attention(
+            canon(q, heads), canon(k, kv_heads), canon(v, kv_heads), g_q, g_k, canon(v_first, kv_heads), vr_coef, gate_logits,
+            float(gate_scale), float(eps), 1.0 / math.sqrt(q.shape[-1]) if sm_scale is None else float(sm_scale), bool(causal), int(q_start),
+            rope_cos, rope_sin, -1 if rope_q_pos0 is None else int(rope_q_pos0), int(rope_k_pos0), bool(qk_norm), bool(out_bshd), inference)
+        return (y.permute(1, 0, 2, 3).reshape(q.shape) if heads else y), lse
+    return _native.load().attention(q, k, v, g_q, g_k, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale, causal, q_start, rope_cos,
+                                    rope_sin, rope_q_pos0, rope_k_pos0, _call_flags(qk_norm, inference), heads, kv_heads, out_bshd, with_lse)
 
 
 def _call_flags(qk_norm, inference):
@@ -173,9 +191,8 @@ class QKNormFlashAttnFunc(_GradModeAtApply, torch.autograd.Function):
             assert v_first.is_cuda and v_first.is_contiguous()
             if promoted and v_first.ndim == 2:
                 v_first = v_first.unsqueeze(0)
-        return _native.load().attention(Q, K, V, gain, k_gain, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale,
-                                        is_causal, q_start, rope_cos, rope_sin, None, 0, _call_flags(True, QKNormFlashAttnFunc._inference()),
-                                        H, Hkv, False, False)[0]
+        return _attend(Q, K, V, gain, k_gain, v_first, vr_coef, gate_logits, gate_scale, eps, sm_scale, is_causal, q_start, rope_cos,
+                       rope_sin, None, 0, True, QKNormFlashAttnFunc._inference(), H, Hkv, False, False)[0]
 
 
 class TritonFlashAttnQKNormFunc(QKNormFlashAttnFunc):
@@ -208,5 +225,5 @@ class FlashAttnFunc(_GradModeAtApply, torch.autograd.Function):
     def forward(ctx, Q, K, V, q_start=0, is_causal=True, n_kv_heads=None):
         Q, K, V, H, Hkv = _flat_operands(Q, K, V, n_kv_heads, None)
         one = torch.ones(1, dtype=torch.float32, device=Q.device)
-        return _native.load().attention(Q, K, V, one, None, None, None, None, 1.0, 0.0, None, is_causal, q_start, None, None, None, 0,
-                                        _call_flags(False, FlashAttnFunc._inference()), H, Hkv, False, False)[0]
+        return _attend(Q, K, V, one, None, None, None, None, 1.0, 0.0, None, is_causal, q_start, None, None, None, 0, False,
+                       FlashAttnFunc._inference(), H, Hkv, False, False)[0]

@@ -116,9 +116,10 @@ _fwd_op.register_autograd(_autograd_backward, setup_context=_setup_context)
 
 
 def _seen_as_operator(*operands):
-    """Somebody looks at the call as an operator: a compiler, a dispatch or function mode (a selective-checkpoint policy,
-    fake tensors), a function transform (vmap, torch.func.grad) or an operand of a tensor subclass."""
-    return (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+    """Somebody looks at the call as an operator: a compiler, a tracer (torch.jit.trace), a dispatch or function mode (a
+    selective-checkpoint policy, fake tensors), a function transform (vmap, torch.func.grad) or an operand of a tensor
+    subclass."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._are_functorch_transforms_active()
             or any(t is not None and type(t) not in (Tensor, torch.nn.Parameter) for t in operands))
 

@@ -10,7 +10,7 @@ import torch
 
 from oracle import qknorm_attn_oracle as orc
 from sample_efficient_gpt_amd import (CONFIGS, FlashAttnFunc, KVCache, MultiHeadSelfAttention, QKNormFlashAttnFunc,
-                                      SelfDotProductAttnQKNorm, make_inputs, qknorm_attention, qknorm_attention_op)
+                                      SelfDotProductAttnQKNorm, TritonFlashAttnQKNormFunc, make_inputs, qknorm_attention, qknorm_attention_op)
 from tests.parity_util import compare, decode_rounding_model, gen, run_gpu, run_oracle, scalar_gain_scale, value_residual_scale
 
 pytestmark = pytest.mark.gpu
@@ -685,6 +685,46 @@ def test_native_node_keeps_what_python_callers_see(gpu_device):
             qknorm_attention(big, dev["k"].expand(400, -1, -1, -1), dev["v"].expand(400, -1, -1, -1), dev["g_q"])
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def _traced_callers(x, device):
+    """name -> (operands of a layout from a generated case, caller of three tensors)"""
+    g = x["g_q"].to(device)
+    rope = dict(zip(("rope_cos", "rope_sin"), (t.float().to(device) for t in orc.rope_tables(x["k"].shape[2], 10000.0, x["q"].shape[3]))))
+    gate = x["gate_logits"].to(device)
+    canon = lambda s: [s[n].to(device) for n in ("q", "k", "v")]
+    flat = lambda s: [s[n].transpose(0, 1).reshape(-1, *s[n].shape[2:]).contiguous().to(device) for n in ("q", "k", "v")]
+    Hkv = x["k"].shape[1]
+
+    def cached(q, k, v):
+        keys, values = KVCache().append(k, v)
+        return qknorm_attention(q, keys, values, g)
+
+    return {
+        "function": (canon, lambda q, k, v: qknorm_attention(q, k, v, g, gate_logits=gate, out_bshd=True, **rope)),
+        "operator": (canon, lambda q, k, v: qknorm_attention_op(q, k, v, g, **rope)),
+        "cache": (canon, cached),
+        "flat": (flat, lambda q, k, v: QKNormFlashAttnFunc.apply(q, k, v, g, True, 0, None, None, None, gate, 2.0, Hkv)),
+        "reference formula": (flat, lambda q, k, v: TritonFlashAttnQKNormFunc.apply(q, k, v, g, True, 0, None, None, None, None, 2.0, Hkv)),
+        "plain": (flat, lambda q, k, v: FlashAttnFunc.apply(q, k, v, 0, True, Hkv)),
+    }
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("name", ["function", "operator", "cache", "flat", "reference formula", "plain"])
+@pytest.mark.filterwarnings("ignore")
+def test_traced_callers_compute_when_replayed(gpu_device, name, grad):
+    """torch.jit.trace records operators, so what it records has to be one: a trace taken on one set of inputs gives the eager
+    result on another."""
+    a, b = (gen(2, 4, 2, 40, 40, 64, BF16, seed=s, extras=True) for s in (3, 4))
+    layout, caller = _traced_callers(a, gpu_device)[name]
+    first, second = ([t.requires_grad_(grad) for t in layout(x)] for x in (a, b))
+    traced = torch.jit.trace(caller, tuple(first), check_trace=False)
+    assert torch.equal(traced(*second), caller(*second))
+    if grad and name != "cache":
+        d = torch.randn_like(caller(*second))
+        for got, want in zip(torch.autograd.grad(traced(*second), second, d), torch.autograd.grad(caller(*second), second, d)):
+            assert torch.equal(got, want)
 
 
 # ------------------------------------------------------------------ rotary embedding fused into the loads
