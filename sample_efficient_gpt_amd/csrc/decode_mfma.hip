@@ -61,7 +61,7 @@ __device__ __forceinline__ bf16x8 mix8(bf16x8 v, bf16x8 f, float c1, float c2) {
   const u32x4 a = __builtin_bit_cast(u32x4, v), b = __builtin_bit_cast(u32x4, f);
   u32x4 w;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(c1 * bf16lo(a[i]) + c2 * bf16lo(b[i]), c1 * bf16hi(a[i]) + c2 * bf16hi(b[i]));
+  for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(fmaf(c2, bf16lo(b[i]), c1 * bf16lo(a[i])), fmaf(c2, bf16hi(b[i]), c1 * bf16hi(a[i])));
   return as_bf16x8(w);
 }
 // (maximum, sum) of a split from those of its streams, at(w), and the streams' weights; a stream with nothing visible has
