@@ -8,6 +8,8 @@
 // without the interpreter.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/ATen.h>
@@ -254,6 +256,15 @@ struct AttentionNode : torch::autograd::Function<AttentionNode> {
       python_error err;
       err.persist();
       throw err;
+    }
+    if (at::GradMode::is_enabled()) {
+      // create_graph: the gradients depend on every operand and on dy, but have no derivative of their own.  Going back
+      // through them has to fail; without a history it would quietly leave these terms out.
+      torch::autograd::edge_list edges = torch::autograd::get_current_node()->next_edges();
+      edges.push_back(torch::autograd::impl::gradient_edge(dy));
+      const auto refuse = std::make_shared<torch::autograd::Error>("qknorm attention has no second derivative", std::move(edges));
+      for (Tensor* t : {&g.q, &g.k, &g.v, &g.g_q, &g.g_k, &g.v_first, &g.coef, &g.gate})
+        if (t->defined()) torch::autograd::set_history(*t, refuse);
     }
     out[0] = g.q; out[1] = g.k; out[2] = g.v; out[3] = g.g_q; out[4] = g.g_k; out[5] = g.v_first; out[6] = g.coef; out[7] = g.gate;
     return out;

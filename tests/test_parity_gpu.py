@@ -727,6 +727,28 @@ def test_traced_callers_compute_when_replayed(gpu_device, name, grad):
             assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("caller", [qknorm_attention_op, qknorm_attention])
+def test_second_derivatives_are_refused(gpu_device, caller):
+    """First derivatives with create_graph=True are the ordinary ones; going back through them raises instead of leaving the
+    attention's terms out of a gradient penalty."""
+    x = gen(1, 2, 1, 33, 33, 64, BF16, seed=5)
+    q, k, v, g, d_o = (x[n].to(gpu_device) for n in ("q", "k", "v", "g_q", "d_o"))
+    wrt = [t.requires_grad_(True) for t in (q, v, g)]
+    plain = torch.autograd.grad(caller(q, k, v, g), wrt, d_o)
+    first = torch.autograd.grad(caller(q, k, v, g), wrt, d_o, create_graph=True)
+    for a, b in zip(plain, first):
+        assert torch.equal(a, b) and not a.requires_grad
+    for d in first:
+        with pytest.raises(RuntimeError, match="derivative|autograd formula"):
+            (d.float().pow(2).sum() + q.float().pow(2).sum()).backward(retain_graph=True)
+        with pytest.raises(RuntimeError, match="derivative|autograd formula"):
+            torch.autograd.grad(d.float().sum(), q, retain_graph=True, allow_unused=True)
+    only_dy = d_o.clone().requires_grad_(True)  # linear in dy, but that is a derivative too
+    first, = torch.autograd.grad(caller(q, k, v, g), q, only_dy, create_graph=True)
+    with pytest.raises(RuntimeError, match="derivative|autograd formula"):
+        torch.autograd.grad(first.float().sum(), only_dy)
+
+
 # ------------------------------------------------------------------ rotary embedding fused into the loads
 
 
