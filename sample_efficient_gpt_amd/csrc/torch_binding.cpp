@@ -46,6 +46,7 @@ void set_python_error(const LibraryError& e) {
 }
 
 Tensor defined_or_none(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+OptTensor none_or_defined(const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); }
 
 // Everything of a call that is not a differentiable operand.  heads > 0: the flattened [(h b), S, d] layout of the
 // positional drop-ins, head-major (attention.py:199), with `heads` / `kv_heads` heads; 0: canonical [B, heads, S, D].
@@ -55,11 +56,10 @@ struct Call : torch::CustomClassHolder {
   int64_t q_start = 0, q_pos0 = 0, k_pos0 = 0;
   int64_t heads = 0, kv_heads = 0;
   int flags = 0;
-  Tensor cos, sin;
 };
 
 struct Operands {
-  Tensor q, k, v, g_q, g_k, v_first, coef, gate;
+  Tensor q, k, v, g_q, g_k, v_first, coef, gate, cos, sin;
 };
 
 Tensor f32_vector(const Tensor& t, const at::Device& dev) {
@@ -67,6 +67,7 @@ Tensor f32_vector(const Tensor& t, const at::Device& dev) {
   if (t.scalar_type() == at::kFloat && t.device() == dev && t.is_contiguous()) return t;
   return t.detach().to(dev, at::kFloat).reshape({-1}).contiguous();
 }
+Tensor f32_table(const Tensor& t, const at::Device& dev) { return t.defined() ? t.detach().to(dev, at::kFloat).contiguous() : t; }
 Tensor last_dim_contiguous(const Tensor& t) { return !t.defined() || t.stride(-1) == 1 ? t : t.contiguous(); }
 
 struct Sizes {
@@ -111,6 +112,7 @@ void check_operands(const Operands& x, const Call& c) {
   if (x.v_first.defined()) check(x.v_first.sizes() == x.v.sizes() && x.coef.numel() == 2, "v_first must have v's shape, vr_coef two elements");
   if (x.gate.defined())
     check(x.gate.dim() == 3 && x.gate.size(0) == q.B && x.gate.size(1) == q.S && x.gate.size(2) == q.H, "gate_logits must be [B, Sq, H]");
+  if (x.cos.defined()) check(x.cos.dim() == 2 && x.cos.sizes() == x.sin.sizes() && x.cos.size(1) == q.D / 2, "rope tables must be [len, head_dim // 2]");
 }
 
 void fill(segpt_attn_params& p, const Operands& x, const Call& c, const Tensor& y, const Tensor& lse) {
@@ -129,9 +131,9 @@ void fill(segpt_attn_params& p, const Operands& x, const Call& c, const Tensor& 
   p.gate = view3(x.gate);
   p.lse = ptr_of<float>(lse);
   p.g_q = ptr_of<float>(x.g_q); p.g_k = ptr_of<float>(x.g_k); p.vr_coef = ptr_of<float>(x.coef);
-  if (c.cos.defined()) {
-    p.rope_cos = ptr_of<float>(c.cos); p.rope_sin = ptr_of<float>(c.sin);
-    p.rope_len = (int32_t)c.cos.size(0);
+  if (x.cos.defined()) {
+    p.rope_cos = ptr_of<float>(x.cos); p.rope_sin = ptr_of<float>(x.sin);
+    p.rope_len = (int32_t)x.cos.size(0);
     p.rope_q_pos0 = (int32_t)c.q_pos0; p.rope_k_pos0 = (int32_t)c.k_pos0;
   }
 }
@@ -142,10 +144,11 @@ Tensor scratch(const segpt_attn_params& p, int which, const at::Device& dev) {
 }
 void* current_stream(const at::Device& dev) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream(); }
 
-// operands as the kernels take them: fp32 scale vectors, contiguous last dimensions; checked
+// operands as the kernels take them: fp32 scale vectors and tables, contiguous last dimensions; checked
 Operands prepared(const Operands& x, const Call& c) {
   const auto dev = x.q.device();
-  Operands r{x.q, x.k, x.v, f32_vector(x.g_q, dev), f32_vector(x.g_k, dev), x.v_first, f32_vector(x.coef, dev), x.gate};
+  Operands r{x.q, x.k, x.v, f32_vector(x.g_q, dev), f32_vector(x.g_k, dev), x.v_first, f32_vector(x.coef, dev), x.gate,
+             f32_table(x.cos, dev), f32_table(x.sin, dev)};
   check_operands(r, c);
   r.q = last_dim_contiguous(r.q); r.k = last_dim_contiguous(r.k); r.v = last_dim_contiguous(r.v);
   r.v_first = last_dim_contiguous(r.v_first);
@@ -228,14 +231,15 @@ using torch::autograd::variable_list;
 
 struct AttentionNode : torch::autograd::Function<AttentionNode> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g_q, const OptTensor& og_k,
-                               const OptTensor& ov_first, const OptTensor& ocoef, const OptTensor& ogate, c10::intrusive_ptr<Call> call, bool bshd,
-                               bool with_lse) {
+                               const OptTensor& ov_first, const OptTensor& ocoef, const OptTensor& ogate, const OptTensor& ocos,
+                               const OptTensor& osin, c10::intrusive_ptr<Call> call, bool bshd, bool with_lse) {
     const Tensor g_k = defined_or_none(og_k), coef = defined_or_none(ocoef), gate = defined_or_none(ogate);
-    const Operands x = prepared({q, k, v, g_q, g_k, defined_or_none(ov_first), coef, gate}, *call);
+    const Tensor cos = defined_or_none(ocos), sin = defined_or_none(osin);
+    const Operands x = prepared({q, k, v, g_q, g_k, defined_or_none(ov_first), coef, gate, cos, sin}, *call);
     const Tensor y = output_like(x.q, bshd);
     const Forward f = run_forward(x, *call, y);
     // the normalised keys (bf16 path) are kept for the backward: 1/rep of q's size
-    ctx->save_for_backward({x.q, x.k, x.v, g_q, g_k, x.v_first, coef, gate, y, f.lse, f.kv_ws});
+    ctx->save_for_backward({x.q, x.k, x.v, g_q, g_k, x.v_first, coef, gate, cos, sin, y, f.lse, f.kv_ws});
     ctx->saved_data["call"] = c10::IValue::make_capsule(call);
     ctx->set_materialize_grads(false);
     if (!with_lse) return {y};
@@ -243,13 +247,13 @@ struct AttentionNode : torch::autograd::Function<AttentionNode> {
     return {y, f.lse};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    variable_list out(11);
+    variable_list out(13);
     const variable_list s = ctx->get_saved_variables();
     const auto call = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
-    const Tensor dy = grads[0].defined() ? grads[0] : at::zeros_like(s[8]);
+    const Tensor dy = grads[0].defined() ? grads[0] : at::zeros_like(s[10]);
     Grads g;
     try {
-      g = run_backward({s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7]}, *call, s[8], s[9], s[10], dy);
+      g = run_backward({s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8], s[9]}, *call, s[10], s[11], s[12], dy);
     } catch (const LibraryError& e) {  // on the engine's thread: carried to the caller's as the Python exception it is there
       const py::gil_scoped_acquire gil;
       set_python_error(e);
@@ -272,24 +276,24 @@ struct AttentionNode : torch::autograd::Function<AttentionNode> {
 };
 
 c10::intrusive_ptr<Call> make_call(const Tensor& q, double gate_scale, double eps, std::optional<double> sm_scale, bool causal, int64_t q_start,
-                                   const OptTensor& rope_cos, const OptTensor& rope_sin, std::optional<int64_t> rope_q_pos0, int64_t rope_k_pos0,
-                                   int64_t flags, int64_t heads, int64_t kv_heads) {
+                                   std::optional<int64_t> rope_q_pos0, int64_t rope_k_pos0, int64_t flags, int64_t heads, int64_t kv_heads) {
   auto c = c10::make_intrusive<Call>();
   c->gate_scale = gate_scale; c->eps = eps;
   c->sm_scale = sm_scale.has_value() ? *sm_scale : 1.0 / std::sqrt((double)q.size(-1));
   c->causal = causal; c->q_start = q_start; c->flags = (int)flags;
   c->heads = heads; c->kv_heads = kv_heads;
-  check(rope_cos.has_value() == rope_sin.has_value(), "rope_cos and rope_sin go together");
-  if (rope_cos.has_value()) {
-    // fp32 contiguous tables of shape [len, head_dim / 2]; query row i sits at position q_pos0 + i (default q_start, as
-    // in the reference's caller, attention.py:191-204), key row j at k_pos0 + j
-    auto table = [&](const Tensor& t) { return t.detach().to(q.device(), at::kFloat).contiguous(); };
-    c->cos = table(*rope_cos); c->sin = table(*rope_sin);
-    check(c->cos.dim() == 2 && c->cos.sizes() == c->sin.sizes() && c->cos.size(1) == q.size(-1) / 2, "rope tables must be [len, head_dim // 2]");
-    c->q_pos0 = rope_q_pos0.has_value() ? *rope_q_pos0 : q_start;
-    c->k_pos0 = rope_k_pos0;
-  }
+  // query row i sits at position q_pos0 + i (default q_start, as in the reference's caller, attention.py:191-204), key row j
+  // at k_pos0 + j
+  c->q_pos0 = rope_q_pos0.has_value() ? *rope_q_pos0 : q_start;
+  c->k_pos0 = rope_k_pos0;
   return c;
+}
+Operands operands(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g_q, const OptTensor& g_k, const OptTensor& v_first,
+                  const OptTensor& coef, const OptTensor& gate, const OptTensor& rope_cos, const OptTensor& rope_sin) {
+  check(rope_cos.has_value() == rope_sin.has_value(), "rope_cos and rope_sin go together");
+  // the tables take no gradient; detached they still share the caller's version counter
+  auto table = [](const OptTensor& t) { return t.has_value() && t->defined() ? t->detach() : Tensor(); };
+  return {q, k, v, g_q, defined_or_none(g_k), defined_or_none(v_first), defined_or_none(coef), defined_or_none(gate), table(rope_cos), table(rope_sin)};
 }
 
 // The differentiable op.  Nothing is recorded when no gradient can be asked for.  Function transforms and forward-mode
@@ -299,15 +303,15 @@ std::pair<Tensor, Tensor> attention(const Tensor& q, const Tensor& k, const Tens
                                     bool causal, int64_t q_start, const OptTensor& rope_cos, const OptTensor& rope_sin,
                                     std::optional<int64_t> rope_q_pos0, int64_t rope_k_pos0, int64_t flags, int64_t heads, int64_t kv_heads, bool bshd,
                                     bool with_lse) {
-  const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin, rope_q_pos0, rope_k_pos0, flags, heads, kv_heads);
-  const Operands x{q, k, v, g_q, defined_or_none(g_k), defined_or_none(v_first), defined_or_none(coef), defined_or_none(gate)};
+  const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_q_pos0, rope_k_pos0, flags, heads, kv_heads);
+  const Operands x = operands(q, k, v, g_q, g_k, v_first, coef, gate, rope_cos, rope_sin);
   if (const auto& transforms = at::functorch::functorchTLSAccessor()) transforms->checkSupportsCppAutogradFunction();
   const bool grad_mode = at::GradMode::is_enabled();
   bool record = false;
   for (const Tensor* t : {&x.q, &x.k, &x.v, &x.g_q, &x.g_k, &x.v_first, &x.coef, &x.gate})
     record |= t->defined() && ((grad_mode && t->requires_grad()) || t->_fw_grad(0).defined());
   if (record) {
-    const variable_list r = AttentionNode::apply(x.q, x.k, x.v, x.g_q, g_k, v_first, coef, gate, call, bshd, with_lse);
+    const variable_list r = AttentionNode::apply(x.q, x.k, x.v, x.g_q, g_k, v_first, coef, gate, none_or_defined(x.cos), none_or_defined(x.sin), call, bshd, with_lse);
     return {r[0], with_lse ? r[1] : Tensor()};
   }
   const at::NoGradGuard no_grad;
@@ -322,8 +326,8 @@ std::tuple<Tensor, Tensor, Tensor> op_forward(const Tensor& q, const Tensor& k, 
                                               const OptTensor& v_first, const OptTensor& coef, const OptTensor& gate, double gate_scale, double eps,
                                               double sm_scale, bool causal, int64_t q_start, const OptTensor& rope_cos, const OptTensor& rope_sin,
                                               std::optional<int64_t> rope_q_pos0, int64_t rope_k_pos0, int64_t flags, const Tensor& y) {
-  const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin, rope_q_pos0, rope_k_pos0, flags, 0, 0);
-  const Operands x = prepared({q, k, v, g_q, defined_or_none(g_k), defined_or_none(v_first), defined_or_none(coef), defined_or_none(gate)}, *call);
+  const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_q_pos0, rope_k_pos0, flags, 0, 0);
+  const Operands x = prepared(operands(q, k, v, g_q, g_k, v_first, coef, gate, rope_cos, rope_sin), *call);
   const Forward f = run_forward(x, *call, y);
   return {y, f.lse, f.kv_ws};
 }
@@ -332,11 +336,9 @@ std::vector<OptTensor> op_backward(const Tensor& dy, const Tensor& q, const Tens
                                    const Tensor& kv_ws, double gate_scale, double eps, double sm_scale, bool causal, int64_t q_start,
                                    const OptTensor& rope_cos, const OptTensor& rope_sin, std::optional<int64_t> rope_q_pos0, int64_t rope_k_pos0,
                                    int64_t flags) {
-  const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_cos, rope_sin, rope_q_pos0, rope_k_pos0, flags, 0, 0);
-  const Grads g = run_backward({q, k, v, g_q, defined_or_none(g_k), defined_or_none(v_first), defined_or_none(coef), defined_or_none(gate)}, *call, y,
-                               lse, kv_ws, dy);
-  auto opt = [](const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); };
-  return {g.q, g.k, g.v, g.g_q, opt(g.g_k), opt(g.v_first), opt(g.coef), opt(g.gate)};
+  const auto call = make_call(q, gate_scale, eps, sm_scale, causal, q_start, rope_q_pos0, rope_k_pos0, flags, 0, 0);
+  const Grads g = run_backward(operands(q, k, v, g_q, g_k, v_first, coef, gate, rope_cos, rope_sin), *call, y, lse, kv_ws, dy);
+  return {g.q, g.k, g.v, g.g_q, none_or_defined(g.g_k), none_or_defined(g.v_first), none_or_defined(g.coef), none_or_defined(g.gate)};
 }
 
 // KVCache.append in one launch: k and v, [B, Hkv, S, D], become rows length .. length + S - 1 of the two buffers; returns the

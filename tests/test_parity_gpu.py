@@ -728,6 +728,25 @@ def test_traced_callers_compute_when_replayed(gpu_device, name, grad):
 
 
 @pytest.mark.parametrize("caller", [qknorm_attention_op, qknorm_attention])
+def test_rotary_tables_are_saved_variables(gpu_device, caller):
+    """Tables written in place between forward and backward would give the gradients of another function: the backward
+    notices, as for every other operand, and tables pass through saved-tensor hooks."""
+    x = gen(1, 2, 1, 33, 33, 64, BF16, seed=5)
+    q, k, v, g, d_o = (x[n].to(gpu_device) for n in ("q", "k", "v", "g_q", "d_o"))
+    q.requires_grad_(True)
+    for dtype in (F32, torch.float64):  # fp64 tables are converted for the kernels; the caller's are what is watched
+        cos, sin = (t.to(gpu_device, dtype) for t in orc.rope_tables(33, 10000.0, 64))
+        y = caller(q, k, v, g, rope_cos=cos, rope_sin=sin)
+        ref, = torch.autograd.grad(y, q, d_o, retain_graph=True)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(gpu_device)):
+            moved = caller(q, k, v, g, rope_cos=cos, rope_sin=sin)
+        assert torch.equal(torch.autograd.grad(moved, q, d_o)[0], ref)
+        sin.mul_(0.5)
+        with pytest.raises(RuntimeError, match="inplace"):
+            torch.autograd.grad(y, q, d_o)
+
+
+@pytest.mark.parametrize("caller", [qknorm_attention_op, qknorm_attention])
 def test_second_derivatives_are_refused(gpu_device, caller):
     """First derivatives with create_graph=True are the ordinary ones; going back through them raises instead of leaving the
     attention's terms out of a gradient penalty."""
