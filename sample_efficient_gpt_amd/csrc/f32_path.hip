@@ -26,6 +26,9 @@
 #include "common.hpp"
 
 namespace segpt {
+
+int f32_dq_grid(const segpt_attn_params& p);
+
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -151,16 +154,24 @@ __device__ __forceinline__ void load_tile(f32x4v (&x)[T32<D>::kPasses], const fl
 }
 
 // 1/sqrt(mean x^2 + eps) of a row from its sum of squares: v_rsq_f32 (1 ulp) and one Newton step, six instructions for
-// the divide and square root sequences' forty; exactly 1 for plain attention (`norm` is wave-uniform)
+// the divide and square root sequences' forty; exactly 1 for plain attention (`norm` is wave-uniform).  A sum of squares that
+// overflowed has y = 0, and so has the result: the median gives the step's NaN a value.  x must be normal
+// (v_rsq_f32 flushes others): see TINY_EPS.
 __device__ __forceinline__ float inv_rms(float ss, float inv_d, float eps, bool norm) {
   const float x = ss * inv_d + eps;
   const float y = __builtin_amdgcn_rsqf(x);
-  return norm ? fmaf(0.5f * y, fmaf(-x * y, y, 1.0f), y) : 1.0f;
+  return norm ? fmaf(0.5f * y, __builtin_amdgcn_fmed3f(fmaf(-x * y, y, 1.0f), -1.0f, 1.0f), y) : 1.0f;
+}
+// TINY_EPS: eps is no normal number, so a row's mean square on top of it need not be one either; the kernels then take the
+// epilogues' form.  A template parameter: as a branch in the tile loop it cost 3 %.
+inline bool tiny_eps(const segpt_attn_params& p) {
+  constexpr float kSmallestNormal = 1.17549435e-38f;
+  return !(p.flags & SEGPT_FLAG_NO_NORM) && !(p.eps >= kSmallestNormal);
 }
 
 // normalise (and rotate) the rows of a tile and put them into LDS: x * 1/rms(x) * scale.  All rows' sums are formed
 // side by side, and the one branch (rotary tables or not) stands outside the row loop.
-template <int D>
+template <int D, bool TINY_EPS>
 __device__ __forceinline__ void stage_norm(const segpt_attn_params& p, f32x4v (&x)[T32<D>::kPasses], f32x4v scale, int pos0, int last,
                                            float* tile, int lane) {
   using T = T32<D>;
@@ -176,7 +187,7 @@ __device__ __forceinline__ void stage_norm(const segpt_attn_params& p, f32x4v (&
     inv[ps] = row_sum<T::kLPR>((x[ps][0] * x[ps][0] + x[ps][1] * x[ps][1]) + (x[ps][2] * x[ps][2] + x[ps][3] * x[ps][3]));
 #pragma unroll
   for (int ps = 0; ps < T::kPasses; ++ps) {
-    const float n = inv_rms(inv[ps], 1.0f / D, p.eps, norm);
+    const float n = TINY_EPS ? row_normaliser(p, inv[ps], 1.0f / D) : inv_rms(inv[ps], 1.0f / D, p.eps, norm);
     *reinterpret_cast<f32x4v*>(tile + (ps * T::kRPP + lr) * T::kRS + 4 * part) = x[ps] * (n * scale);
   }
 }
@@ -288,7 +299,7 @@ __device__ __forceinline__ float gate_logit(const segpt_attn_params& p, int b, i
 
 // ---- forward.  S^T = Khat Qhat^T (lane = query), running maximum per lane, O^T += V'^T P^T; every wave has its own
 // (maximum, sum, O) over its keys, merged behind the loop.  Grid: heaviest query tiles first.
-template <int D>
+template <int D, bool TINY_EPS>
 __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void fwd_f32_kernel(KArgs a) {
   const segpt_attn_params& p = a.p;
   using T = T32<D>;
@@ -324,7 +335,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void fwd_f32_kernel(KArgs a
     gs[e] = gprod<D>(p, 4 * (lane % T::kLPR) + e) * p.sm_scale * kLog2e;
   }
   f32x4v qf[T::kC];
-  stage_norm<D>(p, qraw, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, kt, lane);
+  stage_norm<D, TINY_EPS>(p, qraw, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, kt, lane);
   wave_sync();
 #pragma unroll
   for (int c = 0; c < T::kC; ++c) qf[c] = frag_rm<D>(kt, c, lane);
@@ -338,7 +349,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void fwd_f32_kernel(KArgs a
   const int n_full = p.causal ? min(p.Sk, q0 + p.q_start + 1) / kRows : p.Sk / kRows;  // tiles that need no mask
 
   for (int jt = wave; jt < n_kt; jt += kWaves) {
-    stage_norm<D>(p, kraw, one, p.rope_k_pos0 + jt * kRows, p.Sk - 1 - jt * kRows, kt, lane);
+    stage_norm<D, TINY_EPS>(p, kraw, one, p.rope_k_pos0 + jt * kRows, p.Sk - 1 - jt * kRows, kt, lane);
     stage_plain<D>(vraw, vt, lane);
     wave_sync();
     if (jt + kWaves < n_kt) {
@@ -414,7 +425,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void fwd_f32_kernel(KArgs a
 // rowsum(dY o Y) (Y is the saved, already gated output, so this equals rowsum(dO o O)), dgate = (1 - sigmoid(z)) delta,
 // the gate-scaled dO,
 // and the workgroup's partial of the combined scale gradient  dg[d] = sum_i sm_scale (a_i q_id) T_id.
-template <int D>
+template <int D, bool TINY_EPS>
 __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dq_f32_kernel(KArgs a) {
   const segpt_attn_params& p = a.p;
   using T = T32<D>;
@@ -448,7 +459,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dq_f32_kernel(KArg
     load_tile<D>(x, row_ptr<float>(p.q, b, h, 0), p.q.stride_s, q0, p.Sq, lane);
     load_tile<D>(dy, row_ptr<float>(p.d_o, b, h, 0), p.d_o.stride_s, q0, p.Sq, lane);
     load_tile<D>(y, row_ptr<float>(p.o, b, h, 0), p.o.stride_s, q0, p.Sq, lane);
-    stage_norm<D>(p, x, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, kt, lane);
+    stage_norm<D, TINY_EPS>(p, x, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, kt, lane);
 #pragma unroll
     for (int ps = 0; ps < T::kPasses; ++ps) {
       const int row = ps * T::kRPP + lane / T::kLPR;
@@ -495,7 +506,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dq_f32_kernel(KArg
   const int n_full = p.causal ? min(p.Sk, q0 + p.q_start + 1) / kRows : p.Sk / kRows;
 
   for (int jt = wave; jt < n_kt; jt += kWaves) {
-    stage_norm<D>(p, kraw, one, p.rope_k_pos0 + jt * kRows, p.Sk - 1 - jt * kRows, kt, lane);
+    stage_norm<D, TINY_EPS>(p, kraw, one, p.rope_k_pos0 + jt * kRows, p.Sk - 1 - jt * kRows, kt, lane);
     stage_plain<D>(vraw, vt, lane);
     wave_sync();
     if (jt + kWaves < n_kt) {
@@ -561,7 +572,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dq_f32_kernel(KArg
 // query tiles and writes its sums to the workspace; the finish kernel adds them over the query heads of the GQA group
 // and the splits.  One workgroup per (key tile, KV head) walking all its query heads would leave the card half empty
 // at small batches and its heaviest workgroup (first keys, every query) alone at the end.
-template <int D>
+template <int D, bool TINY_EPS>
 __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dkdv_f32_kernel(KArgs a) {
   const segpt_attn_params& p = a.p;
   using T = T32<D>;
@@ -597,7 +608,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dkdv_f32_kernel(KA
     f32x4v k[T::kPasses], v[T::kPasses];
     load_tile<D>(k, row_ptr<float>(p.k, b, g, 0), p.k.stride_s, j0, p.Sk, lane);
     if (wave == 0) load_vmix<D>(p, v, b, g, j0, c1, c2, lane);
-    stage_norm<D>(p, k, one, p.rope_k_pos0 + j0, p.Sk - 1 - j0, qt, lane);
+    stage_norm<D, TINY_EPS>(p, k, one, p.rope_k_pos0 + j0, p.Sk - 1 - j0, qt, lane);
     if (wave == 0) stage_plain<D>(v, vtile, lane);
     __syncthreads();
 #pragma unroll
@@ -628,7 +639,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dkdv_f32_kernel(KA
 
   for (; it < n_it; it += step) {
     const int i0 = it * kRows;
-    stage_norm<D>(p, qraw, gs, p.rope_q_pos0 + i0, p.Sq - 1 - i0, qt, lane);
+    stage_norm<D, TINY_EPS>(p, qraw, gs, p.rope_q_pos0 + i0, p.Sq - 1 - i0, qt, lane);
     stage_plain<D>(draw, dt, lane);
     if (hh == 0) { stat[wave][0][ln] = lse_l * kLog2e; stat[wave][1][ln] = delta_l; }
     wave_sync();
@@ -736,11 +747,21 @@ __global__ __launch_bounds__(kThreads) void bwd_finish_f32_kernel(KArgs a) {
   }
 }
 
-template <int D>
+template <int D, bool TINY_EPS>
+int launch_fwd(const KArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((fwd_f32_kernel<D, TINY_EPS>), dim3((unsigned)f32_dq_grid(a.p)), dim3(kThreads), 0, st, a);
+  return (int)hipGetLastError();
+}
+template <int D, bool TINY_EPS>
+int launch_dq(const KArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((bwd_dq_f32_kernel<D, TINY_EPS>), dim3((unsigned)f32_dq_grid(a.p)), dim3(kThreads), 0, st, a);
+  return (int)hipGetLastError();
+}
+template <int D, bool TINY_EPS>
 int launch_dkdv(const KArgs& a, hipStream_t st) {
   const segpt_attn_params& p = a.p;
   const int n_kt = (p.Sk + kRows - 1) / kRows;
-  hipLaunchKernelGGL(bwd_dkdv_f32_kernel<D>, dim3((unsigned)(n_kt * p.B * p.H * a.f32_splits)), dim3(kThreads), 0, st, a);
+  hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, TINY_EPS>), dim3((unsigned)(n_kt * p.B * p.H * a.f32_splits)), dim3(kThreads), 0, st, a);
   const int rc = (int)hipGetLastError();
   if (rc) return rc;
   hipLaunchKernelGGL(bwd_finish_f32_kernel<D>, dim3((unsigned)(a.n_dkdv_blocks + 1)), dim3(kThreads), 0, st, a);
@@ -764,32 +785,31 @@ int f32_dkdv_splits(const segpt_attn_params& p) {
 }
 
 int launch_fwd_f32(const KArgs& a, hipStream_t st) {
-  const dim3 grid((unsigned)f32_dq_grid(a.p)), block(kThreads);
+  const bool tiny = tiny_eps(a.p);
   switch (a.p.D) {
-    case 32: hipLaunchKernelGGL(fwd_f32_kernel<32>, grid, block, 0, st, a); break;
-    case 64: hipLaunchKernelGGL(fwd_f32_kernel<64>, grid, block, 0, st, a); break;
-    case 128: hipLaunchKernelGGL(fwd_f32_kernel<128>, grid, block, 0, st, a); break;
+    case 32: return tiny ? launch_fwd<32, true>(a, st) : launch_fwd<32, false>(a, st);
+    case 64: return tiny ? launch_fwd<64, true>(a, st) : launch_fwd<64, false>(a, st);
+    case 128: return tiny ? launch_fwd<128, true>(a, st) : launch_fwd<128, false>(a, st);
     default: return (int)hipErrorInvalidValue;
   }
-  return (int)hipGetLastError();
 }
 
 int launch_bwd_dq_f32(const KArgs& a, hipStream_t st) {
-  const dim3 grid((unsigned)f32_dq_grid(a.p)), block(kThreads);
+  const bool tiny = tiny_eps(a.p);
   switch (a.p.D) {
-    case 32: hipLaunchKernelGGL(bwd_dq_f32_kernel<32>, grid, block, 0, st, a); break;
-    case 64: hipLaunchKernelGGL(bwd_dq_f32_kernel<64>, grid, block, 0, st, a); break;
-    case 128: hipLaunchKernelGGL(bwd_dq_f32_kernel<128>, grid, block, 0, st, a); break;
+    case 32: return tiny ? launch_dq<32, true>(a, st) : launch_dq<32, false>(a, st);
+    case 64: return tiny ? launch_dq<64, true>(a, st) : launch_dq<64, false>(a, st);
+    case 128: return tiny ? launch_dq<128, true>(a, st) : launch_dq<128, false>(a, st);
     default: return (int)hipErrorInvalidValue;
   }
-  return (int)hipGetLastError();
 }
 
 int launch_bwd_dkdv_f32(const KArgs& a, hipStream_t st) {
+  const bool tiny = tiny_eps(a.p);
   switch (a.p.D) {
-    case 32: return launch_dkdv<32>(a, st);
-    case 64: return launch_dkdv<64>(a, st);
-    case 128: return launch_dkdv<128>(a, st);
+    case 32: return tiny ? launch_dkdv<32, true>(a, st) : launch_dkdv<32, false>(a, st);
+    case 64: return tiny ? launch_dkdv<64, true>(a, st) : launch_dkdv<64, false>(a, st);
+    case 128: return tiny ? launch_dkdv<128, true>(a, st) : launch_dkdv<128, false>(a, st);
     default: return (int)hipErrorInvalidValue;
   }
 }

@@ -102,6 +102,28 @@ def test_fp32_tile_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_rows_whose_mean_square_leaves_the_normal_range(gpu_device, D):
+    """A key whose sum of squares overflows has the normaliser 0, like a key of zeros, and poisons nobody; keys so small
+    that their mean square is subnormal (eps = 0) are normalised like any others."""
+    x = gen(1, 2, 1, 70, 70, D, F32, seed=65)
+    row = lambda k, j, f: torch.cat([k[:, :, :j], k[:, :, j:j + 1] * f, k[:, :, j + 1:]], 2)
+    print(f"huge key, D={D}", flush=True)
+    got = run_gpu(dict(x, k=row(x["k"], 33, 1e25)), gpu_device)
+    ref = run_oracle(dict(x, k=row(x["k"], 33, 0.0)))
+    compare(got, ref, F32, names=["y", "lse", "dq", "dv", "dg_q", "dg_k"])
+    assert (got["dk"][:, :, 33] == 0).all()
+    keep = [j for j in range(70) if j != 33]
+    compare({"dk": got["dk"][:, :, keep]}, {"dk": ref["dk"][:, :, keep]}, F32)
+    print(f"tiny keys, D={D}", flush=True)
+    small = dict(x, k=x["k"] * torch.where(torch.arange(70) % 3 == 0, 1e-20, 1.0).reshape(1, 1, 70, 1))
+    got, ref = (f(small, backward=False, eps=0.0) for f in (lambda x, **kw: run_gpu(x, gpu_device, **kw), run_oracle))
+    # a square of 1e-40 is rounded to a multiple of 2^-149, 0.7e-5 of it, and so is their mean: up to 0.7e-5 on the key and,
+    # logits of up to about 5, 4e-5 on a probability
+    for n in ("y", "lse"):
+        assert (got[n].double() - ref[n].reshape(got[n].shape)).abs().max() < 1e-4, n
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_forward_rounding_does_not_grow_with_the_head_size(gpu_device, D):
     """Scores are sums of D products; added up one after the other their error grows with D and y's distance to float64
     was 2.9e-7 in norm for a call of this length at head_dim 128.  Bound: four roundings of half a unit in the last place
