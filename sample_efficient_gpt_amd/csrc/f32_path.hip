@@ -74,6 +74,9 @@ __device__ __forceinline__ f32x16 add_chains(f32x16 (&s)[N]) {
       for (int r = 0; r < 16; ++r) s[i][r] += s[i + n][r];
   return s[0];
 }
+// probability of a score that carries log2 e, from the row's natural lse: one rounding, of the difference (lse * log2 e
+// rounded first is off by half a unit at |lse|, for every key of the row alike)
+__device__ __forceinline__ float prob(float s, float lse) { return __builtin_amdgcn_exp2f(fmaf(lse, -kLog2e, s)); }
 __device__ __forceinline__ int crow(int r, int hh) { return 8 * (r >> 2) + 4 * hh + (r & 3); }
 
 // Work items are listed heaviest first.  When the whole grid is resident at once (up to two workgroups on each of 256
@@ -489,7 +492,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dq_f32_kernel(KArg
     df[c] = frag_rm<D>(vt, c, lane);
   }
   const float delta = dsm[wave][ln];
-  const float lse2 = p.lse[row_base + min(q0 + ln, p.Sq - 1)] * kLog2e;
+  const float lse = p.lse[row_base + min(q0 + ln, p.Sq - 1)];
   wave_sync();
   f32x4v kraw[T::kPasses], vraw[T::kPasses];
   if (wave < n_kt) {
@@ -516,7 +519,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dq_f32_kernel(KArg
     f32x16 s = product_rm<D, 2>(kt, qf, lane);
     const f32x16 dp = product_rm<D, 2>(vt, df, lane);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(s[r] - lse2);
+    for (int r = 0; r < 16; ++r) s[r] = prob(s[r], lse);
     if (jt >= n_full) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
@@ -641,7 +644,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dkdv_f32_kernel(KA
     const int i0 = it * kRows;
     stage_norm<D, TINY_EPS>(p, qraw, gs, p.rope_q_pos0 + i0, p.Sq - 1 - i0, qt, lane);
     stage_plain<D>(draw, dt, lane);
-    if (hh == 0) { stat[wave][0][ln] = lse_l * kLog2e; stat[wave][1][ln] = delta_l; }
+    if (hh == 0) { stat[wave][0][ln] = lse_l; stat[wave][1][ln] = delta_l; }
     wave_sync();
     if (it + step < n_it) request(it + step);
     f32x16 s = product_rm<D, kSums>(qt, kf, lane);
@@ -650,7 +653,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dkdv_f32_kernel(KA
     for (int q = 0; q < 4; ++q) {
       const f32x4v ls = *reinterpret_cast<const f32x4v*>(&stat[wave][0][8 * q + 4 * hh]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[4 * q + e] = __builtin_amdgcn_exp2f(s[4 * q + e] - ls[e]);
+      for (int e = 0; e < 4; ++e) s[4 * q + e] = prob(s[4 * q + e], ls[e]);
     }
     if (i0 + kRows > p.Sq || (p.causal && j0 + kRows - 1 > i0 + p.q_start)) {
 #pragma unroll

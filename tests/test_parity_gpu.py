@@ -137,6 +137,29 @@ def test_fp32_forward_rounding_does_not_grow_with_the_head_size(gpu_device, D):
     assert (y.cpu().double() - ref).norm() <= 4 * 2.0**-24 * ref.norm()
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_backward_rounds_the_row_statistic_once(gpu_device, D):
+    """Two keys of one and the same large score (46 to 63, exact in every order of summation): both probabilities are 1/2, and what
+    the backward makes of them shows the error of exp(score - lse) alone.  Bound: lse below 64 is stored to half a unit, 2^-19; the
+    two constants ln 2 and log2 e miss 1 by 1.1e-8, 7e-7 at 64; exponential, logarithm and products 3e-7.  With lse * log2 e
+    rounded as well it was up to 2.6e-6 more."""
+    n = 512
+    z = lambda s: torch.zeros(n, 1, s, D, device=gpu_device)
+    q, k, v, dy = z(1), z(2), z(2), z(1)
+    q[..., 0] = 46.0 + 17.0 * torch.arange(n, device=gpu_device).reshape(n, 1, 1) / n
+    k[..., 0] = 1.0
+    k[:, :, 1, 1] = 1.0
+    v[:, :, 0, 0], v[:, :, 1, 0] = 1.0, -1.0
+    dy[..., 0] = 1.0
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    y = qknorm_attention(q, k, v, torch.ones(1, device=gpu_device), sm_scale=1.0, q_start=1, qk_norm=False)
+    dq, dv = torch.autograd.grad(y, [q, v], dy)
+    bound = 2.0**-19 + 7e-7 + 3e-7
+    assert (2 * dv[..., 0] - 1).abs().max() <= bound   # p
+    assert (2 * dq[..., 1] + 1).abs().max() <= bound   # p (dp - delta) of the second key
+
+
 # ------------------------------------------------------------------ bf16 MFMA path
 
 
