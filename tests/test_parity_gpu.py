@@ -138,6 +138,21 @@ def test_fp32_forward_rounding_does_not_grow_with_the_head_size(gpu_device, D):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_dq_rounding_does_not_grow_with_the_head_size(gpu_device, D):
+    """dq's scores and its products with dO are sums of D products as well: two sums each put it 6.2 units of 2^-24 from float64 in
+    norm for a call of this length at head_dim 128.  Bound: 5.7, what plain FMA loops with four sums a row reached (5.6)."""
+    rng = torch.Generator().manual_seed(D)
+    ops = torch.randn(3, 4, 212, D, generator=rng), torch.randn(3, 2, 212, D, generator=rng), torch.randn(3, 2, 212, D, generator=rng)
+    dy = torch.randn(3, 4, 212, D, generator=rng)
+    one = torch.ones(1)
+    wide = [t.double().requires_grad_(True) for t in ops]
+    ref, = torch.autograd.grad(orc.attention_forward(*wide, one.double(), qk_norm=False)[0], wide[0], dy.double())
+    q, k, v = (t.to(gpu_device).requires_grad_(True) for t in ops)
+    dq, = torch.autograd.grad(qknorm_attention(q, k, v, one.to(gpu_device), qk_norm=False), q, dy.to(gpu_device))
+    assert (dq.cpu().double() - ref).norm() <= 5.7 * 2.0**-24 * ref.norm()
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_backward_rounds_the_row_statistic_once(gpu_device, D):
     """Two keys of one and the same large score (46 to 63, exact in every order of summation): both probabilities are 1/2, and what
     the backward makes of them shows the error of exp(score - lse) alone.  Bound: lse below 64 is stored to half a unit, 2^-19; the
