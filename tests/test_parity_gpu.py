@@ -154,25 +154,29 @@ def test_fp32_dq_rounding_does_not_grow_with_the_head_size(gpu_device, D):
 
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_backward_rounds_the_row_statistic_once(gpu_device, D):
-    """Two keys of one and the same large score (46 to 63, exact in every order of summation): both probabilities are 1/2, and what
-    the backward makes of them shows the error of exp(score - lse) alone.  Bound: lse below 64 is stored to half a unit, 2^-19; the
-    two constants ln 2 and log2 e miss 1 by 1.1e-8, 7e-7 at 64; exponential, logarithm and products 3e-7.  With lse * log2 e
-    rounded as well it was up to 2.6e-6 more."""
-    n = 512
-    z = lambda s: torch.zeros(n, 1, s, D, device=gpu_device)
-    q, k, v, dy = z(1), z(2), z(2), z(1)
-    q[..., 0] = 46.0 + 17.0 * torch.arange(n, device=gpu_device).reshape(n, 1, 1) / n
+    """All keys have one and the same large score (46 to 60, exact in every order of summation): row i's probabilities are 1/(i+1),
+    and what the backward makes of them shows the error of exp(score - lse) alone.  Bound, relative: lse below 64 is stored to half
+    a unit, 2^-19; the two constants ln 2 and log2 e miss 1 by 1.1e-8, 7e-7 at 64; exponential, logarithm and products 3e-7.
+    With lse * log2 e rounded as well it was up to 2.6e-6 more (5.1e-6 on these inputs)."""
+    n, S = 64, 32
+    eye = torch.eye(S, device=gpu_device)
+    q, k, v, dy = (torch.zeros(n, 1, S, D, device=gpu_device) for _ in range(4))
+    q[..., 0] = 46.0 + 14.0 * torch.arange(n, device=gpu_device).reshape(n, 1, 1) / n
+    k[..., :S] = eye
     k[..., 0] = 1.0
-    k[:, :, 1, 1] = 1.0
-    v[:, :, 0, 0], v[:, :, 1, 0] = 1.0, -1.0
-    dy[..., 0] = 1.0
+    sign = 1.0 - 2.0 * (torch.arange(S, device=gpu_device) % 2)
+    v[..., :S] = sign.unsqueeze(1)
+    dy[..., :S] = eye
     for t in (q, k, v):
         t.requires_grad_(True)
-    y = qknorm_attention(q, k, v, torch.ones(1, device=gpu_device), sm_scale=1.0, q_start=1, qk_norm=False)
-    dq, dv = torch.autograd.grad(y, [q, v], dy)
+    y = qknorm_attention(q, k, v, torch.ones(1, device=gpu_device), sm_scale=1.0, qk_norm=False)
+    dq, dv = (t.double() for t in torch.autograd.grad(y, [q, v], dy))
+    p = torch.tril(torch.ones(S, S, dtype=torch.float64, device=gpu_device)) / torch.arange(1, S + 1, device=gpu_device).unsqueeze(1)
+    ds = p * (sign - (p * sign).sum(-1, keepdim=True))  # dp_ij = sign_j
     bound = 2.0**-19 + 7e-7 + 3e-7
-    assert (2 * dv[..., 0] - 1).abs().max() <= bound   # p
-    assert (2 * dq[..., 1] + 1).abs().max() <= bound   # p (dp - delta) of the second key
+    assert bool(((dv[..., :S].transpose(2, 3) - p).abs() <= bound * p).all())
+    # from the second row on (the first has p (dp - delta) = 0); delta carries y's rounding, 2e-7
+    assert bool(((dq[:, :, 1:, 1:S] - ds[1:, 1:]).abs() <= bound * ds[1:, 1:].abs() + 2e-7 * p[1:, 1:]).all())
 
 
 # ------------------------------------------------------------------ bf16 MFMA path
@@ -271,20 +275,33 @@ def test_bf16_forward_and_dq_workgroup_shapes(gpu_device, B, H, Hkv, Sq, Sk, D, 
     _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, D, seed=62, gen_kw=gen_kw, **kw)
 
 
-def test_bf16_forward_parts_with_scales_beyond_the_bound(gpu_device):
-    """Scale vectors too large for the fixed softmax reference (known on the device only): the two waves of a pair then
-    keep a running one each, and the early rows' second wave sees no key at all."""
-    x = gen(1, 2, 1, 150, 150, 64, BF16, seed=63)
-    x["g_q"] = x["g_q"] * 7.0
-    print("scales beyond the bound", flush=True)
-    ref = run_oracle(x, backward=False)
-    got = run_gpu(x, gpu_device, backward=False)
-    full = run_gpu(dict(x, g_q=x["g_q"].clone()), gpu_device)  # the training forward: never split over workgroups
-    # |logit| <= sqrt(64) * 7 * max g: exp2 arguments carry a relative 2^-8 of two bf16 operands' rounding, 0.25 in the worst
-    # row; the oracle comparison takes the operands' rounding out by tolerance, the two launches have it in common
-    assert torch.isfinite(full["y"].float()).all()
-    assert (full["lse"].double().cpu() - ref["lse"].double().reshape(full["lse"].shape)).abs().max() < 0.25
-    assert (got["lse"].double() - full["lse"].double()).abs().max() < 2.0**-8
+@pytest.mark.parametrize("D,gain", [(64, 7.0), (128, 5.0)])
+def test_bf16_forward_parts_with_scales_beyond_the_bound(gpu_device, D, gain):
+    """Scale vectors too large for the fixed softmax reference (known on the device only): the two waves of a pair then keep a
+    running one each, and the early rows' second wave sees no key at all.  y against the float64 model that rounds where the
+    kernels do, at the ordinary tolerance; lse against the launch whose waves each see all keys: a row sum adds bf16 probabilities
+    (8 significant bits), each rounded by up to 2^-8 of itself against either launch's own reference, 2^-7 between the two."""
+    import tests.parity_util as pu
+    from sample_efficient_gpt_amd import _lib
+    from sample_efficient_gpt_amd.plan import AttnPlan
+
+    x = gen(1, 2, 1, 150, 150, D, BF16, seed=63)
+    x["g_q"] = x["g_q"] * gain
+    assert float((x["g_q"] * x["g_k"]).abs().max()) * D**0.5 * 1.4427 * 1.02 > 64.0
+    flat = lambda t, r=1: t.repeat_interleave(r, dim=1).flatten(0, 1)
+    model = pu.kernel_rounding_model(flat(x["q"]), flat(x["k"], 2), flat(x["v"], 2), x["g_q"].double() * x["g_k"].double(), flat(x["d_o"]),
+                                     eps=1e-6, sm_scale=D**-0.5, causal=True, q_start=0)["y"]
+    plan = AttnPlan({n: (t.to(gpu_device) if t is not None else None) for n, t in x.items()}, backward=False)
+    print(f"scales beyond the bound, D={D}", flush=True)
+    plan.forward()
+    parts = {"y": plan.y.cpu(), "lse": plan.lse.cpu()}
+    plan.forward(flags=_lib.SEGPT_FLAG_RUNNING_MAX)  # always 128-row workgroups
+    whole = {"y": plan.y.cpu(), "lse": plan.lse.cpu()}
+    for got in (parts, whole):
+        err = (got["y"].double().flatten(0, 1) - model).abs()
+        assert bool((err <= 2e-2 + 1e-2 * model.abs()).all()), float(err.max())
+    assert not torch.equal(parts["lse"], whole["lse"])  # two different launches
+    assert (parts["lse"] - whole["lse"]).abs().max() < 2.0**-7
 
 
 def test_bf16_gate_scale_not_positive_takes_the_gated_copy(gpu_device):
