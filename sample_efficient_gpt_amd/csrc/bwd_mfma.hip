@@ -95,7 +95,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   constexpr int MB = D / 32;
   constexpr int kStageBytes = 2 * Z::kTileBytes;
   // the pipeline's numbers: ring_protocol.hpp
-  constexpr ring::Protocol R = ROPE ? ring::dq_rope(Z::kPasses) : ring::dq(Z::kPasses);
+  constexpr ring::Protocol R = PARTS == 1 ? (ROPE ? ring::dq_rope(Z::kPasses) : ring::dq(Z::kPasses))
+                                          : (ROPE ? ring::dq_rope_parts(Z::kPasses) : ring::dq_parts(Z::kPasses));
   static_assert(ring::well_formed(R) && R.stages == kStages && !R.issue_at_top, "tile pipeline");
   static_assert(ROPE ? (R.pre_row_stages == 4 && R.row_stages == 1 && R.early_tiles == R.startup_tiles && !R.wait_before_loop && R.epilogue_row_stages == 2)
                      : (R.pre_row_stages == 0 && R.row_stages == 3 && R.wait_before_loop && R.epilogue_row_stages == 0), "tile pipeline");
@@ -429,8 +430,9 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   // below, which reuses the ring, behind every wave's reads.
   // PARTS == 2: part 1 leaves its T^T in the idle stage 2 (one slot per wave, 16 bytes per lane and access: conflict-free)
   // and is done but for the column sums; part 0 adds it to its own.
-  char* const slot = lds + 2 * kStageBytes + row_wave * (MB * 4096) + lane * 16;
-  static_assert(PARTS == 1 || (kRowWaves * MB * 4096 <= 2 * kStageBytes && BQ * kRedStride * 4 <= 2 * kStageBytes), "slots behind the dg staging area");
+  char* const slot = lds + R.merge_stage_first * kStageBytes + row_wave * (MB * 4096) + lane * 16;
+  static_assert(PARTS == 1 || (kRowWaves * MB * 4096 <= R.merge_stages * kStageBytes && BQ * kRedStride * 4 <= R.scratch_stages * kStageBytes &&
+                               R.scratch_stages <= R.merge_stage_first), "slots behind the dg staging area");
   if constexpr (PARTS == 2) {
     if (part == 1) {
 #pragma unroll
@@ -557,7 +559,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   constexpr int KS = D / 16;
   constexpr int MB = D / 32;
   constexpr int kStageBytes = 2 * Z::kTileBytes;
-  constexpr ring::Protocol R = ring::dkdv(Z::kPasses);  // the pipeline's numbers: ring_protocol.hpp
+  constexpr ring::Protocol R = PARTS == 1 ? ring::dkdv(Z::kPasses) : ring::dkdv_parts(Z::kPasses);  // the pipeline's numbers: ring_protocol.hpp
   static_assert(ring::well_formed(R) && R.stages == kStages && R.row_stages == 2 && !R.wait_before_loop && !R.issue_at_top, "tile pipeline");
   static_assert(R.early_tiles >= ring::kTilesNeededAtLoopStart, "the loop is entered without a further wait");
   static_assert(R.loads_per_tile == 2 * Z::kPasses + 1, "per wave: the two tiles plus one row-statistics load");
@@ -812,7 +814,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   // passed the last iteration's barrier), and from there in the accumulators' layout.  Read row-per-lane from global
   // memory, 8 bytes per lane, every wave-wide load would touch 32 cache lines and the three tensors would keep the
   // address path of the vector memory unit busy for 4-12 us of the launch.
-  static_assert(R.epilogue_row_stages == 3, "k, v, v_first blocks in stages 0, 1, 2");
+  static_assert(R.epilogue_row_stages == (PARTS == 1 ? 3 : 2), "k, v, v_first blocks in stages 0, 1, 2; or in three tiles of stages 0 and 1");
   const bool live = key < p.Sk;
   float c1 = 1.f, c2 = 0.f;
   if (p.vr_coef) { c1 = p.vr_coef[0]; c2 = p.vr_coef[1]; }
@@ -835,8 +837,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
       if (p.vr_coef) issue_tile_pair<D>(fb, fb, tile_lane_offsets<D>(fst, fst, rows_left, src.x, src.y), wave_dst + kStageBytes);
       // The two parts of a key block meet here: part 0 finishes dK, part 1 dV, so each hands the other's half over
       // through the idle stages 2 and 3 (one slot per wave, 16 bytes per lane and access: conflict-free).
-      static_assert(4 * MB * 4096 <= 2 * kStageBytes, "one accumulator per wave in two stages");
-      char* const slot = lds + 2 * kStageBytes + lane * 16;
+      static_assert(4 * MB * 4096 <= R.merge_stages * kStageBytes, "one accumulator per wave in two stages");
+      char* const slot = lds + R.merge_stage_first * kStageBytes + lane * 16;
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -850,7 +852,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
     wait_vmcnt<0>();
     __syncthreads();
     if constexpr (PARTS == 2) {
-      const char* const other = lds + 2 * kStageBytes + lane * 16 + (wave ^ kKeyWaves) * (MB * 4096);
+      const char* const other = lds + R.merge_stage_first * kStageBytes + lane * 16 + (wave ^ kKeyWaves) * (MB * 4096);
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
 #pragma unroll

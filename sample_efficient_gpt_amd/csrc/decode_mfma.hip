@@ -17,6 +17,7 @@
 #include <algorithm>
 
 #include "mfma_common.hpp"
+#include "ring_protocol.hpp"
 
 namespace segpt {
 namespace {
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(kDecThreads, (kDecOcc<D, ROPE, VRES>)) void decode_
   // again as soon as its last reader has its fragments, so K is in flight during the softmax and the V product, V during
   // the next block's scores.  Order of the requests: [tables, K, V, V_first] of block 0, then tables, K, V, V_first of
   // each next block; every wait below leaves exactly the younger ones in flight.
-  constexpr int kTabLoads = TABLES ? 2 * Z::kPasses : 0, kRowLoads = WaveTile<D>::kLoads, kFirstLoads = VRES ? kRowLoads : 0;
+  constexpr ring::DecodeLoads kLoads{TABLES ? 2 * Z::kPasses : 0, WaveTile<D>::kLoads, VRES ? WaveTile<D>::kLoads : 0};
   const char* kbase = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.k, b, g, 0));
   const char* vbase = reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v, b, g, 0));
   const char* fbase = VRES ? reinterpret_cast<const char*>(row_ptr<uint16_t>(p.v_first, b, g, 0)) : nullptr;
@@ -228,7 +229,7 @@ __global__ __launch_bounds__(kDecThreads, (kDecOcc<D, ROPE, VRES>)) void decode_
   wave_lds_sync();
   for (int jb = first; jb < k_hi; jb += kStep) {
     const bool more = jb + kStep < k_hi;
-    if (active) wait_vmcnt<kRowLoads + kFirstLoads>();  // this block's tables and K
+    if (active) wait_vmcnt<ring::decode_kept_at_top(kLoads)>();  // this block's tables and K
     else wait_vmcnt<0>();
     if constexpr (TABLES) {
       __syncthreads();  // every wave's pieces of the tables are there, and nobody reads the other buffer any more
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(kDecThreads, (kDecOcc<D, ROPE, VRES>)) void decode_
       m_run = m_new;
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r] - mu);
-      if (more) wait_vmcnt<kTabLoads + kRowLoads>(); else wait_vmcnt<0>();  // this block's V (and V_first)
+      if (more) wait_vmcnt<ring::decode_kept_before_v(kLoads, true)>(); else wait_vmcnt<ring::decode_kept_before_v(kLoads, false)>();  // this block's V (and V_first)
       const bf16x8 pb[2] = {pack_c_half_sum(s, 0, l_run), pack_c_half_sum(s, 1, l_run)};
       wave_lds_sync();
 #pragma unroll

@@ -115,7 +115,7 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE, PARTS>::kOcc)) void f
   // same time, the scale vector behind them: one memory round trip.  The remaining start-up tiles follow once the
   // query rows sit in registers (run() below).
   constexpr int kQStages = (BQ + 2 * BK - 1) / (2 * BK);  // a stage holds two tiles of BK rows
-  constexpr ring::Protocol R = ring::forward(NS, kQStages, Z::kPasses);  // the pipeline's numbers: ring_protocol.hpp
+  constexpr ring::Protocol R = PARTS == 1 ? ring::forward(NS, kQStages, Z::kPasses) : ring::forward_parts(NS, kQStages, Z::kPasses);  // the pipeline's numbers: ring_protocol.hpp
   static_assert(ring::well_formed(R) && R.loads_per_tile == kLoadsPerTile && !R.wait_before_loop && R.issue_at_top, "tile pipeline");
   static_assert(R.early_tiles >= ring::kTilesNeededAtLoopStart, "the loop is entered without a further wait");
 #pragma unroll
@@ -343,9 +343,10 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE, PARTS>::kOcc)) void f
     // The ring is idle (every wave has passed the last iteration's barrier): part 1 leaves its state there, 16 (8) bytes
     // per lane and access, one slot per wave, and part 0 takes it over.
     constexpr int kSlot = MB * 4096;
-    static_assert(2 * kSlot + 2 * 512 <= NS * kStageBytes, "two slots in the ring");
-    char* const slot = lds + row_wave * kSlot + lane * 16;
-    float2* const stat = reinterpret_cast<float2*>(lds + 2 * kSlot + row_wave * 512) + lane;
+    static_assert(2 * kSlot + 2 * 512 <= R.merge_stages * kStageBytes, "two slots in the ring");
+    char* const slots = lds + R.merge_stage_first * kStageBytes;
+    char* const slot = slots + row_wave * kSlot + lane * 16;
+    float2* const stat = reinterpret_cast<float2*>(slots + 2 * kSlot + row_wave * 512) + lane;
     if (part == 1) {
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)

@@ -1,4 +1,4 @@
-// The tile pipeline of the three ring kernels (forward, dQ, dK/dV), written once as data.
+// The tile pipeline of the three ring kernels (forward, dQ, dK/dV), written once as data; behind them that of the decode kernel.
 //
 // Streamed 64-row tile pairs travel global -> LDS by direct loads that the compiler cannot see, into a ring of
 // `stages` LDS stages (tile t lives in stage t % stages); completion is tracked by hand with s_waitcnt vmcnt(N)
@@ -36,6 +36,10 @@ struct Protocol {
                             // barrier) up to this many row blocks for the epilogue are requested into stages
                             // [0, epilogue_row_stages), awaited, published by one barrier and read into registers
   bool epilogue_reuses_ring = false;  // the epilogue afterwards writes scratch data over the ring's stages
+  int merge_stage_first = 0;  // two waves share the rows of a block: behind the loop they hand accumulators over through
+  int merge_stages = 0;       // stages [merge_stage_first, merge_stage_first + merge_stages): plain stores beside the row
+                              // requests above, read behind the same barrier
+  int scratch_stages = 0;     // with epilogue_reuses_ring: how many stages from 0 on the scratch data takes (0: all)
 };
 
 // An iteration needs its own tile and the next one landed.
@@ -71,12 +75,43 @@ constexpr Protocol dq_rope(int passes) { return Protocol{4, 2 * passes, 3, 3, 1,
 // Behind the loop: the raw k block (and, with a value residual, the raw v and v_first blocks) for the epilogue.
 constexpr Protocol dkdv(int passes) { return Protocol{4, 2 * passes + 1, 2, 2, 2, 3, false, false, 3, 1, 0, 3, false}; }
 
+// The same kernels in 64-row workgroups whose waves split the blocks of a tile.  The forward uses the ring behind its loop for the
+// hand-over alone; dQ leaves stages 2 and 3 to it and its scratch data to 0 and 1 (no barrier between reading
+// the one and writing the other); dK/dV's row blocks are half as large and end before stage 2.
+constexpr Protocol merging(Protocol p, int first, int stages, int scratch_stages = 0, int epilogue_row_stages = -1) {
+  p.merge_stage_first = first;
+  p.merge_stages = stages;
+  p.scratch_stages = scratch_stages;
+  if (epilogue_row_stages >= 0) p.epilogue_row_stages = epilogue_row_stages;
+  return p;
+}
+constexpr Protocol forward_parts(int stages, int q_stages, int passes) { return merging(forward(stages, q_stages, passes), 0, 2); }
+constexpr Protocol dq_parts(int passes) { return merging(dq(passes), 2, 2, 2); }
+constexpr Protocol dq_rope_parts(int passes) { return merging(dq_rope(passes), 2, 2, 2, 1); }
+constexpr Protocol dkdv_parts(int passes) { return merging(dkdv(passes), 2, 2, 0, 2); }
+
 constexpr bool well_formed(const Protocol& p) {
   return p.stages >= 3 && p.early_tiles >= 1 && p.early_tiles <= p.startup_tiles && p.startup_tiles <= p.stages - 1 &&
          p.row_stage_first >= p.early_tiles && p.row_stage_first + p.row_stages <= p.stages && p.keep_tiles >= 0 &&
          p.issue_ahead >= kTilesNeededAtLoopStart && p.pre_row_stages >= 0 && p.pre_row_stages <= p.stages &&
-         p.epilogue_row_stages >= 0 && p.epilogue_row_stages <= p.stages;
+         p.epilogue_row_stages >= 0 && p.epilogue_row_stages <= p.stages &&
+         (p.merge_stages == 0 || (p.merge_stage_first >= p.epilogue_row_stages || p.epilogue_row_stages == 0)) &&
+         p.merge_stage_first + p.merge_stages <= p.stages;
 }
+
+// ---- the split-key decode kernel: one buffer per wave for the K, V (and V_first) rows of a block, two for the table rows of
+// a block, which the four waves of a workgroup share.  Requests in order: [tables, K, V, V_first] of the wave's first block, all
+// awaited; per block: wait, [barrier, tables of the next block into the other buffer], K read, K of the next block, wait, V
+// (and V_first) read, V and V_first of the next block.  Loads of one wave:
+struct DecodeLoads {
+  int tables;  // per block; 0 without staged tables
+  int rows;    // per tensor and block
+  int first;   // V_first; 0 without a value residual
+};
+// the wait at the top of a block: its tables and K have landed, its V and V_first are younger
+constexpr int decode_kept_at_top(const DecodeLoads& d) { return d.rows + d.first; }
+// the wait before the V product: the next block's tables and K are younger, if there is a next block
+constexpr int decode_kept_before_v(const DecodeLoads& d, bool more) { return more ? d.tables + d.rows : 0; }
 
 }  // namespace ring
 }  // namespace segpt

@@ -29,10 +29,10 @@ enum Kind { REQUEST, WAIT, BARRIER, READ };
 struct Op {
   Kind kind;
   int stage;    // REQUEST / READ
-  int content;  // REQUEST / READ: tile index >= 0, kRows, kPreRows, kEpilogueRows or kScratch
+  int content;  // REQUEST / READ: tile index >= 0, kRows, kPreRows, kEpilogueRows, kSlots or kScratch
   int n;        // REQUEST: loads issued by the wave (0: plain LDS stores, e.g. the epilogue's scratch); WAIT: the vmcnt immediate
 };
-constexpr int kRows = -1, kPreRows = -3, kEpilogueRows = -5, kScratch = -4;
+constexpr int kRows = -1, kPreRows = -3, kEpilogueRows = -5, kScratch = -4, kSlots = -6;
 
 // The order of operations of one wave, following fwd_mfma.hip / bwd_mfma.hip:
 //   [first start-up phase: row blocks in stages 0 .., wait for everything, barrier, rows -> registers, barrier;]
@@ -40,8 +40,9 @@ constexpr int kRows = -1, kPreRows = -3, kEpilogueRows = -5, kScratch = -4;
 //             [wait + barrier], fragment request of tile 0;
 //   iteration jt: [request at top], blocks of tile jt (its stage; the second block also requests the row-major
 //             fragments of tile jt+1 from the NEXT stage), [request at bottom], wait, barrier;
-//   [behind the loop: `epilogue_rows` row blocks (at most p.epilogue_row_stages) requested into stages 0 .., wait for
-//    everything, barrier, rows -> registers, barrier, scratch stores over the ring].
+//   [behind the loop: `epilogue_rows` row blocks (at most p.epilogue_row_stages) requested into stages 0 .., beside them the
+//    accumulators that two waves hand over (plain stores), wait for everything, barrier, rows and hand-over -> registers,
+//    barrier if there were rows, scratch stores over the ring; dQ reads the hand-over only behind that second barrier].
 std::vector<Op> wave_program(const Protocol& p, int n_tiles, int row_loads_per_stage, int epilogue_rows = 0) {
   std::vector<Op> ops;
   auto request_tile = [&](int t) { ops.push_back({REQUEST, t % p.stages, t, p.loads_per_tile}); };
@@ -76,15 +77,18 @@ std::vector<Op> wave_program(const Protocol& p, int n_tiles, int row_loads_per_s
     ops.push_back({WAIT, 0, 0, segpt::ring::loads_kept_after_iteration(p, requested)});
     ops.push_back({BARRIER, 0, 0, 0});
   }
-  if (epilogue_rows > 0) {
-    for (int i = 0; i < epilogue_rows; ++i) ops.push_back({REQUEST, i, kEpilogueRows, row_loads_per_stage});
+  const int slots_end = p.merge_stage_first + p.merge_stages;
+  for (int i = p.merge_stage_first; i < slots_end; ++i) ops.push_back({REQUEST, i, kSlots, 0});
+  for (int i = 0; i < epilogue_rows; ++i) ops.push_back({REQUEST, i, kEpilogueRows, row_loads_per_stage});
+  if (epilogue_rows > 0 || p.merge_stages > 0) {
     ops.push_back({WAIT, 0, 0, 0});
     ops.push_back({BARRIER, 0, 0, 0});
-    for (int i = 0; i < epilogue_rows; ++i) ops.push_back({READ, i, kEpilogueRows, 0});
-    if (p.epilogue_reuses_ring) ops.push_back({BARRIER, 0, 0, 0});
   }
+  for (int i = 0; i < epilogue_rows; ++i) ops.push_back({READ, i, kEpilogueRows, 0});
+  if (epilogue_rows > 0 && p.epilogue_reuses_ring) ops.push_back({BARRIER, 0, 0, 0});
+  for (int i = p.merge_stage_first; i < slots_end; ++i) ops.push_back({READ, i, kSlots, 0});
   if (p.epilogue_reuses_ring)
-    for (int i = 0; i < p.stages; ++i) ops.push_back({REQUEST, i, kScratch, 0});
+    for (int i = 0; i < (p.scratch_stages ? p.scratch_stages : p.stages); ++i) ops.push_back({REQUEST, i, kScratch, 0});
   return ops;
 }
 
@@ -156,6 +160,79 @@ std::string check(const Protocol& p, int max_tiles, int min_tiles = 1) {
   return "";
 }
 
+// ---- the split-key decode kernel (decode_mfma.hip).  Buffers: the K, V and V_first rows of a block are a wave's own, the table
+// rows (two buffers) the workgroup's.  A private buffer is readable once its loads were retired by a wait and may be requested
+// over once the reads of it have returned (LDS_DONE); a shared one follows the rules of a stage above.
+enum DecodeBuffer { TAB0, TAB1, KBUF, VBUF, FBUF, kDecodeBuffers };
+constexpr Kind LDS_DONE = (Kind)(READ + 1);
+
+// `reads`: false for a wave of the last workgroup without a (batch, kv head) pair, which only brings its pieces of the tables;
+// reading them stands for what the other waves do with those pieces
+std::vector<Op> decode_program(const segpt::ring::DecodeLoads& d, int n_blocks, bool reads) {
+  std::vector<Op> ops;
+  auto request = [&](int buffer, int block, int loads) { if (loads) ops.push_back({REQUEST, buffer, block, loads}); };
+  if (n_blocks > 0) {
+    request(TAB0, 0, d.tables);
+    if (reads) { request(KBUF, 0, d.rows); request(VBUF, 0, d.rows); request(FBUF, 0, d.first); }
+  }
+  ops.push_back({WAIT, 0, 0, 0});
+  for (int n = 0; n < n_blocks; ++n) {
+    const bool more = n + 1 < n_blocks;
+    ops.push_back({WAIT, 0, 0, reads ? segpt::ring::decode_kept_at_top(d) : 0});
+    if (d.tables) {
+      ops.push_back({BARRIER, 0, 0, 0});
+      if (more) request(TAB0 + (n + 1) % 2, n + 1, d.tables);
+      ops.push_back({READ, TAB0 + n % 2, n, 0});
+    }
+    if (reads) {
+      ops.push_back({READ, KBUF, n, 0});
+      ops.push_back({LDS_DONE, 0, 0, 0});
+      if (more) request(KBUF, n + 1, d.rows);
+      ops.push_back({WAIT, 0, 0, segpt::ring::decode_kept_before_v(d, more)});
+      ops.push_back({READ, VBUF, n, 0});
+      if (d.first) ops.push_back({READ, FBUF, n, 0});
+      ops.push_back({LDS_DONE, 0, 0, 0});
+      if (more) { request(VBUF, n + 1, d.rows); request(FBUF, n + 1, d.first); }
+    }
+  }
+  return ops;
+}
+
+std::string replay_decode(const std::vector<Op>& ops) {
+  struct State { int content = -2, pending = 0, retired_epoch = -1, read_epoch = -1; bool read_open = false; } st[kDecodeBuffers];
+  std::vector<std::pair<int, int>> queue;  // (buffer, content), oldest first
+  int epoch = 0;
+  for (size_t i = 0; i < ops.size(); ++i) {
+    const Op& o = ops[i];
+    const std::string at = "op " + std::to_string(i) + ": buffer " + std::to_string(o.stage) + ", block " + std::to_string(o.content) + ": ";
+    const bool shared = o.stage <= TAB1;
+    State& s = st[o.stage];
+    if (o.kind == REQUEST) {
+      if (s.pending > 0) return at + "requested over a block in flight";
+      if (shared ? s.read_epoch >= epoch : s.read_open) return at + "requested over a block that may still be read";
+      s = State{};
+      s.content = o.content; s.pending = o.n;
+      for (int k = 0; k < o.n; ++k) queue.push_back({o.stage, o.content});
+    } else if (o.kind == WAIT) {
+      while ((int)queue.size() > o.n) {
+        State& r = st[queue.front().first];
+        queue.erase(queue.begin());
+        if (--r.pending == 0) r.retired_epoch = epoch;
+      }
+    } else if (o.kind == BARRIER) {
+      ++epoch;
+    } else if (o.kind == LDS_DONE) {
+      for (State& b : st) b.read_open = false;
+    } else {
+      if (s.content != o.content) return at + "read while the buffer holds block " + std::to_string(s.content);
+      if (s.pending > 0 || (shared && s.retired_epoch >= epoch)) return at + "read before it has landed and been published";
+      s.read_epoch = epoch;
+      s.read_open = true;
+    }
+  }
+  return "";
+}
+
 }  // namespace
 
 int main() {
@@ -178,6 +255,32 @@ int main() {
       failures += !v.empty();
     }
   }
+  // 64-row workgroups: a 64-key tile at either head size, two waves per row block
+  for (const int passes : {2, 4}) {
+    const Named shipped[] = {
+        {"forward, two waves per row block", forward_parts(3, 1, passes)},
+        {"dQ, two waves per row block", dq_parts(passes)},
+        {"dQ with a rotary embedding, two waves per row block", dq_rope_parts(passes)},
+        {"dK/dV, two waves per key block", dkdv_parts(passes)},
+    };
+    for (const Named& k : shipped) {
+      const std::string v = check(k.p, 70, k.p.loads_per_tile == 2 * passes + 1 ? 0 : 1);
+      printf("passes %d  %-82s %s\n", passes, k.name, v.empty() ? "ok" : ("VIOLATION: " + v).c_str());
+      failures += !v.empty();
+    }
+  }
+  // decode: a wave loads the 32 rows of a block in 4 (head_dim 64) or 8 accesses, its quarter of a pair of table tiles in 2 or 4
+  for (const int rows : {4, 8})
+    for (const int tables : {0, rows / 2})
+      for (const int first : {0, rows}) {
+        const DecodeLoads d{tables, rows, first};
+        std::string v;
+        for (int n = 0; n <= 40 && v.empty(); ++n)
+          for (const bool reads : {true, false})
+            if (v.empty()) v = replay_decode(decode_program(d, n, reads));
+        printf("decode: %d loads per tensor, %d of tables, %d of the value residual %34s\n", rows, tables, first, v.empty() ? "ok" : ("VIOLATION: " + v).c_str());
+        failures += !v.empty();
+      }
   const int passes = 2;
   // Other ring depths and borrowed-stage layouts the formulas claim to cover (not shipped): must hold as well.
   for (int stages = 3; stages <= 6; ++stages)
@@ -242,6 +345,44 @@ int main() {
   };
   for (const BrokenOps& k : broken_ops) {
     const std::string v = replay(k.p, k.ops);
+    printf("%-104s %s\n", k.name, v.empty() ? "NOT CAUGHT" : ("caught: " + v).c_str());
+    failures += v.empty();
+  }
+  // ---- the hand-over behind the loop
+  const Protocol fp = forward_parts(3, 1, passes), dp = dq_parts(passes);
+  Protocol dp_scratch = dp;
+  dp_scratch.scratch_stages = 0;  // the scale-gradient staging over all of the ring
+  const std::vector<Op> fwd_ops = wave_program(fp, 11, 2 * fp.loads_per_tile);  // the last tile lies in stage 1, a hand-over stage
+  const int fwd_barriers = 2 + 11 + 1;  // start-up, iterations, hand-over
+  const BrokenOps broken_merge[] = {
+      {"forward reading the other wave's accumulators without the barrier behind their stores", fp, drop(fwd_ops, BARRIER, 0)},
+      {"forward storing its accumulators without the barrier that ends the last iteration", fp, drop_nth(fwd_ops, BARRIER, fwd_barriers - 2)},
+      {"dQ staging the scale gradient over the accumulators it is reading", dp_scratch, wave_program(dp_scratch, 12, 2 * dp.loads_per_tile)},
+  };
+  for (const BrokenOps& k : broken_merge) {
+    const std::string v = replay(k.p, k.ops);
+    printf("%-104s %s\n", k.name, v.empty() ? "NOT CAUGHT" : ("caught: " + v).c_str());
+    failures += v.empty();
+  }
+  // ---- decode: a count that is off, a missing wait or barrier
+  const DecodeLoads dl{2, 4, 4};
+  const std::vector<Op> dec = decode_program(dl, 12, true);
+  auto add_to_waits = [](std::vector<Op> ops, int immediate, int more) {
+    for (Op& o : ops)
+      if (o.kind == WAIT && o.n == immediate) o.n += more;
+    return ops;
+  };
+  struct BrokenDecode { const char* name; std::vector<Op> ops; };
+  const BrokenDecode broken_decode[] = {
+      {"decode leaving one load too many in flight at the top of a block", add_to_waits(dec, decode_kept_at_top(dl), 1)},
+      {"decode counting V_first among the loads younger than V", add_to_waits(dec, decode_kept_before_v(dl, true), dl.first)},
+      {"decode awaiting V as if a next block were in flight behind the last one",
+       [&] { std::vector<Op> o = dec; for (size_t i = o.size(); i-- > 0;) if (o[i].kind == WAIT) { o[i].n = dl.tables + dl.rows; break; } return o; }()},
+      {"decode requesting K over the tile it is reading", drop_nth(dec, LDS_DONE, 0)},
+      {"decode reading the tables without the workgroup's barrier", drop_nth(dec, BARRIER, 3)},
+  };
+  for (const BrokenDecode& k : broken_decode) {
+    const std::string v = replay_decode(k.ops);
     printf("%-104s %s\n", k.name, v.empty() ? "NOT CAUGHT" : ("caught: " + v).c_str());
     failures += v.empty();
   }
