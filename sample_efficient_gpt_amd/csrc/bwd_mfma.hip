@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   constexpr ring::Protocol R = PARTS == 1 ? (ROPE ? ring::dq_rope(Z::kPasses) : ring::dq(Z::kPasses))
                                           : (ROPE ? ring::dq_rope_parts(Z::kPasses) : ring::dq_parts(Z::kPasses));
   static_assert(ring::well_formed(R) && R.stages == kStages && !R.issue_at_top, "tile pipeline");
-  static_assert(ROPE ? (R.pre_row_stages == 4 && R.row_stages == 1 && R.early_tiles == R.startup_tiles && !R.wait_before_loop && R.epilogue_row_stages == 2)
+  static_assert(ROPE ? (R.pre_row_stages == 4 && R.row_stages == 1 && R.early_tiles == R.startup_tiles && !R.wait_before_loop && R.epilogue_row_stages == (PARTS == 1 ? 2 : 1))
                      : (R.pre_row_stages == 0 && R.row_stages == 3 && R.wait_before_loop && R.epilogue_row_stages == 0), "tile pipeline");
   const segpt_attn_params& p = a.p;
   __shared__ __attribute__((aligned(1024))) char lds[kStages * kStageBytes];
