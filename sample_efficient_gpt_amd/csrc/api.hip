@@ -70,6 +70,16 @@ bool gated_do_copy(const segpt_attn_params& p) {
   return p.gate.ptr && (p.dtype == SEGPT_DTYPE_FP32 || !(p.gate_scale > 0.f));
 }
 
+// fp32: dK and dV of a key tile come in one part per query head of the group and share of the query tiles, [B * H, splits, Sk, D].
+// A single part per kv head fits into contiguous dk and dv themselves: the finish kernel reads a piece before it writes it.
+bool f32_part_in_place(const segpt_attn_params& p) {
+  auto packed = [&](const segpt_tensor4& t) {
+    const int64_t head = (int64_t)p.Sk * p.D;
+    return t.ptr && t.stride_s == p.D && (t.stride_h == head || p.Hkv == 1) && (t.stride_b == p.Hkv * head || p.B == 1);
+  };
+  return p.H == p.Hkv && f32_dkdv_splits(p) == 1 && packed(p.dk) && packed(p.dv);
+}
+
 WsLayout bwd_layout(const segpt_attn_params& p) {
   WsLayout w;
   size_t off = 0;
@@ -87,7 +97,7 @@ WsLayout bwd_layout(const segpt_attn_params& p) {
   w.dcoef_part = off;
   off += align_up((size_t)dkdv_blocks(p) * 2 * sizeof(float));
   w.f32_dk_part = w.f32_dv_part = off;
-  if (p.dtype == SEGPT_DTYPE_FP32) {
+  if (p.dtype == SEGPT_DTYPE_FP32 && !f32_part_in_place(p)) {
     const size_t part = align_up((size_t)p.B * p.H * f32_dkdv_splits(p) * p.Sk * p.D * sizeof(float));
     w.f32_dv_part = off + part;
     off += 2 * part;
@@ -372,8 +382,9 @@ static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage
   a.dg_part = reinterpret_cast<float*>(ws + w.dg_part);
   a.dcoef_part = reinterpret_cast<float*>(ws + w.dcoef_part);
   if (p->dtype == SEGPT_DTYPE_FP32) {
-    a.f32_dk_part = reinterpret_cast<float*>(ws + w.f32_dk_part);
-    a.f32_dv_part = reinterpret_cast<float*>(ws + w.f32_dv_part);
+    const bool in_place = f32_part_in_place(*p);
+    a.f32_dk_part = reinterpret_cast<float*>(in_place ? p->dk.ptr : ws + w.f32_dk_part);
+    a.f32_dv_part = reinterpret_cast<float*>(in_place ? p->dv.ptr : ws + w.f32_dv_part);
     a.f32_splits = f32_dkdv_splits(*p);
   } else {
     a.nlse2 = reinterpret_cast<float*>(ws + w.nlse2);

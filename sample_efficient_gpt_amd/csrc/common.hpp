@@ -35,6 +35,7 @@ struct KArgs {
   float* fwd_stat;
   int32_t fwd_splits, fwd_chunk;
   // fp32 backward: dKhat and dV of one query head and one share of the query tiles, [B*H, f32_splits, Sk, D] each
+  // (dk and dv themselves where there is one of each per kv head)
   float* f32_dk_part;
   float* f32_dv_part;
   int32_t f32_splits;

@@ -255,6 +255,27 @@ def test_decode_partials_fit_the_scratch_of_a_split(lib, D):
             assert Sk < 256 or part <= keys, (B, H, Hkv, Sq, Sk)
 
 
+def test_fp32_backward_needs_partials_only_where_there_are_several(lib):
+    """dK and dV of a key tile come in one part per query head of the group and share of the query tiles; a single part is formed in
+    contiguous dk and dv and needs no workspace beside the row statistics and the scale-gradient partials (one row of D per 32
+    query rows)."""
+    B, D = 16, 64
+
+    def ws(H, Hkv, S, bshd=False):
+        p = _lib.new_params()
+        p.dtype, p.B, p.H, p.Hkv, p.Sq, p.Sk, p.D, p.causal = _lib.SEGPT_DTYPE_FP32, B, H, Hkv, S, S, D, 1
+        p.dk = p.dv = _lib.Tensor4(4096, S * Hkv * D, *((D, Hkv * D) if bshd else (S * D, D)))
+        return lib.segpt_attn_workspace_bytes(p, _lib.SEGPT_WS_BWD)
+
+    kv = lambda H, S: 2 * B * H * S * D * 4  # dK and dV of H heads
+    small = lambda H, S: B * H * S * 4 + B * H * -(-S // 32) * D * 4
+    for H, S in ((8, 2048), (4, 128), (1, 100)):
+        assert ws(H, H, S) < small(H, S) + kv(H, S) // 16, (H, S)
+    assert ws(8, 8, 2048, bshd=True) >= small(8, 2048) + kv(8, 2048)  # the parts are [B, H, S, D]
+    assert ws(8, 4, 2048) >= small(8, 2048) + kv(8, 2048)
+    assert ws(1, 1, 256) >= small(1, 256) + 2 * kv(1, 256)  # two shares: the launch does not fill the card
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libsegpt_attn.so"))
