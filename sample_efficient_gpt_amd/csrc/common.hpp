@@ -77,19 +77,6 @@ __device__ __forceinline__ float bf16hi(uint32_t w) { return __uint_as_float(w &
 template <typename T>
 struct Elem;
 template <>
-struct Elem<float> {
-  static constexpr int kVec = 4;  // elements per 16-byte access
-  static __device__ __forceinline__ void load(const float* p, float (&out)[4]) {
-    float4 v = *reinterpret_cast<const float4*>(p);
-    out[0] = v.x; out[1] = v.y; out[2] = v.z; out[3] = v.w;
-  }
-  static __device__ __forceinline__ void store(float* p, const float (&in)[4]) {
-    *reinterpret_cast<float4*>(p) = make_float4(in[0], in[1], in[2], in[3]);
-  }
-  static __device__ __forceinline__ float load1(const float* p) { return *p; }
-  static __device__ __forceinline__ void store1(float* p, float v) { *p = v; }
-};
-template <>
 struct Elem<uint16_t> {  // bf16 bits
   static constexpr int kVec = 8;
   static __device__ __forceinline__ void load(const uint16_t* p, float (&out)[8]) {
@@ -103,8 +90,6 @@ struct Elem<uint16_t> {  // bf16 bits
     v.z = pack_bf16x2(in[4], in[5]); v.w = pack_bf16x2(in[6], in[7]);
     *reinterpret_cast<uint4*>(p) = v;
   }
-  static __device__ __forceinline__ float load1(const uint16_t* p) { return bf16_to_f32(*p); }
-  static __device__ __forceinline__ void store1(uint16_t* p, float v) { *p = f32_to_bf16(v); }
 };
 
 template <typename T>

@@ -551,8 +551,10 @@ bool wide_fwd(const segpt_attn_params& p) { return p.D != 64 || p.Sk > 2048; }
 // 512 (72 workgroups) 9.8 / 8.2, 4 x 512 (288) 10.7 / 9.3, 6 x 512 (432) 11.7 / 12.9, 2 x 2048 (576) 34.7 / 28.2, 3 x 2048 (864) 39.8 /
 // 40.9, 1 x 4096 (576) 66.7 / 50.6; 8 / 8 heads, 1 x 4096 (256) 61.2 / 34.1; head_dim 128 (one workgroup per CU with 64-key
 // tiles), 16 / 4 heads, 2 x 512 (128) 13.9 / 10.9, 4 x 512 (256) 14.9 / 16.1, 1 x 2048 (256) 36.7 / 31.2, 2 x 2048 (512) 47 / 60.
-// Without QK-norm (or on request) the softmax keeps a running reference; a row's probabilities are then rounded against
-// ONE reference, whatever the launch, so those calls stay with 1.
+// Calls whose softmax keeps a running reference by their flags stay with 1: with 2 each half rounds its probabilities against a
+// reference of its own, which moves every output within bf16 rounding, and their results are kept as they are.  It is not a
+// matter of accuracy (2.4e-3 to 2.7e-3 from float64 either way) and costs time without QK-norm, 1 against 2: 1 x 512 13.0 / 10.7, 4
+// x 512 14.3 / 12.2, 2 x 2048 41 / 35, 8 / 8 heads, 1 x 4096 87 / 39; head_dim 128, 2 x 512 17.8 / 13.4, 1 x 2048 48 / 36.5.
 int fwd_parts(const segpt_attn_params& p) {
   if (p.flags & (SEGPT_FLAG_RUNNING_MAX | SEGPT_FLAG_NO_NORM)) return 1;
   const int64_t wgs = (int64_t)p.B * p.H * ((p.Sq + 127) / 128), tiles = (p.Sk + kBK - 1) / kBK;
