@@ -185,6 +185,8 @@ const char* segpt_strerror(int code);
  * SEGPT_WS_KV follows p->flags: a decode-shaped forward with SEGPT_FLAG_DECODE needs only the split-key partial
  * results (a small fraction of the cache), every other call the normalised keys (and mixed values), with the flag
  * plus the partial results where splitting the keys pays.
+ * SEGPT_WS_BWD on the fp32 path follows dk and dv: contiguous ones may hold what other strides need scratch for, so size with
+ * the tensors of the call.
  * Replaces the in-op allocations of triton_flash_attn_qknorm.py:286-287 / :320-323: the caller
  * allocates. */
 size_t segpt_attn_workspace_bytes(const segpt_attn_params* p, int which);

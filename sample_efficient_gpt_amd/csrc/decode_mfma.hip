@@ -94,8 +94,8 @@ __device__ __forceinline__ void wait_lds_reads() {
 // Bound by HBM: every K and V row once.  What the memory system needs for that is whole lines and requests that stay in
 // flight, so K, V, V_first and the tables all travel by direct global->LDS loads into swizzled tiles (see the request
 // order below).  Before, every lane loaded 16-byte pieces of its own row and, with a rotary embedding, of the two
-// table rows, by each wave for itself.  Both kernels, B = 32, 18 / 6 heads, 8192 keys, head_dim 64 (403 MB): 121 -> 77.6 us
-// with a rotary embedding, 83 -> 76 without; B = 8, 16 / 4 heads, 5001 keys, head_dim 128 (82 MB): 34.0 -> 23.5 us; MERGED,
+// table rows, by each wave for itself.  Both kernels, B = 32, 18 / 6 heads, 8192 keys, head_dim 64 (403 MB): 121 -> 76.8 us
+// with a rotary embedding, 83 -> 77 without; B = 8, 16 / 4 heads, 5001 keys, head_dim 128 (82 MB): 34.0 -> 22.8 us; MERGED,
 // 4 x 18 / 6 heads, 4 queries, 3000 keys: 18.5 -> 16.1.
 //
 // The operands are rounded where the training kernels round them: keys normalised in fp32, then to bf16; probabilities
