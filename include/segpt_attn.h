@@ -234,6 +234,35 @@ int segpt_attn_fwd_noalloc(const segpt_attn_params* p, void* stream);
 int segpt_kv_append(int dtype, int B, int Hkv, int S, int D, const segpt_tensor4* k, const segpt_tensor4* v,
                     const segpt_tensor4* k_to, const segpt_tensor4* v_to, void* stream);
 
+/* y = x W^T in bf16 (fp32 accumulation) for the few rows of a generation step: up to SEGPT_LINEAR_MAX_SEGMENTS weight matrices
+ * against the same rows in one launch.  Output column j of row m of a segment goes to
+ *   out[m * stride_m + (j / width) * stride_h + j % width]    (elements),
+ * so that a column block of heads can be written straight into a key/value cache.  Replaces the projections of one token,
+ * attention.py:179-182, :248 and :259, and the cache's concatenations, :20-27. */
+#define SEGPT_LINEAR_MAX_ROWS 16
+#define SEGPT_LINEAR_MAX_SEGMENTS 4
+
+typedef struct segpt_linear_segment {
+  const void* w;    /* [n, K] bf16 device */
+  int64_t w_stride; /* elements between rows */
+  void* out;        /* bf16 device */
+  int64_t stride_m, stride_h;
+  int32_t n, width; /* output columns; columns per head */
+} segpt_linear_segment;
+
+typedef struct segpt_linear_rows_params {
+  uint32_t struct_bytes; /* sizeof(segpt_linear_rows_params) */
+  int32_t M, K;          /* rows of x, at most SEGPT_LINEAR_MAX_ROWS; columns, a multiple of 32 */
+  int32_t n_segments;
+  const void* x; /* [M, K] bf16 device */
+  int64_t x_stride;
+  segpt_linear_segment seg[SEGPT_LINEAR_MAX_SEGMENTS];
+} segpt_linear_rows_params;
+
+/* Rows of x and of the weights are whole 16-byte pieces at 16-byte aligned addresses (SEGPT_E_ALIGN / SEGPT_E_STRIDE otherwise,
+ * nothing launched); the outputs must not overlap x, the weights or each other. */
+int segpt_linear_rows(const segpt_linear_rows_params* p, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

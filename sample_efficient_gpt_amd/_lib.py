@@ -36,6 +36,7 @@ EXPORTED_SYMBOLS = (
     "segpt_attn_fwd_stage",
     "segpt_attn_fwd_noalloc",
     "segpt_kv_append",
+    "segpt_linear_rows",
 )
 
 
@@ -73,6 +74,16 @@ class AttnParams(C.Structure):
         ("rope_cos", C.c_void_p), ("rope_sin", C.c_void_p),
         ("rope_len", C.c_int32), ("rope_q_pos0", C.c_int32), ("rope_k_pos0", C.c_int32), ("reserved0", C.c_int32),
     ]
+
+
+class LinearSegment(C.Structure):
+    _fields_ = [("w", C.c_void_p), ("w_stride", C.c_int64), ("out", C.c_void_p), ("stride_m", C.c_int64), ("stride_h", C.c_int64),
+                ("n", C.c_int32), ("width", C.c_int32)]
+
+
+class LinearRowsParams(C.Structure):
+    _fields_ = [("struct_bytes", C.c_uint32), ("M", C.c_int32), ("K", C.c_int32), ("n_segments", C.c_int32),
+                ("x", C.c_void_p), ("x_stride", C.c_int64), ("seg", LinearSegment * 4)]
 
 
 _lib = None
@@ -117,6 +128,8 @@ def load():
         lib.segpt_attn_fwd_noalloc.argtypes = [C.POINTER(AttnParams), C.c_void_p]
         lib.segpt_kv_append.restype = C.c_int
         lib.segpt_kv_append.argtypes = [C.c_int] * 5 + [C.POINTER(Tensor4)] * 4 + [C.c_void_p]
+        lib.segpt_linear_rows.restype = C.c_int
+        lib.segpt_linear_rows.argtypes = [C.POINTER(LinearRowsParams), C.c_void_p]
         ver = lib.segpt_abi_version()
         if ver != SEGPT_ABI_VERSION:
             raise RuntimeError(f"libsegpt_attn.so ABI version {ver}, binding expects {SEGPT_ABI_VERSION}")

@@ -13,7 +13,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libsegpt_attn.so")
 BINDING_PATH = os.path.join(PKG_DIR, "_segpt_torch.so")  # native host side for PyTorch callers, linked against LIB_PATH
-SOURCES = ["api.hip", "f32_path.hip", "pre_post.hip", "fwd_mfma.hip", "bwd_mfma.hip", "decode_mfma.hip"]
+SOURCES = ["api.hip", "f32_path.hip", "pre_post.hip", "fwd_mfma.hip", "bwd_mfma.hip", "decode_mfma.hip", "linear_rows.hip"]
 # Per-source flags.  The forward never needs more than 256 registers, but at head_dim 128 it runs one
 # workgroup per CU and the compiler would then move every MFMA result into the accumulation registers
 # (one v_accvgpr_read per score before exp2); keeping the ordinary-register form is 8 % faster there.

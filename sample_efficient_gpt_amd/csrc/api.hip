@@ -365,6 +365,28 @@ int segpt_kv_append(int dtype, int B, int Hkv, int S, int D, const segpt_tensor4
   return launch_kv_append(a, reinterpret_cast<hipStream_t>(stream));
 }
 
+int segpt_linear_rows(const segpt_linear_rows_params* p, void* stream) {
+  if (!p) return SEGPT_E_NULL;
+  if (p->struct_bytes != sizeof(segpt_linear_rows_params)) return SEGPT_E_STRUCT;
+  if (p->M <= 0 || p->M > SEGPT_LINEAR_MAX_ROWS || p->K <= 0 || p->K % 32 || p->n_segments <= 0 || p->n_segments > SEGPT_LINEAR_MAX_SEGMENTS)
+    return SEGPT_E_SHAPE;
+  auto check_rows = [&](const void* ptr, int64_t stride) {
+    if (!ptr) return SEGPT_E_NULL;
+    if (!aligned16(ptr)) return SEGPT_E_ALIGN;
+    return stride < p->K || stride % 8 ? SEGPT_E_STRIDE : SEGPT_OK;
+  };
+  int rc = p->M == 1 ? check_rows(p->x, p->K) : check_rows(p->x, p->x_stride);  // one row has no stride
+  for (int i = 0; i < p->n_segments && !rc; ++i) {
+    const segpt_linear_segment& s = p->seg[i];
+    if (s.n <= 0 || s.n > (1 << 24) || s.width <= 0) return SEGPT_E_SHAPE;
+    if (!s.out) return SEGPT_E_NULL;
+    if (s.stride_m < 0 || s.stride_h < 0) return SEGPT_E_STRIDE;
+    rc = check_rows(s.w, s.w_stride);
+  }
+  if (rc) return rc;
+  return launch_linear_rows(*p, reinterpret_cast<hipStream_t>(stream));
+}
+
 static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage_hi, void* stream) {
   if (!p_in) return SEGPT_E_NULL;
   segpt_attn_params p_copy = *p_in;

@@ -185,6 +185,8 @@ struct KvAppendArgs {
   int32_t B, Hkv, S, chunks;  // chunks: 16-byte pieces per row
 };
 int launch_kv_append(const KvAppendArgs& a, hipStream_t st);
+constexpr int kMaxLinearRows = SEGPT_LINEAR_MAX_ROWS;
+int launch_linear_rows(const segpt_linear_rows_params& p, hipStream_t st);
 
 // host-side launchers (one per translation unit); each returns a hipError_t as int
 int launch_fwd_f32(const KArgs& a, hipStream_t st);

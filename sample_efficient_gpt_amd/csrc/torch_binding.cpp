@@ -14,12 +14,14 @@
 
 #include <ATen/ATen.h>
 #include <ATen/FuncTorchTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 
 #include <cmath>
 #include <optional>
 #include <string>
+#include <tuple>
 
 #include "segpt_attn.h"
 
@@ -368,6 +370,97 @@ std::optional<std::pair<Tensor, Tensor>> kv_append(const Tensor& kbuf, const Ten
   return std::make_pair(kbuf.narrow(2, 0, need), vbuf.narrow(2, 0, need));
 }
 
+// One token of each sequence through the attention module with its cache: projections (and the gate's) with the new key and
+// value written into the buffers at row `length`, attention, output projection; (out, keys, values), the latter the filled
+// prefixes.  Four kernels (with the merge) and one way through the interpreter; as separate torch calls around
+// `attention` the step was seven launches and 105 us of host work for 31 us of kernels.
+// None (nothing done, the caller takes the separate calls) for whatever those treat otherwise: recorded gradients or tangents,
+// autocast, types or sizes that differ, rows that are not whole 16-byte pieces, full buffers.
+std::optional<std::tuple<Tensor, Tensor, Tensor>> generation_step(const Tensor& x, const Tensor& w_qkv, const Tensor& w_out, const OptTensor& ow_gate,
+                                                                  const Tensor& gain, const Tensor& cos, const Tensor& sin, const Tensor& kbuf,
+                                                                  const Tensor& vbuf, int64_t length, int64_t heads, int64_t kv_heads, int64_t flags) {
+  const Tensor w_gate = defined_or_none(ow_gate);
+  const auto dev = x.device();
+  if (!x.is_cuda() || x.dim() != 3 || x.size(1) != 1 || x.size(0) < 1 || x.size(0) > SEGPT_LINEAR_MAX_ROWS || w_qkv.dim() != 2) return std::nullopt;
+  if (at::autocast::is_autocast_enabled(at::kCUDA)) return std::nullopt;
+  const int64_t B = x.size(0), K = x.size(2), D = K / heads, q_cols = heads * D, kv_cols = kv_heads * D;
+  if (K % heads || K % 32 || (D != 64 && D != 128) || w_qkv.size(0) != q_cols + 2 * kv_cols || w_qkv.size(1) != K) return std::nullopt;
+  if (w_out.dim() != 2 || w_out.size(0) != K || w_out.size(1) != q_cols) return std::nullopt;
+  if (w_gate.defined() && (w_gate.dim() != 2 || w_gate.size(0) != heads || w_gate.size(1) != K)) return std::nullopt;
+  if ((gain.numel() != 1 && gain.numel() != D) || cos.dim() != 2 || cos.sizes() != sin.sizes() || cos.size(1) != D / 2) return std::nullopt;
+  const bool grad_mode = at::GradMode::is_enabled();
+  auto left_alone = [&](const Tensor& t) { return !(grad_mode && t.requires_grad()) && !t._fw_grad(0).defined() && t.device() == dev; };
+  auto rows = [&](const Tensor& t) {  // bf16 rows of whole, aligned 16-byte pieces
+    return left_alone(t) && t.scalar_type() == at::kBFloat16 && t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  for (const Tensor* t : {&x, &w_qkv, &w_out, &w_gate})
+    if (t->defined() && !(rows(*t) && (t->size(0) == 1 || (t->stride(0) >= K && t->stride(0) % 8 == 0)))) return std::nullopt;
+  for (const Tensor* t : {&gain, &cos, &sin})
+    if (!left_alone(*t)) return std::nullopt;
+  const int64_t need = length + 1;
+  for (const Tensor* t : {&kbuf, &vbuf})
+    if (t->dim() != 4 || t->size(0) != B || t->size(1) != kv_heads || t->size(2) < need || t->size(3) != D || !rows(*t) ||
+        (t->is_inference() && !c10::InferenceMode::is_enabled()))
+      return std::nullopt;
+
+  const Tensor g32 = f32_vector(gain, dev), cos32 = f32_table(cos, dev), sin32 = f32_table(sin, dev);
+  segpt_attn_params p{};
+  p.struct_bytes = sizeof(p);
+  p.dtype = SEGPT_DTYPE_BF16;
+  p.B = (int32_t)B; p.H = (int32_t)heads; p.Hkv = (int32_t)kv_heads; p.Sq = 1; p.Sk = (int32_t)need; p.D = (int32_t)D;
+  p.causal = 1;
+  p.q_start = p.rope_q_pos0 = (int32_t)length;
+  p.gq_numel = (int32_t)g32.numel();
+  p.eps = 1e-6f; p.sm_scale = (float)(1.0 / std::sqrt((double)D)); p.gate_scale = 2.0f;  // attention.py:51-80, :248
+  p.flags = (int)flags;
+  p.k = view4(kbuf, 0); p.v = view4(vbuf, 0);
+  p.g_q = ptr_of<float>(g32);
+  p.rope_cos = ptr_of<float>(cos32); p.rope_sin = ptr_of<float>(sin32);
+  p.rope_len = (int32_t)cos32.size(0);
+  // one buffer for what lives during the step: q, y, lse, gate logits, the attention's own scratch
+  auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  const size_t row_bytes = up((size_t)(B * q_cols) * 2), lse_bytes = up((size_t)(B * heads) * 4), gate_bytes = w_gate.defined() ? up((size_t)(B * heads) * 2) : 0;
+  const size_t ws_bytes = segpt_attn_workspace_bytes(&p, SEGPT_WS_KV);
+  const Tensor buf = at::empty({(int64_t)(2 * row_bytes + lse_bytes + gate_bytes + up(ws_bytes))}, at::TensorOptions().dtype(at::kByte).device(dev));
+  char* at = static_cast<char*>(buf.data_ptr());
+  p.q = {at, q_cols, D, q_cols};
+  p.o = {at + row_bytes, q_cols, D, q_cols};
+  p.lse = reinterpret_cast<float*>(at + 2 * row_bytes);
+  if (gate_bytes) p.gate = {at + 2 * row_bytes + lse_bytes, heads, heads, 1};
+  p.kv_workspace = at + 2 * row_bytes + lse_bytes + gate_bytes;
+  p.kv_workspace_bytes = up(ws_bytes);
+  const Tensor out = at::empty({B, 1, K}, x.options());
+
+  segpt_linear_rows_params in{}, proj{};
+  in.struct_bytes = proj.struct_bytes = sizeof(in);
+  in.M = proj.M = (int32_t)B;
+  in.K = (int32_t)K;
+  in.x = x.data_ptr();
+  in.x_stride = x.stride(0);
+  auto weight_row = [&](const Tensor& w, int64_t row) { return static_cast<const char*>(w.data_ptr()) + row * w.stride(0) * 2; };
+  auto cache_row = [&](const Tensor& t) { return static_cast<char*>(t.data_ptr()) + length * t.stride(2) * 2; };
+  in.seg[in.n_segments++] = {weight_row(w_qkv, 0), w_qkv.stride(0), at, q_cols, D, (int32_t)q_cols, (int32_t)D};
+  in.seg[in.n_segments++] = {weight_row(w_qkv, q_cols), w_qkv.stride(0), cache_row(kbuf), kbuf.stride(0), kbuf.stride(1), (int32_t)kv_cols, (int32_t)D};
+  in.seg[in.n_segments++] = {weight_row(w_qkv, q_cols + kv_cols), w_qkv.stride(0), cache_row(vbuf), vbuf.stride(0), vbuf.stride(1), (int32_t)kv_cols, (int32_t)D};
+  if (gate_bytes) in.seg[in.n_segments++] = {w_gate.data_ptr(), w_gate.stride(0), at + 2 * row_bytes + lse_bytes, heads, 0, (int32_t)heads, (int32_t)heads};
+  proj.K = (int32_t)q_cols;
+  proj.x = at + row_bytes;
+  proj.x_stride = q_cols;
+  proj.seg[proj.n_segments++] = {w_out.data_ptr(), w_out.stride(0), out.data_ptr(), K, 0, (int32_t)K, (int32_t)K};
+
+  const c10::DeviceGuard guard(dev);
+  void* const stream = current_stream(dev);
+  int rc = segpt_linear_rows(&in, stream);
+  if (rc < 0) return std::nullopt;
+  if (rc) throw LibraryError(rc, "segpt_linear_rows");
+  for (const Tensor* t : {&kbuf, &vbuf}) torch::autograd::impl::bump_version(*t);
+  rc = segpt_attn_fwd(&p, stream);
+  if (rc) throw LibraryError(rc, "segpt_attn_fwd");
+  rc = segpt_linear_rows(&proj, stream);
+  if (rc) throw LibraryError(rc, "segpt_linear_rows");
+  return std::make_tuple(out, kbuf.narrow(2, 0, need), vbuf.narrow(2, 0, need));
+}
+
 // What torch raises (out of memory, an error from a saved-tensor hook) keeps its Python type across the binding
 template <typename R, typename... A>
 auto bound(R (*f)(A...)) {
@@ -406,4 +499,5 @@ PYBIND11_MODULE(_segpt_torch, m) {
   m.def("op_forward", bound(&op_forward));
   m.def("op_backward", bound(&op_backward));
   m.def("kv_append", bound(&kv_append));
+  m.def("generation_step", bound(&generation_step));
 }

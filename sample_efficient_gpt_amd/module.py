@@ -5,8 +5,10 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from torch.nn.modules import module as _module
+
 from . import _native
-from .function import QKNormFlashAttnFunc
+from .function import QKNormFlashAttnFunc, _call_flags
 from .library_op import _seen_as_operator
 
 
@@ -96,6 +98,17 @@ class KVCache:
         return self._mbuf[:, :, : self.length]
 
 
+def _weight_of(layer):
+    """The weight of a `_Linear` whose call is nothing but `x W^T`, else None: no hook, replaced forward, bias or module of
+    another class (adapters, parametrizations, quantised layers) stands in between."""
+    if type(layer) is not _Linear or type(layer.linear) is not nn.Linear or layer.linear.bias is not None:
+        return None
+    for m in (layer, layer.linear):
+        if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+            return None
+    return layer.linear.weight
+
+
 class _Linear(nn.Module):
     """Bias-free linear layer with the reference's parameter name (`<name>.linear.weight`) and
     initialisation (core.py:11-23)."""
@@ -177,11 +190,37 @@ class MultiHeadSelfAttention(nn.Module):
                 raise ValueError(f"{self.gating=} is undefined")
             self.attn_gate = _Linear(gate_in, gate_out, device=device, dtype=dtype)
 
+    def _generation_step(self, x, kv_cache):
+        """One token of each of a few sequences as one native call: ``(attn_out, keys, values)``, or None where the layers
+        around the attention are to be called one by one (see ``generation_step`` in csrc/torch_binding.cpp)."""
+        if self.value_residual or (self.gating and self.gating != "per-head") or type(kv_cache) is not KVCache or kv_cache._kbuf is None:
+            return None
+        if _module._global_forward_hooks or _module._global_forward_pre_hooks:
+            return None
+        w_qkv, w_out = _weight_of(self.qkv), _weight_of(self.out)
+        w_gate = _weight_of(self.attn_gate) if self.gating else None
+        if w_qkv is None or w_out is None or (self.gating and w_gate is None):
+            return None
+        gain = self.sdpa_qknorm.gain if self.qknorm else self._unit_gain
+        cos, sin = self.rope.cos, self.rope.sin
+        if _seen_as_operator(x, w_qkv, w_out, w_gate, gain, cos, sin, kv_cache._kbuf, kv_cache._vbuf):
+            return None
+        step = _native.load().generation_step(x, w_qkv, w_out, w_gate, gain, cos, sin, kv_cache._kbuf, kv_cache._vbuf, kv_cache.length,
+                                              self.n_heads, self.n_kv_heads, _call_flags(self.qknorm, True))
+        if step is not None:
+            kv_cache.length += 1
+            kv_cache.keys, kv_cache.values = step[1:]
+        return step
+
     def forward(self, x, token_positions=None, v1=None, kv_cache: KVCache | None = None):
         from .function import _canon
         from .library_op import qknorm_attention_op
 
         b, S, d_model = x.shape
+        if S == 1 and kv_cache is not None and x.is_cuda and not torch.compiler.is_compiling():
+            step = self._generation_step(x, kv_cache)
+            if step is not None:
+                return step[0], step[2] if v1 is None or self.always_return_values else None
         H, Hkv = self.n_heads, self.n_kv_heads
         d = d_model // H
         q_out, kv_out = H * d, Hkv * d

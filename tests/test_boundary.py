@@ -223,6 +223,29 @@ def test_module_interface():
     assert list(sig.parameters) == ["Q", "K", "V", "is_causal", "q_start"]
 
 
+def test_linear_rows_rejects_bad_arguments_before_any_launch(lib):
+    """segpt_linear_rows returns its error codes without a device."""
+    def call(M=2, K=64, x=256, xs=64, n_segments=1, w=512, ws=64, out=1024, n=5, width=5, sm=5, sh=0, struct_bytes=None):
+        p = _lib.LinearRowsParams()
+        p.struct_bytes = C.sizeof(p) if struct_bytes is None else struct_bytes
+        p.M, p.K, p.n_segments, p.x, p.x_stride = M, K, n_segments, x, xs
+        for i in range(4):
+            p.seg[i] = _lib.LinearSegment(w, ws, out, sm, sh, n, width)
+        return lib.segpt_linear_rows(p, None)
+
+    codes = {k: int(v) for k, v in re.findall(r"#define\s+SEGPT_E_(\w+)\s+\(?(-?\d+)", open(HEADER).read())}
+    assert lib.segpt_linear_rows(None, None) == codes["NULL"]
+    assert call(struct_bytes=8) == codes["STRUCT"]
+    for bad in (dict(M=0), dict(M=17), dict(K=0), dict(K=48), dict(n_segments=0), dict(n_segments=5), dict(n=0), dict(n=(1 << 24) + 1), dict(width=0)):
+        assert call(**bad) == codes["SHAPE"], bad
+    for bad in (dict(x=None), dict(w=None), dict(out=None)):
+        assert call(**bad) == codes["NULL"], bad
+    for bad in (dict(x=264), dict(w=520)):
+        assert call(**bad) == codes["ALIGN"], bad
+    for bad in (dict(xs=63), dict(xs=68), dict(ws=32), dict(ws=68), dict(sm=-1), dict(sh=-1)):
+        assert call(**bad) == codes["STRIDE"], bad
+
+
 def test_kv_append_rejects_bad_arguments_before_any_launch(lib):
     """segpt_kv_append returns its error codes without a device."""
     t = lambda ptr=256, sb=4096, sh=1024, ss=64: _lib.Tensor4(ptr, sb, sh, ss)

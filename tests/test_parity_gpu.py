@@ -1557,6 +1557,114 @@ def test_kv_cache_append_is_the_two_copies(gpu_device, dtype, D):
     assert keys.requires_grad and torch.equal(keys[:, :, -2:], k)
 
 
+@pytest.mark.parametrize("M,K,ns", [(1, 32, (1,)), (2, 288, (16, 15)), (15, 1152, (1152, 384, 384, 18)), (16, 2048, (17, 64)), (3, 2080, (33,))])
+def test_linear_rows(gpu_device, M, K, ns):
+    """segpt_linear_rows at the edges of its tiles (rows, columns, steps shared out unevenly over the waves, more than one batch
+    of them) and with heads scattered over a larger buffer.  Bound: one rounding to bf16 of a sum whose fp32 additions err by
+    2^-24 of the summed magnitudes each, at most K / 32 / 8 * 2 + 8 of them in a row."""
+    import ctypes
+
+    from sample_efficient_gpt_amd import _lib
+    g = torch.Generator().manual_seed(M + K)
+    n = lambda *s: torch.randn(*s, generator=g).to(BF16).to(gpu_device)
+    x = n(M, K + 8)[:, :K]
+    p = _lib.LinearRowsParams()
+    p.struct_bytes, p.M, p.K, p.n_segments, p.x, p.x_stride = ctypes.sizeof(p), M, K, len(ns), x.data_ptr(), x.stride(0)
+    ws, outs = [n(c, K) for c in ns], []
+    for i, c in enumerate(ns):
+        width = 16 if c % 16 == 0 else c
+        outs.append(torch.full((M, c // width, 3, width), 7.0, dtype=BF16, device=gpu_device))
+        p.seg[i] = _lib.LinearSegment(ws[i].data_ptr(), K, outs[i][:, :, 1].data_ptr(), outs[i].stride(0), outs[i].stride(1), c, width)
+    print(f"linear_rows M={M} K={K} ns={ns}", flush=True)
+    assert _lib.load().segpt_linear_rows(p, torch.cuda.current_stream(gpu_device).cuda_stream) == 0
+    torch.cuda.synchronize()
+    for w, o in zip(ws, outs):
+        want = x.double() @ w.double().T
+        slack = (x.double().abs() @ w.double().abs().T) * (K / 128 + 8) * 2.0**-24
+        assert bool(((o[:, :, 1].reshape(M, -1).double() - want).abs() <= want.abs() * 2.0**-8 + slack).all())
+        assert bool((o[:, :, 0] == 7).all()) and bool((o[:, :, 2] == 7).all())
+
+
+@pytest.mark.parametrize("b,H,Hkv,d,gating,qknorm", [(1, 18, 6, 64, "per-head", True), (3, 6, 2, 64, False, True), (16, 4, 4, 128, "per-head", False)])
+def test_mhsa_module_generation_step_is_the_separate_calls(gpu_device, b, H, Hkv, d, gating, qknorm):
+    """A cached token as one native call against the same module whose layers are called one by one (a hook on a layer asks
+    for that): the same new rows of the cache and outputs but for the order of the projections' sums, the earlier rows
+    untouched, and every caller that has to see the layers still does."""
+    S0, d_model = 70, H * d
+    m, _, _ = _module_and_oracle_weights(gpu_device, BF16, d_model, H, Hkv, qknorm, False, gating, seed=31)
+    x = torch.randn(b, S0 + 2, d_model, generator=torch.Generator().manual_seed(32)).to(BF16).to(gpu_device)
+    seen = []
+
+    def run(hooked):
+        cache = KVCache(capacity=S0 + 2)
+        with torch.no_grad():
+            m(x[:, :S0], kv_cache=cache)
+            prompt = cache.keys.clone(), cache.values.clone()
+            hook = m.qkv.linear.register_forward_hook(lambda *_: seen.append(1)) if hooked else None
+            version = cache._kbuf._version
+            outs = [m(x[:, t : t + 1], kv_cache=cache) for t in (S0, S0 + 1)]
+            assert cache._kbuf._version > version
+            if hooked:
+                hook.remove()
+        assert cache.length == S0 + 2 and cache.keys.shape == (b, Hkv, S0 + 2, d)
+        assert torch.equal(cache.keys[:, :, :S0], prompt[0]) and torch.equal(cache.values[:, :, :S0], prompt[1])
+        assert all(v.data_ptr() == cache._vbuf.data_ptr() and v.shape[2] == S0 + 1 + i for i, (_, v) in enumerate(outs))
+        return torch.cat([o for o, _ in outs], 1), cache
+
+    print(f"generation step b={b} H={H} d={d}", flush=True)
+    (y, cache), (want, want_cache) = run(False), run(True)
+    assert len(seen) == 2
+    for a, r in ((cache.keys, want_cache.keys), (cache.values, want_cache.values)):
+        assert torch.allclose(a.float(), r.float(), rtol=2.0**-7, atol=1e-5)  # neighbouring bf16 values
+    assert torch.allclose(y.float(), want.float(), atol=2e-2, rtol=1e-2)
+    real = _native_module().generation_step
+    args = lambda xt, length: (xt, m.qkv.linear.weight, m.out.linear.weight, m.attn_gate.linear.weight if gating else None, torch.ones(1, device=gpu_device),
+                               m.rope.cos, m.rope.sin, cache._kbuf, cache._vbuf, length, H, Hkv, 4)
+    token = x[:, :1].clone()
+    with torch.no_grad():
+        before = cache._kbuf.clone()
+        assert real(*args(token, cache._kbuf.shape[2])) is None                       # the buffers are full
+        assert real(*args(x[:, :2], 0)) is None and real(*args(token.float(), 0)) is None
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert real(*args(token, 0)) is None
+        assert torch.equal(cache._kbuf.view(torch.int16), before.view(torch.int16))
+    assert real(*args(token.requires_grad_(), 0)) is None
+
+
+def _native_module():
+    from sample_efficient_gpt_amd import _native
+    return _native.load()
+
+
+def test_generation_step_in_a_graph(gpu_device):
+    """A captured step replayed with new tokens and eager work in between equals the eager step bit for bit."""
+    H, Hkv, d, S0 = 6, 2, 64, 200
+    m, _, _ = _module_and_oracle_weights(gpu_device, BF16, H * d, H, Hkv, True, False, "per-head", seed=41)
+    x = torch.randn(2, S0 + 1, H * d, generator=torch.Generator().manual_seed(42)).to(BF16).to(gpu_device)
+    cache, token = KVCache(capacity=S0 + 1), x[:, S0:].clone()
+
+    def step():
+        cache.length = S0
+        return m(token, kv_cache=cache)[0]
+
+    with torch.no_grad():
+        m(x[:, :S0], kv_cache=cache)
+        step()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = step()
+        for i in range(4):
+            token.copy_(torch.randn(token.shape, generator=torch.Generator().manual_seed(i)).to(BF16))
+            eager = step().clone()
+            row = cache.keys[:, :, S0].clone()
+            cache._kbuf[:, :, S0].zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, eager) and torch.equal(cache._kbuf[:, :, S0], row), i
+
+
 def test_mhsa_module_prefill_with_grad_then_cached_steps_without(gpu_device):
     """A prefill that runs with gradients enabled (its mixed values are not kept in the cache) followed by
     generation steps under no_grad: the first cached step mixes every row the cache is still missing, and the value
