@@ -86,17 +86,26 @@ extern "C" {
                                     and the SDPA call attention.py:233-240.  Logits are then unbounded: the bf16
                                     forward always keeps a running row maximum */
 
+#define SEGPT_FLAG_F32_SPLIT 16  /* fp32: kv_workspace is scratch of SEGPT_WS_F32_FWD / SEGPT_WS_F32_BWD bytes, 256 B aligned, and the
+                                    call may run on the bf16 matrix pipe, every fp32 operand as a sum of three bf16 numbers
+                                    (no less accurate, faster; contents undefined on entry and exit).  No effect where that
+                                    size is 0, and ignored for bf16 and by segpt_attn_fwd_noalloc */
+
 /* which scratch buffer segpt_attn_workspace_bytes() sizes */
 #define SEGPT_WS_KV 0  /* kv_workspace: bf16 copies of the normalised keys (and mixed values); forward AND backward */
 #define SEGPT_WS_BWD 1 /* workspace: per-row statistics, normalised queries, partial sums; backward only            */
+#define SEGPT_WS_F32_FWD 2 /* fp32 with SEGPT_FLAG_F32_SPLIT: kv_workspace of the forward ... */
+#define SEGPT_WS_F32_BWD 3 /* ... and of the backward, which does not need the forward's; 0 where the call runs without */
 
 /* the two stages segpt_attn_fwd() runs, in this order */
-#define SEGPT_FWD_STAGE_PRE 0  /* bf16: key/value pre-pass (skipped with SEGPT_FLAG_KV_PREPARED); fp32: nothing */
+#define SEGPT_FWD_STAGE_PRE 0  /* bf16: key/value pre-pass (skipped with SEGPT_FLAG_KV_PREPARED); fp32: nothing, or
+                                    the operands as bf16 numbers (SEGPT_FLAG_F32_SPLIT) */
 #define SEGPT_FWD_STAGE_ATTN 1 /* the attention kernel: writes o and lse                                         */
 
 /* the four stages segpt_attn_bwd() runs, in this order */
 #define SEGPT_BWD_STAGE_PRE 0    /* bf16: key/value pre-pass (skipped with SEGPT_FLAG_KV_PREPARED): normalised
-                                    Khat (and V' = c1 v + c2 v_first) into kv_workspace; fp32: nothing  */
+                                    Khat (and V' = c1 v + c2 v_first) into kv_workspace; fp32: nothing,
+                                    or the operands as bf16 numbers (SEGPT_FLAG_F32_SPLIT), delta and dgate */
 #define SEGPT_BWD_STAGE_DQ 1     /* dQ, delta, dgate and the per-workgroup partials of the scale gradient; on
                                     the bf16 path also Qhat for stage 2 (a positive gate factor is folded
                                     into the row statistics; fp32, or a gate scale <= 0, adds a gate-scaled
@@ -158,7 +167,8 @@ typedef struct segpt_attn_params {
   size_t workspace_bytes;
   void* kv_workspace; /* bf16 forward and backward: >= segpt_attn_workspace_bytes(p, SEGPT_WS_KV), 256 B aligned.
                          Written by the key/value pre-pass of either call; a backward that gets the buffer its
-                         forward used may set SEGPT_FLAG_KV_PREPARED.  Ignored (may be NULL) for fp32. */
+                         forward used may set SEGPT_FLAG_KV_PREPARED.  fp32: ignored (may be NULL) without
+                         SEGPT_FLAG_F32_SPLIT. */
   size_t kv_workspace_bytes;
 
   /* optional rotary embedding of q and k, fused into the loads (the step before the op in the reference:

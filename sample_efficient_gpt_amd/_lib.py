@@ -19,10 +19,13 @@ SEGPT_FLAG_KV_PREPARED = 1
 SEGPT_FLAG_RUNNING_MAX = 2
 SEGPT_FLAG_DECODE = 4
 SEGPT_FLAG_NO_NORM = 8
+SEGPT_FLAG_F32_SPLIT = 16
 SEGPT_E_SCRATCH_LIMIT = -13
 SEGPT_NOALLOC_SCRATCH_BYTES = 16 << 20
 SEGPT_WS_KV = 0
 SEGPT_WS_BWD = 1
+SEGPT_WS_F32_FWD = 2
+SEGPT_WS_F32_BWD = 3
 FWD_STAGES = ("pre", "attn")  # SEGPT_FWD_STAGE_* = index
 BWD_STAGES = ("pre", "dq", "dkdv", "reduce")  # SEGPT_BWD_STAGE_* = index
 

@@ -13,7 +13,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libsegpt_attn.so")
 BINDING_PATH = os.path.join(PKG_DIR, "_segpt_torch.so")  # native host side for PyTorch callers, linked against LIB_PATH
-SOURCES = ["api.hip", "f32_path.hip", "pre_post.hip", "fwd_mfma.hip", "bwd_mfma.hip", "decode_mfma.hip", "linear_rows.hip"]
+SOURCES = ["api.hip", "f32_path.hip", "f32_split.hip", "pre_post.hip", "fwd_mfma.hip", "bwd_mfma.hip", "decode_mfma.hip", "linear_rows.hip"]
 # Per-source flags.  The forward never needs more than 256 registers, but at head_dim 128 it runs one
 # workgroup per CU and the compiler would then move every MFMA result into the accumulation registers
 # (one v_accvgpr_read per score before exp2); keeping the ordinary-register form is 8 % faster there.
@@ -22,7 +22,8 @@ SOURCES = ["api.hip", "f32_path.hip", "pre_post.hip", "fwd_mfma.hip", "bwd_mfma.
 EXTRA_FLAGS = {"fwd_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-sched-strategy=max-ilp"],
                "decode_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                # one workgroup per CU at head_dim 128 as above: dK/dV 49 -> 43 us at B = 2, H = 4, S = 500
-               "f32_path.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+               "f32_path.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+               "f32_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 # -packed-fp32-ops is switched off: hipcc -O3 otherwise forms v_pk_*_f32 from ordinary float code.
 HIPCC_FLAGS = [

@@ -176,6 +176,21 @@ int check_common(const segpt_attn_params* p) {
   return SEGPT_OK;
 }
 
+// fp32: scratch of the kernels that take every operand as three bf16 numbers, 0 where they are not the faster ones
+size_t f32_split_scratch(const segpt_attn_params& p, bool bwd) {
+  if (p.dtype != SEGPT_DTYPE_FP32 || (p.D != 32 && p.D != 64 && p.D != 128)) return 0;
+  return align_up(f32_split_bytes(p, bwd));
+}
+int bind_split(KArgs& a, bool bwd) {
+  const segpt_attn_params& p = a.p;
+  const size_t need = (p.flags & SEGPT_FLAG_F32_SPLIT) ? f32_split_scratch(p, bwd) : 0;
+  if (!need) return SEGPT_OK;
+  if (!p.kv_workspace || p.kv_workspace_bytes < need) return SEGPT_E_WORKSPACE;
+  if (reinterpret_cast<uintptr_t>(p.kv_workspace) & 255u) return SEGPT_E_ALIGN;
+  a.f32_split = reinterpret_cast<char*>(p.kv_workspace);
+  return SEGPT_OK;
+}
+
 // fills the kernel arguments that both directions share
 void bind_kv(KArgs& a) {
   const segpt_attn_params& p = a.p;
@@ -244,6 +259,7 @@ size_t segpt_attn_workspace_bytes(const segpt_attn_params* p, int which) {
   if (p->dtype == SEGPT_DTYPE_BF16 && p->D != 64 && p->D != 128) return 0;
   if (which == SEGPT_WS_KV) return kv_layout(*p).total_split;
   if (which == SEGPT_WS_BWD) return bwd_layout(*p).total;
+  if (which == SEGPT_WS_F32_FWD || which == SEGPT_WS_F32_BWD) return f32_split_scratch(*p, which == SEGPT_WS_F32_BWD);
   return 0;
 }
 
@@ -256,6 +272,7 @@ static int fwd_stage_impl(const segpt_attn_params* p, int stage_lo, int stage_hi
   KArgs a{};
   a.p = *p;
   bind_kv(a);
+  if ((rc = bind_split(a, false))) return rc;
   a.fwd_splits = 1;
   if (p->dtype == SEGPT_DTYPE_BF16) {
     const KvLayout kv = kv_layout(*p);
@@ -270,8 +287,11 @@ static int fwd_stage_impl(const segpt_attn_params* p, int stage_lo, int stage_hi
   const bool decode = use_decode(p);
   for (int stage = stage_lo; stage <= stage_hi; ++stage) {
     switch (stage) {
-      case SEGPT_FWD_STAGE_PRE: rc = (f32 || decode || (p->flags & SEGPT_FLAG_KV_PREPARED)) ? 0 : launch_kv_prep(a, st); break;
-      case SEGPT_FWD_STAGE_ATTN: rc = f32 ? launch_fwd_f32(a, st) : (decode ? launch_fwd_decode_bf16(a, st) : launch_fwd_bf16(a, st)); break;
+      case SEGPT_FWD_STAGE_PRE:
+        if (f32) rc = a.f32_split ? launch_split_prep(a, false, st) : 0;
+        else rc = (decode || (p->flags & SEGPT_FLAG_KV_PREPARED)) ? 0 : launch_kv_prep(a, st);
+        break;
+      case SEGPT_FWD_STAGE_ATTN: rc = f32 ? (a.f32_split ? launch_fwd_split(a, st) : launch_fwd_f32(a, st)) : (decode ? launch_fwd_decode_bf16(a, st) : launch_fwd_bf16(a, st)); break;
       default: return SEGPT_E_STAGE;
     }
     if (rc) return rc;
@@ -316,7 +336,7 @@ int segpt_attn_fwd_noalloc(const segpt_attn_params* p, void* stream) {
   segpt_attn_params q = *p;
   q.kv_workspace = nullptr;
   q.kv_workspace_bytes = 0;
-  q.flags &= ~SEGPT_FLAG_KV_PREPARED;  // the scratch is shared by every call on this GPU: never assume its contents
+  q.flags &= ~(SEGPT_FLAG_KV_PREPARED | SEGPT_FLAG_F32_SPLIT);  // the scratch is shared by every call on this GPU: never assume its contents
   if (q.dtype == SEGPT_DTYPE_BF16) {
     if (q.B > 0 && q.H > 0 && q.Hkv > 0 && q.Sq > 0 && q.Sk > 0 && (q.D == 64 || q.D == 128) &&
         kv_layout(q).total > (size_t)SEGPT_NOALLOC_SCRATCH_BYTES)
@@ -413,6 +433,8 @@ static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage
     a.qhat = reinterpret_cast<uint16_t*>(ws + w.qhat);
   }
   bind_kv(a);
+  if ((rc = bind_split(a, true))) return rc;
+  if (p->dtype == SEGPT_DTYPE_FP32) a.f32_parts = a.f32_split ? f32_split_parts(*p) : p->H / p->Hkv * a.f32_splits;
   a.n_dq_blocks = dq_blocks(*p);
   a.n_dkdv_blocks = dkdv_blocks(*p);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
@@ -420,10 +442,15 @@ static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage
   for (int stage = stage_lo; stage <= stage_hi; ++stage) {
     switch (stage) {
       case SEGPT_BWD_STAGE_PRE:
-        rc = (f32 || (p->flags & SEGPT_FLAG_KV_PREPARED)) ? 0 : launch_kv_prep(a, st);
+        if (f32) rc = a.f32_split ? launch_split_prep(a, true, st) : 0;
+        else rc = (p->flags & SEGPT_FLAG_KV_PREPARED) ? 0 : launch_kv_prep(a, st);
         break;
-      case SEGPT_BWD_STAGE_DKDV: rc = f32 ? launch_bwd_dkdv_f32(a, st) : launch_bwd_dkdv_bf16(a, st); break;
-      case SEGPT_BWD_STAGE_DQ: rc = f32 ? launch_bwd_dq_f32(a, st) : launch_bwd_dq_bf16(a, st); break;
+      case SEGPT_BWD_STAGE_DKDV:
+        rc = f32 ? (a.f32_split ? launch_bwd_dkdv_split(a, st) : launch_bwd_dkdv_f32(a, st)) : launch_bwd_dkdv_bf16(a, st);
+        break;
+      case SEGPT_BWD_STAGE_DQ:
+        rc = f32 ? (a.f32_split ? launch_bwd_dq_split(a, st) : launch_bwd_dq_f32(a, st)) : launch_bwd_dq_bf16(a, st);
+        break;
       case SEGPT_BWD_STAGE_REDUCE: rc = launch_bwd_reduce(a, st); break;
       default: return SEGPT_E_STAGE;
     }

@@ -38,7 +38,8 @@ struct KArgs {
   // (dk and dv themselves where there is one of each per kv head)
   float* f32_dk_part;
   float* f32_dv_part;
-  int32_t f32_splits;
+  int32_t f32_splits, f32_parts;  // f32_parts: parts of dK, dV per kv head
+  char* f32_split;  // fp32 calls with SEGPT_FLAG_F32_SPLIT: operands as three bf16 numbers each (kv_workspace; f32_split.hip), else null
 };
 
 // Row normaliser 1/sqrt(mean x^2 + eps) from the row's sum of squares ss (inv_d = 1/D); exactly 1 for plain
@@ -192,6 +193,12 @@ int launch_linear_rows(const segpt_linear_rows_params& p, hipStream_t st);
 int launch_fwd_f32(const KArgs& a, hipStream_t st);
 int launch_bwd_dkdv_f32(const KArgs& a, hipStream_t st);
 int launch_bwd_dq_f32(const KArgs& a, hipStream_t st);
+int launch_split_prep(const KArgs& a, bool bwd, hipStream_t st);  // fp32 on the bf16 matrix pipe (f32_split.hip)
+int launch_fwd_split(const KArgs& a, hipStream_t st);
+int launch_bwd_dq_split(const KArgs& a, hipStream_t st);
+int launch_bwd_dkdv_split(const KArgs& a, hipStream_t st);
+int f32_split_parts(const segpt_attn_params& p);
+size_t f32_split_bytes(const segpt_attn_params& p, bool bwd);  // scratch its operands take
 int launch_fwd_bf16(const KArgs& a, hipStream_t st);
 int launch_bwd_dkdv_bf16(const KArgs& a, hipStream_t st);
 int launch_bwd_dq_bf16(const KArgs& a, hipStream_t st);

@@ -1,0 +1,705 @@
+// fp32 forward and backward on the bf16 matrix pipe: every fp32 operand as the sum of three bf16 numbers.
+//
+// x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1) (round to nearest: 24 bits and the signs of
+// the remainders, so the sum is x itself but for the last bit of what lies below bf16's smallest numbers).  A product of two such
+// numbers is six matrix instructions, x0 y0 + (x0 y1 + x1 y0 + x1 y1 + x0 y2 + x2 y0), each product exact and summed in fp32;
+// what is left out is below 2^-25 of |x y|.  v_mfma_f32_32x32x16_bf16 does eight times the products of
+// v_mfma_f32_32x32x2_f32 in half the time, so six of them take 3/8 of the fp32 instructions' time, and a sum of 64 products is 4 (and
+// 20 small ones) roundings deep instead of 32: norm-wise distance of a 32x32 tile of products to float64, 64 / 128 columns:
+// fp32 instructions 1.5e-7 / 1.95e-7, one accumulator for all six 1.1e-7 / 1.6e-7, the largest product on its own 4.9e-8 / 6.4e-8.
+//
+// Range: the parts of a value of 2^-102 (2e-31) and more are normal numbers, smaller ones lose their last bits (dO of 1e-32: as above; of
+// 1e-35: 8e-5 from float64).  An infinity among the operands gives NaN where the fp32 instructions give an infinity or NaN.
+//
+// What that takes: nothing may be split inside a loop that runs once per pair of tiles.  A pre-pass rotates, normalises
+// and splits every row once and leaves 32-row tiles as matrix-instruction operands, 1 KB (64 lanes x 16 bytes) each, in the order they
+// are used: [unit][x0, x1, x2], D / 16 units a tile.
+//   rm  (contraction over the columns): unit u, lane (ln, hh): columns 16 u + 8 hh .. + 7 of row ln.
+//   tr  (contraction over the rows): unit 2 mb + s: column MB ln + mb (MB = D / 32) of the rows 16 s + 8 (i / 4) + 4 hh + i % 4,
+//       i = 0..7, which are the rows that registers 8 s .. 8 s + 7 of a C tile hold: scores need no shuffle to be the other operand.
+// The streamed operands then travel from the L2 straight into registers, without LDS, without a barrier in the loops; the 32
+// stationary rows of a workgroup lie in LDS once for its four waves, which share out the streamed tiles as in f32_path.hip.
+//
+// What bounds it: the streamed tiles, 24 / 36 / 48 KB (forward / dQ / dK/dV at head_dim 64) per 32x32 scores and wave, of which a
+// CU gets about 19 bytes a cycle (11 TB/s) whether they are hits in the L2 or requests of a deeper look-ahead: matrix pipe 27 % busy,
+// and neither forming the next scores beside this tile's exponentials nor two accumulators more for shorter chains of dependent
+// products moved a kernel.  Kernels, us, fp32 instructions -> here: 2 x 8 / 4 heads, 1000 tokens of 64 forward 37 -> 5.4 + 21, dQ 47 ->
+// 26, dK/dV 62 -> 32, the pre-pass of the backward 11; the step 143 -> 110.  8 x 18 / 6 heads of 2048 tokens 3556 -> 2428, 1 x 4 / 2
+// heads of 1000 x 128 214 -> 119.
+#include <algorithm>
+
+#include "f32_common.hpp"
+
+namespace segpt {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kUnitBytes = 3 * 1024;
+template <int D>
+constexpr int kUnits = D / 16;
+template <int D>
+constexpr int kTileBytes = kUnits<D> * kUnitBytes;
+
+struct Split3 {
+  bf16x8 p[3];
+};
+// The streamed tiles come in as halves of 32 columns (rm) or of one block mb (tr), two units each, MB = D / 32 halves a
+// tile: twelve matrix instructions (384 cycles).
+struct Half {
+  Split3 u[2];
+};
+constexpr int kHalfBytes = 2 * kUnitBytes;
+
+// where the pre-pass leaves its tiles
+struct SplitMap {
+  char *k_rm, *v, *k_tr, *q_rm, *q_tr, *d_rm, *d_tr;  // v: tr for the forward, rm for the backward
+  float* stat;                                        // [B * H][query tiles][lse of 32 rows, delta of 32 rows]
+};
+__device__ __forceinline__ int tiles_of(int n) { return (n + kRows - 1) / kRows; }
+template <int D>
+__device__ __forceinline__ SplitMap split_map(const KArgs& a) {
+  const int64_t kv = (int64_t)a.p.B * a.p.Hkv * tiles_of(a.p.Sk) * kTileBytes<D>, q = (int64_t)a.p.B * a.p.H * tiles_of(a.p.Sq) * kTileBytes<D>;
+  SplitMap m;
+  m.k_rm = a.f32_split;
+  m.v = m.k_rm + kv;
+  m.k_tr = m.v + kv;
+  m.q_rm = m.k_tr + kv;
+  m.q_tr = m.q_rm + q;
+  m.d_rm = m.q_tr + q;
+  m.d_tr = m.d_rm + q;
+  m.stat = reinterpret_cast<float*>(m.d_tr + q);
+  return m;
+}
+
+// Nothing is scheduled across: every half is requested two steps before its use and not earlier.  Left to itself the compiler
+// hoists a whole iteration's requests and spills (dQ and dK/dV at head_dim 64: 72 and 112 registers).
+__device__ __forceinline__ void step_end() { __builtin_amdgcn_sched_barrier(0); }
+
+__device__ __forceinline__ f32x16 mfma16(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+
+__device__ __forceinline__ Split3 split8(const float (&x)[8]) {
+  Split3 s;
+  u32x4 w[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      w[k][i] = pack_bf16x2(a, b);
+      a -= bf16lo(w[k][i]);
+      b -= bf16hi(w[k][i]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) s.p[k] = __builtin_bit_cast(bf16x8, w[k]);
+  return s;
+}
+
+__device__ __forceinline__ Split3 load_unit(const char* unit, int lane) {
+  Split3 s;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) s.p[k] = *reinterpret_cast<const bf16x8*>(unit + k * 1024 + lane * 16);
+  return s;
+}
+__device__ __forceinline__ Half load_half(const char* half, int lane) { return {{load_unit(half, lane), load_unit(half + kUnitBytes, lane)}}; }
+__device__ __forceinline__ void store_unit(char* unit, const Split3& s, int lane) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(unit + k * 1024 + lane * 16) = s.p[k];
+}
+
+// units u0, u0 + step, ... of a row-major fp32 tile in LDS
+template <int D>
+__device__ __forceinline__ void emit_rm(const float* tile, char* dst, int lane, int u0 = 0, int step = 1) {
+  for (int u = u0; u < kUnits<D>; u += step) {
+    const f32x4v* src = reinterpret_cast<const f32x4v*>(tile + (lane & 31) * T32<D>::kRS + 16 * u + 8 * (lane >> 5));
+    const f32x4v lo = src[0], hi = src[1];
+    const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    store_unit(dst + u * kUnitBytes, split8(x), lane);
+  }
+}
+template <int D>
+__device__ __forceinline__ void emit_tr(const float* tile, char* dst, int lane) {
+  constexpr int MB = T32<D>::kMB;
+#pragma unroll
+  for (int u = 0; u < kUnits<D>; ++u) {
+    const float* src = tile + MB * (lane & 31) + u / 2;
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = src[crow(8 * (u % 2) + i, lane >> 5) * T32<D>::kRS];
+    store_unit(dst + u * kUnitBytes, split8(x), lane);
+  }
+}
+
+// the five small products of a pair and the large one, into accumulators of their own or into one
+__device__ __forceinline__ f32x16 small5(const Split3& a, const Split3& b, f32x16 c) {
+  c = mfma16(a.p[0], b.p[2], c);
+  c = mfma16(a.p[2], b.p[0], c);
+  c = mfma16(a.p[1], b.p[1], c);
+  c = mfma16(a.p[0], b.p[1], c);
+  return mfma16(a.p[1], b.p[0], c);
+}
+// X . B^T over the columns: C rows = rows of the streamed tile, C columns = the 32 stationary rows, whose rm units lie in LDS
+struct Dot {
+  f32x16 large = zero16(), small = zero16();
+  __device__ __forceinline__ void add(const Half& a, const char* b_lds, int lane) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const Split3 b = load_unit(b_lds + u * kUnitBytes, lane);
+      small = small5(a.u[u], b, small);
+      large = mfma16(a.u[u].p[0], b.p[0], large);
+    }
+  }
+  __device__ __forceinline__ f32x16 sum() const {
+    f32x16 s;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = large[r] + small[r];
+    return s;
+  }
+};
+// scores (registers = rows of the streamed tile) as the other operand of the product over those rows
+struct Scores3 {
+  Split3 s[2];
+};
+__device__ __forceinline__ Scores3 split_scores(const f32x16& w) {
+  Scores3 b;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const float x[8] = {w[8 * s], w[8 * s + 1], w[8 * s + 2], w[8 * s + 3], w[8 * s + 4], w[8 * s + 5], w[8 * s + 6], w[8 * s + 7]};
+    b.s[s] = split8(x);
+  }
+  return b;
+}
+// acc += (block mb of a tile)^T . w over the 32 rows; the tile's sum is formed by itself and added once
+__device__ __forceinline__ void add_tr(const Half& a, const Scores3& w, f32x16& acc) {
+  f32x16 t = small5(a.u[0], w.s[0], zero16());
+  t = small5(a.u[1], w.s[1], t);
+  t = mfma16(a.u[0].p[0], w.s[0].p[0], t);
+  t = mfma16(a.u[1].p[0], w.s[1].p[0], t);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] += t[r];
+}
+
+// ---- pre-pass: one wave per (tile, tensor, layout).  Forward: keys rm, values tr.  Backward: query and dO tiles in both layouts
+// first (four waves of a workgroup on one query tile), then keys rm, keys tr, values rm; the wave of dO's rm tile also owns
+// what belongs to a query row: delta = rowsum(dY o Y), dgate, and the gate factor goes into dO here.
+template <int D, bool BWD>
+__global__ __launch_bounds__(kThreads) void split_prep_kernel(KArgs a) {
+  const segpt_attn_params& p = a.p;
+  using T = T32<D>;
+  __shared__ __attribute__((aligned(16))) float tiles[kWaves][T::kTile];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const SplitMap m = split_map<D>(a);
+  const int n_qt = tiles_of(p.Sq), n_kt = tiles_of(p.Sk);
+  float* tile = tiles[wave];
+  int64_t job = (int64_t)blockIdx.x * kWaves + wave;
+  const int64_t q_jobs = BWD ? (int64_t)p.B * p.H * n_qt * 4 : 0;
+  f32x4v x[T::kPasses];
+  if (BWD && job < q_jobs) {
+    const int kind = (int)(job & 3);
+    const int64_t t = job >> 2;
+    const int qt = (int)(t % n_qt), hb = (int)(t / n_qt), b = hb / p.H, h = hb % p.H, q0 = qt * kRows;
+    if (kind < 2) {
+      load_tile<D>(x, row_ptr<float>(p.q, b, h, 0), p.q.stride_s, q0, p.Sq, lane);
+      f32x4v gs;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) gs[e] = gprod<D>(p, 4 * (lane % T::kLPR) + e) * p.sm_scale * kLog2e;
+      stage_norm<D, true>(p, x, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, tile, lane);
+    } else {
+      load_tile<D>(x, row_ptr<float>(p.d_o, b, h, 0), p.d_o.stride_s, q0, p.Sq, lane);
+      f32x4v y[T::kPasses];
+      if (kind == 2) load_tile<D>(y, row_ptr<float>(p.o, b, h, 0), p.o.stride_s, q0, p.Sq, lane);
+#pragma unroll
+      for (int ps = 0; ps < T::kPasses; ++ps) {
+        const int row = ps * T::kRPP + lane / T::kLPR;
+        float sg = 0.f;
+        if (p.gate.ptr) sg = sigmoidf_acc(gate_logit(p, b, h, min(q0 + row, p.Sq - 1)));
+        if (kind == 2) {
+          const f32x4v d = x[ps] * y[ps];
+          const float delta = row_sum<T::kLPR>((d[0] + d[1]) + (d[2] + d[3]));
+          if (lane % T::kLPR == 0) {
+            m.stat[t * 64 + row] = p.lse[((int64_t)b * p.H + h) * p.Sq + min(q0 + row, p.Sq - 1)];
+            m.stat[t * 64 + 32 + row] = delta;
+            if (p.gate.ptr && q0 + row < p.Sq)
+              reinterpret_cast<float*>(p.dgate.ptr)[(int64_t)b * p.dgate.stride_b + (int64_t)(q0 + row) * p.dgate.stride_s + (int64_t)h * p.dgate.stride_h] = (1.0f - sg) * delta;
+          }
+        }
+        if (p.gate.ptr) x[ps] *= p.gate_scale * sg;
+      }
+      stage_plain<D>(x, tile, lane);
+    }
+    wave_sync();
+    char* const dst = (kind == 0 ? m.q_rm : kind == 1 ? m.q_tr : kind == 2 ? m.d_rm : m.d_tr) + t * kTileBytes<D>;
+    if (kind & 1) emit_tr<D>(tile, dst, lane);
+    else emit_rm<D>(tile, dst, lane);
+    return;
+  }
+  job -= q_jobs;
+  constexpr int kKinds = BWD ? 3 : 2;
+  const int kind = (int)(job % kKinds);
+  const int64_t t = job / kKinds;
+  if (t >= (int64_t)p.B * p.Hkv * n_kt) return;
+  const int kt = (int)(t % n_kt), bg = (int)(t / n_kt), b = bg / p.Hkv, g = bg % p.Hkv, j0 = kt * kRows;
+  const bool values = kind == kKinds - 1;
+  if (values) {
+    float c1 = 1.f, c2 = 0.f;
+    if (p.vr_coef) { c1 = p.vr_coef[0]; c2 = p.vr_coef[1]; }
+    load_vmix<D>(p, x, b, g, j0, c1, c2, lane);
+    stage_plain<D>(x, tile, lane);
+  } else {
+    load_tile<D>(x, row_ptr<float>(p.k, b, g, 0), p.k.stride_s, j0, p.Sk, lane);
+    const f32x4v one = {1.f, 1.f, 1.f, 1.f};
+    stage_norm<D, true>(p, x, one, p.rope_k_pos0 + j0, p.Sk - 1 - j0, tile, lane);
+  }
+  wave_sync();
+  char* const dst = (values ? m.v : kind == 0 ? m.k_rm : m.k_tr) + t * kTileBytes<D>;
+  if (kind == 1) emit_tr<D>(tile, dst, lane);  // forward: values, backward: keys
+  else emit_rm<D>(tile, dst, lane);
+}
+
+// Which tile a workgroup takes: (tile, heaviest first; (batch, kv head); member of the pair: query head or part).  Up to 1024
+// workgroups, most of them resident at once, as in f32_path.hip.  More: one pair after the other on each XCD, so that the
+// streamed tiles of the resident workgroups (2.4 MB a pair at 2048 keys of 64) stay in its L2; with all pairs in turn they came
+// out of the memory side at its 7 TB/s.  `pair` is past the last one for the workgroups that fill up the last round.
+struct Item {
+  int tile, pair, member;
+};
+constexpr int kPinnedGrid = 1024;
+__device__ __forceinline__ Item split_item(int tiles, int pairs, int members) {
+  Item it;
+  if ((int64_t)tiles * pairs * members <= kPinnedGrid) {
+    const int id = work_item(), rest = id % (pairs * members);
+    it.tile = id / (pairs * members);
+    it.pair = rest / members;
+    it.member = rest % members;
+  } else {
+    const int k = blockIdx.x / 8, per = tiles * members, rest = k % per;
+    it.pair = 8 * (k / per) + blockIdx.x % 8;
+    it.tile = rest / members;
+    it.member = rest % members;
+  }
+  return it;
+}
+
+// ---- forward, as fwd_f32_kernel
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
+  const segpt_attn_params& p = a.p;
+  using T = T32<D>;
+  // in the loop Qhat's units (and before it one fp32 tile behind them), after it the four waves' results
+  __shared__ __attribute__((aligned(16))) char lds[std::max(kTileBytes<D> + 4 * T::kTile, 4 * kWaves * T::kTile)];
+  char* const qs = lds;
+  float* const tiles = reinterpret_cast<float*>(lds);
+  __shared__ float msm[kWaves][32], lsm[kWaves][32];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 31, hh = lane >> 5;
+  const int n_qt = tiles_of(p.Sq), rep = p.H / p.Hkv;
+  const Item item = split_item(n_qt, p.B * p.Hkv, rep);
+  if (item.pair >= p.B * p.Hkv) return;
+  const int b = item.pair / p.Hkv, g = item.pair % p.Hkv, h = g * rep + item.member;
+  const int qt = n_qt - 1 - item.tile, q0 = qt * kRows;
+  int kend = p.Sk;
+  if (p.causal) kend = min(p.Sk, q0 + kRows + p.q_start);
+  const int n_kt = tiles_of(kend);
+  const SplitMap m = split_map<D>(a);
+  const int64_t first = ((int64_t)b * p.Hkv + g) * tiles_of(p.Sk) * kTileBytes<D>;
+  const char *ktiles = m.k_rm + first, *vtiles = m.v + first;
+  // step i of a tile uses half i of its keys, then of its values; requested kAhead steps before
+  constexpr int MB = T::kMB, kSteps = 2 * MB, kAhead = D == 64 ? 3 : MB == 1 ? 1 : 2;
+  Half half[kSteps];
+  auto source = [&](int jt, int i) {
+    return (i < MB ? ktiles : vtiles) + (int64_t)jt * kTileBytes<D> + i % MB * kHalfBytes;
+  };
+  if (wave < n_kt) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) half[i] = load_half(source(wave, i), lane);
+  }
+  {
+    f32x4v qraw[T::kPasses], gs;
+    load_tile<D>(qraw, row_ptr<float>(p.q, b, h, 0), p.q.stride_s, q0, p.Sq, lane);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) gs[e] = gprod<D>(p, 4 * (lane % T::kLPR) + e) * p.sm_scale * kLog2e;
+    float* const tile = reinterpret_cast<float*>(lds + kTileBytes<D>);  // every wave writes the same values
+    stage_norm<D, true>(p, qraw, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, tile, lane);
+    wave_sync();
+    emit_rm<D>(tile, qs, lane, wave, kWaves);
+  }
+  __syncthreads();
+
+  f32x16 o[T::kMB];
+#pragma unroll
+  for (int mb = 0; mb < T::kMB; ++mb) o[mb] = zero16();
+  float mrow = -INFINITY, l = 0.f;  // l: this lane's half of the keys
+  const int qlim = p.causal ? min(q0 + ln + p.q_start, p.Sk - 1) : p.Sk - 1;  // last visible key
+  const int n_full = p.causal ? min(p.Sk, q0 + p.q_start + 1) / kRows : p.Sk / kRows;  // tiles that need no mask
+
+  for (int jt = wave; jt < n_kt; jt += kWaves) {
+    const int next = jt + kWaves < n_kt ? jt + kWaves : jt;  // past the end: this tile's once more, unused
+    auto request = [&](int i) { half[i % kSteps] = load_half(i < kSteps ? source(jt, i) : source(next, i - kSteps), lane); };
+    Dot dot;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      request(i + kAhead);
+      dot.add(half[i], qs + i * kHalfBytes, lane);
+      step_end();
+    }
+    f32x16 s = dot.sum();
+    if (jt >= n_full) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (jt * kRows + crow(r, hh) > qlim) s[r] = -INFINITY;
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    mx = fmaxf(mrow, half_max(mx));
+    const float mu = mx == -INFINITY ? 0.f : mx;
+    if (__builtin_amdgcn_ballot_w64(mx > mrow) != 0) {  // some row has a new maximum
+      const float corr = __builtin_amdgcn_exp2f(mrow - mu);
+      l *= corr;
+#pragma unroll
+      for (int mb = 0; mb < T::kMB; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[mb][r] *= corr;
+      mrow = mx;
+    }
+    float part[2] = {0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = __builtin_amdgcn_exp2f(s[r] - mu);
+      part[r & 1] += s[r];
+    }
+    l += part[0] + part[1];
+    const Scores3 probs = split_scores(s);
+#pragma unroll
+    for (int i = MB; i < kSteps; ++i) {
+      step_end();
+      request(i + kAhead);
+      add_tr(half[i], probs, o[i - MB]);
+    }
+    step_end();
+  }
+
+  const float lt = half_sum(l);
+  if (hh == 0) { msm[wave][ln] = mrow; lsm[wave][ln] = lt; }
+  __syncthreads();  // nobody reads Qhat any more
+  put_rows<D>(tiles + wave * T::kTile, o, lane);
+  __syncthreads();
+  merge_waves<D>(p, b, h, q0, msm, lsm, tiles, T::kTile, tid);
+}
+
+// the rm units of a workgroup's stationary rows into LDS
+template <int D>
+__device__ __forceinline__ void fetch_units(char* lds, const char* tile, int tid) {
+#pragma unroll
+  for (int i = 0; i < kTileBytes<D>; i += 16 * kThreads)
+    if (kTileBytes<D> % (16 * kThreads) == 0 || i + 16 * tid < kTileBytes<D>)
+      *reinterpret_cast<u32x4*>(lds + i + 16 * tid) = *reinterpret_cast<const u32x4*>(tile + i + 16 * tid);
+}
+
+// ---- dQ: S^T and dP^T (lane = query), T^T += Khat^T dS^T
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void bwd_dq_split_kernel(KArgs a) {
+  const segpt_attn_params& p = a.p;
+  using T = T32<D>;
+  // in the loop the units of Qhat and dO, after it the four waves' results
+  __shared__ __attribute__((aligned(16))) char lds[std::max(2 * kTileBytes<D>, 4 * kWaves * T::kTile)];
+  char *const qs = lds, *const ds = lds + kTileBytes<D>;
+  float* const tiles = reinterpret_cast<float*>(lds);
+  __shared__ __attribute__((aligned(16))) float red[kWaves * D];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 31, hh = lane >> 5;
+  const int n_qt = tiles_of(p.Sq), rep = p.H / p.Hkv;
+  const Item item = split_item(n_qt, p.B * p.Hkv, rep);
+  if (item.pair >= p.B * p.Hkv) return;
+  const int b = item.pair / p.Hkv, g = item.pair % p.Hkv, h = g * rep + item.member;
+  const int qt = n_qt - 1 - item.tile, q0 = qt * kRows;
+  int kend = p.Sk;
+  if (p.causal) kend = min(p.Sk, q0 + kRows + p.q_start);
+  const int n_kt = tiles_of(kend);
+  const SplitMap m = split_map<D>(a);
+  const int64_t first = ((int64_t)b * p.Hkv + g) * tiles_of(p.Sk) * kTileBytes<D>, mine = ((int64_t)b * p.H + h) * n_qt + qt;
+  const char *ktiles = m.k_rm + first, *vtiles = m.v + first, *kttiles = m.k_tr + first;
+  // step i of a tile: half i of the keys (scores), of the values (dP), of the keys again (T)
+  constexpr int MB = T::kMB, kSteps = 3 * MB, kAhead = MB == 1 ? 2 : 3;
+  Half half[kSteps];
+  auto source = [&](int jt, int i) {
+    return (i < MB ? ktiles : i < 2 * MB ? vtiles : kttiles) + (int64_t)jt * kTileBytes<D> + i % MB * kHalfBytes;
+  };
+  if (wave < n_kt) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) half[i] = load_half(source(wave, i), lane);
+  }
+  fetch_units<D>(qs, m.q_rm + mine * kTileBytes<D>, tid);
+  fetch_units<D>(ds, m.d_rm + mine * kTileBytes<D>, tid);
+  const float lse = m.stat[mine * 64 + ln], delta = m.stat[mine * 64 + 32 + ln];
+  __syncthreads();
+  f32x16 t[T::kMB];
+#pragma unroll
+  for (int mb = 0; mb < T::kMB; ++mb) t[mb] = zero16();
+  const int qlim = p.causal ? min(q0 + ln + p.q_start, p.Sk - 1) : p.Sk - 1;
+  const int n_full = p.causal ? min(p.Sk, q0 + p.q_start + 1) / kRows : p.Sk / kRows;
+
+  for (int jt = wave; jt < n_kt; jt += kWaves) {
+    const int next = jt + kWaves < n_kt ? jt + kWaves : jt;
+    auto request = [&](int i) { half[i % kSteps] = load_half(i < kSteps ? source(jt, i) : source(next, i - kSteps), lane); };
+    Dot dot[2];
+#pragma unroll
+    for (int i = 0; i < 2 * MB; ++i) {
+      request(i + kAhead);
+      dot[i / MB].add(half[i], (i < MB ? qs : ds) + i % MB * kHalfBytes, lane);
+      step_end();
+    }
+    f32x16 s = dot[0].sum();
+    const f32x16 dp = dot[1].sum();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = prob(s[r], lse);
+    if (jt >= n_full) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (jt * kRows + crow(r, hh) > qlim) s[r] = 0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] *= dp[r] - delta;
+    const Scores3 grads = split_scores(s);
+#pragma unroll
+    for (int i = 2 * MB; i < kSteps; ++i) {
+      step_end();
+      request(i + kAhead);
+      add_tr(half[i], grads, t[i - 2 * MB]);
+    }
+    step_end();
+  }
+
+  __syncthreads();
+  put_rows<D>(tiles + wave * T::kTile, t, lane);
+  __syncthreads();
+  finish_dq<D>(a, b, h, q0, (int)mine, tiles, T::kTile, red, tid);
+}
+
+// ---- dK, dV of one kv head: S = Qhat Khat^T and dP = dO V'^T (lane = key), dV^T += dO^T P, dK^T += Qhat^T dS.  The query tiles
+// that see the keys, of all query heads of the group one after the other, are dealt out to 4 f32_parts waves; a workgroup
+// leaves one part of the sum (bwd_dkdv_f32_kernel leaves one per query head and share: twice the traffic at two heads a group).
+template <int D>
+__global__ __launch_bounds__(kThreads, (D == 128 ? 1 : 2)) void bwd_dkdv_split_kernel(KArgs a) {
+  const segpt_attn_params& p = a.p;
+  using T = T32<D>;
+  __shared__ __attribute__((aligned(16))) char lds[std::max(2 * kTileBytes<D>, 4 * kWaves * T::kTile)];  // as above: Khat and V'
+  char *const ks = lds, *const vs = lds + kTileBytes<D>;
+  float* const tiles = reinterpret_cast<float*>(lds);
+  __shared__ __attribute__((aligned(16))) float stat[kWaves][64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 31, hh = lane >> 5;
+  const Item item = split_item(tiles_of(p.Sk), p.B * p.Hkv, a.f32_parts);  // the first key tiles are the heaviest
+  if (item.pair >= p.B * p.Hkv) return;
+  const int kt_i = item.tile, part_i = item.member, bg = item.pair;
+  const int b = bg / p.Hkv, g = bg % p.Hkv, rep = p.H / p.Hkv;
+  const int j0 = kt_i * kRows;
+  const SplitMap m = split_map<D>(a);
+  const int n_qt = tiles_of(p.Sq);
+  const int first = p.causal ? max(0, j0 - p.q_start) / kRows : 0;  // the first tile that holds a query seeing key j0
+  const int step = kWaves * a.f32_parts;
+  const int64_t mine = ((int64_t)bg * tiles_of(p.Sk) + kt_i) * kTileBytes<D>, head = (int64_t)(b * p.H + g * rep) * n_qt;
+  const char *qrm = m.q_rm + head * kTileBytes<D>, *qtr = m.q_tr + head * kTileBytes<D>;
+  const char *drm = m.d_rm + head * kTileBytes<D>, *dtr = m.d_tr + head * kTileBytes<D>;
+  const float* stats = m.stat + head * 64;
+  int it = first + part_i * kWaves + wave, left = rep;  // tile within its head, query heads still to come with this one
+  auto settle = [&](int& tile, int& heads) {  // tiles past a head's last one are the next head's first visible ones
+    while (tile >= n_qt && heads > 0) { tile -= n_qt - first; --heads; }
+  };
+  if (first < n_qt) settle(it, left);
+  else left = 0;
+  // step i of a tile: half i of the queries (scores), of dO (dP), of dO again (dV), of the queries again (dK)
+  constexpr int MB = T::kMB, kSteps = 4 * MB, kAhead = 3;
+  Half half[kSteps];
+  auto source = [&](int tile, int i) {
+    return (i < MB ? qrm : i < 2 * MB ? drm : i < 3 * MB ? dtr : qtr) + (int64_t)tile * kTileBytes<D> + i % MB * kHalfBytes;
+  };
+  float st = 0.f;
+  int at = (rep - left) * n_qt + it;  // tile within the group
+  if (left > 0) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) half[i] = load_half(source(at, i), lane);
+    st = stats[(int64_t)at * 64 + lane];
+  }
+  fetch_units<D>(ks, m.k_rm + mine, tid);
+  fetch_units<D>(vs, m.v + mine, tid);
+  __syncthreads();
+  f32x16 dk[T::kMB], dv[T::kMB];
+#pragma unroll
+  for (int mb = 0; mb < T::kMB; ++mb) dk[mb] = dv[mb] = zero16();
+
+  while (left > 0) {
+    const int i0 = it * kRows;
+    int next_left = left;
+    it += step;
+    settle(it, next_left);
+    const int next = next_left > 0 ? (rep - next_left) * n_qt + it : at;
+    auto request = [&](int i) { half[i % kSteps] = load_half(i < kSteps ? source(at, i) : source(next, i - kSteps), lane); };
+    stat[wave][lane] = st;
+    st = stats[(int64_t)next * 64 + lane];
+    wave_sync();
+    Dot dot[2];
+#pragma unroll
+    for (int i = 0; i < 2 * MB; ++i) {
+      request(i + kAhead);
+      dot[i / MB].add(half[i], (i < MB ? ks : vs) + i % MB * kHalfBytes, lane);
+      step_end();
+    }
+    f32x16 s = dot[0].sum();
+    const f32x16 dp = dot[1].sum();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4v ls = *reinterpret_cast<const f32x4v*>(&stat[wave][8 * q + 4 * hh]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[4 * q + e] = prob(s[4 * q + e], ls[e]);
+    }
+    if (i0 + kRows > p.Sq || (p.causal && j0 + kRows - 1 > i0 + p.q_start)) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = i0 + crow(r, hh);
+        if (i >= p.Sq || (p.causal && j0 + ln > i + p.q_start)) s[r] = 0.f;
+      }
+    }
+    const Scores3 probs = split_scores(s);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4v de = *reinterpret_cast<const f32x4v*>(&stat[wave][32 + 8 * q + 4 * hh]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[4 * q + e] *= dp[4 * q + e] - de[e];
+    }
+    const Scores3 grads = split_scores(s);
+#pragma unroll
+    for (int i = 2 * MB; i < kSteps; ++i) {
+      step_end();
+      request(i + kAhead);
+      if (i < 3 * MB) add_tr(half[i], probs, dv[i - 2 * MB]);
+      else add_tr(half[i], grads, dk[i - 3 * MB]);
+    }
+    step_end();
+    wave_sync();
+    at = next;
+    left = next_left;
+  }
+
+  const int part = tid % T::kLPR;
+  const int64_t out = ((int64_t)bg * a.f32_parts + part_i) * p.Sk * D;
+  auto leave = [&](const f32x16 (&acc)[T::kMB], float* to) {
+    __syncthreads();
+    put_rows<D>(tiles + wave * T::kTile, acc, lane);
+    __syncthreads();
+#pragma unroll
+    for (int row = tid / T::kLPR; row < kRows; row += kThreads / T::kLPR)
+      if (j0 + row < p.Sk)
+        *reinterpret_cast<f32x4v*>(to + out + (int64_t)(j0 + row) * D + 4 * part) = sum_waves<D>(tiles, T::kTile, row, part);
+  };
+  leave(dk, a.f32_dk_part);
+  leave(dv, a.f32_dv_part);
+}
+
+int n_tiles(int n) { return (n + kRows - 1) / kRows; }
+
+dim3 split_grid(int tiles, int pairs, int members) {
+  const int64_t n = (int64_t)tiles * pairs * members;
+  return dim3((unsigned)(n <= kPinnedGrid ? n : (int64_t)8 * ((pairs + 7) / 8) * tiles * members));
+}
+
+template <int D>
+int launch_prep(const KArgs& a, bool bwd, hipStream_t st) {
+  const segpt_attn_params& p = a.p;
+  const int64_t kv = (int64_t)p.B * p.Hkv * n_tiles(p.Sk), q = (int64_t)p.B * p.H * n_tiles(p.Sq);
+  const int64_t jobs = bwd ? 4 * q + 3 * kv : 2 * kv;
+  const dim3 grid((unsigned)((jobs + kWaves - 1) / kWaves)), block(kThreads);
+  if (bwd) hipLaunchKernelGGL((split_prep_kernel<D, true>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((split_prep_kernel<D, false>), grid, block, 0, st, a);
+  return (int)hipGetLastError();
+}
+template <int D>
+int launch_attn(const KArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(fwd_split_kernel<D>, split_grid(n_tiles(a.p.Sq), a.p.B * a.p.Hkv, a.p.H / a.p.Hkv), dim3(kThreads), 0, st, a);
+  return (int)hipGetLastError();
+}
+template <int D>
+int launch_dq(const KArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(bwd_dq_split_kernel<D>, split_grid(n_tiles(a.p.Sq), a.p.B * a.p.Hkv, a.p.H / a.p.Hkv), dim3(kThreads), 0, st, a);
+  return (int)hipGetLastError();
+}
+template <int D>
+int launch_dkdv(const KArgs& a, hipStream_t st) {
+  const segpt_attn_params& p = a.p;
+  hipLaunchKernelGGL(bwd_dkdv_split_kernel<D>, split_grid(n_tiles(p.Sk), p.B * p.Hkv, a.f32_parts), dim3(kThreads), 0, st, a);
+  const int rc = (int)hipGetLastError();
+  return rc ? rc : launch_finish_f32(a, st);
+}
+
+}  // namespace
+
+// Parts of dK and dV per kv head: one resident round of 512 workgroups, every wave with a tile; never more than the
+// workspace of the other kernels has, one per query head and f32_dkdv_splits.
+int f32_split_parts(const segpt_attn_params& p) {
+  const int units = n_tiles(p.Sk) * p.B * p.Hkv, rep = p.H / p.Hkv;
+  const int want = (512 + units - 1) / units, most = (rep * n_tiles(p.Sq) + kWaves - 1) / kWaves;
+  return std::max(1, std::min({want, most, rep * f32_dkdv_splits(p)}));
+}
+// Where splitting pays.  The pre-pass is a launch more (4 to 6 us, 11 for a backward of 16 heads of 1000 tokens) and 6 bytes an
+// element written and read again, so a key has to be used by several workgroups and a wave has to have a few tiles.  Us of a call, plain
+// operands, fp32 instructions -> here:
+//   forward  head_dim 128, 4 heads:  128 tokens 13.3 -> 16.5, 192: 20.0 -> 19.1, 1000: 60.9 -> 35.2;  16 heads: 192 20.2 -> 20.1, 512 35.0 -> 29.1
+//            64, 16 heads:  256 11.6 -> 13.5, 512 18.7 -> 17.8, 1000 33.3 -> 29.4;  32 heads: 512 21.3 -> 24.0, 768 45.0 -> 38.6; 144 heads of 2048 859 -> 530
+//            32, 12 heads:  512 11.7 -> 12.4, 768 16.6 -> 15.1;  48 heads: 256 9.4 -> 11.4, 384 14.5 -> 13.7
+//   backward head_dim 128:  64 tokens, 4 heads 39 -> 31, 1000 153 -> 83;  16 heads: 128 43 -> 38, 512 123 -> 80
+//            64, 16 heads:  256 31 -> 33, 384 47 -> 42, 1000 112 -> 85;  32 heads: 192 38 -> 35, 384 67 -> 56
+//            32, 12 heads:  384 27 -> 30, 512 33.5 -> 33.1, 768 54 -> 43;  48 heads: 192 29 -> 33, 384 54 -> 43
+bool f32_split_pays(const segpt_attn_params& p, bool bwd) {
+  const int n_qt = n_tiles(p.Sq), n_kt = n_tiles(p.Sk);
+  const int64_t heads = (int64_t)p.B * p.H, pairs = heads * n_qt * n_kt;
+  if ((int64_t)(p.H / p.Hkv) * n_qt < 8 && !(bwd && p.D == 128)) return false;  // one query against a long cache: split keys used once or twice
+  if (p.D == 128) return bwd || n_kt >= 6;
+  if (p.D == 64) return bwd ? n_kt >= 12 : n_kt >= 24 || (n_kt >= 16 && heads <= 16);
+  return pairs >= (bwd ? 3072 : 5000);
+}
+size_t f32_split_bytes(const segpt_attn_params& p, bool bwd) {
+  if (!f32_split_pays(p, bwd)) return 0;
+  const size_t tile = (size_t)p.D * (kUnitBytes / 16), kv = (size_t)p.B * p.Hkv * n_tiles(p.Sk), q = (size_t)p.B * p.H * n_tiles(p.Sq);
+  return bwd ? (3 * kv + 4 * q) * tile + q * 64 * sizeof(float) : 2 * kv * tile;
+}
+
+int launch_split_prep(const KArgs& a, bool bwd, hipStream_t st) {
+  switch (a.p.D) {
+    case 32: return launch_prep<32>(a, bwd, st);
+    case 64: return launch_prep<64>(a, bwd, st);
+    case 128: return launch_prep<128>(a, bwd, st);
+    default: return (int)hipErrorInvalidValue;
+  }
+}
+int launch_fwd_split(const KArgs& a, hipStream_t st) {
+  switch (a.p.D) {
+    case 32: return launch_attn<32>(a, st);
+    case 64: return launch_attn<64>(a, st);
+    case 128: return launch_attn<128>(a, st);
+    default: return (int)hipErrorInvalidValue;
+  }
+}
+int launch_bwd_dq_split(const KArgs& a, hipStream_t st) {
+  switch (a.p.D) {
+    case 32: return launch_dq<32>(a, st);
+    case 64: return launch_dq<64>(a, st);
+    case 128: return launch_dq<128>(a, st);
+    default: return (int)hipErrorInvalidValue;
+  }
+}
+int launch_bwd_dkdv_split(const KArgs& a, hipStream_t st) {
+  switch (a.p.D) {
+    case 32: return launch_dkdv<32>(a, st);
+    case 64: return launch_dkdv<64>(a, st);
+    case 128: return launch_dkdv<128>(a, st);
+    default: return (int)hipErrorInvalidValue;
+  }
+}
+
+}  // namespace segpt

@@ -299,6 +299,37 @@ def test_fp32_backward_needs_partials_only_where_there_are_several(lib):
     assert ws(1, 1, 256) >= small(1, 256) + 2 * kv(1, 256)  # two shares: the launch does not fill the card
 
 
+def test_fp32_split_scratch(lib):
+    """SEGPT_FLAG_F32_SPLIT: sizes (0 where the other kernels are taken: short calls, a query or two against a long cache), what the
+    flag asks of kv_workspace, and no effect without it or on bf16."""
+
+    def params(Sq, Sk, D=64, **kw):
+        p = _valid_params(dtype=_lib.SEGPT_DTYPE_FP32, D=D)
+        p.Sq, p.Sk, p.flags = Sq, Sk, _lib.SEGPT_FLAG_F32_SPLIT
+        p.workspace, p.workspace_bytes = 0x20000, 1 << 40
+        for name in ("q", "o", "d_o", "dq"):
+            setattr(p, name, _lib.Tensor4(0x10000, 6 * Sq * D, Sq * D, D))
+        for name in ("k", "v", "dk", "dv"):
+            setattr(p, name, _lib.Tensor4(0x10000, 2 * Sk * D, Sk * D, D))
+        return p
+
+    size = lambda p: [lib.segpt_attn_workspace_bytes(p, w) for w in (_lib.SEGPT_WS_F32_FWD, _lib.SEGPT_WS_F32_BWD)]
+    for D in (32, 64, 128):
+        assert size(params(1, 8192, D))[0] == 0
+        kv, q = 2 * 2 * 32 * 32 * D, 2 * 6 * 32 * 32 * D  # elements of K and of Q in whole tiles
+        assert size(params(1000, 1000, D)) == [2 * kv * 6, 3 * kv * 6 + 4 * q * 6 + 2 * 6 * 32 * 64 * 4]
+    assert size(params(128, 128)) == [0, 0]
+    p = _valid_params(); p.Sq = p.Sk = 1000
+    assert size(p) == [0, 0]
+    for call, i in ((lib.segpt_attn_fwd, 0), (lib.segpt_attn_bwd, 1)):
+        p = params(1000, 1000); p.kv_workspace, p.kv_workspace_bytes = None, 0
+        assert call(p, None) == -7
+        p = params(1000, 1000); p.kv_workspace_bytes = size(p)[i] - 1
+        assert call(p, None) == -7
+        p = params(1000, 1000); p.kv_workspace, p.kv_workspace_bytes = 0x40010, 1 << 40
+        assert call(p, None) == -10
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libsegpt_attn.so"))

@@ -102,6 +102,54 @@ def test_fp32_tile_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize(
+    "B,H,Hkv,Sq,Sk,kw,gen_kw",
+    [
+        (2, 4, 2, 769, 769, {}, {}),                                                      # one row past 24 tiles
+        (1, 8, 8, 895, 895, {"rope": True, "gate_scale": -1.5}, {"extras": True}),         # one short of 28; one head a group
+        (2, 9, 3, 640, 833, {"q_start": 193, "rope": True}, {"extras": True, "scalar_gain": True}),
+        (2, 6, 2, 545, 801, {"causal": False}, {"scalar_gain": True, "no_gk": True}),
+        (1, 8, 2, 830, 790, {}, {}),                                                      # queries that see every key
+        (2, 4, 1, 800, 800, {"qk_norm": False}, {"scalar_gain": True, "no_gk": True}),
+        (4, 8, 2, 200, 900, {"q_start": 3}, {}),                                          # keys that no query sees
+        (5, 9, 3, 769, 769, {}, {}),  # more than 1024 workgroups, (batch, kv head) pairs that are no multiple of the XCDs
+    ],
+)
+def test_fp32_split_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
+    """Calls long enough for the three-way bf16 splits (operands as sums of three bf16 numbers on the bf16 matrix pipe): tile edges,
+    shares of the query tiles over the heads of a group, both orders of the workgroups; the same 1e-5."""
+    from sample_efficient_gpt_amd import _lib
+
+    p = _lib.new_params()
+    p.dtype, p.B, p.H, p.Hkv, p.Sq, p.Sk, p.D = _lib.SEGPT_DTYPE_FP32, B, H, Hkv, Sq, Sk, D
+    for which in (_lib.SEGPT_WS_F32_FWD, _lib.SEGPT_WS_F32_BWD):
+        assert _lib.load().segpt_attn_workspace_bytes(p, which) > 0
+    kw = dict(kw)
+    if kw.pop("rope", False):
+        kw["rope"] = orc.rope_tables(1000, 10000.0, D)
+    _case(gpu_device, F32, B, H, Hkv, Sq, Sk, D, gen_kw=gen_kw, seed=72, **kw)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_split_is_no_less_accurate(gpu_device, D):
+    """Distance to float64 in norm, in units of 2^-24, of y, dq, dk, dv of a call that the splits take.  With the fp32 matrix instruction
+    it was 3.31, 6.36, 7.60, 6.09 at its largest over the three head sizes, the bounds; with the splits 2.64, 5.74, 6.09, 4.82."""
+    rng = torch.Generator().manual_seed(D)
+    S = 770
+    ops = [torch.randn(2, h, S, D, generator=rng) for h in (4, 2, 2)]
+    dy, one = torch.randn(2, 4, S, D, generator=rng), torch.ones(1)
+    wide = [t.double().requires_grad_(True) for t in ops]
+    y64 = orc.attention_forward(*wide, one.double(), qk_norm=True)[0]
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in ops]
+    y = qknorm_attention(*leaves, one.to(gpu_device))
+    got = [y, *torch.autograd.grad(y, leaves, dy.to(gpu_device))]
+    ref = [y64, *torch.autograd.grad(y64, wide, dy.double())]
+    err = [((a.detach().cpu().double() - b).norm() / b.norm()).item() * 2**24 for a, b in zip(got, ref)]
+    print("units of 2^-24:", " ".join(f"{e:.2f}" for e in err), flush=True)
+    assert all(e <= bound for e, bound in zip(err, (3.31, 6.36, 7.60, 6.09)))
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_rows_whose_mean_square_leaves_the_normal_range(gpu_device, D):
     """A key whose sum of squares overflows has the normaliser 0, like a key of zeros, and poisons nobody; keys so small
     that their mean square is subnormal (eps = 0) are normalised like any others."""
