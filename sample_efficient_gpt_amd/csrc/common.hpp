@@ -127,11 +127,19 @@ __device__ __forceinline__ void reduce_scale_grad(const KArgs& a, int tid, float
   const int D = p.D;
   const int lanes = THREADS / D;  // threads cooperating on one d
   const int d = tid % D, sl = tid / D;
-  // eight independent chains hide the load latency
+  // eight independent chains, 32 loads in flight: as one batch of eight after the other the 512 rows of an fp32 backward of 16 heads and 1000
+  // tokens were 16 round trips to memory (finish kernel of the fp32 path, which this one workgroup bound: 9.2 -> 6.9 us)
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   const float* src = a.dg_part + d;
   const int n = a.n_dq_blocks;
   int blk = sl;
+  for (; blk + 31 * lanes < n; blk += 32 * lanes) {
+    float v[32];
+#pragma unroll
+    for (int u = 0; u < 32; ++u) v[u] = src[(int64_t)(blk + u * lanes) * D];
+#pragma unroll
+    for (int u = 0; u < 32; ++u) acc[u % 8] += v[u];
+  }
   for (; blk + 7 * lanes < n; blk += 8 * lanes) {
     float v[8];
 #pragma unroll

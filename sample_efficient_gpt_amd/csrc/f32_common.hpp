@@ -63,8 +63,8 @@ __device__ __forceinline__ int crow(int r, int hh) { return 8 * (r >> 2) + 4 * h
 // CUs) or nearly so, the CU that got item i also gets item i + 256: every second round of 256 is dealt in reverse, so
 // that a heavy item shares its CU with a light one (512 items: forward 37.8 -> 31.8 us, dQ 51 -> 43).  Larger grids
 // balance by themselves and keep the plain order (dK/dV 3 % slower reversed at 9216 items).
-__device__ __forceinline__ int work_item() {
-  const int id = blockIdx.x, n = gridDim.x, round = id >> 8;
+__device__ __forceinline__ int work_item(int id, int n) {
+  const int round = id >> 8;
   if (n > 1024 || !(round & 1)) return id;
   const int x = id & 255;
   return (round << 8) + 256 <= n ? (round << 8) + 248 - (x & 248) + (x & 7) : n - 1 - x;

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void fwd_f32_kernel(KArgs a
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
   const int n_qt = (p.Sq + kRows - 1) / kRows, heads = p.B * p.H;
-  const int item = work_item();
+  const int item = work_item(blockIdx.x, gridDim.x);
   const int qt = n_qt - 1 - item / heads, hb = item % heads;
   const int b = hb / p.H, h = hb % p.H, g = h / (p.H / p.Hkv);
   const int q0 = qt * kRows;
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dq_f32_kernel(KArg
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
   const int n_qt = (p.Sq + kRows - 1) / kRows, heads = p.B * p.H;
-  const int item = work_item();
+  const int item = work_item(blockIdx.x, gridDim.x);
   const int qt = n_qt - 1 - item / heads, hb = item % heads;
   const int b = hb / p.H, h = hb % p.H, g = h / (p.H / p.Hkv);
   const int q0 = qt * kRows;
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(kThreads, T32<D>::kOcc) void bwd_dkdv_f32_kernel(KA
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
   const int units = p.B * p.H * a.f32_splits;  // heaviest key tiles (the first ones) first
-  const int item = work_item();
+  const int item = work_item(blockIdx.x, gridDim.x);
   const int kt_i = item / units;
   int rest = item % units;
   const int split = rest % a.f32_splits;
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(kThreads) void bwd_finish_f32_kernel(KArgs a) {
   __shared__ float tot[D];
   const int tid = threadIdx.x;
   if (blockIdx.x == 0) {
-    reduce_scale_grad<kThreads>(a, tid, red, tot);
+    if (!a.f32_split) reduce_scale_grad<kThreads>(a, tid, red, tot);  // the other dK/dV kernel has done it
     return;
   }
   const int part = tid % T::kLPR;

@@ -24,8 +24,8 @@
 // CU gets about 19 bytes a cycle (11 TB/s) whether they are hits in the L2 or requests of a deeper look-ahead: matrix pipe 27 % busy,
 // and neither forming the next scores beside this tile's exponentials nor two accumulators more for shorter chains of dependent
 // products moved a kernel.  Kernels, us, fp32 instructions -> here: 2 x 8 / 4 heads, 1000 tokens of 64 forward 37 -> 5.4 + 21, dQ 47 ->
-// 26, dK/dV 62 -> 32, the pre-pass of the backward 11; the step 143 -> 110.  8 x 18 / 6 heads of 2048 tokens 3556 -> 2428, 1 x 4 / 2
-// heads of 1000 x 128 214 -> 119.
+// 26, dK/dV 62 -> 32, the pre-pass of the backward 11; the step 143 -> 102.  8 x 18 / 6 heads of 2048 tokens 3556 -> 2191, 1 x 4 / 2
+// heads of 1000 x 128 214 -> 115.
 #include <algorithm>
 
 #include "f32_common.hpp"
@@ -266,17 +266,17 @@ __global__ __launch_bounds__(kThreads) void split_prep_kernel(KArgs a) {
 struct Item {
   int tile, pair, member;
 };
-constexpr int kPinnedGrid = 1024;
-__device__ __forceinline__ Item split_item(int tiles, int pairs, int members) {
+constexpr int kPinnedGrid = 1024, kXcds = 8;
+__device__ __forceinline__ Item split_item(int block, int tiles, int pairs, int members) {
   Item it;
   if ((int64_t)tiles * pairs * members <= kPinnedGrid) {
-    const int id = work_item(), rest = id % (pairs * members);
+    const int id = work_item(block, tiles * pairs * members), rest = id % (pairs * members);
     it.tile = id / (pairs * members);
     it.pair = rest / members;
     it.member = rest % members;
   } else {
-    const int k = blockIdx.x / 8, per = tiles * members, rest = k % per;
-    it.pair = 8 * (k / per) + blockIdx.x % 8;
+    const int k = block / 8, per = tiles * members, rest = k % per;
+    it.pair = 8 * (k / per) + block % 8;
     it.tile = rest / members;
     it.member = rest % members;
   }
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
   const int n_qt = tiles_of(p.Sq), rep = p.H / p.Hkv;
-  const Item item = split_item(n_qt, p.B * p.Hkv, rep);
+  const Item item = split_item(blockIdx.x, n_qt, p.B * p.Hkv, rep);
   if (item.pair >= p.B * p.Hkv) return;
   const int b = item.pair / p.Hkv, g = item.pair % p.Hkv, h = g * rep + item.member;
   const int qt = n_qt - 1 - item.tile, q0 = qt * kRows;
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_split_kernel(KArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
   const int n_qt = tiles_of(p.Sq), rep = p.H / p.Hkv;
-  const Item item = split_item(n_qt, p.B * p.Hkv, rep);
+  const Item item = split_item(blockIdx.x, n_qt, p.B * p.Hkv, rep);
   if (item.pair >= p.B * p.Hkv) return;
   const int b = item.pair / p.Hkv, g = item.pair % p.Hkv, h = g * rep + item.member;
   const int qt = n_qt - 1 - item.tile, q0 = qt * kRows;
@@ -484,6 +484,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_split_kernel(KArgs a) {
 // ---- dK, dV of one kv head: S = Qhat Khat^T and dP = dO V'^T (lane = key), dV^T += dO^T P, dK^T += Qhat^T dS.  The query tiles
 // that see the keys, of all query heads of the group one after the other, are dealt out to 4 f32_parts waves; a workgroup
 // leaves one part of the sum (bwd_dkdv_f32_kernel leaves one per query head and share: twice the traffic at two heads a group).
+// The first workgroup adds up the scale gradient behind the others' back: in the finish kernel it was the longest one (finish 6.9 -> 4.7 us at 512 rows,
+// 109 -> 24 at 9216; the other seven of the first kXcds workgroups keep the rest on their XCDs).
 template <int D>
 __global__ __launch_bounds__(kThreads, (D == 128 ? 1 : 2)) void bwd_dkdv_split_kernel(KArgs a) {
   const segpt_attn_params& p = a.p;
@@ -495,7 +497,11 @@ __global__ __launch_bounds__(kThreads, (D == 128 ? 1 : 2)) void bwd_dkdv_split_k
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
-  const Item item = split_item(tiles_of(p.Sk), p.B * p.Hkv, a.f32_parts);  // the first key tiles are the heaviest
+  if (blockIdx.x < kXcds) {
+    if (blockIdx.x == 0) reduce_scale_grad<kThreads>(a, tid, tiles, tiles + kThreads);
+    return;
+  }
+  const Item item = split_item(blockIdx.x - kXcds, tiles_of(p.Sk), p.B * p.Hkv, a.f32_parts);  // the first key tiles are the heaviest
   if (item.pair >= p.B * p.Hkv) return;
   const int kt_i = item.tile, part_i = item.member, bg = item.pair;
   const int b = bg / p.Hkv, g = bg % p.Hkv, rep = p.H / p.Hkv;
@@ -604,9 +610,9 @@ __global__ __launch_bounds__(kThreads, (D == 128 ? 1 : 2)) void bwd_dkdv_split_k
 
 int n_tiles(int n) { return (n + kRows - 1) / kRows; }
 
-dim3 split_grid(int tiles, int pairs, int members) {
+dim3 split_grid(int tiles, int pairs, int members, int extra = 0) {
   const int64_t n = (int64_t)tiles * pairs * members;
-  return dim3((unsigned)(n <= kPinnedGrid ? n : (int64_t)8 * ((pairs + 7) / 8) * tiles * members));
+  return dim3((unsigned)(extra + (n <= kPinnedGrid ? n : (int64_t)8 * ((pairs + 7) / 8) * tiles * members)));
 }
 
 template <int D>
@@ -632,7 +638,7 @@ int launch_dq(const KArgs& a, hipStream_t st) {
 template <int D>
 int launch_dkdv(const KArgs& a, hipStream_t st) {
   const segpt_attn_params& p = a.p;
-  hipLaunchKernelGGL(bwd_dkdv_split_kernel<D>, split_grid(n_tiles(p.Sk), p.B * p.Hkv, a.f32_parts), dim3(kThreads), 0, st, a);
+  hipLaunchKernelGGL(bwd_dkdv_split_kernel<D>, split_grid(n_tiles(p.Sk), p.B * p.Hkv, a.f32_parts, kXcds), dim3(kThreads), 0, st, a);
   const int rc = (int)hipGetLastError();
   return rc ? rc : launch_finish_f32(a, st);
 }
