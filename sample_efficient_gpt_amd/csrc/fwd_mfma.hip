@@ -414,7 +414,9 @@ __global__ __launch_bounds__(kThreadsM, (FwdShape<D, WIDE, PARTS>::kOcc)) void f
 // Adds up the shares of the query tiles that were split: D/4 lanes across a row, G groups of them across the shares.
 // Few rows want the shares side by side (4608 rows, 16 shares: 8.9 us with G = 1, 6.4 with a wave per row), many rows are
 // better off with more rows per wave (73728 rows, 2 shares: 5.2 and 11.4 us).  Fixed order: deterministic.
-constexpr int kMergeThreads = 256, kMergeFewRows = 8192;
+// Bound by its chain of loads: a lane's first kMergeEarly shares and the gate are one round trip to memory, where statistics, then
+// values, then the gate were three (18 / 6 heads, 256 queries, 8192 keys, the whole call: 30.3 -> 29.9 us).
+constexpr int kMergeThreads = 256, kMergeFewRows = 8192, kMergeEarly = 4;
 template <int D, int G>
 __global__ __launch_bounds__(kMergeThreads) void fwd_merge_kernel(KArgs a) {
   const segpt_attn_params& p = a.p;
@@ -431,19 +433,37 @@ __global__ __launch_bounds__(kMergeThreads) void fwd_merge_kernel(KArgs a) {
   const int64_t at = ((int64_t)b * p.H + h) * a.fwd_splits * p.Sq + i;
   const float2* stat = reinterpret_cast<const float2*>(a.fwd_stat) + at;
   const float* o = a.fwd_part + at * D + 4 * part;
-  float m = -INFINITY;
-  for (int s = gi; s < n; s += G) m = fmaxf(m, stat[(int64_t)s * p.Sq].x);
+  uint16_t gate = 0;
+  if (p.gate.ptr)
+    gate = reinterpret_cast<const uint16_t*>(p.gate.ptr)[(int64_t)b * p.gate.stride_b + (int64_t)i * p.gate.stride_s + (int64_t)h * p.gate.stride_h];
+  auto stat_of = [&](int s) { return stat[(int64_t)s * p.Sq]; };
+  auto row_of = [&](int s) { return *reinterpret_cast<const float4*>(o + (int64_t)s * p.Sq * D); };
+  // the first shares are requested together, statistics and values
+  float2 ml[kMergeEarly];
+  float4 t[kMergeEarly];
+#pragma unroll
+  for (int u = 0; u < kMergeEarly; ++u) {
+    const int s = min(gi + G * u, n - 1);  // past the end: the last share once more, unused
+    ml[u] = stat_of(s);
+    t[u] = row_of(s);
+  }
+  float m = ml[0].x;
+#pragma unroll
+  for (int u = 1; u < kMergeEarly; ++u) m = fmaxf(m, ml[u].x);
+  for (int s = gi + G * kMergeEarly; s < n; s += G) m = fmaxf(m, stat_of(s).x);
 #pragma unroll
   for (int x = LPR * RPW; x < 64; x <<= 1) m = fmaxf(m, __shfl_xor(m, x, 64));
   float l = 0.f, y[4] = {0.f, 0.f, 0.f, 0.f};
+  auto add_share = [&](float2 x, float4 v) {
+    const float w = fast_exp2(x.x - m);  // a share without a visible key has (-inf, 0): weight 0
+    l += w * x.y;
+    y[0] += w * v.x; y[1] += w * v.y; y[2] += w * v.z; y[3] += w * v.w;
+  };
+#pragma unroll
+  for (int u = 0; u < kMergeEarly; ++u)
+    if (gi + G * u < n) add_share(ml[u], t[u]);
 #pragma unroll 4
-  for (int s = gi; s < n; s += G) {
-    const float2 ml = stat[(int64_t)s * p.Sq];
-    const float4 t = *reinterpret_cast<const float4*>(o + (int64_t)s * p.Sq * D);
-    const float w = fast_exp2(ml.x - m);  // a share without a visible key has (-inf, 0): weight 0
-    l += w * ml.y;
-    y[0] += w * t.x; y[1] += w * t.y; y[2] += w * t.z; y[3] += w * t.w;
-  }
+  for (int s = gi + G * kMergeEarly; s < n; s += G) add_share(stat_of(s), row_of(s));
 #pragma unroll
   for (int x = LPR * RPW; x < 64; x <<= 1) {
     l += __shfl_xor(l, x, 64);
@@ -451,10 +471,7 @@ __global__ __launch_bounds__(kMergeThreads) void fwd_merge_kernel(KArgs a) {
     for (int e = 0; e < 4; ++e) y[e] += __shfl_xor(y[e], x, 64);
   }
   float f = 1.0f / l;
-  if (p.gate.ptr) {
-    const float z = bf16_to_f32(reinterpret_cast<const uint16_t*>(p.gate.ptr)[(int64_t)b * p.gate.stride_b + (int64_t)i * p.gate.stride_s + (int64_t)h * p.gate.stride_h]);
-    f *= p.gate_scale / (1.0f + __expf(-z));
-  }
+  if (p.gate.ptr) f *= p.gate_scale / (1.0f + __expf(-bf16_to_f32(gate)));
   if (gi == 0) {
     if (part == 0) p.lse[((int64_t)b * p.H + h) * p.Sq + i] = (m + __log2f(l)) * kLn2;
     const u32x2 w = {pack_bf16x2(y[0] * f, y[1] * f), pack_bf16x2(y[2] * f, y[3] * f)};

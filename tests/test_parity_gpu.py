@@ -1076,6 +1076,9 @@ def test_decode_mixes_a_value_residual_before_it_rounds(gpu_device, B, H, Hkv, S
     (1, 2, 1, 1500, 1500, 128, {"qk_norm": False}, {"head_scales": True}, True),              # shares whose keys some rows do not see
     (1, 8, 2, 257, 2113, 64, {"q_start": 1856, "qk_norm": False}, {"head_scales": True}, False),
     (1, 4, 2, 200, 1900, 64, {"causal": False}, {}, False),
+    (1, 1, 1, 70, 5000, 64, {"q_start": 4930}, {"extras": True}, False),                      # 20 shares: more than a lane requests up front
+    (1, 1, 1, 70, 5000, 128, {"q_start": 4930}, {}, False),                                   # 40
+    (1, 4, 4, 2100, 8192, 64, {"q_start": 6092}, {"extras": True}, False),                    # 8400 rows: one lane takes all 5 shares of its columns
 ])
 def test_forward_only_split_keys(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw, use_rope):
     """Forward-only calls with few query tiles share out the keys of a tile (partials in the kv workspace, merged by a
