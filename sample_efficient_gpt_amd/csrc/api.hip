@@ -435,6 +435,7 @@ static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage
   bind_kv(a);
   if ((rc = bind_split(a, true))) return rc;
   if (p->dtype == SEGPT_DTYPE_FP32) a.f32_parts = a.f32_split ? f32_split_parts(*p) : p->H / p->Hkv * a.f32_splits;
+  a.f32_both = a.f32_split && stage_lo <= SEGPT_BWD_STAGE_DQ && stage_hi >= SEGPT_BWD_STAGE_DKDV && f32_split_both(a);
   a.n_dq_blocks = dq_blocks(*p);
   a.n_dkdv_blocks = dkdv_blocks(*p);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
@@ -446,10 +447,12 @@ static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage
         else rc = (p->flags & SEGPT_FLAG_KV_PREPARED) ? 0 : launch_kv_prep(a, st);
         break;
       case SEGPT_BWD_STAGE_DKDV:
-        rc = f32 ? (a.f32_split ? launch_bwd_dkdv_split(a, st) : launch_bwd_dkdv_f32(a, st)) : launch_bwd_dkdv_bf16(a, st);
+        if (a.f32_both) rc = launch_finish_f32(a, st);
+        else rc = f32 ? (a.f32_split ? launch_bwd_dkdv_split(a, st) : launch_bwd_dkdv_f32(a, st)) : launch_bwd_dkdv_bf16(a, st);
         break;
       case SEGPT_BWD_STAGE_DQ:
-        rc = f32 ? (a.f32_split ? launch_bwd_dq_split(a, st) : launch_bwd_dq_f32(a, st)) : launch_bwd_dq_bf16(a, st);
+        if (a.f32_both) rc = launch_bwd_both_split(a, st);
+        else rc = f32 ? (a.f32_split ? launch_bwd_dq_split(a, st) : launch_bwd_dq_f32(a, st)) : launch_bwd_dq_bf16(a, st);
         break;
       case SEGPT_BWD_STAGE_REDUCE: rc = launch_bwd_reduce(a, st); break;
       default: return SEGPT_E_STAGE;

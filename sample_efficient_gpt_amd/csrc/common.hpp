@@ -39,6 +39,7 @@ struct KArgs {
   float* f32_dk_part;
   float* f32_dv_part;
   int32_t f32_splits, f32_parts;  // f32_parts: parts of dK, dV per kv head
+  bool f32_both;  // dQ and dK/dV share a launch
   char* f32_split;  // fp32 calls with SEGPT_FLAG_F32_SPLIT: operands as three bf16 numbers each (kv_workspace; f32_split.hip), else null
 };
 
@@ -205,6 +206,9 @@ int launch_split_prep(const KArgs& a, bool bwd, hipStream_t st);  // fp32 on the
 int launch_fwd_split(const KArgs& a, hipStream_t st);
 int launch_bwd_dq_split(const KArgs& a, hipStream_t st);
 int launch_bwd_dkdv_split(const KArgs& a, hipStream_t st);
+bool f32_split_both(const KArgs& a);  // dQ and dK/dV of a whole backward in one launch
+int launch_bwd_both_split(const KArgs& a, hipStream_t st);
+int launch_finish_f32(const KArgs& a, hipStream_t st);
 int f32_split_parts(const segpt_attn_params& p);
 size_t f32_split_bytes(const segpt_attn_params& p, bool bwd);  // scratch its operands take
 int launch_fwd_bf16(const KArgs& a, hipStream_t st);

@@ -7,7 +7,6 @@ namespace segpt {
 
 int f32_dq_grid(const segpt_attn_params& p);
 int f32_dkdv_splits(const segpt_attn_params& p);
-int launch_finish_f32(const KArgs& a, hipStream_t st);
 
 namespace {
 

@@ -369,7 +369,7 @@ __global__ __launch_bounds__(kThreads) void bwd_finish_f32_kernel(KArgs a) {
   __shared__ float tot[D];
   const int tid = threadIdx.x;
   if (blockIdx.x == 0) {
-    if (!a.f32_split) reduce_scale_grad<kThreads>(a, tid, red, tot);  // the other dK/dV kernel has done it
+    if (!a.f32_split || a.f32_both) reduce_scale_grad<kThreads>(a, tid, red, tot);  // else the other dK/dV kernel has done it
     return;
   }
   const int part = tid % T::kLPR;

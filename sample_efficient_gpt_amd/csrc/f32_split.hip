@@ -401,20 +401,22 @@ __device__ __forceinline__ void fetch_units(char* lds, const char* tile, int tid
 }
 
 // ---- dQ: S^T and dP^T (lane = query), T^T += Khat^T dS^T
+// `lds` holds in the loop the units of Qhat and dO (of Khat and V' below), after it the four waves' results
 template <int D>
-__global__ __launch_bounds__(kThreads, 2) void bwd_dq_split_kernel(KArgs a) {
+constexpr int kBwdLds = std::max(2 * kTileBytes<D>, 4 * kWaves * T32<D>::kTile);
+template <int D>
+constexpr int kBwdRed = kWaves * std::max(D, 64);
+template <int D>
+__device__ __forceinline__ void bwd_dq_split(const KArgs& a, int block, char* lds, float* red) {
   const segpt_attn_params& p = a.p;
   using T = T32<D>;
-  // in the loop the units of Qhat and dO, after it the four waves' results
-  __shared__ __attribute__((aligned(16))) char lds[std::max(2 * kTileBytes<D>, 4 * kWaves * T::kTile)];
   char *const qs = lds, *const ds = lds + kTileBytes<D>;
   float* const tiles = reinterpret_cast<float*>(lds);
-  __shared__ __attribute__((aligned(16))) float red[kWaves * D];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
   const int n_qt = tiles_of(p.Sq), rep = p.H / p.Hkv;
-  const Item item = split_item(blockIdx.x, n_qt, p.B * p.Hkv, rep);
+  const Item item = split_item(block, n_qt, p.B * p.Hkv, rep);
   if (item.pair >= p.B * p.Hkv) return;
   const int b = item.pair / p.Hkv, g = item.pair % p.Hkv, h = g * rep + item.member;
   const int qt = n_qt - 1 - item.tile, q0 = qt * kRows;
@@ -484,24 +486,17 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_split_kernel(KArgs a) {
 // ---- dK, dV of one kv head: S = Qhat Khat^T and dP = dO V'^T (lane = key), dV^T += dO^T P, dK^T += Qhat^T dS.  The query tiles
 // that see the keys, of all query heads of the group one after the other, are dealt out to 4 f32_parts waves; a workgroup
 // leaves one part of the sum (bwd_dkdv_f32_kernel leaves one per query head and share: twice the traffic at two heads a group).
-// The first workgroup adds up the scale gradient behind the others' back: in the finish kernel it was the longest one (finish 6.9 -> 4.7 us at 512 rows,
-// 109 -> 24 at 9216; the other seven of the first kXcds workgroups keep the rest on their XCDs).
 template <int D>
-__global__ __launch_bounds__(kThreads, (D == 128 ? 1 : 2)) void bwd_dkdv_split_kernel(KArgs a) {
+__device__ __forceinline__ void bwd_dkdv_split(const KArgs& a, int block, char* lds, float* stat_lds) {
   const segpt_attn_params& p = a.p;
   using T = T32<D>;
-  __shared__ __attribute__((aligned(16))) char lds[std::max(2 * kTileBytes<D>, 4 * kWaves * T::kTile)];  // as above: Khat and V'
   char *const ks = lds, *const vs = lds + kTileBytes<D>;
   float* const tiles = reinterpret_cast<float*>(lds);
-  __shared__ __attribute__((aligned(16))) float stat[kWaves][64];
+  float(*const stat)[64] = reinterpret_cast<float(*)[64]>(stat_lds);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
-  if (blockIdx.x < kXcds) {
-    if (blockIdx.x == 0) reduce_scale_grad<kThreads>(a, tid, tiles, tiles + kThreads);
-    return;
-  }
-  const Item item = split_item(blockIdx.x - kXcds, tiles_of(p.Sk), p.B * p.Hkv, a.f32_parts);  // the first key tiles are the heaviest
+  const Item item = split_item(block, tiles_of(p.Sk), p.B * p.Hkv, a.f32_parts);  // the first key tiles are the heaviest
   if (item.pair >= p.B * p.Hkv) return;
   const int kt_i = item.tile, part_i = item.member, bg = item.pair;
   const int b = bg / p.Hkv, g = bg % p.Hkv, rep = p.H / p.Hkv;
@@ -608,6 +603,38 @@ __global__ __launch_bounds__(kThreads, (D == 128 ? 1 : 2)) void bwd_dkdv_split_k
   leave(dv, a.f32_dv_part);
 }
 
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void bwd_dq_split_kernel(KArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[kBwdLds<D>];
+  __shared__ __attribute__((aligned(16))) float red[kBwdRed<D>];
+  bwd_dq_split<D>(a, blockIdx.x, lds, red);
+}
+// On its own the dK/dV launch's first workgroup adds up the scale gradient behind the others' back: in the finish kernel it was the longest one (finish
+// 6.9 -> 4.7 us at 512 rows, 109 -> 24 at 9216; the other seven of the first kXcds workgroups keep the rest on their XCDs).
+template <int D>
+__global__ __launch_bounds__(kThreads, (D == 128 ? 1 : 2)) void bwd_dkdv_split_kernel(KArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[kBwdLds<D>];
+  __shared__ __attribute__((aligned(16))) float stat[kBwdRed<D>];
+  if (blockIdx.x < kXcds) {
+    float* const sums = reinterpret_cast<float*>(lds);
+    if (blockIdx.x == 0) reduce_scale_grad<kThreads>(a, threadIdx.x, sums, sums + kThreads);
+    return;
+  }
+  bwd_dkdv_split<D>(a, blockIdx.x - kXcds, lds, stat);
+}
+// Both, dK/dV first: they need the pre-pass and not each other, so the heavy dQ workgroups fill the causal tail of dK/dV and a launch is saved; the
+// finish kernel adds up the scale gradient.  For grids of one or two resident rounds each, where the tail counts (f32_split_both).  Step, us, two
+// launches -> one: 2 x 8 / 4 heads of 64, 1000 tokens 103.4 -> 101.0, 400 tokens 59.2 -> 54.7; 1 x 4 heads, 700 tokens 61.0 -> 55.6; 4 x 8
+// heads, 1000 tokens (1024 dQ workgroups) 202.9 -> 201.8; 3 x 6 / 2 heads of 32, 1000 tokens 77.1 -> 74.9.  head_dim 128 has its own register
+// bound for dK/dV; larger grids want a pair's tiles pinned to an XCD and have the longer sum of the scale gradient.
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void bwd_both_split_kernel(KArgs a, int n_dkdv) {
+  __shared__ __attribute__((aligned(16))) char lds[kBwdLds<D>];
+  __shared__ __attribute__((aligned(16))) float red[kBwdRed<D>];
+  if ((int)blockIdx.x < n_dkdv) bwd_dkdv_split<D>(a, blockIdx.x, lds, red);
+  else bwd_dq_split<D>(a, blockIdx.x - n_dkdv, lds, red);
+}
+
 int n_tiles(int n) { return (n + kRows - 1) / kRows; }
 
 dim3 split_grid(int tiles, int pairs, int members, int extra = 0) {
@@ -698,6 +725,21 @@ int launch_bwd_dq_split(const KArgs& a, hipStream_t st) {
     case 128: return launch_dq<128>(a, st);
     default: return (int)hipErrorInvalidValue;
   }
+}
+bool f32_split_both(const KArgs& a) {
+  const segpt_attn_params& p = a.p;
+  return p.D != 128 && n_tiles(p.Sq) * (int64_t)p.B * p.H <= kPinnedGrid && n_tiles(p.Sk) * (int64_t)p.B * p.Hkv * a.f32_parts <= kPinnedGrid;
+}
+int launch_bwd_both_split(const KArgs& a, hipStream_t st) {
+  const segpt_attn_params& p = a.p;
+  const int n_dkdv = n_tiles(p.Sk) * p.B * p.Hkv * a.f32_parts, n_dq = n_tiles(p.Sq) * p.B * p.H;
+  const dim3 grid((unsigned)(n_dkdv + n_dq)), block(kThreads);
+  switch (p.D) {
+    case 32: hipLaunchKernelGGL(bwd_both_split_kernel<32>, grid, block, 0, st, a, n_dkdv); break;
+    case 64: hipLaunchKernelGGL(bwd_both_split_kernel<64>, grid, block, 0, st, a, n_dkdv); break;
+    default: return (int)hipErrorInvalidValue;
+  }
+  return (int)hipGetLastError();
 }
 int launch_bwd_dkdv_split(const KArgs& a, hipStream_t st) {
   switch (a.p.D) {
