@@ -130,6 +130,32 @@ def test_fp32_split_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
     _case(gpu_device, F32, B, H, Hkv, Sq, Sk, D, gen_kw=gen_kw, seed=72, **kw)
 
 
+@pytest.mark.parametrize("B,H,Hkv,S,D,extras", [(1, 4, 2, 401, 64, True), (4, 12, 4, 300, 32, False), (4, 8, 4, 1024, 64, False), (4, 8, 4, 1025, 64, True)])
+def test_fp32_split_backward_in_one_launch_is_its_stages(gpu_device, B, H, Hkv, S, D, extras):
+    """dQ and dK/dV of a whole backward share a launch up to 1024 workgroups each (the third case; the fourth has more); the stages run one
+    by one.  Both are within 8 units of 2^-24 of float64 in norm (test_fp32_split_is_no_less_accurate), so within 16 of each other."""
+    from sample_efficient_gpt_amd import _lib
+    from sample_efficient_gpt_amd.plan import AttnPlan
+
+    x = gen(B, H, Hkv, S, S, D, F32, seed=51, extras=extras)
+    plan = AttnPlan({n: None if t is None else t.to(gpu_device) for n, t in x.items()})
+    need = plan.lib.segpt_attn_workspace_bytes(plan.p, _lib.SEGPT_WS_F32_BWD)
+    assert need > 0
+    plan.forward()
+    scratch = torch.empty(need, dtype=torch.uint8, device=gpu_device)
+    plan.p.kv_workspace, plan.p.kv_workspace_bytes = scratch.data_ptr(), need
+    plan.base_flags |= _lib.SEGPT_FLAG_F32_SPLIT
+    grads = [t for t in (plan.dq, plan.dk, plan.dv, plan.dg_q, plan.dg_k, plan.dv_first, plan.dgate) if t is not None]
+    plan.backward()
+    whole = [t.clone() for t in grads]
+    for t in grads:
+        t.fill_(float("nan"))
+    for stage in range(4):
+        plan.backward_stage(stage)
+    for w, t in zip(whole, grads):
+        assert (w.double() - t.double()).norm() <= 16 * 2.0**-24 * w.double().norm()
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_split_is_no_less_accurate(gpu_device, D):
     """Distance to float64 in norm, in units of 2^-24, of y, dq, dk, dv of a call that the splits take.  With the fp32 matrix instruction
