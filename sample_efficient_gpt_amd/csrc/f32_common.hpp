@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "work_order.hpp"
 
 namespace segpt {
 
@@ -57,17 +58,6 @@ __device__ __forceinline__ f32x16 add_chains(f32x16 (&s)[N]) {
 // rounded first is off by half a unit at |lse|, for every key of the row alike)
 __device__ __forceinline__ float prob(float s, float lse) { return __builtin_amdgcn_exp2f(fmaf(lse, -kLog2e, s)); }
 __device__ __forceinline__ int crow(int r, int hh) { return 8 * (r >> 2) + 4 * hh + (r & 3); }
-
-// Work items are listed heaviest first.  When the whole grid is resident at once (up to two workgroups on each of 256
-// CUs) or nearly so, the CU that got item i also gets item i + 256: every second round of 256 is dealt in reverse, so
-// that a heavy item shares its CU with a light one (512 items: forward 37.8 -> 31.8 us, dQ 51 -> 43).  Larger grids
-// balance by themselves and keep the plain order (dK/dV 3 % slower reversed at 9216 items).
-__device__ __forceinline__ int work_item(int id, int n) {
-  const int round = id >> 8;
-  if (n > 1024 || !(round & 1)) return id;
-  const int x = id & 255;
-  return (round << 8) + 256 <= n ? (round << 8) + 248 - (x & 248) + (x & 7) : n - 1 - x;
-}
 
 // LDS regions here are private to a wave: program order is enough, the compiler only has to keep it
 __device__ __forceinline__ void wave_sync() {

@@ -259,30 +259,6 @@ __global__ __launch_bounds__(kThreads) void split_prep_kernel(KArgs a) {
   else emit_rm<D>(tile, dst, lane);
 }
 
-// Which tile a workgroup takes: (tile, heaviest first; (batch, kv head); member of the pair: query head or part).  Up to 1024
-// workgroups, most of them resident at once, as in f32_path.hip.  More: one pair after the other on each XCD, so that the
-// streamed tiles of the resident workgroups (2.4 MB a pair at 2048 keys of 64) stay in its L2; with all pairs in turn they came
-// out of the memory side at its 7 TB/s.  `pair` is past the last one for the workgroups that fill up the last round.
-struct Item {
-  int tile, pair, member;
-};
-constexpr int kPinnedGrid = 1024, kXcds = 8;
-__device__ __forceinline__ Item split_item(int block, int tiles, int pairs, int members) {
-  Item it;
-  if ((int64_t)tiles * pairs * members <= kPinnedGrid) {
-    const int id = work_item(block, tiles * pairs * members), rest = id % (pairs * members);
-    it.tile = id / (pairs * members);
-    it.pair = rest / members;
-    it.member = rest % members;
-  } else {
-    const int k = block / 8, per = tiles * members, rest = k % per;
-    it.pair = 8 * (k / per) + block % 8;
-    it.tile = rest / members;
-    it.member = rest % members;
-  }
-  return it;
-}
-
 // ---- forward, as fwd_f32_kernel
 template <int D>
 __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
@@ -297,8 +273,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
   const int n_qt = tiles_of(p.Sq), rep = p.H / p.Hkv;
-  const Item item = split_item(blockIdx.x, n_qt, p.B * p.Hkv, rep);
-  if (item.pair >= p.B * p.Hkv) return;
+  const Item item = split_item(blockIdx.x, n_qt, p.B * p.Hkv, rep, 2 * (int64_t)tiles_of(p.Sk) * kTileBytes<D>);
   const int b = item.pair / p.Hkv, g = item.pair % p.Hkv, h = g * rep + item.member;
   const int qt = n_qt - 1 - item.tile, q0 = qt * kRows;
   int kend = p.Sk;
@@ -416,8 +391,7 @@ __device__ __forceinline__ void bwd_dq_split(const KArgs& a, int block, char* ld
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
   const int n_qt = tiles_of(p.Sq), rep = p.H / p.Hkv;
-  const Item item = split_item(block, n_qt, p.B * p.Hkv, rep);
-  if (item.pair >= p.B * p.Hkv) return;
+  const Item item = split_item(block, n_qt, p.B * p.Hkv, rep, 3 * (int64_t)tiles_of(p.Sk) * kTileBytes<D>);
   const int b = item.pair / p.Hkv, g = item.pair % p.Hkv, h = g * rep + item.member;
   const int qt = n_qt - 1 - item.tile, q0 = qt * kRows;
   int kend = p.Sk;
@@ -496,8 +470,7 @@ __device__ __forceinline__ void bwd_dkdv_split(const KArgs& a, int block, char* 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
-  const Item item = split_item(block, tiles_of(p.Sk), p.B * p.Hkv, a.f32_parts);  // the first key tiles are the heaviest
-  if (item.pair >= p.B * p.Hkv) return;
+  const Item item = split_item(block, tiles_of(p.Sk), p.B * p.Hkv, a.f32_parts, 4 * (int64_t)(p.H / p.Hkv) * tiles_of(p.Sq) * kTileBytes<D>);  // the first key tiles are the heaviest
   const int kt_i = item.tile, part_i = item.member, bg = item.pair;
   const int b = bg / p.Hkv, g = bg % p.Hkv, rep = p.H / p.Hkv;
   const int j0 = kt_i * kRows;
@@ -638,8 +611,7 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_both_split_kernel(KArgs a, in
 int n_tiles(int n) { return (n + kRows - 1) / kRows; }
 
 dim3 split_grid(int tiles, int pairs, int members, int extra = 0) {
-  const int64_t n = (int64_t)tiles * pairs * members;
-  return dim3((unsigned)(extra + (n <= kPinnedGrid ? n : (int64_t)8 * ((pairs + 7) / 8) * tiles * members)));
+  return dim3((unsigned)(extra + (int64_t)tiles * pairs * members));
 }
 
 template <int D>

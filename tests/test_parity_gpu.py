@@ -113,6 +113,8 @@ def test_fp32_tile_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
         (2, 4, 1, 800, 800, {"qk_norm": False}, {"scalar_gain": True, "no_gk": True}),
         (4, 8, 2, 200, 900, {"q_start": 3}, {}),                                          # keys that no query sees
         (5, 9, 3, 769, 769, {}, {}),  # more than 1024 workgroups, (batch, kv head) pairs that are no multiple of the XCDs
+        (1, 44, 1, 770, 770, {}, {}),  # the same with one pair for all XCDs
+        (1, 27, 3, 1290, 1290, {}, {}),  # three pairs: two and one at a time; dK/dV between 512 and 1024 workgroups, more than an L2 streamed
     ],
 )
 def test_fp32_split_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
@@ -127,6 +129,7 @@ def test_fp32_split_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
     kw = dict(kw)
     if kw.pop("rope", False):
         kw["rope"] = orc.rope_tables(1000, 10000.0, D)
+    print(f"split edges B={B} H={H} Hkv={Hkv} Sq={Sq} Sk={Sk} D={D}", flush=True)
     _case(gpu_device, F32, B, H, Hkv, Sq, Sk, D, gen_kw=gen_kw, seed=72, **kw)
 
 
