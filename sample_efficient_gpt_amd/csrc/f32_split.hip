@@ -660,13 +660,20 @@ int f32_split_parts(const segpt_attn_params& p) {
 //   backward head_dim 128:  64 tokens, 4 heads 39 -> 31, 1000 153 -> 83;  16 heads: 128 43 -> 38, 512 123 -> 80
 //            64, 16 heads:  256 31 -> 33, 384 47 -> 42, 1000 112 -> 85;  32 heads: 192 38 -> 35, 384 67 -> 56
 //            32, 12 heads:  384 27 -> 30, 512 33.5 -> 33.1, 768 54 -> 43;  48 heads: 192 29 -> 33, 384 54 -> 43
+// Few workgroups that read a key tile (users: query tiles of the group's heads), forward; the backward gains there too:
+//   forward  128, 16 heads:  256 20.5 -> 21.1, 384 27.4 -> 24.9;  32 heads: 256 21.1 -> 24.3, 320 27.5 -> 30.2, 384 33.3 -> 33.3, 512 54 -> 36;
+//            64 heads: 256 33.9 -> 30.0;  8 heads: 256 20.4 -> 19.6;  8 x 32 / 4 heads, one query, 4096 keys 228 -> 153
+//            64, 17 heads:  512 19.4 -> 21.4;  8 x 32 / 4 heads, one query, 4096 keys 107 -> 75
+//            32, 128 heads:  256 16.6 -> 18.8, 384 27.2 -> 28.4, 448 35 -> 32;  256 heads: 256 30.4 -> 29.8, 320 41 -> 36;  48 heads: 384 14.0 -> 14.4, 448 16.1 -> 16.0
+//   backward 128, one query:  4 heads, 2048 keys 180 -> 89;  8 x 32 / 4 heads, 4096 keys 2735 -> 601;  32 x 16 heads, one key 86 -> 66
 bool f32_split_pays(const segpt_attn_params& p, bool bwd) {
   const int n_qt = n_tiles(p.Sq), n_kt = n_tiles(p.Sk);
-  const int64_t heads = (int64_t)p.B * p.H, pairs = heads * n_qt * n_kt;
-  if ((int64_t)(p.H / p.Hkv) * n_qt < 8 && !(bwd && p.D == 128)) return false;  // one query against a long cache: split keys used once or twice
-  if (p.D == 128) return bwd || n_kt >= 6;
+  const int64_t heads = (int64_t)p.B * p.H, pairs = heads * n_qt * n_kt, grid = heads * n_qt;
+  const int64_t users = (int64_t)(p.H / p.Hkv) * n_qt;  // workgroups that read a key tile
+  if (users < 8 && !(bwd && p.D == 128)) return false;  // one query against a long cache: split keys used once or twice
+  if (p.D == 128) return bwd || (n_kt >= 6 && (n_kt >= 12 || users >= 12 || grid <= 64 || grid >= 512));
   if (p.D == 64) return bwd ? n_kt >= 12 : n_kt >= 24 || (n_kt >= 16 && heads <= 16);
-  return pairs >= (bwd ? 3072 : 5000);
+  return bwd ? pairs >= 3072 : pairs >= 5000 && (n_kt >= 14 || users >= 14 || grid >= 2560);
 }
 size_t f32_split_bytes(const segpt_attn_params& p, bool bwd) {
   if (!f32_split_pays(p, bwd)) return 0;

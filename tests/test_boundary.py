@@ -300,7 +300,7 @@ def test_fp32_backward_needs_partials_only_where_there_are_several(lib):
 
 
 def test_fp32_split_scratch(lib):
-    """SEGPT_FLAG_F32_SPLIT: sizes (0 where the other kernels are taken: short calls, a query or two against a long cache), what the
+    """SEGPT_FLAG_F32_SPLIT: sizes (0 where the other kernels are taken: short calls, forwards of a query or two against a long cache), what the
     flag asks of kv_workspace, and no effect without it or on bf16."""
 
     def params(Sq, Sk, D=64, **kw):
@@ -315,10 +315,17 @@ def test_fp32_split_scratch(lib):
 
     size = lambda p: [lib.segpt_attn_workspace_bytes(p, w) for w in (_lib.SEGPT_WS_F32_FWD, _lib.SEGPT_WS_F32_BWD)]
     for D in (32, 64, 128):
-        assert size(params(1, 8192, D))[0] == 0
+        few = size(params(1, 8192, D))
+        assert few[0] == 0 and (few[1] > 0) == (D == 128)  # the backward is the faster one at head_dim 128, whatever the queries
         kv, q = 2 * 2 * 32 * 32 * D, 2 * 6 * 32 * 32 * D  # elements of K and of Q in whole tiles
         assert size(params(1000, 1000, D)) == [2 * kv * 6, 3 * kv * 6 + 4 * q * 6 + 2 * 6 * 32 * 64 * 4]
     assert size(params(128, 128)) == [0, 0]
+    # head_dim 128: few users of a short key tile are not worth the forward's pre-pass in launches of 65 to 511 workgroups
+    heads = lambda n, S, D: (lambda p: (setattr(p, "H", n), setattr(p, "Hkv", n), setattr(p, "B", 1), size(p))[-1])(params(S, S, D))
+    assert heads(32, 256, 128)[0] == 0 and heads(32, 256, 128)[1] > 0
+    assert heads(8, 256, 128)[0] > 0 and heads(64, 256, 128)[0] > 0 and heads(32, 384, 128)[0] > 0
+    # head_dim 32: the same below 14 key tiles up to 2559 workgroups
+    assert heads(128, 256, 32)[0] == 0 and heads(128, 448, 32)[0] > 0 and heads(320, 256, 32)[0] > 0
     p = _valid_params(); p.Sq = p.Sk = 1000
     assert size(p) == [0, 0]
     for call, i in ((lib.segpt_attn_fwd, 0), (lib.segpt_attn_bwd, 1)):
