@@ -9,7 +9,7 @@
 // fp32 instructions 1.5e-7 / 1.95e-7, one accumulator for all six 1.1e-7 / 1.6e-7, the largest product on its own 4.9e-8 / 6.4e-8.
 //
 // Range: the parts of a value of 2^-102 (2e-31) and more are normal numbers, smaller ones lose their last bits (dO of 1e-32: as above; of
-// 1e-35: 8e-5 from float64).  An infinity among the operands gives NaN where the fp32 instructions give an infinity or NaN.
+// 1e-35: 8e-5 from float64).  Infinities and finite values beyond bf16's largest: see split8.
 //
 // What that takes: nothing may be split inside a loop that runs once per pair of tiles.  A pre-pass rotates, normalises
 // and splits every row once and leaves 32-row tiles as matrix-instruction operands, 1 KB (64 lanes x 16 bytes) each, in the order they
@@ -79,23 +79,45 @@ __device__ __forceinline__ void step_end() { __builtin_amdgcn_sched_barrier(0); 
 
 __device__ __forceinline__ f32x16 mfma16(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 
+// Beyond bf16's range: a finite value there keeps bf16's largest number as its first part, the rest goes into the other two.  An infinity is
+// the third part alone, which meets only the other operand's first part: the product is that infinity, or NaN where the other
+// operand is 0, as with the fp32 instructions (as the first part it met the remainders of either sign).
+constexpr float kBf16Max = 3.38953139e38f;
+template <int N>
+__device__ __forceinline__ bool beyond_bf16(const float (&x)[N]) {
+  float m = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) m = fmaxf(m, fabsf(x[i]));  // NaN needs nothing: every part of it is NaN
+  return __builtin_amdgcn_ballot_w64(m > kBf16Max) != 0;
+}
+template <bool BEYOND>
 __device__ __forceinline__ Split3 split8(const float (&x)[8]) {
   Split3 s;
   u32x4 w[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float a = x[2 * i], b = x[2 * i + 1];
+    float v[2] = {x[2 * i], x[2 * i + 1]}, first[2] = {v[0], v[1]};
+    if (BEYOND) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      w[k][i] = pack_bf16x2(a, b);
-      a -= bf16lo(w[k][i]);
-      b -= bf16hi(w[k][i]);
+      for (int e = 0; e < 2; ++e) {
+        const bool inf = __builtin_isinf(v[e]);
+        first[e] = inf ? 0.f : fabsf(v[e]) > kBf16Max ? copysignf(kBf16Max, v[e]) : v[e];
+      }
     }
+    w[0][i] = pack_bf16x2(first[0], first[1]);
+    float a = v[0] - bf16lo(w[0][i]), b = v[1] - bf16hi(w[0][i]);
+    if (BEYOND) {
+      w[1][i] = pack_bf16x2(__builtin_isinf(v[0]) ? 0.f : a, __builtin_isinf(v[1]) ? 0.f : b);
+    } else {
+      w[1][i] = pack_bf16x2(a, b);
+    }
+    w[2][i] = pack_bf16x2(a - bf16lo(w[1][i]), b - bf16hi(w[1][i]));
   }
 #pragma unroll
   for (int k = 0; k < 3; ++k) s.p[k] = __builtin_bit_cast(bf16x8, w[k]);
   return s;
 }
+__device__ __forceinline__ Split3 split_row(const float (&x)[8]) { return beyond_bf16(x) ? split8<true>(x) : split8<false>(x); }
 
 __device__ __forceinline__ Split3 load_unit(const char* unit, int lane) {
   Split3 s;
@@ -116,7 +138,7 @@ __device__ __forceinline__ void emit_rm(const float* tile, char* dst, int lane, 
     const f32x4v* src = reinterpret_cast<const f32x4v*>(tile + (lane & 31) * T32<D>::kRS + 16 * u + 8 * (lane >> 5));
     const f32x4v lo = src[0], hi = src[1];
     const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    store_unit(dst + u * kUnitBytes, split8(x), lane);
+    store_unit(dst + u * kUnitBytes, split_row(x), lane);
   }
 }
 template <int D>
@@ -128,7 +150,7 @@ __device__ __forceinline__ void emit_tr(const float* tile, char* dst, int lane) 
     float x[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = src[crow(8 * (u % 2) + i, lane >> 5) * T32<D>::kRS];
-    store_unit(dst + u * kUnitBytes, split8(x), lane);
+    store_unit(dst + u * kUnitBytes, split_row(x), lane);
   }
 }
 
@@ -162,14 +184,23 @@ struct Dot {
 struct Scores3 {
   Split3 s[2];
 };
-__device__ __forceinline__ Scores3 split_scores(const f32x16& w) {
+template <bool BEYOND>
+__device__ __forceinline__ Scores3 split16(const float (&w)[16]) {
   Scores3 b;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     const float x[8] = {w[8 * s], w[8 * s + 1], w[8 * s + 2], w[8 * s + 3], w[8 * s + 4], w[8 * s + 5], w[8 * s + 6], w[8 * s + 7]};
-    b.s[s] = split8(x);
+    b.s[s] = split8<BEYOND>(x);
   }
   return b;
+}
+// probabilities (at most 1) never leave bf16's range, their gradients may
+template <bool PROBS>
+__device__ __forceinline__ Scores3 split_scores(const f32x16& w) {
+  float x[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) x[r] = w[r];
+  return !PROBS && beyond_bf16(x) ? split16<true>(x) : split16<false>(x);
 }
 // acc += (block mb of a tile)^T . w over the 32 rows; the tile's sum is formed by itself and added once
 __device__ __forceinline__ void add_tr(const Half& a, const Scores3& w, f32x16& acc) {
@@ -348,7 +379,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
       part[r & 1] += s[r];
     }
     l += part[0] + part[1];
-    const Scores3 probs = split_scores(s);
+    const Scores3 probs = split_scores<true>(s);
 #pragma unroll
     for (int i = MB; i < kSteps; ++i) {
       step_end();
@@ -441,7 +472,7 @@ __device__ __forceinline__ void bwd_dq_split(const KArgs& a, int block, char* ld
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] *= dp[r] - delta;
-    const Scores3 grads = split_scores(s);
+    const Scores3 grads = split_scores<false>(s);
 #pragma unroll
     for (int i = 2 * MB; i < kSteps; ++i) {
       step_end();
@@ -540,14 +571,14 @@ __device__ __forceinline__ void bwd_dkdv_split(const KArgs& a, int block, char* 
         if (i >= p.Sq || (p.causal && j0 + ln > i + p.q_start)) s[r] = 0.f;
       }
     }
-    const Scores3 probs = split_scores(s);
+    const Scores3 probs = split_scores<true>(s);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const f32x4v de = *reinterpret_cast<const f32x4v*>(&stat[wave][32 + 8 * q + 4 * hh]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) s[4 * q + e] *= dp[4 * q + e] - de[e];
     }
-    const Scores3 grads = split_scores(s);
+    const Scores3 grads = split_scores<false>(s);
 #pragma unroll
     for (int i = 2 * MB; i < kSteps; ++i) {
       step_end();

@@ -178,6 +178,60 @@ def test_fp32_split_is_no_less_accurate(gpu_device, D):
     assert all(e <= bound for e, bound in zip(err, (3.31, 6.36, 7.60, 6.09)))
 
 
+def _fp32_both_ways(x, device):
+    """y, dq, dk, dv with the three-bf16 kernels (the call as users make it) and with the fp32 instructions (without the flag)."""
+    from sample_efficient_gpt_amd import _lib
+    from sample_efficient_gpt_amd.plan import AttnPlan
+
+    plan = AttnPlan({n: None if t is None else t.to(device) for n, t in x.items()})
+    for which in (_lib.SEGPT_WS_F32_FWD, _lib.SEGPT_WS_F32_BWD):
+        assert plan.lib.segpt_attn_workspace_bytes(plan.p, which) > 0
+    plan.forward()
+    plan.backward()
+    torch.cuda.synchronize()
+    got = run_gpu(x, device)
+    return [got[n] for n in ("y", "dq", "dk", "dv")], [t.cpu() for t in (plan.y, plan.dq, plan.dk, plan.dv)]
+
+
+def _within(a, b, units):
+    """Distance in norm of the finite values, in units of 2^-24; the others have to agree."""
+    fa, fb = torch.isfinite(a), torch.isfinite(b)
+    assert torch.equal(fa, fb) and torch.equal(a.isinf(), b.isinf()) and torch.equal(a[a.isinf()], b[b.isinf()])
+    a, b = a.double()[fa], b.double()[fb]
+    assert (a - b).norm() <= units * 2.0**-24 * b.norm()
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_split_values_beyond_bf16s_range(gpu_device, D):
+    """Infinities and finite values above bf16's largest number in v and dO: infinite, NaN and finite results stand where the fp32
+    instructions have them.  Both are within 8 units of 2^-24 of float64 (test_fp32_split_is_no_less_accurate), so within 16 of each other."""
+    base = gen(1, 8, 4, 800, 800, D, F32, seed=67, scalar_gain=True, no_gk=True)
+
+    def run(name, row, value):
+        x = dict(base, **{name: base[name].clone()})
+        x[name][0, 1, row, 3] = value
+        print(f"{name}[{row}] = {value}, D={D}", flush=True)
+        return _fp32_both_ways(x, gpu_device)
+
+    new, old = run("v", 500, float("inf"))
+    assert new[0].isinf().sum() == 2 * 300 and new[0].isnan().sum() == old[0].isnan().sum()
+    for a, b in zip(new, old):
+        _within(a, b, 16)
+    for row in (0, 400):
+        new, old = run("d_o", row, float("-inf"))
+        assert new[3].isinf().any()
+        for a, b in zip(new, old):
+            _within(a, b, 16)
+    # query 0 sees key 0 alone: its row of y is v's, and dv gets dO's times the other probabilities
+    for value in (3.4e38, -3.3962e38):
+        new, old = run("v", 0, value)
+        assert torch.isfinite(new[0]).all() and new[0][0, 2, 0, 3] == torch.tensor(value)
+        _within(new[0], old[0], 16)
+        new, old = run("d_o", 0, value)
+        assert torch.isfinite(new[3]).all()
+        _within(new[3], old[3], 16)
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_rows_whose_mean_square_leaves_the_normal_range(gpu_device, D):
     """A key whose sum of squares overflows has the normaliser 0, like a key of zeros, and poisons nobody; keys so small
