@@ -143,8 +143,8 @@ inline bool tiny_eps(const segpt_attn_params& p) {
 }
 
 // normalise (and rotate) the rows of a tile and put them into LDS: x * 1/rms(x) * scale.  All rows' sums are formed
-// side by side, and the one branch (rotary tables or not) stands outside the row loop.
-template <int D, bool TINY_EPS>
+// side by side, and the one branch (rotary tables or not) stands outside the row loop.  KEEP: they stay in the registers too.
+template <int D, bool TINY_EPS, bool KEEP = false>
 __device__ __forceinline__ void stage_norm(const segpt_attn_params& p, f32x4v (&x)[T32<D>::kPasses], f32x4v scale, int pos0, int last,
                                            float* tile, int lane) {
   using T = T32<D>;
@@ -161,7 +161,9 @@ __device__ __forceinline__ void stage_norm(const segpt_attn_params& p, f32x4v (&
 #pragma unroll
   for (int ps = 0; ps < T::kPasses; ++ps) {
     const float n = TINY_EPS ? row_normaliser(p, inv[ps], 1.0f / D) : inv_rms(inv[ps], 1.0f / D, p.eps, norm);
-    *reinterpret_cast<f32x4v*>(tile + (ps * T::kRPP + lr) * T::kRS + 4 * part) = x[ps] * (n * scale);
+    const f32x4v y = x[ps] * (n * scale);
+    if (KEEP) x[ps] = y;
+    *reinterpret_cast<f32x4v*>(tile + (ps * T::kRPP + lr) * T::kRS + 4 * part) = y;
   }
 }
 template <int D>

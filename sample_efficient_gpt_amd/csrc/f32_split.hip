@@ -8,8 +8,8 @@
 // 20 small ones) roundings deep instead of 32: norm-wise distance of a 32x32 tile of products to float64, 64 / 128 columns:
 // fp32 instructions 1.5e-7 / 1.95e-7, one accumulator for all six 1.1e-7 / 1.6e-7, the largest product on its own 4.9e-8 / 6.4e-8.
 //
-// Range: the parts of a value of 2^-102 (2e-31) and more are normal numbers, smaller ones lose their last bits (dO of 1e-32: as above; of
-// 1e-35: 8e-5 from float64).  Infinities and finite values beyond bf16's largest: see split8.
+// Range: the last bits of a value below 2^-109 are none of bf16's any more.  Operand tiles with such values are kept with scaled parts
+// and take a slower form of the products (see kPart).  Infinities and finite values beyond bf16's largest: see split8.
 //
 // What that takes: nothing may be split inside a loop that runs once per pair of tiles.  A pre-pass rotates, normalises
 // and splits every row once and leaves 32-row tiles as matrix-instruction operands, 1 KB (64 lanes x 16 bytes) each, in the order they
@@ -56,20 +56,26 @@ constexpr int kHalfBytes = 2 * kUnitBytes;
 struct SplitMap {
   char *k_rm, *v, *k_tr, *q_rm, *q_tr, *d_rm, *d_tr;  // v: tr for the forward, rm for the backward
   float* stat;                                        // [B * H][query tiles][lse of 32 rows, delta of 32 rows]
+  uint32_t *k_small, *v_small, *q_small, *d_small;    // a tile's parts are scaled (kPart)
 };
 __device__ __forceinline__ int tiles_of(int n) { return (n + kRows - 1) / kRows; }
 template <int D>
-__device__ __forceinline__ SplitMap split_map(const KArgs& a) {
-  const int64_t kv = (int64_t)a.p.B * a.p.Hkv * tiles_of(a.p.Sk) * kTileBytes<D>, q = (int64_t)a.p.B * a.p.H * tiles_of(a.p.Sq) * kTileBytes<D>;
+__device__ __forceinline__ SplitMap split_map(const KArgs& a, bool bwd) {
+  const int64_t kvt = (int64_t)a.p.B * a.p.Hkv * tiles_of(a.p.Sk), qt = bwd ? (int64_t)a.p.B * a.p.H * tiles_of(a.p.Sq) : 0;
+  const int64_t kv = kvt * kTileBytes<D>, q = qt * kTileBytes<D>;
   SplitMap m;
   m.k_rm = a.f32_split;
   m.v = m.k_rm + kv;
-  m.k_tr = m.v + kv;
-  m.q_rm = m.k_tr + kv;
+  m.k_tr = m.v + kv;  // from here on to stat: backward only
+  m.q_rm = m.k_tr + (bwd ? kv : 0);
   m.q_tr = m.q_rm + q;
   m.d_rm = m.q_tr + q;
   m.d_tr = m.d_rm + q;
   m.stat = reinterpret_cast<float*>(m.d_tr + q);
+  m.k_small = reinterpret_cast<uint32_t*>(m.stat + qt * 64);
+  m.v_small = m.k_small + kvt;
+  m.q_small = m.v_small + kvt;
+  m.d_small = m.q_small + qt;
   return m;
 }
 
@@ -90,8 +96,16 @@ __device__ __forceinline__ bool beyond_bf16(const float (&x)[N]) {
   for (int i = 0; i < N; ++i) m = fmaxf(m, fabsf(x[i]));  // NaN needs nothing: every part of it is NaN
   return __builtin_amdgcn_ballot_w64(m > kBf16Max) != 0;
 }
+// Small values: the second part of a value is up to 2^16, the third up to 2^24 below it.  Where bits would fall below bf16's last, 2^-133, the
+// second part is kept times kPart and the third times kPart^2, and no bit is lost whose product fp32 could hold.  That is a property of
+// a tile (its flag in SplitMap); a wave that meets such a tile takes all its tiles through a loop of its own, in which the products of each
+// scale are formed apart.  dO of 1e-35: gradients were 6e-5 from float64, now 3.4e-7 (fp32 instructions 4e-7).  The flags and split_lanes
+// cost 1 to 4 % (backward of 2 x 8 / 4 heads, 1000 tokens 75.9 -> 78.1 us); scaling always and no second loop cost 5 to 8 %.
+constexpr float kPart = 128.f, kSmall = 7.888609052e-31f;  // 2^-100
+__device__ __forceinline__ bool any_lane(bool x) { return __builtin_amdgcn_ballot_w64(x) != 0; }
+__device__ __forceinline__ bool is_small(float x) { return x != 0.f && fabsf(x) < kSmall; }
 template <bool BEYOND>
-__device__ __forceinline__ Split3 split8(const float (&x)[8]) {
+__device__ __forceinline__ Split3 split8(const float (&x)[8], float part) {
   Split3 s;
   u32x4 w[3];
 #pragma unroll
@@ -105,19 +119,19 @@ __device__ __forceinline__ Split3 split8(const float (&x)[8]) {
       }
     }
     w[0][i] = pack_bf16x2(first[0], first[1]);
-    float a = v[0] - bf16lo(w[0][i]), b = v[1] - bf16hi(w[0][i]);
+    const float a = (v[0] - bf16lo(w[0][i])) * part, b = (v[1] - bf16hi(w[0][i])) * part;
     if (BEYOND) {
       w[1][i] = pack_bf16x2(__builtin_isinf(v[0]) ? 0.f : a, __builtin_isinf(v[1]) ? 0.f : b);
     } else {
       w[1][i] = pack_bf16x2(a, b);
     }
-    w[2][i] = pack_bf16x2(a - bf16lo(w[1][i]), b - bf16hi(w[1][i]));
+    w[2][i] = pack_bf16x2((a - bf16lo(w[1][i])) * part, (b - bf16hi(w[1][i])) * part);
   }
 #pragma unroll
   for (int k = 0; k < 3; ++k) s.p[k] = __builtin_bit_cast(bf16x8, w[k]);
   return s;
 }
-__device__ __forceinline__ Split3 split_row(const float (&x)[8]) { return beyond_bf16(x) ? split8<true>(x) : split8<false>(x); }
+__device__ __forceinline__ Split3 split_row(const float (&x)[8], float part) { return beyond_bf16(x) ? split8<true>(x, part) : split8<false>(x, part); }
 
 __device__ __forceinline__ Split3 load_unit(const char* unit, int lane) {
   Split3 s;
@@ -131,18 +145,34 @@ __device__ __forceinline__ void store_unit(char* unit, const Split3& s, int lane
   for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(unit + k * 1024 + lane * 16) = s.p[k];
 }
 
+// any small value in the tile that a wave holds?
+template <int D>
+__device__ __forceinline__ bool tile_small(const f32x4v (&x)[T32<D>::kPasses]) {
+  uint32_t m = ~0u;
+#pragma unroll
+  for (int ps = 0; ps < T32<D>::kPasses; ++ps)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m = min(m, (__float_as_uint(x[ps][e]) << 1) - 1);  // the sign goes, zero becomes the largest
+  return any_lane(m < (__float_as_uint(kSmall) << 1) - 1);
+}
+// the flags of n tiles; the first 64 are requested early
+__device__ __forceinline__ uint32_t first_flags(const uint32_t* flags, int n, int lane) { return lane < n ? flags[lane] : 0; }
+__device__ __forceinline__ bool any_small(uint32_t first, const uint32_t* flags, int n, int lane) {
+  for (int i = lane + 64; i < n; i += 64) first |= flags[i];
+  return any_lane(first);
+}
 // units u0, u0 + step, ... of a row-major fp32 tile in LDS
 template <int D>
-__device__ __forceinline__ void emit_rm(const float* tile, char* dst, int lane, int u0 = 0, int step = 1) {
+__device__ __forceinline__ void emit_rm(const float* tile, char* dst, int lane, float part, int u0 = 0, int step = 1) {
   for (int u = u0; u < kUnits<D>; u += step) {
     const f32x4v* src = reinterpret_cast<const f32x4v*>(tile + (lane & 31) * T32<D>::kRS + 16 * u + 8 * (lane >> 5));
     const f32x4v lo = src[0], hi = src[1];
     const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    store_unit(dst + u * kUnitBytes, split_row(x), lane);
+    store_unit(dst + u * kUnitBytes, split_row(x, part), lane);
   }
 }
 template <int D>
-__device__ __forceinline__ void emit_tr(const float* tile, char* dst, int lane) {
+__device__ __forceinline__ void emit_tr(const float* tile, char* dst, int lane, float part) {
   constexpr int MB = T32<D>::kMB;
 #pragma unroll
   for (int u = 0; u < kUnits<D>; ++u) {
@@ -150,7 +180,7 @@ __device__ __forceinline__ void emit_tr(const float* tile, char* dst, int lane) 
     float x[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = src[crow(8 * (u % 2) + i, lane >> 5) * T32<D>::kRS];
-    store_unit(dst + u * kUnitBytes, split_row(x), lane);
+    store_unit(dst + u * kUnitBytes, split_row(x, part), lane);
   }
 }
 
@@ -162,6 +192,21 @@ __device__ __forceinline__ f32x16 small5(const Split3& a, const Split3& b, f32x1
   c = mfma16(a.p[0], b.p[1], c);
   return mfma16(a.p[1], b.p[0], c);
 }
+// the same where the second parts of a, b or both are scaled by 1 / fa, 1 / fb, the third parts by the squares
+__device__ __forceinline__ f32x16 scaled5(const Split3& a, float fa, const Split3& b, float fb, f32x16 c) {
+  const int ia[5] = {0, 2, 1, 0, 1}, ib[5] = {2, 0, 1, 1, 0};
+  const float f[5] = {fb * fb, fa * fa, fa * fb, fb, fa};
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const f32x16 t = mfma16(a.p[ia[i]], b.p[ib[i]], zero16());
+#pragma unroll
+    for (int r = 0; r < 16; ++r) c[r] = fmaf(t[r], f[i], c[r]);
+    step_end();  // one product's 16 registers at a time
+  }
+  return c;
+}
+// what a tile's *_small flag means for its products (wave-uniform)
+__device__ __forceinline__ float part_scale(bool small) { return small ? 1.f / kPart : 1.f; }
 // X . B^T over the columns: C rows = rows of the streamed tile, C columns = the 32 stationary rows, whose rm units lie in LDS
 struct Dot {
   f32x16 large = zero16(), small = zero16();
@@ -171,6 +216,17 @@ struct Dot {
       const Split3 b = load_unit(b_lds + u * kUnitBytes, lane);
       small = small5(a.u[u], b, small);
       large = mfma16(a.u[u].p[0], b.p[0], large);
+    }
+  }
+  // the same for all units of a streamed tile, which come in one by one
+  template <int D>
+  __device__ __forceinline__ void add_scaled(const char* a_tile, bool a_small, const char* b_lds, bool b_small, int lane) {
+    const float fa = part_scale(a_small), fb = part_scale(b_small);
+#pragma unroll 1
+    for (int u = 0; u < kUnits<D>; ++u) {
+      const Split3 a = load_unit(a_tile + u * kUnitBytes, lane), b = load_unit(b_lds + u * kUnitBytes, lane);
+      small = scaled5(a, fa, b, fb, small);
+      large = mfma16(a.p[0], b.p[0], large);
     }
   }
   __device__ __forceinline__ f32x16 sum() const {
@@ -185,29 +241,53 @@ struct Scores3 {
   Split3 s[2];
 };
 template <bool BEYOND>
-__device__ __forceinline__ Scores3 split16(const float (&w)[16]) {
+__device__ __forceinline__ Scores3 split16(const f32x16& w, float part) {
   Scores3 b;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     const float x[8] = {w[8 * s], w[8 * s + 1], w[8 * s + 2], w[8 * s + 3], w[8 * s + 4], w[8 * s + 5], w[8 * s + 6], w[8 * s + 7]};
-    b.s[s] = split8<BEYOND>(x);
+    b.s[s] = split8<BEYOND>(x, part);
   }
   return b;
 }
-// probabilities (at most 1) never leave bf16's range, their gradients may
-template <bool PROBS>
-__device__ __forceinline__ Scores3 split_scores(const f32x16& w) {
-  float x[16];
+// Probabilities or, GRADS, their gradients.  The scores of a column (a lane and the one 32 on) add up among themselves: where the largest of
+// them is small, all are taken 2^64 times as large and their sum is multiplied by f.  (The forward's need no look, a row's largest is or was 1.)
+struct LaneScores {
+  Scores3 s;
+  float f;
+};
+template <bool GRADS>
+__device__ __forceinline__ LaneScores split_lanes(f32x16& w) {
+  float m = 0.f;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) x[r] = w[r];
-  return !PROBS && beyond_bf16(x) ? split16<true>(x) : split16<false>(x);
+  for (int r = 0; r < 16; ++r) m = fmaxf(m, fabsf(w[r]));  // NaN needs nothing: every part of it is NaN
+  m = half_max(m);  // two lanes hold a column
+  LaneScores x;
+  x.f = 1.f;
+  f32x16 v = w;
+  if (any_lane(is_small(m))) {
+    const bool up = is_small(m);
+    x.f = up ? 0x1p-64f : 1.f;
+    const float f = up ? 0x1p64f : 1.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] *= f;
+  }
+  x.s = GRADS && any_lane(m > kBf16Max) ? split16<true>(v, 1.f) : split16<false>(v, 1.f);
+  return x;
 }
 // acc += (block mb of a tile)^T . w over the 32 rows; the tile's sum is formed by itself and added once
-__device__ __forceinline__ void add_tr(const Half& a, const Scores3& w, f32x16& acc) {
-  f32x16 t = small5(a.u[0], w.s[0], zero16());
-  t = small5(a.u[1], w.s[1], t);
+__device__ __forceinline__ f32x16 add_large(const Half& a, const Scores3& w, f32x16 t) {
   t = mfma16(a.u[0].p[0], w.s[0].p[0], t);
-  t = mfma16(a.u[1].p[0], w.s[1].p[0], t);
+  return mfma16(a.u[1].p[0], w.s[1].p[0], t);
+}
+__device__ __forceinline__ void add_tr(const Half& a, const Scores3& w, f32x16& acc, float f = 1.f) {
+  const f32x16 t = add_large(a, w, small5(a.u[1], w.s[1], small5(a.u[0], w.s[0], zero16())));
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = fmaf(t[r], f, acc[r]);
+}
+__device__ __forceinline__ void add_tr_scaled(const Half& a, bool a_small, const Scores3& w, f32x16& acc) {  // w: always scaled
+  const float fa = part_scale(a_small), fw = 1.f / kPart;
+  const f32x16 t = add_large(a, w, scaled5(a.u[1], fa, w.s[1], fw, scaled5(a.u[0], fa, w.s[0], fw, zero16())));
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] += t[r];
 }
@@ -222,7 +302,7 @@ __global__ __launch_bounds__(kThreads) void split_prep_kernel(KArgs a) {
   __shared__ __attribute__((aligned(16))) float tiles[kWaves][T::kTile];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const SplitMap m = split_map<D>(a);
+  const SplitMap m = split_map<D>(a, BWD);
   const int n_qt = tiles_of(p.Sq), n_kt = tiles_of(p.Sk);
   float* tile = tiles[wave];
   int64_t job = (int64_t)blockIdx.x * kWaves + wave;
@@ -237,7 +317,7 @@ __global__ __launch_bounds__(kThreads) void split_prep_kernel(KArgs a) {
       f32x4v gs;
 #pragma unroll
       for (int e = 0; e < 4; ++e) gs[e] = gprod<D>(p, 4 * (lane % T::kLPR) + e) * p.sm_scale * kLog2e;
-      stage_norm<D, true>(p, x, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, tile, lane);
+      stage_norm<D, true, true>(p, x, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, tile, lane);
     } else {
       load_tile<D>(x, row_ptr<float>(p.d_o, b, h, 0), p.d_o.stride_s, q0, p.Sq, lane);
       f32x4v y[T::kPasses];
@@ -263,8 +343,10 @@ __global__ __launch_bounds__(kThreads) void split_prep_kernel(KArgs a) {
     }
     wave_sync();
     char* const dst = (kind == 0 ? m.q_rm : kind == 1 ? m.q_tr : kind == 2 ? m.d_rm : m.d_tr) + t * kTileBytes<D>;
-    if (kind & 1) emit_tr<D>(tile, dst, lane);
-    else emit_rm<D>(tile, dst, lane);
+    const bool small = tile_small<D>(x);
+    if (!(kind & 1) && lane == 0) (kind ? m.d_small : m.q_small)[t] = small;
+    if (kind & 1) emit_tr<D>(tile, dst, lane, small ? kPart : 1.f);
+    else emit_rm<D>(tile, dst, lane, small ? kPart : 1.f);
     return;
   }
   job -= q_jobs;
@@ -282,12 +364,14 @@ __global__ __launch_bounds__(kThreads) void split_prep_kernel(KArgs a) {
   } else {
     load_tile<D>(x, row_ptr<float>(p.k, b, g, 0), p.k.stride_s, j0, p.Sk, lane);
     const f32x4v one = {1.f, 1.f, 1.f, 1.f};
-    stage_norm<D, true>(p, x, one, p.rope_k_pos0 + j0, p.Sk - 1 - j0, tile, lane);
+    stage_norm<D, true, true>(p, x, one, p.rope_k_pos0 + j0, p.Sk - 1 - j0, tile, lane);
   }
   wave_sync();
   char* const dst = (values ? m.v : kind == 0 ? m.k_rm : m.k_tr) + t * kTileBytes<D>;
-  if (kind == 1) emit_tr<D>(tile, dst, lane);  // forward: values, backward: keys
-  else emit_rm<D>(tile, dst, lane);
+  const bool small = tile_small<D>(x);
+  if ((values || kind == 0) && lane == 0) (values ? m.v_small : m.k_small)[t] = small;
+  if (kind == 1) emit_tr<D>(tile, dst, lane, small ? kPart : 1.f);  // forward: values, backward: keys
+  else emit_rm<D>(tile, dst, lane, small ? kPart : 1.f);
 }
 
 // ---- forward, as fwd_f32_kernel
@@ -310,28 +394,32 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
   int kend = p.Sk;
   if (p.causal) kend = min(p.Sk, q0 + kRows + p.q_start);
   const int n_kt = tiles_of(kend);
-  const SplitMap m = split_map<D>(a);
-  const int64_t first = ((int64_t)b * p.Hkv + g) * tiles_of(p.Sk) * kTileBytes<D>;
+  const SplitMap m = split_map<D>(a, false);
+  const int64_t kv0 = ((int64_t)b * p.Hkv + g) * tiles_of(p.Sk), first = kv0 * kTileBytes<D>;
   const char *ktiles = m.k_rm + first, *vtiles = m.v + first;
+  const uint32_t *k_small = m.k_small + kv0, *v_small = m.v_small + kv0;
   // step i of a tile uses half i of its keys, then of its values; requested kAhead steps before
   constexpr int MB = T::kMB, kSteps = 2 * MB, kAhead = D == 64 ? 3 : MB == 1 ? 1 : 2;
   Half half[kSteps];
   auto source = [&](int jt, int i) {
     return (i < MB ? ktiles : vtiles) + (int64_t)jt * kTileBytes<D> + i % MB * kHalfBytes;
   };
+  const uint32_t flags = first_flags(k_small, n_kt, lane) | first_flags(v_small, n_kt, lane);
   if (wave < n_kt) {
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) half[i] = load_half(source(wave, i), lane);
   }
+  bool q_small;
   {
     f32x4v qraw[T::kPasses], gs;
     load_tile<D>(qraw, row_ptr<float>(p.q, b, h, 0), p.q.stride_s, q0, p.Sq, lane);
 #pragma unroll
     for (int e = 0; e < 4; ++e) gs[e] = gprod<D>(p, 4 * (lane % T::kLPR) + e) * p.sm_scale * kLog2e;
     float* const tile = reinterpret_cast<float*>(lds + kTileBytes<D>);  // every wave writes the same values
-    stage_norm<D, true>(p, qraw, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, tile, lane);
+    stage_norm<D, true, true>(p, qraw, gs, p.rope_q_pos0 + q0, p.Sq - 1 - q0, tile, lane);
     wave_sync();
-    emit_rm<D>(tile, qs, lane, wave, kWaves);
+    q_small = tile_small<D>(qraw);
+    emit_rm<D>(tile, qs, lane, q_small ? kPart : 1.f, wave, kWaves);
   }
   __syncthreads();
 
@@ -342,17 +430,8 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
   const int qlim = p.causal ? min(q0 + ln + p.q_start, p.Sk - 1) : p.Sk - 1;  // last visible key
   const int n_full = p.causal ? min(p.Sk, q0 + p.q_start + 1) / kRows : p.Sk / kRows;  // tiles that need no mask
 
-  for (int jt = wave; jt < n_kt; jt += kWaves) {
-    const int next = jt + kWaves < n_kt ? jt + kWaves : jt;  // past the end: this tile's once more, unused
-    auto request = [&](int i) { half[i % kSteps] = load_half(i < kSteps ? source(jt, i) : source(next, i - kSteps), lane); };
-    Dot dot;
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      request(i + kAhead);
-      dot.add(half[i], qs + i * kHalfBytes, lane);
-      step_end();
-    }
-    f32x16 s = dot.sum();
+  // S^T of a tile: mask, maximum, probabilities
+  auto softmax = [&](int jt, f32x16& s) {
     if (jt >= n_full) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
@@ -363,7 +442,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
     for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
     mx = fmaxf(mrow, half_max(mx));
     const float mu = mx == -INFINITY ? 0.f : mx;
-    if (__builtin_amdgcn_ballot_w64(mx > mrow) != 0) {  // some row has a new maximum
+    if (any_lane(mx > mrow)) {  // some row has a new maximum
       const float corr = __builtin_amdgcn_exp2f(mrow - mu);
       l *= corr;
 #pragma unroll
@@ -379,7 +458,23 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
       part[r & 1] += s[r];
     }
     l += part[0] + part[1];
-    const Scores3 probs = split_scores<true>(s);
+  };
+  const bool small = any_small(flags, k_small, n_kt, lane) | any_small(0, v_small, n_kt, lane) | q_small;
+  int jt = wave;
+#pragma unroll 1
+  for (; !small && jt < n_kt; jt += kWaves) {
+    const int next = jt + kWaves < n_kt ? jt + kWaves : jt;  // past the end: this tile's once more, unused
+    auto request = [&](int i) { half[i % kSteps] = load_half(i < kSteps ? source(jt, i) : source(next, i - kSteps), lane); };
+    Dot dot;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      request(i + kAhead);
+      dot.add(half[i], qs + i * kHalfBytes, lane);
+      step_end();
+    }
+    f32x16 s = dot.sum();
+    softmax(jt, s);
+    const Scores3 probs = split16<false>(s, 1.f);
 #pragma unroll
     for (int i = MB; i < kSteps; ++i) {
       step_end();
@@ -387,6 +482,20 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(KArgs a) {
       add_tr(half[i], probs, o[i - MB]);
     }
     step_end();
+  }
+#pragma unroll 1
+  for (; jt < n_kt; jt += kWaves) {  // some tile has small values
+    const bool ks = k_small[jt], vs = v_small[jt];
+    Dot dot;
+    dot.add_scaled<D>(source(jt, 0), ks, qs, q_small, lane);
+    f32x16 s = dot.sum();
+    softmax(jt, s);
+    const Scores3 probs = split16<false>(s, kPart);
+#pragma unroll
+    for (int i = MB; i < kSteps; ++i) {
+      step_end();
+      add_tr_scaled(load_half(source(jt, i), lane), vs, probs, o[i - MB]);
+    }
   }
 
   const float lt = half_sum(l);
@@ -428,8 +537,10 @@ __device__ __forceinline__ void bwd_dq_split(const KArgs& a, int block, char* ld
   int kend = p.Sk;
   if (p.causal) kend = min(p.Sk, q0 + kRows + p.q_start);
   const int n_kt = tiles_of(kend);
-  const SplitMap m = split_map<D>(a);
-  const int64_t first = ((int64_t)b * p.Hkv + g) * tiles_of(p.Sk) * kTileBytes<D>, mine = ((int64_t)b * p.H + h) * n_qt + qt;
+  const SplitMap m = split_map<D>(a, true);
+  const int64_t kv0 = ((int64_t)b * p.Hkv + g) * tiles_of(p.Sk), first = kv0 * kTileBytes<D>, mine = ((int64_t)b * p.H + h) * n_qt + qt;
+  const uint32_t *k_small = m.k_small + kv0, *v_small = m.v_small + kv0;
+  const bool q_small = m.q_small[mine], d_small = m.d_small[mine];
   const char *ktiles = m.k_rm + first, *vtiles = m.v + first, *kttiles = m.k_tr + first;
   // step i of a tile: half i of the keys (scores), of the values (dP), of the keys again (T)
   constexpr int MB = T::kMB, kSteps = 3 * MB, kAhead = MB == 1 ? 2 : 3;
@@ -437,6 +548,7 @@ __device__ __forceinline__ void bwd_dq_split(const KArgs& a, int block, char* ld
   auto source = [&](int jt, int i) {
     return (i < MB ? ktiles : i < 2 * MB ? vtiles : kttiles) + (int64_t)jt * kTileBytes<D> + i % MB * kHalfBytes;
   };
+  const uint32_t flags = first_flags(k_small, n_kt, lane) | first_flags(v_small, n_kt, lane);
   if (wave < n_kt) {
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) half[i] = load_half(source(wave, i), lane);
@@ -451,7 +563,22 @@ __device__ __forceinline__ void bwd_dq_split(const KArgs& a, int block, char* ld
   const int qlim = p.causal ? min(q0 + ln + p.q_start, p.Sk - 1) : p.Sk - 1;
   const int n_full = p.causal ? min(p.Sk, q0 + p.q_start + 1) / kRows : p.Sk / kRows;
 
-  for (int jt = wave; jt < n_kt; jt += kWaves) {
+  // dS^T of a tile
+  auto gradient = [&](int jt, f32x16& s, const f32x16& dp) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = prob(s[r], lse);
+    if (jt >= n_full) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (jt * kRows + crow(r, hh) > qlim) s[r] = 0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] *= dp[r] - delta;
+  };
+  const bool small = any_small(flags, k_small, n_kt, lane) | any_small(0, v_small, n_kt, lane) | q_small | d_small;
+  int jt = wave;
+#pragma unroll 1
+  for (; !small && jt < n_kt; jt += kWaves) {
     const int next = jt + kWaves < n_kt ? jt + kWaves : jt;
     auto request = [&](int i) { half[i % kSteps] = load_half(i < kSteps ? source(jt, i) : source(next, i - kSteps), lane); };
     Dot dot[2];
@@ -462,24 +589,30 @@ __device__ __forceinline__ void bwd_dq_split(const KArgs& a, int block, char* ld
       step_end();
     }
     f32x16 s = dot[0].sum();
-    const f32x16 dp = dot[1].sum();
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = prob(s[r], lse);
-    if (jt >= n_full) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (jt * kRows + crow(r, hh) > qlim) s[r] = 0.f;
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] *= dp[r] - delta;
-    const Scores3 grads = split_scores<false>(s);
+    gradient(jt, s, dot[1].sum());
+    const LaneScores grads = split_lanes<true>(s);
 #pragma unroll
     for (int i = 2 * MB; i < kSteps; ++i) {
       step_end();
       request(i + kAhead);
-      add_tr(half[i], grads, t[i - 2 * MB]);
+      add_tr(half[i], grads.s, t[i - 2 * MB], grads.f);
     }
     step_end();
+  }
+#pragma unroll 1
+  for (; jt < n_kt; jt += kWaves) {  // some tile has small values
+    const bool kf = k_small[jt], vf = v_small[jt];
+    Dot dot[2];
+    dot[0].add_scaled<D>(source(jt, 0), kf, qs, q_small, lane);
+    dot[1].add_scaled<D>(source(jt, MB), vf, ds, d_small, lane);
+    f32x16 s = dot[0].sum();
+    gradient(jt, s, dot[1].sum());
+    const Scores3 grads = split16<true>(s, kPart);
+#pragma unroll
+    for (int i = 2 * MB; i < kSteps; ++i) {
+      step_end();
+      add_tr_scaled(load_half(source(jt, i), lane), kf, grads, t[i - 2 * MB]);
+    }
   }
 
   __syncthreads();
@@ -505,14 +638,16 @@ __device__ __forceinline__ void bwd_dkdv_split(const KArgs& a, int block, char* 
   const int kt_i = item.tile, part_i = item.member, bg = item.pair;
   const int b = bg / p.Hkv, g = bg % p.Hkv, rep = p.H / p.Hkv;
   const int j0 = kt_i * kRows;
-  const SplitMap m = split_map<D>(a);
+  const SplitMap m = split_map<D>(a, true);
   const int n_qt = tiles_of(p.Sq);
   const int first = p.causal ? max(0, j0 - p.q_start) / kRows : 0;  // the first tile that holds a query seeing key j0
   const int step = kWaves * a.f32_parts;
+  const bool k_small = m.k_small[(int64_t)bg * tiles_of(p.Sk) + kt_i], v_small = m.v_small[(int64_t)bg * tiles_of(p.Sk) + kt_i];
   const int64_t mine = ((int64_t)bg * tiles_of(p.Sk) + kt_i) * kTileBytes<D>, head = (int64_t)(b * p.H + g * rep) * n_qt;
   const char *qrm = m.q_rm + head * kTileBytes<D>, *qtr = m.q_tr + head * kTileBytes<D>;
   const char *drm = m.d_rm + head * kTileBytes<D>, *dtr = m.d_tr + head * kTileBytes<D>;
   const float* stats = m.stat + head * 64;
+  const uint32_t *q_small = m.q_small + head, *d_small = m.d_small + head;
   int it = first + part_i * kWaves + wave, left = rep;  // tile within its head, query heads still to come with this one
   auto settle = [&](int& tile, int& heads) {  // tiles past a head's last one are the next head's first visible ones
     while (tile >= n_qt && heads > 0) { tile -= n_qt - first; --heads; }
@@ -526,6 +661,7 @@ __device__ __forceinline__ void bwd_dkdv_split(const KArgs& a, int block, char* 
     return (i < MB ? qrm : i < 2 * MB ? drm : i < 3 * MB ? dtr : qtr) + (int64_t)tile * kTileBytes<D> + i % MB * kHalfBytes;
   };
   float st = 0.f;
+  const uint32_t flags = first_flags(q_small, rep * n_qt, lane) | first_flags(d_small, rep * n_qt, lane);
   int at = (rep - left) * n_qt + it;  // tile within the group
   if (left > 0) {
 #pragma unroll
@@ -539,25 +675,8 @@ __device__ __forceinline__ void bwd_dkdv_split(const KArgs& a, int block, char* 
 #pragma unroll
   for (int mb = 0; mb < T::kMB; ++mb) dk[mb] = dv[mb] = zero16();
 
-  while (left > 0) {
-    const int i0 = it * kRows;
-    int next_left = left;
-    it += step;
-    settle(it, next_left);
-    const int next = next_left > 0 ? (rep - next_left) * n_qt + it : at;
-    auto request = [&](int i) { half[i % kSteps] = load_half(i < kSteps ? source(at, i) : source(next, i - kSteps), lane); };
-    stat[wave][lane] = st;
-    st = stats[(int64_t)next * 64 + lane];
-    wave_sync();
-    Dot dot[2];
-#pragma unroll
-    for (int i = 0; i < 2 * MB; ++i) {
-      request(i + kAhead);
-      dot[i / MB].add(half[i], (i < MB ? ks : vs) + i % MB * kHalfBytes, lane);
-      step_end();
-    }
-    f32x16 s = dot[0].sum();
-    const f32x16 dp = dot[1].sum();
+  // S and dP of a tile to P and dS
+  auto probabilities = [&](int i0, f32x16& s) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const f32x4v ls = *reinterpret_cast<const f32x4v*>(&stat[wave][8 * q + 4 * hh]);
@@ -571,25 +690,78 @@ __device__ __forceinline__ void bwd_dkdv_split(const KArgs& a, int block, char* 
         if (i >= p.Sq || (p.causal && j0 + ln > i + p.q_start)) s[r] = 0.f;
       }
     }
-    const Scores3 probs = split_scores<true>(s);
+  };
+  auto gradients = [&](f32x16& s, const f32x16& dp) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const f32x4v de = *reinterpret_cast<const f32x4v*>(&stat[wave][32 + 8 * q + 4 * hh]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) s[4 * q + e] *= dp[4 * q + e] - de[e];
     }
-    const Scores3 grads = split_scores<false>(s);
+  };
+  const bool small = any_small(flags, q_small, rep * n_qt, lane) | any_small(0, d_small, rep * n_qt, lane) | k_small | v_small;
+#pragma unroll 1
+  while (left > 0 && !small) {
+    int next_it = it + step, next_left = left;
+    settle(next_it, next_left);
+    const int next = next_left > 0 ? (rep - next_left) * n_qt + next_it : at;
+    auto request = [&](int i) { half[i % kSteps] = load_half(i < kSteps ? source(at, i) : source(next, i - kSteps), lane); };
+    stat[wave][lane] = st;
+    st = stats[(int64_t)next * 64 + lane];
+    wave_sync();
+    Dot dot[2];
+#pragma unroll
+    for (int i = 0; i < 2 * MB; ++i) {
+      request(i + kAhead);
+      dot[i / MB].add(half[i], (i < MB ? ks : vs) + i % MB * kHalfBytes, lane);
+      step_end();
+    }
+    f32x16 s = dot[0].sum();
+    const f32x16 dp = dot[1].sum();
+    probabilities(it * kRows, s);
+    const LaneScores probs = split_lanes<false>(s);
+    gradients(s, dp);
+    const LaneScores grads = split_lanes<true>(s);
 #pragma unroll
     for (int i = 2 * MB; i < kSteps; ++i) {
       step_end();
       request(i + kAhead);
-      if (i < 3 * MB) add_tr(half[i], probs, dv[i - 2 * MB]);
-      else add_tr(half[i], grads, dk[i - 3 * MB]);
+      if (i < 3 * MB) add_tr(half[i], probs.s, dv[i - 2 * MB], probs.f);
+      else add_tr(half[i], grads.s, dk[i - 3 * MB], grads.f);
     }
     step_end();
     wave_sync();
-    at = next;
+    it = next_it;
     left = next_left;
+    at = next;
+  }
+#pragma unroll 1
+  while (left > 0) {  // some tile has small values
+    const bool qf = q_small[at], df = d_small[at];
+    wave_sync();
+    stat[wave][lane] = stats[(int64_t)at * 64 + lane];
+    wave_sync();
+    Dot dot[2];
+    dot[0].add_scaled<D>(source(at, 0), qf, ks, k_small, lane);
+    dot[1].add_scaled<D>(source(at, MB), df, vs, v_small, lane);
+    f32x16 s = dot[0].sum();
+    probabilities(it * kRows, s);
+    const Scores3 probs = split16<false>(s, kPart);
+#pragma unroll
+    for (int i = 2 * MB; i < 3 * MB; ++i) {
+      step_end();
+      add_tr_scaled(load_half(source(at, i), lane), df, probs, dv[i - 2 * MB]);
+    }
+    gradients(s, dot[1].sum());
+    const Scores3 grads = split16<true>(s, kPart);
+#pragma unroll
+    for (int i = 3 * MB; i < kSteps; ++i) {
+      step_end();
+      add_tr_scaled(load_half(source(at, i), lane), qf, grads, dk[i - 3 * MB]);
+    }
+    it += step;
+    settle(it, left);
+    at = (rep - left) * n_qt + it;
   }
 
   const int part = tid % T::kLPR;
@@ -709,7 +881,7 @@ bool f32_split_pays(const segpt_attn_params& p, bool bwd) {
 size_t f32_split_bytes(const segpt_attn_params& p, bool bwd) {
   if (!f32_split_pays(p, bwd)) return 0;
   const size_t tile = (size_t)p.D * (kUnitBytes / 16), kv = (size_t)p.B * p.Hkv * n_tiles(p.Sk), q = (size_t)p.B * p.H * n_tiles(p.Sq);
-  return bwd ? (3 * kv + 4 * q) * tile + q * 64 * sizeof(float) : 2 * kv * tile;
+  return (bwd ? (3 * kv + 4 * q) * tile + q * (64 * sizeof(float) + 2 * sizeof(uint32_t)) : 2 * kv * tile) + kv * 2 * sizeof(uint32_t);
 }
 
 int launch_split_prep(const KArgs& a, bool bwd, hipStream_t st) {

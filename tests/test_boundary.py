@@ -313,12 +313,13 @@ def test_fp32_split_scratch(lib):
             setattr(p, name, _lib.Tensor4(0x10000, 2 * Sk * D, Sk * D, D))
         return p
 
+    up = lambda n: -(-n // 256) * 256
     size = lambda p: [lib.segpt_attn_workspace_bytes(p, w) for w in (_lib.SEGPT_WS_F32_FWD, _lib.SEGPT_WS_F32_BWD)]
     for D in (32, 64, 128):
         few = size(params(1, 8192, D))
         assert few[0] == 0 and (few[1] > 0) == (D == 128)  # the backward is the faster one at head_dim 128, whatever the queries
-        kv, q = 2 * 2 * 32 * 32 * D, 2 * 6 * 32 * 32 * D  # elements of K and of Q in whole tiles
-        assert size(params(1000, 1000, D)) == [2 * kv * 6, 3 * kv * 6 + 4 * q * 6 + 2 * 6 * 32 * 64 * 4]
+        kv, q = 2 * 2 * 32, 2 * 6 * 32  # tiles of 32 rows of K and of Q: three bf16 numbers an element, two flags; lse and delta of the queries
+        assert size(params(1000, 1000, D)) == [up(kv * (2 * 32 * D * 6 + 8)), up(kv * (3 * 32 * D * 6 + 8) + q * (4 * 32 * D * 6 + 8 + 64 * 4))]
     assert size(params(128, 128)) == [0, 0]
     # head_dim 128: few users of a short key tile are not worth the forward's pre-pass in launches of 65 to 511 workgroups
     heads = lambda n, S, D: (lambda p: (setattr(p, "H", n), setattr(p, "Hkv", n), setattr(p, "B", 1), size(p))[-1])(params(S, S, D))

@@ -233,6 +233,52 @@ def test_fp32_split_values_beyond_bf16s_range(gpu_device, D):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_split_small_values(gpu_device, D):
+    """The calls are linear in v (y) and in dO (dq, dk, dv): scaled by 2^-112 (1e-34) they give the same numbers times 2^-112, within the 16
+    units of two results that are 8 from float64 each; products that end among the subnormal numbers lose up to 2^-150, 2^-38 of a result of
+    ordinary size, 0.05 units for 800 of them.  With some rows scaled and others not, in one tile and in a tile of their own, every row
+    of y and dq scales with its own operand (the values of its keys, its dO) alone."""
+    x = gen(1, 8, 4, 800, 800, D, F32, seed=68, scalar_gain=True, no_gk=True)
+    f = 2.0**-112
+    (y, dq, dk, dv), _ = _fp32_both_ways(x, gpu_device)
+    print(f"small values, D={D}", flush=True)
+    small_y = _fp32_both_ways(dict(x, v=x["v"] * f), gpu_device)[0][0]
+    small = _fp32_both_ways(dict(x, d_o=x["d_o"] * f), gpu_device)[0][1:]
+    for a, b in zip((small_y, *small), (y, dq, dk, dv)):
+        _within(a.double() / f, b.double(), 16)
+    scale = torch.ones(800, 1)
+    scale[100:101] = scale[320:352] = scale[700:750] = f
+    got = _fp32_both_ways(dict(x, d_o=x["d_o"] * scale), gpu_device)[0]
+    _within(got[1].double() / scale.double(), dq.double(), 16)
+    scale = torch.where(torch.arange(800).unsqueeze(1) < 40, f, 1.0)  # queries 0 .. 39 see small values alone
+    got, old = _fp32_both_ways(dict(x, v=x["v"] * scale), gpu_device)
+    _within(got[0][:, :, :40].double() / f, y[:, :, :40].double(), 16)
+    for a, b in zip(got, old):
+        _within(a, b, 16)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_split_small_probabilities(gpu_device, D):
+    """Keys that every query ignores: with logits 78 below the others' (112.5 in base 2) their probabilities are 2^-114 to 2^-122, and their
+    rows of dv and dk have the accuracy that the logits allow: five roundings of them (the scale vector's three, Qhat's, the sum's) are
+    5 * 112.5 * ln 2 * 2^-24 = 2.3e-5 of a probability.  Unscaled, the parts of the smallest ones are off by 2^-12."""
+    x = gen(1, 8, 4, 800, 800, D, F32, seed=69, scalar_gain=True, no_gk=True)
+    x["q"] *= 0.05
+    x["q"][..., 0] = 1.0
+    x["k"][..., 0] = 0.0
+    ignored = torch.arange(0, 800, 3)[1:]
+    x["k"][:, :, ignored, 0] = -78.0 * D**0.5 / 1.3
+    print(f"small probabilities, D={D}", flush=True)
+    got, ref = run_gpu(x, gpu_device, qk_norm=False), run_oracle(x, qk_norm=False)
+    late = ignored[(ignored > 400) & (ignored < 700)]
+    assert 2.0**-126 < ref["dv"][:, :, late].abs().max() < 2.0**-110
+    for n in ("dk", "dv"):
+        for rows in (late, late + 1):
+            a, b = got[n][:, :, rows, 1:].double(), ref[n][:, :, rows, 1:]  # column 0 of dk is the sum of dS, which all but cancels
+            assert (a - b).norm() <= 5 * 112.5 * math.log(2) * 2.0**-24 * b.norm(), n
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_rows_whose_mean_square_leaves_the_normal_range(gpu_device, D):
     """A key whose sum of squares overflows has the normaliser 0, like a key of zeros, and poisons nobody; keys so small
     that their mean square is subnormal (eps = 0) are normalised like any others."""
