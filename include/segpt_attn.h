@@ -93,7 +93,8 @@ extern "C" {
 
 /* which scratch buffer segpt_attn_workspace_bytes() sizes */
 #define SEGPT_WS_KV 0  /* kv_workspace: bf16 copies of the normalised keys (and mixed values); forward AND backward */
-#define SEGPT_WS_BWD 1 /* workspace: per-row statistics, normalised queries, partial sums; backward only            */
+#define SEGPT_WS_BWD 1 /* workspace: per-row statistics, normalised queries, partial sums; backward only.  Follows flags:
+                          with SEGPT_FLAG_F32_SPLIT an fp32 call needs less of it                                   */
 #define SEGPT_WS_F32_FWD 2 /* fp32 with SEGPT_FLAG_F32_SPLIT: kv_workspace of the forward ... */
 #define SEGPT_WS_F32_BWD 3 /* ... and of the backward, which does not need the forward's; 0 where the call runs without */
 

@@ -64,20 +64,28 @@ KvLayout kv_layout(const segpt_attn_params& p) {
   return w;
 }
 
-// The backward keeps a gate-scaled copy of dO on the fp32 path and, on the bf16 path, only for a gate scale that is
+// fp32: scratch of the kernels that take every operand as three bf16 numbers, 0 where they are not the faster ones
+size_t f32_split_scratch(const segpt_attn_params& p, bool bwd) {
+  if (p.dtype != SEGPT_DTYPE_FP32 || (p.D != 32 && p.D != 64 && p.D != 128)) return 0;
+  return align_up(f32_split_bytes(p, bwd));
+}
+bool f32_split_runs(const segpt_attn_params& p, bool bwd) { return (p.flags & SEGPT_FLAG_F32_SPLIT) && f32_split_scratch(p, bwd); }
+
+// The backward keeps a gate-scaled copy of dO with the fp32 instructions and, on the bf16 path, only for a gate scale that is
 // not positive: a positive gate factor travels to the dK/dV kernel inside the two row statistics instead.
 bool gated_do_copy(const segpt_attn_params& p) {
-  return p.gate.ptr && (p.dtype == SEGPT_DTYPE_FP32 || !(p.gate_scale > 0.f));
+  return p.gate.ptr && (p.dtype == SEGPT_DTYPE_FP32 ? !f32_split_runs(p, true) : !(p.gate_scale > 0.f));
 }
 
-// fp32: dK and dV of a key tile come in one part per query head of the group and share of the query tiles, [B * H, splits, Sk, D].
-// A single part per kv head fits into contiguous dk and dv themselves: the finish kernel reads a piece before it writes it.
+// fp32: dK and dV of a key tile come in parts, [B * Hkv, parts, Sk, D]: one per query head of the group and share of the query tiles, or
+// as many as f32_split_parts.  A single part fits into contiguous dk and dv themselves: the finish kernel reads a piece before it writes it.
+int f32_parts(const segpt_attn_params& p) { return f32_split_runs(p, true) ? f32_split_parts(p) : p.H / p.Hkv * f32_dkdv_splits(p); }
 bool f32_part_in_place(const segpt_attn_params& p) {
   auto packed = [&](const segpt_tensor4& t) {
     const int64_t head = (int64_t)p.Sk * p.D;
     return t.ptr && t.stride_s == p.D && (t.stride_h == head || p.Hkv == 1) && (t.stride_b == p.Hkv * head || p.B == 1);
   };
-  return p.H == p.Hkv && f32_dkdv_splits(p) == 1 && packed(p.dk) && packed(p.dv);
+  return f32_parts(p) == 1 && packed(p.dk) && packed(p.dv);
 }
 
 WsLayout bwd_layout(const segpt_attn_params& p) {
@@ -85,7 +93,7 @@ WsLayout bwd_layout(const segpt_attn_params& p) {
   size_t off = 0;
   const size_t rows = (size_t)p.B * p.H * p.Sq;
   w.delta = off;
-  off += align_up(rows * sizeof(float));
+  if (!f32_split_runs(p, true)) off += align_up(rows * sizeof(float));
   w.nlse2 = off;
   if (p.dtype == SEGPT_DTYPE_BF16) off += align_up(rows * sizeof(float));
   w.do_eff = off;
@@ -98,7 +106,7 @@ WsLayout bwd_layout(const segpt_attn_params& p) {
   off += align_up((size_t)dkdv_blocks(p) * 2 * sizeof(float));
   w.f32_dk_part = w.f32_dv_part = off;
   if (p.dtype == SEGPT_DTYPE_FP32 && !f32_part_in_place(p)) {
-    const size_t part = align_up((size_t)p.B * p.H * f32_dkdv_splits(p) * p.Sk * p.D * sizeof(float));
+    const size_t part = align_up((size_t)p.B * p.Hkv * f32_parts(p) * p.Sk * p.D * sizeof(float));
     w.f32_dv_part = off + part;
     off += 2 * part;
   }
@@ -176,15 +184,10 @@ int check_common(const segpt_attn_params* p) {
   return SEGPT_OK;
 }
 
-// fp32: scratch of the kernels that take every operand as three bf16 numbers, 0 where they are not the faster ones
-size_t f32_split_scratch(const segpt_attn_params& p, bool bwd) {
-  if (p.dtype != SEGPT_DTYPE_FP32 || (p.D != 32 && p.D != 64 && p.D != 128)) return 0;
-  return align_up(f32_split_bytes(p, bwd));
-}
 int bind_split(KArgs& a, bool bwd) {
   const segpt_attn_params& p = a.p;
-  const size_t need = (p.flags & SEGPT_FLAG_F32_SPLIT) ? f32_split_scratch(p, bwd) : 0;
-  if (!need) return SEGPT_OK;
+  if (!f32_split_runs(p, bwd)) return SEGPT_OK;
+  const size_t need = f32_split_scratch(p, bwd);
   if (!p.kv_workspace || p.kv_workspace_bytes < need) return SEGPT_E_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(p.kv_workspace) & 255u) return SEGPT_E_ALIGN;
   a.f32_split = reinterpret_cast<char*>(p.kv_workspace);
@@ -434,7 +437,7 @@ static int bwd_stage_impl(const segpt_attn_params* p_in, int stage_lo, int stage
   }
   bind_kv(a);
   if ((rc = bind_split(a, true))) return rc;
-  if (p->dtype == SEGPT_DTYPE_FP32) a.f32_parts = a.f32_split ? f32_split_parts(*p) : p->H / p->Hkv * a.f32_splits;
+  if (p->dtype == SEGPT_DTYPE_FP32) a.f32_parts = f32_parts(*p);
   a.f32_both = a.f32_split && stage_lo <= SEGPT_BWD_STAGE_DQ && stage_hi >= SEGPT_BWD_STAGE_DKDV && f32_split_both(a);
   a.n_dq_blocks = dq_blocks(*p);
   a.n_dkdv_blocks = dkdv_blocks(*p);

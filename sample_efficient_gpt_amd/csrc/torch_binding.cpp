@@ -144,14 +144,25 @@ Tensor scratch(const segpt_attn_params& p, int which, const at::Device& dev) {
   const size_t n = segpt_attn_workspace_bytes(&p, which);
   return at::empty({(int64_t)(n < 256 ? 256 : n)}, at::TensorOptions().dtype(at::kByte).device(dev));
 }
-// fp32: scratch of the kernels that run on the bf16 matrix pipe, where those are the faster ones; held until the launch
-Tensor f32_scratch(segpt_attn_params& p, int which, const at::Device& dev) {
-  if (p.dtype != SEGPT_DTYPE_FP32 || segpt_attn_workspace_bytes(&p, which) == 0) return Tensor();
-  const Tensor t = scratch(p, which, dev);
-  p.flags |= SEGPT_FLAG_F32_SPLIT;
-  p.kv_workspace = t.data_ptr();
-  p.kv_workspace_bytes = (size_t)t.numel();
-  return t;
+// fp32: scratch of the kernels that run on the bf16 matrix pipe, where those are the faster ones; held until the launch.  It is several
+// times the operands: `rest` allocates what else the launch needs, and where the two do not fit, the call runs without.
+template <typename F>
+Tensor f32_scratch(segpt_attn_params& p, int which, const at::Device& dev, F rest) {
+  if (p.dtype == SEGPT_DTYPE_FP32 && segpt_attn_workspace_bytes(&p, which) != 0) {
+    const segpt_attn_params without = p;
+    try {
+      const Tensor t = scratch(p, which, dev);
+      p.flags |= SEGPT_FLAG_F32_SPLIT;
+      p.kv_workspace = t.data_ptr();
+      p.kv_workspace_bytes = (size_t)t.numel();
+      rest();
+      return t;
+    } catch (const c10::OutOfMemoryError&) {
+      p = without;
+    }
+  }
+  rest();
+  return Tensor();
 }
 void* current_stream(const at::Device& dev) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream(); }
 
@@ -184,7 +195,7 @@ Forward run_forward(const Operands& x, const Call& c, const Tensor& y) {
   r.kv_ws = scratch(p, SEGPT_WS_KV, dev);
   p.kv_workspace = r.kv_ws.data_ptr();
   p.kv_workspace_bytes = (size_t)r.kv_ws.numel();
-  const Tensor f32_ws = f32_scratch(p, SEGPT_WS_F32_FWD, dev);
+  const Tensor f32_ws = f32_scratch(p, SEGPT_WS_F32_FWD, dev, [] {});
   const c10::DeviceGuard guard(dev);  // the launch goes to the tensors' device, whatever the current one is
   const int rc = segpt_attn_fwd(&p, current_stream(dev));
   if (rc) throw LibraryError(rc, "segpt_attn_fwd");
@@ -218,10 +229,12 @@ Grads run_backward(const Operands& raw, const Call& c, const Tensor& y, const Te
     p.dq = view4(g.q, c.heads); p.dk = view4(g.k, c.kv_heads); p.dv = view4(g.v, c.kv_heads); p.dv_first = view4(g.v_first, c.kv_heads);
     p.dgate = view3(g.gate);
     p.dg_q = ptr_of<float>(g.g_q); p.dg_k = ptr_of<float>(g.g_k); p.dvr_coef = ptr_of<float>(g.coef);
-    const Tensor ws = scratch(p, SEGPT_WS_BWD, dev);
-    p.workspace = ws.data_ptr(); p.workspace_bytes = (size_t)ws.numel();
     p.kv_workspace = kv_ws.data_ptr(); p.kv_workspace_bytes = (size_t)kv_ws.numel();
-    const Tensor f32_ws = f32_scratch(p, SEGPT_WS_F32_BWD, dev);
+    Tensor ws;
+    const Tensor f32_ws = f32_scratch(p, SEGPT_WS_F32_BWD, dev, [&] {
+      ws = scratch(p, SEGPT_WS_BWD, dev);
+      p.workspace = ws.data_ptr(); p.workspace_bytes = (size_t)ws.numel();
+    });
     const c10::DeviceGuard guard(dev);
     const int rc = segpt_attn_bwd(&p, current_stream(dev));
     if (rc) throw LibraryError(rc, "segpt_attn_bwd");

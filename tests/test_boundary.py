@@ -329,6 +329,13 @@ def test_fp32_split_scratch(lib):
     assert heads(128, 256, 32)[0] == 0 and heads(128, 448, 32)[0] > 0 and heads(320, 256, 32)[0] > 0
     p = _valid_params(); p.Sq = p.Sk = 1000
     assert size(p) == [0, 0]
+    # the other workspace follows the flag: no delta, no copy of a gated dO, parts of dK and dV per kv head and not per query head
+    ws = lambda p: lib.segpt_attn_workspace_bytes(p, _lib.SEGPT_WS_BWD)
+    p, rows, kv_rows = params(1000, 1000), 2 * 6 * 1000, 2 * 2 * 1000
+    p.gate = _lib.Tensor3(0x10000, 6000, 6, 1)
+    with_flag = ws(p)
+    p.flags = 0
+    assert with_flag < 2 * 4 * kv_rows * 64 * 4 + (1 << 20) and ws(p) > with_flag + rows * 65 * 4
     for call, i in ((lib.segpt_attn_fwd, 0), (lib.segpt_attn_bwd, 1)):
         p = params(1000, 1000); p.kv_workspace, p.kv_workspace_bytes = None, 0
         assert call(p, None) == -7

@@ -178,6 +178,35 @@ def test_fp32_split_is_no_less_accurate(gpu_device, D):
     assert all(e <= bound for e, bound in zip(err, (3.31, 6.36, 7.60, 6.09)))
 
 
+def test_fp32_without_room_for_the_split_operands(gpu_device):
+    """Where the scratch of the three-bf16 kernels does not fit, a step that fits without it runs with the fp32 instructions instead of out of
+    memory; against a plan that never asks for the scratch, at 1e-5."""
+    from sample_efficient_gpt_amd import _lib
+    from sample_efficient_gpt_amd.plan import AttnPlan
+
+    x = {n: None if t is None else t.to(gpu_device) for n, t in gen(4, 8, 2, 2048, 2048, 64, F32, seed=66).items()}
+    plan = AttnPlan(x)
+    plan.forward()
+    plan.backward()
+    want = [t.clone() for t in (plan.y, plan.dq, plan.dk, plan.dv)]
+    need = plan.lib.segpt_attn_workspace_bytes(plan.p, _lib.SEGPT_WS_F32_BWD)
+    step = 2 * x["q"].nbytes + 2 * x["k"].nbytes + plan.ws.numel()  # y, dq, dk, dv, workspace
+    assert need > 100 << 20 and step < 90 << 20
+    del plan
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(gpu_device).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(gpu_device) + step + (24 << 20)) / total, gpu_device)
+        leaves = [x[n].requires_grad_(True) for n in ("q", "k", "v")]
+        y = qknorm_attention(*leaves, x["g_q"], x["g_k"])
+        got = [y.detach(), *torch.autograd.grad(y, leaves, x["d_o"])]
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, gpu_device)
+    for a, b in zip(got, want):
+        assert torch.allclose(a, b, atol=1e-5, rtol=1e-5)
+
+
 def _fp32_both_ways(x, device):
     """y, dq, dk, dv with the three-bf16 kernels (the call as users make it) and with the fp32 instructions (without the flag)."""
     from sample_efficient_gpt_amd import _lib
