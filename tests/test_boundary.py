@@ -223,6 +223,29 @@ def test_module_interface():
     assert list(sig.parameters) == ["Q", "K", "V", "is_causal", "q_start"]
 
 
+def test_generation_step_leaves_replaced_layers_alone(monkeypatch):
+    """The native step multiplies by the weights itself, so a layer whose call is anything else has none to give."""
+    import torch.nn as nn
+    import torch.nn.functional as F
+
+    from sample_efficient_gpt_amd import module as M
+
+    plain = lambda: M._Linear(8, 8)
+    layer = plain()
+    assert M._weight_of(layer) is layer.linear.weight and not M._linear_replaced()
+    for where, other in ((nn.Linear, lambda self, x: 2 * x), (nn.Linear, print), (M._Linear, lambda self, x: 2 * x), (F, lambda x, w, b=None: 2 * x)):
+        with monkeypatch.context() as m:
+            m.setattr(where, "linear" if where is F else "forward", other)
+            assert M._linear_replaced(), where
+    assert not M._linear_replaced()
+    for spoil in (lambda l: l.register_forward_hook(print), lambda l: l.linear.register_forward_pre_hook(print), lambda l: setattr(l, "forward", print),
+                  lambda l: setattr(l.linear, "forward", print), lambda l: setattr(l.linear, "bias", nn.Parameter(l.linear.weight[0].detach())),
+                  lambda l: nn.utils.parametrizations.weight_norm(l.linear)):
+        layer = plain()
+        spoil(layer)
+        assert M._weight_of(layer) is None
+
+
 def test_linear_rows_rejects_bad_arguments_before_any_launch(lib):
     """segpt_linear_rows returns its error codes without a device."""
     def call(M=2, K=64, x=256, xs=64, n_segments=1, w=512, ws=64, out=1024, n=5, width=5, sm=5, sh=0, struct_bytes=None):
