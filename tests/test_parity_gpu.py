@@ -1802,7 +1802,7 @@ def test_mhsa_module_generation_step_is_the_separate_calls(gpu_device, b, H, Hkv
     S0, d_model = 70, H * d
     m, _, _ = _module_and_oracle_weights(gpu_device, BF16, d_model, H, Hkv, qknorm, False, gating, seed=31)
     x = torch.randn(b, S0 + 2, d_model, generator=torch.Generator().manual_seed(32)).to(BF16).to(gpu_device)
-    seen = []
+    seen, native = [], _record_generation_steps(m)
 
     def run(hooked):
         cache = KVCache(capacity=S0 + 2)
@@ -1821,8 +1821,15 @@ def test_mhsa_module_generation_step_is_the_separate_calls(gpu_device, b, H, Hkv
         return torch.cat([o for o, _ in outs], 1), cache
 
     print(f"generation step b={b} H={H} d={d}", flush=True)
-    (y, cache), (want, want_cache) = run(False), run(True)
-    assert len(seen) == 2
+    y, cache = run(False)
+    assert native == [True, True] and not seen  # both tokens were native steps
+    want, want_cache = run(True)
+    assert len(seen) == 2 and native == [True, True, False, False]
+    with torch.no_grad(), pytest.MonkeyPatch.context() as patch:  # a layer that is replaced for all is called too
+        patch.setattr(torch.nn.Linear, "forward", lambda self, t: torch.zeros(*t.shape[:-1], self.out_features, dtype=t.dtype, device=t.device))
+        other = KVCache(capacity=2)
+        other.append(cache.keys[:, :, :1].contiguous(), cache.values[:, :, :1].contiguous())
+        assert not m(x[:, :1], kv_cache=other)[0].any() and not other.keys[:, :, 1].any()
     for a, r in ((cache.keys, want_cache.keys), (cache.values, want_cache.values)):
         assert torch.allclose(a.float(), r.float(), rtol=2.0**-7, atol=1e-5)  # neighbouring bf16 values
     assert torch.allclose(y.float(), want.float(), atol=2e-2, rtol=1e-2)
@@ -1831,6 +1838,10 @@ def test_mhsa_module_generation_step_is_the_separate_calls(gpu_device, b, H, Hkv
                                m.rope.cos, m.rope.sin, cache._kbuf, cache._vbuf, length, H, Hkv, 4)
     token = x[:, :1].clone()
     with torch.no_grad():
+        # accepted as it stands; what follows differs from it in one argument each
+        row = cache._kbuf[:, :, 0].clone(), cache._vbuf[:, :, 0].clone()
+        assert real(*args(token, 0)) is not None
+        cache._kbuf[:, :, 0], cache._vbuf[:, :, 0] = row
         before = cache._kbuf.clone()
         assert real(*args(token, cache._kbuf.shape[2])) is None                       # the buffers are full
         assert real(*args(x[:, :2], 0)) is None and real(*args(token.float(), 0)) is None
@@ -1838,6 +1849,19 @@ def test_mhsa_module_generation_step_is_the_separate_calls(gpu_device, b, H, Hkv
             assert real(*args(token, 0)) is None
         assert torch.equal(cache._kbuf.view(torch.int16), before.view(torch.int16))
     assert real(*args(token.requires_grad_(), 0)) is None
+
+
+def _record_generation_steps(m):
+    """Whether each cached token that `m` is given takes the native step."""
+    steps, real = [], m._generation_step
+
+    def record(*args):
+        step = real(*args)
+        steps.append(step is not None)
+        return step
+
+    m._generation_step = record
+    return steps
 
 
 def _native_module():
@@ -1850,7 +1874,7 @@ def test_generation_step_in_a_graph(gpu_device):
     H, Hkv, d, S0 = 6, 2, 64, 200
     m, _, _ = _module_and_oracle_weights(gpu_device, BF16, H * d, H, Hkv, True, False, "per-head", seed=41)
     x = torch.randn(2, S0 + 1, H * d, generator=torch.Generator().manual_seed(42)).to(BF16).to(gpu_device)
-    cache, token = KVCache(capacity=S0 + 1), x[:, S0:].clone()
+    cache, token, native = KVCache(capacity=S0 + 1), x[:, S0:].clone(), _record_generation_steps(m)
 
     def step():
         cache.length = S0
@@ -1863,6 +1887,7 @@ def test_generation_step_in_a_graph(gpu_device):
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             y = step()
+        assert native == [True, True]
         for i in range(4):
             token.copy_(torch.randn(token.shape, generator=torch.Generator().manual_seed(i)).to(BF16))
             eager = step().clone()
