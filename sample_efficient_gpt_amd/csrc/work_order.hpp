@@ -8,18 +8,26 @@ namespace segpt {
 
 // Work items are listed heaviest first.  When the whole grid is resident at once (up to two workgroups on each of 256
 // CUs) or nearly so, the CU that got item i also gets item i + 256: every second round of 256 is dealt in reverse, so
-// that a heavy item shares its CU with a light one (512 items: forward 37.8 -> 31.8 us, dQ 51 -> 43).  Larger grids
+// that a heavy item shares its CU with a light one (2 x 8 / 4 heads of 1000 tokens, us: forward 39.7 -> 33.8, backward 121 -> 109).  Larger grids
 // balance by themselves and keep the plain order (dK/dV 3 % slower reversed at 9216 items).
 __attribute__((always_inline)) constexpr int work_item(int id, int n) {
   const int round = id >> 8;
   if (n > 1024 || !(round & 1)) return id;
+  return (round << 8) + 255 < n ? (round << 8) + 255 - (id & 255) : n - 1 - (id & 255);
+}
+// The same with whole rounds reversed in eights, which keeps an item's XCD: where the items of an XCD share what they stream (split_item).  Three-bf16
+// kernels, us, work_item -> this: 2 x 8 / 4 heads of 1000 tokens forward 27.8 -> 26.4, 18 / 6 heads of 512 backward 51.5 -> 47.9.  The fp32 instructions'
+// kernels do not gain: backward 109 -> 113.
+__attribute__((always_inline)) constexpr int work_item_xcd(int id, int n) {
+  const int round = id >> 8;
+  if (n > 1024 || !(round & 1)) return id;
   const int x = id & 255;
-  return (round << 8) + 256 <= n ? (round << 8) + 248 - (x & 248) + (x & 7) : n - 1 - x;
+  return (round << 8) + 255 < n ? (round << 8) + 248 - (x & 248) + (x & 7) : n - 1 - x;
 }
 
 // Which tile a workgroup takes: (tile, heaviest first; (batch, kv head); member of the pair: query head or part).  The streamed
 // tiles of the pairs that an XCD works on at a time should stay in its L2 (2.4 MB a pair at 2048 keys of 64).
-//   * Up to 512 workgroups, resident at once: in work_item's order; from 256 on with the pairs before the members, so that an XCD
+//   * Up to 512 workgroups, resident at once: in work_item_xcd's order; from 256 on with the pairs before the members, so that an XCD
 //     sees every eighth pair with all its members (us, members before pairs -> this: forward of 8 x 32 / 4 heads, one query, 4096 keys of 64 148 ->
 //     75, fp32 instructions 107; fewer workgroups do not fill the memory side and are 5 % faster spread: 16 / 4 heads, 64 queries, 2048 keys 33.9, 35.2).
 //     Up to 1024 the same if what an XCD then streams is no more than a few times its L2: it balances the causal tail (4 x 8 heads of 1000
@@ -38,7 +46,7 @@ __attribute__((always_inline)) constexpr Item split_item(int block, int tiles, i
   const int per = tiles * members;
   const int64_t total = (int64_t)per * pairs;
   if (total <= kResident || (total <= kPinnedGrid && stream * (pairs % kXcds ? pairs : pairs / kXcds) <= kStreamLimit)) {
-    const int n = per * pairs, id = work_item(block, n), rest = id % (pairs * members);
+    const int n = per * pairs, id = work_item_xcd(block, n), rest = id % (pairs * members);
     it.tile = id / (pairs * members);
     it.pair = n < 256 ? rest / members : rest % pairs;
     it.member = n < 256 ? rest % members : rest / pairs;

@@ -40,6 +40,17 @@ const char* check(F order, int tiles, int pairs, int members, int64_t stream, in
 
 int main() {
   int cases = 0, caught = 0;
+  for (int n = 1; n <= 1300; ++n) {
+    std::vector<int> plain(n), xcd(n);
+    for (int id = 0; id < n; ++id) {
+      ++plain.at(work_item(id, n));
+      ++xcd.at(work_item_xcd(id, n));
+      // whole rounds keep an item's XCD; without that the rounds themselves are mirrored
+      if (id / 256 * 256 + 256 <= n && work_item_xcd(id, n) % kXcds != id % kXcds) return 1;
+      if (n <= 1024 && id / 256 % 2 && id / 256 * 256 + 256 <= n && work_item(id, n) != id / 256 * 256 + 255 - id % 256) return 1;
+    }
+    if (std::count(plain.begin(), plain.end(), 1) != n || std::count(xcd.begin(), xcd.end(), 1) != n) return 1;
+  }
   for (int tiles : {1, 2, 3, 7, 8, 31, 64, 257})
     for (int pairs = 1; pairs <= 41; ++pairs)
       for (int members : {1, 2, 3, 5, 8, 32})
