@@ -402,7 +402,8 @@ std::optional<std::pair<Tensor, Tensor>> kv_append(const Tensor& kbuf, const Ten
 // autocast, types or sizes that differ, rows that are not whole 16-byte pieces, full buffers.
 std::optional<std::tuple<Tensor, Tensor, Tensor>> generation_step(const Tensor& x, const Tensor& w_qkv, const Tensor& w_out, const OptTensor& ow_gate,
                                                                   const Tensor& gain, const Tensor& cos, const Tensor& sin, const Tensor& kbuf,
-                                                                  const Tensor& vbuf, int64_t length, int64_t heads, int64_t kv_heads, int64_t flags) {
+                                                                  const Tensor& vbuf, int64_t length, int64_t heads, int64_t kv_heads, int64_t flags,
+                                                                  double eps, double gate_scale) {
   const Tensor w_gate = defined_or_none(ow_gate);
   const auto dev = x.device();
   if (!x.is_cuda() || x.dim() != 3 || x.size(1) != 1 || x.size(0) < 1 || x.size(0) > SEGPT_LINEAR_MAX_ROWS || w_qkv.dim() != 2) return std::nullopt;
@@ -435,7 +436,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> generation_step(const Tensor& 
   p.causal = 1;
   p.q_start = p.rope_q_pos0 = (int32_t)length;
   p.gq_numel = (int32_t)g32.numel();
-  p.eps = 1e-6f; p.sm_scale = (float)(1.0 / std::sqrt((double)D)); p.gate_scale = 2.0f;  // attention.py:51-80, :248
+  p.eps = (float)eps; p.sm_scale = (float)(1.0 / std::sqrt((double)D)); p.gate_scale = (float)gate_scale;
   p.flags = (int)flags;
   p.k = view4(kbuf, 0); p.v = view4(vbuf, 0);
   p.g_q = ptr_of<float>(g32);

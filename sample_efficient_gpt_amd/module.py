@@ -99,12 +99,18 @@ class KVCache:
         return self._mbuf[:, :, : self.length]
 
 
+# what the module asks of the attention, in a prompt and in a generation step alike (attention.py:51-80, :248)
+_EPS, _GATE_SCALE = 1e-6, 2.0
+
+_LINEAR_FILE, _LINEAR_PRODUCT = nn.Linear.extra_repr.__code__.co_filename, torch._C._nn.linear
+
+
 def _linear_replaced():
-    """Somebody has put another function in the place of the layers' forward, for all of them, or of the product it calls (their code
-    is not from the file that the class's other methods are from)."""
+    """Somebody has put another function in the place of the layers' forward, for all of them (its code is not from the class's file), or
+    of the product it calls."""
     try:
-        return (nn.Linear.forward.__code__.co_filename != nn.Linear.extra_repr.__code__.co_filename
-                or _Linear.forward.__code__.co_filename != _Linear.__init__.__code__.co_filename or F.linear is not torch._C._nn.linear)
+        return (nn.Linear.forward.__code__.co_filename != _LINEAR_FILE or _Linear.forward.__code__ is not _LAYER_CODE
+                or F.linear is not _LINEAR_PRODUCT)
     except AttributeError:
         return True
 
@@ -132,6 +138,9 @@ class _Linear(nn.Module):
 
     def forward(self, x):
         return self.linear(x)
+
+
+_LAYER_CODE = _Linear.forward.__code__
 
 
 class MultiHeadSelfAttention(nn.Module):
@@ -217,7 +226,7 @@ class MultiHeadSelfAttention(nn.Module):
         if _seen_as_operator(x, w_qkv, w_out, w_gate, gain, cos, sin, kv_cache._kbuf, kv_cache._vbuf):
             return None
         step = _native.load().generation_step(x, w_qkv, w_out, w_gate, gain, cos, sin, kv_cache._kbuf, kv_cache._vbuf, kv_cache.length,
-                                              self.n_heads, self.n_kv_heads, _call_flags(self.qknorm, True))
+                                              self.n_heads, self.n_kv_heads, _call_flags(self.qknorm, True), _EPS, _GATE_SCALE)
         if step is not None:
             kv_cache.length += 1
             kv_cache.keys, kv_cache.values = step[1:]
@@ -277,10 +286,10 @@ class MultiHeadSelfAttention(nn.Module):
             gate_logits = self.attn_gate(x[..., :d])
         gain = self.sdpa_qknorm.gain if self.qknorm else self._unit_gain
         # the registered op: one opaque node under torch.compile and non-reentrant checkpointing
-        y = qknorm_attention_op(q, k, v, gain, None, v_first=v_first, vr_coef=vr_coef, gate_logits=gate_logits, gate_scale=2.0,
-                             causal=True, q_start=q_start, rope_cos=self.rope.cos, rope_sin=self.rope.sin,
+        y = qknorm_attention_op(q, k, v, gain, None, v_first=v_first, vr_coef=vr_coef, gate_logits=gate_logits, gate_scale=_GATE_SCALE,
+                             eps=_EPS, causal=True, q_start=q_start, rope_cos=self.rope.cos, rope_sin=self.rope.sin,
                              rope_q_pos0=q_start, rope_k_pos0=0, qk_norm=self.qknorm, out_bshd=True)
         attn_cat = y.permute(0, 2, 1, 3).reshape(b, S, H * d)  # a view: the kernel wrote this layout
         if self.gating == "elementwise":
-            attn_cat = (2.0 * self.attn_gate(x).sigmoid()) * attn_cat
+            attn_cat = (_GATE_SCALE * self.attn_gate(x).sigmoid()) * attn_cat
         return self.out(attn_cat), v_mixed  # later layers take the second one as v1

@@ -1835,7 +1835,7 @@ def test_mhsa_module_generation_step_is_the_separate_calls(gpu_device, b, H, Hkv
     assert torch.allclose(y.float(), want.float(), atol=2e-2, rtol=1e-2)
     real = _native_module().generation_step
     args = lambda xt, length: (xt, m.qkv.linear.weight, m.out.linear.weight, m.attn_gate.linear.weight if gating else None, torch.ones(1, device=gpu_device),
-                               m.rope.cos, m.rope.sin, cache._kbuf, cache._vbuf, length, H, Hkv, 4)
+                               m.rope.cos, m.rope.sin, cache._kbuf, cache._vbuf, length, H, Hkv, 4, 1e-6, 2.0)
     token = x[:, :1].clone()
     with torch.no_grad():
         # accepted as it stands; what follows differs from it in one argument each
@@ -1849,6 +1849,27 @@ def test_mhsa_module_generation_step_is_the_separate_calls(gpu_device, b, H, Hkv
             assert real(*args(token, 0)) is None
         assert torch.equal(cache._kbuf.view(torch.int16), before.view(torch.int16))
     assert real(*args(token.requires_grad_(), 0)) is None
+
+
+def test_generation_step_asks_for_the_prompts_attention(gpu_device, monkeypatch):
+    """eps and gate scale have one place: changed there, prompt and token change alike (the last row of a prompt is the token behind its
+    other rows, within two roundings to bf16 of the projections)."""
+    from sample_efficient_gpt_amd import module
+
+    monkeypatch.setattr(module, "_EPS", 0.5)
+    monkeypatch.setattr(module, "_GATE_SCALE", 3.0)
+    H, Hkv, d, S = 6, 2, 64, 40
+    m, _, _ = _module_and_oracle_weights(gpu_device, BF16, H * d, H, Hkv, True, False, "per-head", seed=43)
+    x = torch.randn(2, S, H * d, generator=torch.Generator().manual_seed(44)).to(BF16).to(gpu_device)
+    native, cache = _record_generation_steps(m), KVCache()
+    with torch.no_grad():
+        whole = m(x)[0][:, -1:]
+        m(x[:, :-1], kv_cache=cache)
+        token = m(x[:, -1:], kv_cache=cache)[0]
+        monkeypatch.undo()
+        before = m(x)[0][:, -1:]
+    assert native == [True]
+    assert (token - whole).float().norm() <= 0.01 * whole.float().norm() < 0.1 * (before - whole).float().norm()
 
 
 def _record_generation_steps(m):
