@@ -1,9 +1,9 @@
 // fp32 forward and backward on the bf16 matrix pipe: every fp32 operand as the sum of three bf16 numbers.
 //
 // x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1) (round to nearest: 24 bits and the signs of
-// the remainders, so the sum is x itself but for the last bit of what lies below bf16's smallest numbers).  A product of two such
-// numbers is six matrix instructions, x0 y0 + (x0 y1 + x1 y0 + x1 y1 + x0 y2 + x2 y0), each product exact and summed in fp32;
-// what is left out is below 2^-25 of |x y|.  v_mfma_f32_32x32x16_bf16 does eight times the products of
+// the remainders, so the sum is x itself).  The method is Henry, Tang and Heinecke's, "Leveraging the bfloat16 Artificial Intelligence
+// Datatype for Higher-Precision Computations" (2019).  A product of two such numbers is six matrix instructions, x0 y0 + (x0 y1 + x1 y0 +
+// x1 y1 + x0 y2 + x2 y0), each product exact and summed in fp32; what is left out is below 2^-24 of |x y|.  v_mfma_f32_32x32x16_bf16 does eight times the products of
 // v_mfma_f32_32x32x2_f32 in half the time, so six of them take 3/8 of the fp32 instructions' time, and a sum of 64 products is 4 (and
 // 20 small ones) roundings deep instead of 32: norm-wise distance of a 32x32 tile of products to float64, 64 / 128 columns:
 // fp32 instructions 1.5e-7 / 1.95e-7, one accumulator for all six 1.1e-7 / 1.6e-7, the largest product on its own 4.9e-8 / 6.4e-8.
@@ -854,29 +854,31 @@ int f32_split_parts(const segpt_attn_params& p) {
   const int want = (512 + units - 1) / units, most = (rep * n_tiles(p.Sq) + kWaves - 1) / kWaves;
   return std::max(1, std::min({want, most, rep * f32_dkdv_splits(p)}));
 }
-// Where splitting pays.  The pre-pass is a launch more (4 to 6 us, 11 for a backward of 16 heads of 1000 tokens) and 6 bytes an
-// element written and read again, so a key has to be used by several workgroups and a wave has to have a few tiles.  Us of a call, plain
-// operands, fp32 instructions -> here:
-//   forward  head_dim 128, 4 heads:  128 tokens 13.3 -> 16.5, 192: 20.0 -> 19.1, 1000: 60.9 -> 35.2;  16 heads: 192 20.2 -> 20.1, 512 35.0 -> 29.1
-//            64, 16 heads:  256 11.6 -> 13.5, 512 18.7 -> 17.8, 1000 33.3 -> 29.4;  32 heads: 512 21.3 -> 24.0, 768 45.0 -> 38.6; 144 heads of 2048 859 -> 530
-//            32, 12 heads:  512 11.7 -> 12.4, 768 16.6 -> 15.1;  48 heads: 256 9.4 -> 11.4, 384 14.5 -> 13.7
-//   backward head_dim 128:  64 tokens, 4 heads 39 -> 31, 1000 153 -> 83;  16 heads: 128 43 -> 38, 512 123 -> 80
-//            64, 16 heads:  256 31 -> 33, 384 47 -> 42, 1000 112 -> 85;  32 heads: 192 38 -> 35, 384 67 -> 56
-//            32, 12 heads:  384 27 -> 30, 512 33.5 -> 33.1, 768 54 -> 43;  48 heads: 192 29 -> 33, 384 54 -> 43
-// Few workgroups that read a key tile (users: query tiles of the group's heads), forward; the backward gains there too:
-//   forward  128, 16 heads:  256 20.5 -> 21.1, 384 27.4 -> 24.9;  32 heads: 256 21.1 -> 24.3, 320 27.5 -> 30.2, 384 33.3 -> 33.3, 512 54 -> 36;
-//            64 heads: 256 33.9 -> 30.0;  8 heads: 256 20.4 -> 19.6;  8 x 32 / 4 heads, one query, 4096 keys 228 -> 153
-//            64, 17 heads:  512 19.4 -> 21.4;  8 x 32 / 4 heads, one query, 4096 keys 107 -> 75
-//            32, 128 heads:  256 16.6 -> 18.8, 384 27.2 -> 28.4, 448 35 -> 32;  256 heads: 256 30.4 -> 29.8, 320 41 -> 36;  48 heads: 384 14.0 -> 14.4, 448 16.1 -> 16.0
-//   backward 128, one query:  4 heads, 2048 keys 180 -> 89;  8 x 32 / 4 heads, 4096 keys 2735 -> 601;  32 x 16 heads, one key 86 -> 66
+// Where splitting pays.  The pre-pass is a launch more (4 to 7 us, 12 for a backward of 16 heads of 1000 tokens) and 6 bytes an
+// element written and read again, so a key has to be used by several workgroups (`users`) and a wave has to have a few tiles.  The fp32 instructions'
+// times go in steps, rounds of 256 or 512 resident workgroups of `n_kt` tiles; hence lines in n_kt and in workgroups (`grid`).  Us of a call, plain
+// operands, fp32 instructions -> here; two heads a group where no other is given:
+//   forward  128, 4 heads:  128 tokens 13.4 -> 18.2, 192 19.7 -> 20.8, 1000 59.7 -> 36.8;  16 heads: 192 19.9 -> 21.4, 512 34.5 -> 28.3
+//            one head a group:  8 heads: 256 20.5 -> 21.6, 320 26.6 -> 24.1;  16: 256 20.5 -> 23.2, 320 26.6 -> 25.8;  32: 256 20.9 -> 26.2, 320 27.4 -> 30.2, 400 46 -> 35;
+//            64: 256 34.3 -> 31.4;  four a group:  32: 256 20.9 -> 22.3, 320 27.3 -> 26.4;  8 x 32 / 4 heads, one query, 4096 keys 227 -> 156
+//            64, 16 heads:  256 10.9 -> 13.6, 384 14.5 -> 15.5, 512 17.8 -> 17.0, 1000 32.6 -> 26.2;  32 heads: 512 20.4 -> 19.8, 768 40 -> 33; 144 heads of 2048 842 -> 505
+//            one head a group:  8 heads: 512 17.7 -> 16.7;  12: 512 17.6 -> 19.2, 600 20.9 -> 21.4;  16: 512 17.7 -> 18.3, 600 22.3 -> 21.4;  17: 512 19.3 -> 21.5
+//            32, 12 heads:  512 11.1 -> 12.7, 768 15.6 -> 15.4;  24: 512 12.1 -> 13.9;  48 heads: 256 8.6 -> 11.5, 384 13.6 -> 13.4
+//            one head a group:  24: 640 14.4 -> 16.6;  48: 448 15.9 -> 16.5, 480 18.8 -> 17.8;  80: 448 24.0 -> 25.2;  128: 256 16.6 -> 18.8, 384 27 -> 28, 448 35 -> 32;
+//            256: 320 41 -> 36;  four a group:  256: 160 18.1 -> 17.5
+//   backward 128:  4 heads: 64 tokens 48 -> 33, 1000 153 -> 81;  16 heads: 128 49 -> 38, 512 125 -> 73;  one query: 4 heads, 2048 keys 180 -> 89, 8 x 32 / 4
+//            heads, 4096 keys 2730 -> 605;  32 x 16 heads, one key 86 -> 66
+//            64, 16 heads:  256 34 -> 29, 384 48 -> 38, 1000 110 -> 76;  32 heads: 192 39 -> 32, 384 65 -> 44
+//            32, 12 heads:  384 29 -> 26, 512 34 -> 32, 768 55 -> 40;  48 heads: 192 31 -> 29, 384 54 -> 40;  one head a group, 128: 128 28 -> 31, 256 57 -> 56
 bool f32_split_pays(const segpt_attn_params& p, bool bwd) {
-  const int n_qt = n_tiles(p.Sq), n_kt = n_tiles(p.Sk);
+  const int n_qt = n_tiles(p.Sq), n_kt = n_tiles(p.Sk), rep = p.H / p.Hkv;
   const int64_t heads = (int64_t)p.B * p.H, pairs = heads * n_qt * n_kt, grid = heads * n_qt;
-  const int64_t users = (int64_t)(p.H / p.Hkv) * n_qt;  // workgroups that read a key tile
+  const int64_t users = (int64_t)rep * n_qt;  // workgroups that read a key tile
   if (users < 8 && !(bwd && p.D == 128)) return false;  // one query against a long cache: split keys used once or twice
-  if (p.D == 128) return bwd || (n_kt >= 6 && (n_kt >= 12 || users >= 12 || grid <= 64 || grid >= 512));
-  if (p.D == 64) return bwd ? n_kt >= 12 : n_kt >= 24 || (n_kt >= 16 && heads <= 16);
-  return bwd ? pairs >= 3072 : pairs >= 5000 && (n_kt >= 14 || users >= 14 || grid >= 2560);
+  if (p.D == 128) return bwd || n_kt >= 13 || (n_kt >= 10 && (grid <= 192 || users >= 24)) || (n_kt >= 6 && grid >= 512);
+  if (p.D == 64) return bwd ? n_kt >= 12 : n_kt >= 24 || (n_kt >= 16 && heads <= 16 && (heads <= 8 || n_kt >= 19 || users >= 32));
+  if (bwd) return pairs >= 3072;
+  return pairs >= 5000 && (n_kt >= 24 || (n_kt >= 15 && grid > 512) || (n_kt >= 14 && grid >= 1792) || grid >= 2560 || (rep >= 4 && users >= 14 && grid > 512));
 }
 size_t f32_split_bytes(const segpt_attn_params& p, bool bwd) {
   if (!f32_split_pays(p, bwd)) return 0;

@@ -344,12 +344,13 @@ def test_fp32_split_scratch(lib):
         kv, q = 2 * 2 * 32, 2 * 6 * 32  # tiles of 32 rows of K and of Q: three bf16 numbers an element, two flags; lse and delta of the queries
         assert size(params(1000, 1000, D)) == [up(kv * (2 * 32 * D * 6 + 8)), up(kv * (3 * 32 * D * 6 + 8) + q * (4 * 32 * D * 6 + 8 + 64 * 4))]
     assert size(params(128, 128)) == [0, 0]
-    # head_dim 128: few users of a short key tile are not worth the forward's pre-pass in launches of 65 to 511 workgroups
+    # head_dim 128: short keys are not worth the forward's pre-pass in launches of fewer than 512 workgroups
     heads = lambda n, S, D: (lambda p: (setattr(p, "H", n), setattr(p, "Hkv", n), setattr(p, "B", 1), size(p))[-1])(params(S, S, D))
     assert heads(32, 256, 128)[0] == 0 and heads(32, 256, 128)[1] > 0
-    assert heads(8, 256, 128)[0] > 0 and heads(64, 256, 128)[0] > 0 and heads(32, 384, 128)[0] > 0
-    # head_dim 32: the same below 14 key tiles up to 2559 workgroups
+    assert heads(8, 256, 128)[0] == 0 and heads(64, 256, 128)[0] > 0 and heads(32, 416, 128)[0] > 0 and heads(8, 320, 128)[0] > 0
+    # the same at the other head sizes
     assert heads(128, 256, 32)[0] == 0 and heads(128, 448, 32)[0] > 0 and heads(320, 256, 32)[0] > 0
+    assert heads(16, 512, 64)[0] == 0 and heads(8, 512, 64)[0] > 0 and heads(17, 768, 64)[0] > 0
     p = _valid_params(); p.Sq = p.Sk = 1000
     assert size(p) == [0, 0]
     # the other workspace follows the flag: no delta, no copy of a gated dO, parts of dK and dV per kv head and not per query head
