@@ -88,8 +88,9 @@ extern "C" {
 
 #define SEGPT_FLAG_F32_SPLIT 16  /* fp32: kv_workspace is scratch of SEGPT_WS_F32_FWD / SEGPT_WS_F32_BWD bytes, 256 B aligned, and the
                                     call may run on the bf16 matrix pipe, every fp32 operand as a sum of three bf16 numbers
-                                    (no less accurate, faster; contents undefined on entry and exit).  No effect where that
-                                    size is 0, and ignored for bf16 and by segpt_attn_fwd_noalloc */
+                                    (no less accurate, faster; contents undefined on entry and exit, kept between the
+                                    stages of a call that is run stage by stage).  No effect where that size is 0, and
+                                    ignored for bf16 and by segpt_attn_fwd_noalloc */
 
 /* which scratch buffer segpt_attn_workspace_bytes() sizes */
 #define SEGPT_WS_KV 0  /* kv_workspace: bf16 copies of the normalised keys (and mixed values); forward AND backward */
