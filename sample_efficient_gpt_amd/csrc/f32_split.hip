@@ -23,9 +23,9 @@
 // What bounds it: the streamed tiles, 24 / 36 / 48 KB (forward / dQ / dK/dV at head_dim 64) per 32x32 scores and wave, of which a
 // CU gets about 19 bytes a cycle (11 TB/s) whether they are hits in the L2 or requests of a deeper look-ahead: matrix pipe 27 % busy,
 // and neither forming the next scores beside this tile's exponentials nor two accumulators more for shorter chains of dependent
-// products moved a kernel.  Kernels, us, fp32 instructions -> here: 2 x 8 / 4 heads, 1000 tokens of 64 forward 37 -> 5.4 + 21, dQ 47 ->
-// 26, dK/dV 62 -> 32, the pre-pass of the backward 11; the step 143 -> 102.  8 x 18 / 6 heads of 2048 tokens 3556 -> 2191, 1 x 4 / 2
-// heads of 1000 x 128 214 -> 115.
+// products moved a kernel.  Kernels, us, fp32 instructions -> here: 2 x 8 / 4 heads, 1000 tokens of 64 forward 37 -> 6.9 + 23, dQ and dK/dV 47 +
+// 62 -> 60, the pre-pass of the backward 13; the step 143 -> 99.  8 x 18 / 6 heads of 2048 tokens 3453 -> 2250, 1 x 4 / 2 heads of 1000 x
+// 128 213 -> 117.
 #include <algorithm>
 
 #include "f32_common.hpp"
@@ -100,7 +100,8 @@ __device__ __forceinline__ bool beyond_bf16(const float (&x)[N]) {
 // second part is kept times kPart and the third times kPart^2, and no bit is lost whose product fp32 could hold.  That is a property of
 // a tile (its flag in SplitMap); a wave that meets such a tile takes all its tiles through a loop of its own, in which the products of each
 // scale are formed apart.  dO of 1e-35: gradients were 6e-5 from float64, now 3.4e-7 (fp32 instructions 4e-7).  The flags and split_lanes
-// cost 1 to 4 % (backward of 2 x 8 / 4 heads, 1000 tokens 75.9 -> 78.1 us); scaling always and no second loop cost 5 to 8 %.
+// cost 1 to 4 % (backward of 2 x 8 / 4 heads, 1000 tokens 75.9 -> 78.1 us); scaling always and no second loop cost 5 to 8 %.  The same call with
+// one such row: 97, with v and dO of 1e-33: 106, its forward 28 -> 49 (fp32 instructions 111 and 36).
 constexpr float kPart = 128.f, kSmall = 7.888609052e-31f;  // 2^-100
 __device__ __forceinline__ bool any_lane(bool x) { return __builtin_amdgcn_ballot_w64(x) != 0; }
 __device__ __forceinline__ bool is_small(float x) { return x != 0.f && fabsf(x) < kSmall; }
@@ -799,9 +800,9 @@ __global__ __launch_bounds__(kThreads, (D == 128 ? 1 : 2)) void bwd_dkdv_split_k
   bwd_dkdv_split<D>(a, blockIdx.x - kXcds, lds, stat);
 }
 // Both, dK/dV first: they need the pre-pass and not each other, so the heavy dQ workgroups fill the causal tail of dK/dV and a launch is saved; the
-// finish kernel adds up the scale gradient.  For grids of one or two resident rounds each, where the tail counts (f32_split_both).  Step, us, two
-// launches -> one: 2 x 8 / 4 heads of 64, 1000 tokens 103.4 -> 101.0, 400 tokens 59.2 -> 54.7; 1 x 4 heads, 700 tokens 61.0 -> 55.6; 4 x 8
-// heads, 1000 tokens (1024 dQ workgroups) 202.9 -> 201.8; 3 x 6 / 2 heads of 32, 1000 tokens 77.1 -> 74.9.  head_dim 128 has its own register
+// finish kernel adds up the scale gradient.  For grids of one or two resident rounds each, where the tail counts (f32_split_both).  Backward, us, two
+// launches -> one: 2 x 8 / 4 heads of 64, 1000 tokens 75.5 -> 76.3, 400 tokens 41.7 -> 38.8; 1 x 4 heads, 700 tokens 43.2 -> 39.1; 4 x 8
+// heads, 1000 tokens (1024 dQ workgroups) 143.3 -> 142.7; 3 x 6 / 2 heads of 32, 1000 tokens 56.5 -> 53.8.  head_dim 128 has its own register
 // bound for dK/dV; larger grids want a pair's tiles pinned to an XCD and have the longer sum of the scale gradient.
 template <int D>
 __global__ __launch_bounds__(kThreads, 2) void bwd_both_split_kernel(KArgs a, int n_dkdv) {
