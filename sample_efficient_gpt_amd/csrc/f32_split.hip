@@ -802,7 +802,8 @@ __global__ __launch_bounds__(kThreads, (D == 128 ? 1 : 2)) void bwd_dkdv_split_k
 // Both, dK/dV first: they need the pre-pass and not each other, so the heavy dQ workgroups fill the causal tail of dK/dV and a launch is saved; the
 // finish kernel adds up the scale gradient.  For grids of one or two resident rounds each, where the tail counts (f32_split_both).  Backward, us, two
 // launches -> one: 2 x 8 / 4 heads of 64, 1000 tokens 75.5 -> 76.3, 400 tokens 41.7 -> 38.8; 1 x 4 heads, 700 tokens 43.2 -> 39.1; 4 x 8
-// heads, 1000 tokens (1024 dQ workgroups) 143.3 -> 142.7; 3 x 6 / 2 heads of 32, 1000 tokens 56.5 -> 53.8.  head_dim 128 has its own register
+// heads, 1000 tokens (1024 dQ workgroups) 143.3 -> 142.7; 3 x 6 / 2 heads of 32, 1000 tokens 56.5 -> 53.8.  And where what dQ streams stays in the
+// L2 beside what dK/dV does (32 / 4 heads, 256 queries, 8192 keys 361 -> 410; 16 / 2 heads, 2048 tokens 223 -> 255; 32 / 1 heads, 900 tokens 147 -> 137).  head_dim 128 has its own register
 // bound for dK/dV; larger grids want a pair's tiles pinned to an XCD and have the longer sum of the scale gradient.
 template <int D>
 __global__ __launch_bounds__(kThreads, 2) void bwd_both_split_kernel(KArgs a, int n_dkdv) {
@@ -913,7 +914,8 @@ int launch_bwd_dq_split(const KArgs& a, hipStream_t st) {
 }
 bool f32_split_both(const KArgs& a) {
   const segpt_attn_params& p = a.p;
-  return p.D != 128 && n_tiles(p.Sq) * (int64_t)p.B * p.H <= kPinnedGrid && n_tiles(p.Sk) * (int64_t)p.B * p.Hkv * a.f32_parts <= kPinnedGrid;
+  return p.D != 128 && n_tiles(p.Sq) * (int64_t)p.B * p.H <= kPinnedGrid && n_tiles(p.Sk) * (int64_t)p.B * p.Hkv * a.f32_parts <= kPinnedGrid &&
+         stream_per_xcd(p.B * p.Hkv, 3 * (int64_t)n_tiles(p.Sk) * p.D * (kUnitBytes / 16)) <= kL2Bytes;
 }
 int launch_bwd_both_split(const KArgs& a, hipStream_t st) {
   const segpt_attn_params& p = a.p;

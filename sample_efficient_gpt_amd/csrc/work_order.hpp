@@ -39,13 +39,14 @@ struct Item {
   int tile, pair, member;
 };
 constexpr int kPinnedGrid = 1024, kResident = 512, kXcds = 8;
-constexpr int64_t kStreamLimit = 16 << 20;
-// `stream`: bytes of the streamed tiles of one pair
+constexpr int64_t kL2Bytes = 4 << 20, kStreamLimit = 4 * kL2Bytes;
+// `stream`: bytes of the streamed tiles of one pair.  What an XCD streams in work_item_xcd's order:
+__attribute__((always_inline)) constexpr int64_t stream_per_xcd(int pairs, int64_t stream) { return stream * (pairs % kXcds ? pairs : pairs / kXcds); }
 __attribute__((always_inline)) constexpr Item split_item(int block, int tiles, int pairs, int members, int64_t stream) {
   Item it{};
   const int per = tiles * members;
   const int64_t total = (int64_t)per * pairs;
-  if (total <= kResident || (total <= kPinnedGrid && stream * (pairs % kXcds ? pairs : pairs / kXcds) <= kStreamLimit)) {
+  if (total <= kResident || (total <= kPinnedGrid && stream_per_xcd(pairs, stream) <= kStreamLimit)) {
     const int n = per * pairs, id = work_item_xcd(block, n), rest = id % (pairs * members);
     it.tile = id / (pairs * members);
     it.pair = n < 256 ? rest / members : rest % pairs;

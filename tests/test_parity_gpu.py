@@ -133,10 +133,11 @@ def test_fp32_split_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
     _case(gpu_device, F32, B, H, Hkv, Sq, Sk, D, gen_kw=gen_kw, seed=72, **kw)
 
 
-@pytest.mark.parametrize("B,H,Hkv,S,D,extras", [(1, 4, 2, 401, 64, True), (4, 12, 4, 300, 32, False), (4, 8, 4, 1024, 64, False), (4, 8, 4, 1025, 64, True)])
+@pytest.mark.parametrize("B,H,Hkv,S,D,extras", [(1, 4, 2, 401, 64, True), (4, 12, 4, 300, 32, False), (4, 8, 4, 1024, 64, False), (4, 8, 4, 1025, 64, True),
+                                               (1, 5, 5, 2700, 64, False), (1, 4, 1, 3700, 32, True)])
 def test_fp32_split_backward_in_one_launch_is_its_stages(gpu_device, B, H, Hkv, S, D, extras):
-    """dQ and dK/dV of a whole backward share a launch up to 1024 workgroups each (the third case; the fourth has more); the stages run one
-    by one.  Both are within 8 units of 2^-24 of float64 in norm (test_fp32_split_is_no_less_accurate), so within 16 of each other."""
+    """dQ and dK/dV of a whole backward share a launch up to 1024 workgroups each (the third case; the fourth has more) while what dQ streams
+    fits an L2 (the last two do not); the stages run one by one.  Both are within 8 units of 2^-24 of float64 in norm (test_fp32_split_is_no_less_accurate), so within 16 of each other."""
     from sample_efficient_gpt_amd import _lib
     from sample_efficient_gpt_amd.plan import AttnPlan
 
