@@ -853,7 +853,13 @@ int launch_dkdv(const KArgs& a, hipStream_t st) {
 // workspace of the other kernels has, one per query head and f32_dkdv_splits.
 int f32_split_parts(const segpt_attn_params& p) {
   const int units = n_tiles(p.Sk) * p.B * p.Hkv, rep = p.H / p.Hkv;
-  const int want = (512 + units - 1) / units, most = (rep * n_tiles(p.Sq) + kWaves - 1) / kWaves;
+  int want = (kResident + units - 1) / units;
+  const int most = (rep * n_tiles(p.Sq) + kWaves - 1) / kWaves;
+  // Less than two rounds of workgroups that all walk more than an L2 holds: the heaviest of them alone take as long as the rest, so two parts each.
+  // Backward, us, one part -> two (fp32 instructions): 12 / 3 heads of 64, 8192 tokens 3241 -> 2432 (3135); 20 / 5 heads, 4096 tokens 1223 -> 1050 (1361);
+  // 32 / 4 heads of 128, 4096 tokens 4364 -> 2991 (5247).  One head a group walks less: 5 heads, 4096 tokens 293 -> 296.
+  const bool walks = stream_per_xcd(p.B * p.Hkv, 4 * (int64_t)rep * n_tiles(p.Sq) * p.D * (kUnitBytes / 16)) > kStreamLimit;
+  if (want == 1 && units <= 2 * kResident && walks && rep > 1) want = 2;
   return std::max(1, std::min({want, most, rep * f32_dkdv_splits(p)}));
 }
 // Where splitting pays.  The pre-pass is a launch more (4 to 7 us, 12 for a backward of 16 heads of 1000 tokens) and 6 bytes an
