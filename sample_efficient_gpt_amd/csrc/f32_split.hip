@@ -878,11 +878,15 @@ int f32_split_parts(const segpt_attn_params& p) {
 //            heads, 4096 keys 2730 -> 605;  32 x 16 heads, one key 86 -> 66
 //            64, 16 heads:  256 34 -> 29, 384 48 -> 38, 1000 110 -> 76;  32 heads: 192 39 -> 32, 384 65 -> 44
 //            32, 12 heads:  384 29 -> 26, 512 34 -> 32, 768 55 -> 40;  48 heads: 192 31 -> 29, 384 54 -> 40;  one head a group, 128: 128 28 -> 31, 256 57 -> 56
+// One or two kv heads whose dK/dV workgroups each walk all queries of very many tiles, backward: the streams outgrow every cache
+//   64, one kv head:  16 heads of 4096 tokens (2048 users) 1097 -> 998, 12 of 6000 (2256) 1737 -> 1811, 16 of 6000 2275 -> 2350, 32 of 4096 2157 -> 2180;  two: 32 of 8192 8252 -> 8585
+//   32, one kv head:  64 heads of 4096 tokens (8192) 2342 -> 2245, of 8192 8979 -> 9150
 bool f32_split_pays(const segpt_attn_params& p, bool bwd) {
   const int n_qt = n_tiles(p.Sq), n_kt = n_tiles(p.Sk), rep = p.H / p.Hkv;
   const int64_t heads = (int64_t)p.B * p.H, pairs = heads * n_qt * n_kt, grid = heads * n_qt;
   const int64_t users = (int64_t)rep * n_qt;  // workgroups that read a key tile
   if (users < 8 && !(bwd && p.D == 128)) return false;  // one query against a long cache: split keys used once or twice
+  if (bwd && p.D <= 64 && p.B * p.Hkv <= 2 && users > (p.D == 64 ? 2200 : 12000)) return false;
   if (p.D == 128) return bwd || n_kt >= 13 || (n_kt >= 10 && (grid <= 192 || users >= 24)) || (n_kt >= 6 && grid >= 512);
   if (p.D == 64) return bwd ? n_kt >= 12 : n_kt >= 24 || (n_kt >= 16 && heads <= 16 && (heads <= 8 || n_kt >= 19 || users >= 32));
   if (bwd) return pairs >= 3072;

@@ -31,9 +31,9 @@ __attribute__((always_inline)) constexpr int work_item_xcd(int id, int n) {
 //     sees every eighth pair with all its members (us, members before pairs -> this: forward of 8 x 32 / 4 heads, one query, 4096 keys of 64 148 ->
 //     75, fp32 instructions 107; fewer workgroups do not fill the memory side and are 5 % faster spread: 16 / 4 heads, 64 queries, 2048 keys 33.9, 35.2).
 //     Up to 1024 the same if what an XCD then streams is no more than a few times its L2: it balances the causal tail (4 x 8 heads of 1000
-//     tokens: backward 138, 141 in the order below; 20 / 5 heads, 4096 tokens: 1534, 1203, fp32 instructions 1376).
+//     tokens: backward 138, 141 in the order below; forward of 32 x 16 / 4 heads, 64 queries, 2048 keys: 210, 159, fp32 instructions 189).
 //   * More: eight pairs at a time, one on each XCD; the last pairs % 8 as four, two and one, each on two, four or all XCDs, so that none idles
-//     (us, the last ones on an XCD each -> this: 32 heads on one kv head, 4096 tokens of 64: forward 2417 -> 398, backward 4962 -> 2190; 18 / 6
+//     (us, the last ones on an XCD each -> this: 8 heads on one kv head, 8192 tokens of 64: forward 2273 -> 393, backward 4487 -> 1799; 18 / 6
 //     heads, 8192 tokens 1098 -> 856, 3768 -> 3640).
 struct Item {
   int tile, pair, member;

@@ -348,7 +348,10 @@ def test_fp32_split_scratch(lib):
     heads = lambda n, S, D: (lambda p: (setattr(p, "H", n), setattr(p, "Hkv", n), setattr(p, "B", 1), size(p))[-1])(params(S, S, D))
     assert heads(32, 256, 128)[0] == 0 and heads(32, 256, 128)[1] > 0
     assert heads(8, 256, 128)[0] == 0 and heads(64, 256, 128)[0] > 0 and heads(32, 416, 128)[0] > 0 and heads(8, 320, 128)[0] > 0
-    # the same at the other head sizes
+    # one or two kv heads under very many query tiles are left to the fp32 instructions in the backward
+    group = lambda n, S, D: (lambda p: (setattr(p, "H", n), setattr(p, "Hkv", 1), setattr(p, "B", 1), size(p))[-1])(params(S, S, D))
+    assert group(16, 4096, 64)[1] > 0 and group(16, 6000, 64)[1] == 0 and group(16, 6000, 64)[0] > 0 and group(16, 6000, 128)[1] > 0
+    # the forward's lines at the other head sizes
     assert heads(128, 256, 32)[0] == 0 and heads(128, 448, 32)[0] > 0 and heads(320, 256, 32)[0] > 0
     assert heads(16, 512, 64)[0] == 0 and heads(8, 512, 64)[0] > 0 and heads(17, 768, 64)[0] > 0
     p = _valid_params(); p.Sq = p.Sk = 1000
