@@ -115,6 +115,7 @@ def test_fp32_tile_edges(gpu_device, B, H, Hkv, Sq, Sk, D, kw, gen_kw):
         (5, 9, 3, 769, 769, {}, {}),  # more than 1024 workgroups, (batch, kv head) pairs that are no multiple of the XCDs
         (1, 44, 1, 770, 770, {}, {}),  # the same with one pair for all XCDs
         (3, 10, 5, 1100, 1100, {}, {}),  # dK/dV: 525 workgroups would take one part each, two where they walk more than an L2 holds
+        (4, 8, 4, 1025, 1025, {}, {"extras": True}),  # one part of dK and dV for two heads a group, formed in place
         (1, 27, 3, 1290, 1290, {}, {}),  # three pairs: two and one at a time; dK/dV between 512 and 1024 workgroups, more than an L2 streamed
     ],
 )
