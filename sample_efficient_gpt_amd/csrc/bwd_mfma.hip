@@ -554,6 +554,7 @@ template <int D, bool ROPE, int PARTS>
 __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kernel(KArgs a) {
   using Z = Swz<D>;
   static_assert(PARTS == 1 || PARTS == 2, "a tile has two 32-query blocks");
+  constexpr bool PIPE = PARTS == 1;
   constexpr int BKV = kBwdRows / PARTS;
   constexpr int kKeyWaves = 4 / PARTS;  // waves side by side along the keys
   constexpr int KS = D / 16;
@@ -571,7 +572,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: everything derived from it stays scalar
   const int ln = lane & 31, hh = lane >> 5;
-  const int rep = p.H / p.Hkv;
+  const int rep = __builtin_amdgcn_readfirstlane(p.H / p.Hkv);  // divided in vector registers
   const int n_kvt = (p.Sk + BKV - 1) / BKV;
   // Workgroup 0 is an extra one: dispatched first, it only folds the dQ kernel's per-workgroup partials of the
   // scale-vector gradient (complete: that kernel ran before this one on the stream) while the others compute.
@@ -586,8 +587,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
     if (tid < 2) a.dcoef_part[(int64_t)bid * 2 + tid] = 0.f;
     return;
   }
-  wg.tile = n_kvt - 1 - wg.tile;  // early key tiles see the most queries: issue them first
-  const int b = wg.b, g = wg.g;
+  wg.tile = __builtin_amdgcn_readfirstlane(n_kvt - 1 - wg.tile);  // early key tiles see the most queries: issue them first
+  const int b = __builtin_amdgcn_readfirstlane(wg.b), g = __builtin_amdgcn_readfirstlane(wg.g);
   const int k0 = wg.tile * BKV;
   const int key_wave = PARTS == 1 ? wave : wave % kKeyWaves, part = PARTS == 1 ? 0 : wave / kKeyWaves;
   const int kw0 = k0 + key_wave * 32;
@@ -598,7 +599,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   int qt_start = 0;
   if (p.causal) qt_start = min(max(0, k0 - p.q_start) / kBK, n_qt);
   const int n_vis = n_qt - qt_start;  // visible query tiles per head
-  const int n_it = n_vis * rep;       // streamed tiles in total
+  const int n_it = __builtin_amdgcn_readfirstlane(n_vis * rep);  // streamed tiles in total
 
   // ---- staging of one (head, query tile): Qhat and dO tiles plus the two row statistics, all by direct
   // global->LDS loads.  Every wave issues the same number of loads (waves 2/3 repeat the statistics load
@@ -609,22 +610,38 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   const float* const stat_arr = (wave & 1) ? a.delta : a.nlse2;
   const uint32_t dstep = do_contig ? (uint32_t)D * 2 : (uint32_t)p.d_o.stride_s * 2;
   const TileLaneOff<D> full_tile = tile_lane_offsets<D>(D * 2, dstep, kBK, src.x, src.y);
-  // The stream of (head, query tile) pairs is walked by running pointers kept beside the compute loop's own
-  // counters (three tiles ahead of it): per tile a few scalar additions, per head one address computation.
-  const char* q_it = nullptr;
-  const char* d_it = nullptr;
-  const float* s_it = nullptr;
-  int left_it = 0, iss_h = 0, iss_t = 0, iss_stage = 0;
-  auto set_head = [&](int hq) {
-    const int h = g * rep + hq, i0 = qt_start * kBK;
-    const int64_t row = ((int64_t)b * p.H + h) * p.Sq + i0;
-    q_it = reinterpret_cast<const char*>(a.qhat + row * D);
-    d_it = do_contig ? reinterpret_cast<const char*>(reinterpret_cast<const uint16_t*>(a.do_eff) + row * D)
-                     : reinterpret_cast<const char*>(row_ptr<uint16_t>(p.d_o, b, h, i0));
-    s_it = stat_arr + row;
-    left_it = p.Sq - i0;
+  // The stream of (query tile, head) pairs is walked by running pointers kept beside the compute loop's own counters
+  // (three tiles ahead of it): per tile a few scalar additions.
+  // PARTS == 1: from the last tile down, every head of the group at a tile before the next tile.  All workgroups of a
+  // (batch, kv head) pair start at the same tile and stay together, so that a tile comes into the XCD's L2 once for all of them.
+  // Head by head and upwards from the diagonal every workgroup was somewhere else: L2 misses per launch (128-byte lines),
+  // 4 x 16 / 4 heads, 4096 tokens, head_dim 128 9.8 M -> 4.0 M, 2 x 18 / 6 heads, 8192 tokens, head_dim 64 10.7 M -> 3.9 M.
+  // PARTS == 2, head by head and upwards: these launches' streams fit the L2 anyway, and in step their workgroups
+  // only queue for the same lines (8 x 18 / 6 heads, 999 tokens: the whole step 177.3 us, in step 178.5).
+  constexpr bool kInStep = PARTS == 1;
+  int iss_h = 0, iss_t = 0, iss_stage = 0, issued = 0;
+  const int i_first = kInStep ? (n_qt - 1) * kBK : qt_start * kBK;  // first query of the stream's first tile
+  const int64_t row_first = ((int64_t)b * p.H + g * rep) * p.Sq + i_first;
+  const int64_t q_head = (int64_t)p.Sq * D * 2, d_head = do_contig ? q_head : (int64_t)p.d_o.stride_h * 2;
+  const char* q_it = reinterpret_cast<const char*>(a.qhat + row_first * D);
+  const char* d_it = do_contig ? reinterpret_cast<const char*>(reinterpret_cast<const uint16_t*>(a.do_eff) + row_first * D)
+                               : reinterpret_cast<const char*>(row_ptr<uint16_t>(p.d_o, b, g * rep, i_first));
+  const float* s_it = stat_arr + row_first;
+  int left_it = p.Sq - i_first;
+  auto move = [&](int tiles, int heads) {
+    const int rows = tiles * kBK;
+    q_it += heads * q_head + (int64_t)rows * D * 2;
+    d_it += heads * d_head + (int64_t)rows * dstep;
+    s_it += heads * p.Sq + rows;
+    left_it -= rows;
   };
-  if (n_it > 0) set_head(0);
+  auto advance = [&]() {
+    if constexpr (kInStep) {
+      if (++iss_h == rep) { iss_h = 0; move(-1, 1 - rep); } else move(0, 1);
+    } else {
+      if (++iss_t == n_vis) { iss_t = 0; move(1 - n_vis, 1); } else move(1, 0);
+    }
+  };
   const uint32_t lane4 = lane * 4;
   auto issue_next = [&]() {
     const uint32_t dst = lds0 + iss_stage * kStageBytes + wave * 1024;
@@ -637,15 +654,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
       gload_lds4_so(s_it, (uint32_t)min(lane, left_it - 1) * 4, sdst);
     }
     iss_stage = iss_stage == kStages - 1 ? 0 : iss_stage + 1;
-    if (++iss_t == n_vis) {
-      iss_t = 0;
-      if (++iss_h < rep) set_head(iss_h);
-    } else {
-      q_it += kBK * D * 2;
-      d_it += (int64_t)kBK * dstep;
-      s_it += kBK;
-      left_it -= kBK;
-    }
+    if (++issued < n_it) advance();
   };
 
   // ---- start-up: streamed tiles 0 and 1 into stages 0 and 1, and with them the workgroup's 128 Khat and V' rows
@@ -699,113 +708,327 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   const uint32_t st_lane = ldl0 + 16 * hh + part * 32 * 4;
 
   bf16x8 qf[KS], df[KS];
-  auto request_rowmajor = [&](uint32_t rm, int qb) {  // qb is a compile-time constant at every call site
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      qf[ks] = swz_frag_rm<D>(rm, qb, ks);
-      df[ks] = swz_frag_rm<D>(rm + Z::kTileBytes, qb, ks);
-    }
-  };
-  // one 32-query block (qb = 0/1, compile-time) of the tile whose stage the pointers address;
-  // ib = first query of the block; the row-major fragments of the block after it start at next_rm.
-  // The mask variant is compile-time so that a whole block is one straight-line scheduling region:
-  // 0 none, 1 causal diagonal only (every query of the block exists), 2 diagonal and / or end of the queries.
-  auto step = [&](auto masked_c, uint32_t tr, uint32_t st, int qb, int ib, uint32_t next_rm, int next_qb) {
-    constexpr int MASK = decltype(masked_c)::value;
-    // head_dim 128 (one wave per SIMD, nothing else to hide the exp2 phase behind): the compiler's interleaving
-    // strategy for exp2 work between MFMA chains, measured -3 % on this kernel; at head_dim 64 it changes nothing
-    if constexpr (D == 128) __builtin_amdgcn_iglp_opt(3);
-    // accumulators of S and dP start from -lse2 / -delta of the 16 query rows their registers map to
-    f32x16 s, dpv;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const f32x4 l4 = lds_read_f4(st + (32 * qb + 8 * c) * 4);
-      const f32x4 d4 = lds_read_f4(st + (64 + 32 * qb + 8 * c) * 4);
-      s[4 * c] = l4[0]; s[4 * c + 1] = l4[1]; s[4 * c + 2] = l4[2]; s[4 * c + 3] = l4[3];
-      dpv[4 * c] = d4[0]; dpv[4 * c + 1] = d4[1]; dpv[4 * c + 2] = d4[2]; dpv[4 * c + 3] = d4[3];
-    }
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) s = mfma32(qf[ks], kreg[ks], s);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) dpv = mfma32(df[ks], vreg[ks], dpv);
-    bf16x8 dT[MB][2], qT[MB][2];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      dT[mb][0] = swz_frag_tr<D>(tr + Z::kTileBytes, mb, 2 * qb);
-      qT[mb][0] = swz_frag_tr<D>(tr, mb, 2 * qb);
-      dT[mb][1] = swz_frag_tr<D>(tr + Z::kTileBytes, mb, 2 * qb + 1);
-      qT[mb][1] = swz_frag_tr<D>(tr, mb, 2 * qb + 1);
-    }
-    if (MASK != 0) {  // block touches the diagonal or the end of the queries
-      // register r holds query ib + 4hh + c_r with c_r = 8(r/4) + r%4 a compile-time constant.
-      // masked iff key > query + q_start  <=>  c_r < key - q_start - ib - 4hh,   or query >= Sq
-      const int t = p.causal ? key - p.q_start - ib - 4 * hh : -1;
-      const int u = p.Sq - ib - 4 * hh;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int c = 8 * (r >> 2) + (r & 3);
-        if (MASK == 1 ? c < t : (c < t || c >= u)) s[r] = -INFINITY;
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = fast_exp2(s[r]);
-      dpv[r] *= s[r];
-    }
-    const bf16x8 p0 = pack_c_half(s, 0), p1 = pack_c_half(s, 1);
-    const bf16x8 ds0 = pack_c_half(dpv, 0), ds1 = pack_c_half(dpv, 1);
-    request_rowmajor(next_rm, next_qb);  // unconditional: past the last block the fragments are simply unused
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      dvacc[mb] = mfma32(dT[mb][0], p0, dvacc[mb]);
-      dkacc[mb] = mfma32(qT[mb][0], ds0, dkacc[mb]);
-    }
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      dvacc[mb] = mfma32(dT[mb][1], p1, dvacc[mb]);
-      dkacc[mb] = mfma32(qT[mb][1], ds1, dkacc[mb]);
-    }
-  };
-
-  // ---- pipeline start-up: tiles 0 and 1 have landed (first wait above), tile 2 is in flight
-  if (n_it > 0) request_rowmajor(rm_lane, 0);
-  // Per head the visible query tiles t = 0 .. n_vis-1 (first query (qt_start + t) * 64) fall into runs for this
-  // wave: [0, t_diag) touch the causal diagonal (those before t_full lie inside Sq and need the diagonal test only),
-  // [t_diag, t_end) need no mask, [t_end, n_vis) run past Sq.  Each run is its own loop so that a loop body holds
-  // one variant of the block (whole-block scheduling regions, no accumulator copies at joins).
+  // The visible query tiles t = 0 .. n_vis-1 (first query (qt_start + t) * 64) fall into runs for this wave: [0, t_diag)
+  // touch the causal diagonal (those before t_full lie inside Sq and need the diagonal test only), [t_diag, t_end) need
+  // no mask, [t_end, n_vis) run past Sq.  Each run is its own loop so that a loop body holds one variant of the block
+  // (whole-block scheduling regions, no accumulator copies at joins).
   int t_diag = 0;
   if (p.causal) t_diag = min(max((max(kw0 + 31 - p.q_start, 0) + kBK - 1) / kBK - qt_start, 0), n_vis);
   const int t_full = min(max(p.Sq / kBK - qt_start, 0), n_vis);  // tiles whose 64 queries all exist
   const int t_end = max(t_full, t_diag);
-  int stage = 0, it = 0;
-  auto run_tiles = [&](auto masked_c, int t_lo, int t_hi) {
-    constexpr int MASK = decltype(masked_c)::value;
-    for (int t = t_lo; t < t_hi; ++t, ++it) {
-      const int nstage = stage == kStages - 1 ? 0 : stage + 1;
-      const int i0 = (qt_start + t) * kBK;
-      const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
-      const uint32_t st = st_lane + stage * 512;
-      // on the diagonal a block whose last query still lies before this wave's first key is masked entirely:
-      // it only passes the fragment request on (wave-uniform, so the barrier below is reached all the same)
-      if constexpr (PARTS == 1) {
-        if (MASK == 1 && kw0 > i0 + 31 + p.q_start) request_rowmajor(rm, 1); else step(masked_c, tr, st, 0, i0, rm, 1);
-        if (MASK == 1 && kw0 > i0 + 63 + p.q_start) request_rowmajor(rm_lane + nstage * kStageBytes, 0);
-        else step(masked_c, tr, st, 1, i0 + 32, rm_lane + nstage * kStageBytes, 0);
-      } else {
+  if constexpr (PARTS == 1) {
+    // A software pipeline over 32-query blocks, laid out instruction by instruction: step n computes the scores and dP of
+    // block n + 1 (first half: kA matrix instructions) while the vector unit turns those of block n into P and dS, then
+    // adds block n to dV and dK (second half: kB) while the row-major fragments and row statistics of block n + 2 come in.
+    // A slot is one matrix instruction and what fits beside it, closed by a scheduling barrier, so that the source's order is
+    // the kernel's.  What a slot holds (one wave per SIMD, cycles): a matrix instruction runs for 32 and keeps the vector
+    // port for 16 of them; behind it a plain vector instruction takes 4, an exponential 8, an LDS read 8 (for free in
+    // those 16), a direct load 13.  Left to the compiler, the products of a block ran first and its exponentials next.
+    // The accumulators and the stationary rows live in accumulation registers, scores and dP in ordinary ones; a kernel
+    // of more than 256 registers gets one form for all matrix instructions from the compiler, hence the inline assembly,
+    // whose wait states tests/test_mfma_hazards.py checks on the built code.
+    // dK/dV, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 515 -> 430 (matrix pipe 54 -> 72 % busy; the clock gives part of
+    // it back, 1.98 -> 1.74 GHz); head_dim 64, 2 x 18 / 6 heads, 8192 tokens 587 -> 530 (58 -> 67 %), 8 x 2048 154 -> 149.
+    constexpr int kA = 2 * KS, kB = 4 * MB;
+    // i-th product of the first half: k-step of S (0 .. KS-1) or KS + that of dP.  S leads, so that the statistics from which
+    // dP starts, requested last, have time.
+    constexpr int kOrder64[] = {0, 1, 4, 2, 5, 3, 6, 7}, kOrder128[] = {0, 1, 2, 8, 3, 9, 4, 10, 5, 11, 6, 12, 7, 13, 14, 15};
+    auto order = [&](int i) { return D == 64 ? kOrder64[i & 7] : kOrder128[i]; };
+    f32x16 s0, d0, s1, d1;  // scores and dP of two consecutive blocks
+    uint32_t rm_next = 0, st_next = 0;        // the next tile's row-major fragments and statistics
+    uint32_t rma[KS], tra[2 * MB];            // ... its fragments by k-step, and this tile's transposed ones by column block
+    auto load_stat = [&](f32x16& s, f32x16& d, uint32_t st, int qb, int c) {  // a quarter of -lse2 (c < 4) or -delta
+      const f32x4 v = lds_read_f4(st + ((c & 4 ? 64 : 0) + 32 * qb + 8 * (c & 3)) * 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) (c & 4 ? d : s)[4 * (c & 3) + i] = v[i];
+    };
+    // (s, d): block n, whose first query is ib, number qb of its tile; (sn, dn): block n + 1.  mem and alu: what else
+    // the slots hold, beside the LDS reads and beside the vector instructions.  The mask variant is compile-time: 0 none, 1 causal
+    // diagonal only (every query of the block exists), 2 diagonal and / or end of the queries.
+    auto step = [&](auto masked_c, f32x16& s, f32x16& d, f32x16& sn, f32x16& dn, int qb, int ib, auto mem, auto alu) {
+      constexpr int MASK = decltype(masked_c)::value;
+      // register r holds query ib + 4hh + c_r with c_r = 8(r/4) + r%4 a compile-time constant.
+      // masked iff key > query + q_start  <=>  c_r < key - q_start - ib - 4hh,   or query >= Sq
+      const int t = p.causal ? key - p.q_start - ib - 4 * hh : -1;
+      const int u = p.Sq - ib - 4 * hh;
+      u32x4 pw[2], dw[2];  // P and dS as operands, in halves of 16 queries
+      bf16x8 dT[MB][2], qT[MB][2];
+      auto v_exp = [&](int r) {
+        const int c = 8 * (r >> 2) + (r & 3);
+        if (MASK == 1 ? c < t : MASK == 2 && (c < t || c >= u)) s[r] = -INFINITY;
+        s[r] = fast_exp2(s[r]);
+      };
+      auto v_mul = [&](int r, int n) {
+        for (int i = r; i < r + n; ++i) d[i] *= s[i];
+      };
+      auto v_p = [&](int j, int n) {
+        for (int i = j; i < j + n; ++i) pw[i >> 2][i & 3] = pack_bf16x2(s[2 * i], s[2 * i + 1]);
+      };
+      auto v_ds = [&](int j, int n) {
+        for (int i = j; i < j + n; ++i) dw[i >> 2][i & 3] = pack_bf16x2(d[2 * i], d[2 * i + 1]);
+      };
+#pragma unroll
+      for (int i = 0; i < kA; ++i) {
+        const int o = order(i);
+        if (o < KS) mfma32_fixed(sn, qf[o], kreg[o]);
+        else mfma32_fixed(dn, df[o - KS], vreg[o - KS]);
+        const int half = i / (2 * MB), mb = (i % (2 * MB)) >> 1;
+        (i & 1 ? qT : dT)[mb][half] = frag_tr_at<D>(tra[2 * mb], tra[2 * mb + 1], 2 * qb + half, i & 1 ? 0 : Z::kTileBytes);
+        mem(i);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (D == 128) {
+          v_exp(i);
+          if (i >= 1 && i <= 8) v_mul(i - 1, 1);
+          if (i >= 9 && i <= 12) v_p(i - 9, 1);
+          if (i >= 13) v_ds(i - 13, i == 15 ? 2 : 1);
+        } else {
+          v_exp(2 * i);
+          v_exp(2 * i + 1);
+          if (i >= 1 && i <= 4) v_mul(2 * i - 2, 2);
+          if (i == 5 || i == 6) v_p(2 * i - 10, 2);
+          if (i == 7) v_ds(0, 4);
+        }
+        alu(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int j = 0; j < kB; ++j) {
+        const int half = j / (2 * MB), mb = (j % (2 * MB)) >> 1;
+        if (j & 1) mfma32_acc(dkacc[mb], qT[mb][half], as_bf16x8(dw[half]));
+        else mfma32_acc(dvacc[mb], dT[mb][half], as_bf16x8(pw[half]));
+        const int o = order(j);
+        (o < KS ? qf : df)[o % KS] = as_bf16x8(lds_read16(rma[o % KS] + (o < KS ? 0 : Z::kTileBytes) + qb * 32 * Z::kRB));
+        if (D == 128 && j >= 6 && j < 14) load_stat(s, d, st_next, qb, j - 6);
+        if (D == 64 && j >= 4) {
+          load_stat(s, d, st_next, qb, 2 * (j - 4));
+          load_stat(s, d, st_next, qb, 2 * (j - 4) + 1);
+        }
+        mem(kA + j);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (D == 128) {
+          if (j < 2) v_mul(8 + 3 * j, 3);
+          if (j == 2) { v_mul(14, 2); v_p(4, 1); }
+          if (j == 3) v_p(5, 3);
+          if (j == 4) v_ds(4, 3);
+          if (j == 5) v_ds(7, 1);
+        } else {
+          if (j < 2) v_mul(8 + 4 * j, 4);
+          if (j == 2) v_p(4, 4);
+          if (j == 3) v_ds(4, 4);
+        }
+        alu(kA + j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    auto tr_addr = [&](uint32_t tr, int x) { return tr ^ (uint32_t)(((x >> 1) << 6) ^ (x & 1 ? Z::kHiXor : 0)); };
+#pragma unroll
+    for (int x = 0; x < 2 * MB; ++x) tra[x] = tr_addr(tr_lane, x);
+    if (n_it > 0) {  // tiles 0 and 1 have landed (first wait above): block 0 up to its scores, the fragments of block 1
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          qf[ks] = swz_frag_rm<D>(rm_lane, qb, ks);
+          df[ks] = swz_frag_rm<D>(rm_lane + Z::kTileBytes, qb, ks);
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) load_stat(qb ? s1 : s0, qb ? d1 : d0, st_lane, qb, c);
+        if (qb == 0) {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            mfma32_fixed(s0, qf[ks], kreg[ks]);
+            mfma32_fixed(d0, df[ks], vreg[ks]);
+          }
+          mfma32_fixed_done(s0);
+          mfma32_fixed_done(d0);
+        }
+      }
+    }
+    // the tile requested in an iteration: its rows' lane offsets, cut off at the last query, and where the stream goes on
+    const int q_row = src.x * D * 2, d_row = src.x * (int)dstep;
+    const int64_t q_wrap = -((rep - 1) * q_head + kBK * D * 2), d_wrap = -((rep - 1) * d_head + (int64_t)kBK * dstep);
+    const int s_wrap = -((rep - 1) * p.Sq + kBK);
+    constexpr int kLoads = 2 * Z::kPasses;
+    // slots of the second halves that hold load k (first step: k < kFirst) and, one slot before, its offset
+    constexpr int kFirst = D == 128 ? 5 : 3, kAt0 = D == 128 ? 7 : 4, kAt1 = D == 128 ? 6 : 4, kEvery = D == 128 ? 2 : 1;
+    constexpr int kStatAt = D == 128 ? 11 : 5, kMoveAt = D == 128 ? 12 : 5;
+    auto slot_load = [](int j, int first, int n) { return j >= first && (j - first) % kEvery == 0 && (j - first) / kEvery < n ? (j - first) / kEvery : -1; };
+    int stage = 0, it = 0;
+    iss_stage = R.startup_tiles;  // also where there are fewer tiles than that
+    auto run_tiles = [&](auto masked_c, int t_lo, int t_hi) {
+      for (int x = (t_hi - t_lo) * rep, t = t_hi - 1, hq = 0; x > 0; --x, ++it) {
+        const int nstage = stage == kStages - 1 ? 0 : stage + 1;
+        const int i0 = (qt_start + t) * kBK;
+        uint32_t off = 0, tr_next = 0, tra_next[2 * MB];
+        bool more = false, wrap = false;
+        int64_t q_step = 0, d_step = 0;
+        int s_step = 0, left_step = 0;
+        auto offset = [&](int k) {  // rows past the last query re-read it
+          const int lim = min(left_it, kBK) - 1, row = (k >> 1) * 4 * Z::kRowsPerInst;
+          if (k & 1) off = min(d_row, (lim - row) * (int)dstep) + src.y + row * (int)dstep;
+          else off = min(q_row, (lim - row) * D * 2) + src.y + row * D * 2;
+        };
+        auto load = [&](int k) {
+          const uint32_t dst = lds0 + iss_stage * kStageBytes + wave * 1024 + (k >> 1) * 4096;
+          if (k & 1) gload_lds16_so(d_it, off, dst + Z::kTileBytes);
+          else gload_lds16_so(q_it, off, dst);
+        };
+        step(masked_c, s0, d0, s1, d1, 0, i0,
+             [&](int slot) {
+               const int j = slot - kA;
+               if (slot_load(j, kAt0, kFirst) >= 0) load(slot_load(j, kAt0, kFirst));
+               if (j == 0) {
+                 more = it + R.issue_ahead + 1 < n_it;  // else the last tile is requested once more
+                 wrap = iss_h + 1 == rep;
+                 iss_h = !more ? iss_h : wrap ? 0 : iss_h + 1;
+               }
+               if (j == 1) q_step = more ? (wrap ? q_wrap : q_head) : 0;
+               if (j == 2) d_step = more ? (wrap ? d_wrap : d_head) : 0;
+               if (j == 3) { s_step = more ? (wrap ? s_wrap : p.Sq) : 0; left_step = more && wrap ? kBK : 0; }
+             },
+             [&](int slot) {
+               const int j = slot - kA;
+               if (slot == 0) rm_next = rm_lane + nstage * kStageBytes;
+               // k-step ks is read in slot 0, 1, 2 (head_dim 128) or 2 ks - 2
+#pragma unroll
+               for (int ks = 0; ks < KS; ++ks)
+                 if (D == 64 || ks < 2 ? slot == 0 : j == (ks == 2 ? 0 : 2 * ks - 4)) rma[ks] = rm_next ^ (uint32_t)(ks << 5);
+               if (j == (D == 128 ? 5 : 3)) st_next = st_lane + nstage * 512;
+               if (slot_load(j + 1, kAt0, kFirst) >= 0) offset(slot_load(j + 1, kAt0, kFirst));
+             });
+        step(masked_c, s1, d1, s0, d0, 1, i0 + 32,
+             [&](int slot) {
+               const int j = slot - kA, k = slot_load(j, kAt1, kLoads - kFirst);
+               if (k >= 0) load(kFirst + k);
+               if (j == kStatAt) gload_lds4_so(s_it, off, ldl0 + (iss_stage * 128 + (wave & 1) * 64) * 4);
+               if (j == kMoveAt) q_it += q_step;
+               if (j == kMoveAt + 1) d_it += d_step;
+               if (j == kMoveAt + 2) { s_it += s_step; left_it += left_step; }
+             },
+             [&](int slot) {
+               const int j = slot - kA, k = slot_load(j + 1, kAt1, kLoads - kFirst), x2 = j - (kB / 2 - 2);
+               if (j == kB / 2 - 3) tr_next = tr_lane + nstage * kStageBytes;
+               if (x2 >= 0 && x2 < 2 * MB) tra_next[x2] = tr_addr(tr_next, x2);
+               if (k >= 0) offset(kFirst + k);
+               if (j == kStatAt - 1) off = (uint32_t)min(lane, left_it - 1) * 4;
+             });
+        iss_stage = iss_stage == kStages - 1 ? 0 : iss_stage + 1;
+        wait_vmcnt<ring::loads_kept_after_iteration(R, true)>();
+        // a bare barrier: the reads of this tile have returned (the products above used them), and those of the next tile's
+        // first fragments, still on their way, come from a stage that the next iteration does not refill either
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        stage = nstage;
+#pragma unroll
+        for (int i = 0; i < 2 * MB; ++i) tra[i] = tra_next[i];
+        if (++hq == rep) { hq = 0; --t; }
+      }
+    };
+    run_tiles(IC<2>{}, t_end, n_vis);
+    run_tiles(IC<0>{}, t_diag, t_end);
+    run_tiles(IC<2>{}, min(t_diag, t_full), t_diag);
+    run_tiles(IC<1>{}, 0, min(t_diag, t_full));
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) { mfma32_acc_done(dvacc[mb]); mfma32_acc_done(dkacc[mb]); }
+    static_assert(R.always_requests, "no branch around the loads of an iteration");
+    wait_vmcnt<0>();  // the last tile, requested once more, has left the stages that the epilogue uses
+    __syncthreads();
+  } else {
+    auto request_rowmajor = [&](uint32_t rm, int qb) {  // qb is a compile-time constant at every call site
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        qf[ks] = swz_frag_rm<D>(rm, qb, ks);
+        df[ks] = swz_frag_rm<D>(rm + Z::kTileBytes, qb, ks);
+      }
+    };
+    // one 32-query block (qb = 0/1, compile-time) of the tile whose stage the pointers address;
+    // ib = first query of the block; the row-major fragments of the block after it start at next_rm.
+    // The mask variant is compile-time so that a whole block is one straight-line scheduling region:
+    // 0 none, 1 causal diagonal only (every query of the block exists), 2 diagonal and / or end of the queries.
+    auto step = [&](auto masked_c, uint32_t tr, uint32_t st, int qb, int ib, uint32_t next_rm, int next_qb) {
+      constexpr int MASK = decltype(masked_c)::value;
+      // head_dim 128 (one wave per SIMD, nothing else to hide the exp2 phase behind): the compiler's interleaving
+      // strategy for exp2 work between MFMA chains, measured -3 % on this kernel; at head_dim 64 it changes nothing
+      if constexpr (D == 128) __builtin_amdgcn_iglp_opt(3);
+      // accumulators of S and dP start from -lse2 / -delta of the 16 query rows their registers map to
+      f32x16 s, dpv;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const f32x4 l4 = lds_read_f4(st + (32 * qb + 8 * c) * 4);
+        const f32x4 d4 = lds_read_f4(st + (64 + 32 * qb + 8 * c) * 4);
+        s[4 * c] = l4[0]; s[4 * c + 1] = l4[1]; s[4 * c + 2] = l4[2]; s[4 * c + 3] = l4[3];
+        dpv[4 * c] = d4[0]; dpv[4 * c + 1] = d4[1]; dpv[4 * c + 2] = d4[2]; dpv[4 * c + 3] = d4[3];
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) s = mfma32(qf[ks], kreg[ks], s);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) dpv = mfma32(df[ks], vreg[ks], dpv);
+      bf16x8 dT[MB][2], qT[MB][2];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        dT[mb][0] = swz_frag_tr<D>(tr + Z::kTileBytes, mb, 2 * qb);
+        qT[mb][0] = swz_frag_tr<D>(tr, mb, 2 * qb);
+        dT[mb][1] = swz_frag_tr<D>(tr + Z::kTileBytes, mb, 2 * qb + 1);
+        qT[mb][1] = swz_frag_tr<D>(tr, mb, 2 * qb + 1);
+      }
+      if (MASK != 0) {  // block touches the diagonal or the end of the queries
+        // register r holds query ib + 4hh + c_r with c_r = 8(r/4) + r%4 a compile-time constant.
+        // masked iff key > query + q_start  <=>  c_r < key - q_start - ib - 4hh,   or query >= Sq
+        const int t = p.causal ? key - p.q_start - ib - 4 * hh : -1;
+        const int u = p.Sq - ib - 4 * hh;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int c = 8 * (r >> 2) + (r & 3);
+          if (MASK == 1 ? c < t : (c < t || c >= u)) s[r] = -INFINITY;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[r] = fast_exp2(s[r]);
+        dpv[r] *= s[r];
+      }
+      const bf16x8 p0 = pack_c_half(s, 0), p1 = pack_c_half(s, 1);
+      const bf16x8 ds0 = pack_c_half(dpv, 0), ds1 = pack_c_half(dpv, 1);
+      request_rowmajor(next_rm, next_qb);  // unconditional: past the last block the fragments are simply unused
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        dvacc[mb] = mfma32(dT[mb][0], p0, dvacc[mb]);
+        dkacc[mb] = mfma32(qT[mb][0], ds0, dkacc[mb]);
+      }
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        dvacc[mb] = mfma32(dT[mb][1], p1, dvacc[mb]);
+        dkacc[mb] = mfma32(qT[mb][1], ds1, dkacc[mb]);
+      }
+    };
+
+    // ---- pipeline start-up: tiles 0 and 1 have landed (first wait above), tile 2 is in flight
+    if (n_it > 0) request_rowmajor(rm_lane, 0);
+    int stage = 0, it = 0;
+    auto run_tiles = [&](auto masked_c, int t_lo, int t_hi) {
+      constexpr int MASK = decltype(masked_c)::value;
+      for (int t = t_lo; t < t_hi; ++t, ++it) {
+        const int nstage = stage == kStages - 1 ? 0 : stage + 1;
+        const int i0 = (qt_start + t) * kBK;
+        const uint32_t tr = tr_lane + stage * kStageBytes;
+        const uint32_t st = st_lane + stage * 512;
+        // on the diagonal a block whose last query still lies before this wave's first key is masked entirely:
+        // it only passes the fragment request on (wave-uniform, so the barrier below is reached all the same)
         const int ib = i0 + 32 * part;
         if (MASK == 1 && kw0 > ib + 31 + p.q_start) request_rowmajor(rm_lane + nstage * kStageBytes, 0);
         else step(masked_c, tr, st, 0, ib, rm_lane + nstage * kStageBytes, 0);
+        if (it + R.issue_ahead < n_it) { issue_next(); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
+        __syncthreads();
+        stage = nstage;
       }
-      if (it + R.issue_ahead < n_it) { issue_next(); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
-      __syncthreads();
-      stage = nstage;
+    };
+    for (int hq = 0; hq < rep; ++hq) {
+      run_tiles(IC<1>{}, 0, min(t_diag, t_full));
+      run_tiles(IC<2>{}, min(t_diag, t_full), t_diag);
+      run_tiles(IC<0>{}, t_diag, t_end);
+      run_tiles(IC<2>{}, t_end, n_vis);
     }
-  };
-  for (int hq = 0; hq < rep; ++hq) {
-    run_tiles(IC<1>{}, 0, min(t_diag, t_full));
-    run_tiles(IC<2>{}, min(t_diag, t_full), t_diag);
-    run_tiles(IC<0>{}, t_diag, t_end);
-    run_tiles(IC<2>{}, t_end, n_vis);
   }
 
   // ---- epilogue: lane = key row, registers = head-dim entries.  The rows it reads (the raw key for the normaliser's

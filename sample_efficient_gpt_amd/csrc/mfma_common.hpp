@@ -29,6 +29,20 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// The same instruction with its register files chosen by hand, for loops laid out instruction by instruction: a sum over
+// the whole loop in accumulation registers (_acc), or a short-lived result in ordinary ones with the stationary operand
+// in accumulation registers (_fixed).  The compiler sees neither as a matrix instruction: what it inserts around those
+// (two wait states behind a vector instruction that wrote an operand, twelve before one that reads the result) the caller's
+// order has to provide, and behind the last one the _done form does.
+__device__ __forceinline__ void mfma32_acc(f32x16& acc, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma32_fixed(f32x16& acc, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
+}
+__device__ __forceinline__ void mfma32_fixed_done(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc)); }
+__device__ __forceinline__ void mfma32_acc_done(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc)); }
+
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 // value held by lane l^32 combined with the own value
@@ -182,6 +196,17 @@ __device__ __forceinline__ bf16x8 swz_frag_tr(uint32_t tile_plus_lane_off, int c
   typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
   s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p));
   s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(q));
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8, v);
+}
+
+// the transposed fragment of row step s from the two addresses of its column block (those of row step 0, without `tile`)
+template <int D>
+__device__ __forceinline__ bf16x8 frag_tr_at(uint32_t p, uint32_t q, int s, int tile) {
+  typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
+  s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p + tile + 16 * s * Swz<D>::kRB));
+  s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(q + tile + (16 * s + 8) * Swz<D>::kRB));
   typedef short s16x8 __attribute__((ext_vector_type(8)));
   s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   return __builtin_bit_cast(bf16x8, v);

@@ -39,6 +39,9 @@ struct Protocol {
   int merge_stage_first = 0;  // two waves share the rows of a block: behind the loop they hand accumulators over through
   int merge_stages = 0;       // stages [merge_stage_first, merge_stage_first + merge_stages): plain stores beside the row
                               // requests above, read behind the same barrier
+  bool always_requests = false;  // every iteration requests a tile, past the end the last one once more (never read), so that
+                              // one wait fits all of them and no load sits behind a branch; a wait for everything and a
+                              // barrier follow the loop
   int scratch_stages = 0;     // with epilogue_reuses_ring: how many stages from 0 on the scratch data takes (0: all)
 };
 
@@ -53,7 +56,7 @@ constexpr int loads_kept_before_loop(const Protocol& p, int n_tiles) {
 }
 // vmcnt immediate of the wait that ends an iteration
 constexpr int loads_kept_after_iteration(const Protocol& p, bool requested_a_tile) {
-  return requested_a_tile ? p.keep_tiles * p.loads_per_tile : 0;
+  return requested_a_tile || p.always_requests ? p.keep_tiles * p.loads_per_tile : 0;
 }
 
 // ---- the kernels' protocols.  passes = wave-wide 16-byte loads per wave and [64, D] tile (2 at both head dims).
@@ -73,7 +76,11 @@ constexpr Protocol dq_rope(int passes) { return Protocol{4, 2 * passes, 3, 3, 1,
 // dK/dV: (Qhat, dO) tiles 0 and 1 in stages 0 and 1 with the Khat / V' row blocks in stages 2 and 3, then tile 2;
 // a tile is the two [64, D] tiles plus one row-statistics load.
 // Behind the loop: the raw k block (and, with a value residual, the raw v and v_first blocks) for the epilogue.
-constexpr Protocol dkdv(int passes) { return Protocol{4, 2 * passes + 1, 2, 2, 2, 3, false, false, 3, 1, 0, 3, false}; }
+constexpr Protocol dkdv(int passes, bool always_requests = true) {
+  Protocol p{4, 2 * passes + 1, 2, 2, 2, 3, false, false, 3, 1, 0, 3, false};
+  p.always_requests = always_requests;
+  return p;
+}
 
 // The same kernels in 64-row workgroups whose waves split the blocks of a tile.  The forward uses the ring behind its loop for the
 // hand-over alone; dQ leaves stages 2 and 3 to it and its scratch data to 0 and 1 (no barrier between reading
@@ -88,7 +95,7 @@ constexpr Protocol merging(Protocol p, int first, int stages, int scratch_stages
 constexpr Protocol forward_parts(int stages, int q_stages, int passes) { return merging(forward(stages, q_stages, passes), 0, 2); }
 constexpr Protocol dq_parts(int passes) { return merging(dq(passes), 2, 2, 2); }
 constexpr Protocol dq_rope_parts(int passes) { return merging(dq_rope(passes), 2, 2, 2, 1); }
-constexpr Protocol dkdv_parts(int passes) { return merging(dkdv(passes), 2, 2, 0, 2); }
+constexpr Protocol dkdv_parts(int passes) { return merging(dkdv(passes, false), 2, 2, 0, 2); }
 
 constexpr bool well_formed(const Protocol& p) {
   return p.stages >= 3 && p.early_tiles >= 1 && p.early_tiles <= p.startup_tiles && p.startup_tiles <= p.stages - 1 &&

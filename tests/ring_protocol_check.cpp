@@ -69,12 +69,16 @@ std::vector<Op> wave_program(const Protocol& p, int n_tiles, int row_loads_per_s
   }
   if (n_tiles > 0) ops.push_back({READ, 0, 0, 0});  // row-major fragments of the first block
   for (int jt = 0; jt < n_tiles; ++jt) {
-    const bool requested = jt + p.issue_ahead < n_tiles;
+    const bool requested = p.always_requests || jt + p.issue_ahead < n_tiles;  // past the end: a tile nobody reads
     if (p.issue_at_top && requested) request_tile(jt + p.issue_ahead);
     ops.push_back({READ, jt % p.stages, jt, 0});                                      // both blocks, both orientations
     if (jt + 1 < n_tiles) ops.push_back({READ, (jt + 1) % p.stages, jt + 1, 0});      // next tile's first fragments
     if (!p.issue_at_top && requested) request_tile(jt + p.issue_ahead);
     ops.push_back({WAIT, 0, 0, segpt::ring::loads_kept_after_iteration(p, requested)});
+    ops.push_back({BARRIER, 0, 0, 0});
+  }
+  if (p.always_requests) {
+    ops.push_back({WAIT, 0, 0, 0});
     ops.push_back({BARRIER, 0, 0, 0});
   }
   const int slots_end = p.merge_stage_first + p.merge_stages;

@@ -478,6 +478,25 @@ def test_bf16_dkdv_workgroup_shapes(gpu_device, B, H, Hkv, Sq, Sk, D, kw):
     _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, D, seed=61, gen_kw={"extras": True}, rope=orc.rope_tables(max(Sq, Sk), 10000.0, D), **kw)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,kw", [
+    (4, 66, 66, 33, 40, {"q_start": 7}),        # one streamed tile, requested over and over; its second block has one query
+    (4, 66, 66, 70, 100, {"causal": False}),    # two, the last of six rows
+    (3, 174, 87, 64, 64, {}),                   # two heads, one tile each, nothing but diagonal
+    (2, 198, 66, 97, 300, {}),                  # six; the later key tiles see one query or none
+    (3, 90, 90, 200, 140, {"causal": False}),   # four, and a last key tile of 12 rows
+])
+def test_bf16_dkdv_pipeline_ends(gpu_device, B, H, Hkv, Sq, Sk, D, kw):
+    """dK/dV of launches that fill the card (128-key workgroups), whose pipeline runs two blocks ahead of itself and requests
+    a tile in every iteration, at the shortest streams and at ragged ends.
+    Outliers: a launch that fills the card has millions of entries, and dk of a row that few queries see is a sum of few terms
+    with roundings of 2^-9 each against a result that cancels; over the 198-head case dk is 3.7e-3 from float64 in norm and
+    one entry of 2.5 million is 0.043 away where the elementwise bound says 0.04 (both to all digits also with the products
+    in the order of tiles, head by head).  One in a million may be up to twice the bound away."""
+    assert B * Hkv * (-(-Sk // 128)) > 256
+    _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, D, seed=63, outliers=(1e-6, 2.0), rope=orc.rope_tables(max(Sq, Sk), 10000.0, D), **kw)
+
+
 @pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,kw,gen_kw,use_rope", [
     (1, 2, 1, 65, 65, 64, {}, {"extras": True}, True),                         # one row in the last workgroup, its second wave beyond the end
     (1, 2, 2, 31, 130, 64, {"q_start": 99}, {"extras": True}, False),          # fewer rows than one wave owns
