@@ -95,7 +95,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   constexpr int MB = D / 32;
   constexpr int kStageBytes = 2 * Z::kTileBytes;
   // the pipeline's numbers: ring_protocol.hpp
-  constexpr ring::Protocol R = PARTS == 1 ? (ROPE ? ring::dq_rope(Z::kPasses) : ring::dq(Z::kPasses))
+  constexpr bool PIPE = D == 128 && PARTS == 1;
+  constexpr ring::Protocol R = PARTS == 1 ? (ROPE ? ring::dq_rope(Z::kPasses, PIPE) : ring::dq(Z::kPasses, PIPE))
                                           : (ROPE ? ring::dq_rope_parts(Z::kPasses) : ring::dq_parts(Z::kPasses));
   static_assert(ring::well_formed(R) && R.stages == kStages && !R.issue_at_top, "tile pipeline");
   static_assert(ROPE ? (R.pre_row_stages == 4 && R.row_stages == 1 && R.early_tiles == R.startup_tiles && !R.wait_before_loop && R.epilogue_row_stages == (PARTS == 1 ? 2 : 1))
@@ -322,60 +323,6 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
   const uint32_t rm_lane = lds0 + swz_off_rm<D>(lane) + part * 32 * Z::kRB;
   const uint32_t tr_lane = lds0 + swz_off_tr<D>(lane) + part * 32 * Z::kRB;
   bf16x8 kf[KS], vf[KS];
-  auto request_rowmajor = [&](uint32_t rm, int kb) {  // kb compile-time at every call site
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      kf[ks] = swz_frag_rm<D>(rm, kb, ks);
-      vf[ks] = swz_frag_rm<D>(rm + Z::kTileBytes, kb, ks);
-    }
-  };
-  // one 32-key block: tr = lane address inside the block's stage; `more`: a block follows, its row-major
-  // fragments start at next_rm
-  // MASKED is compile-time so that a whole block is one straight-line scheduling region
-  auto step = [&](auto masked_c, uint32_t tr, int kb, int jb, uint32_t next_rm, int next_kb) {
-    constexpr bool MASKED = decltype(masked_c)::value != 0;
-    // head_dim 128 runs one wave per SIMD with all 256 ordinary registers in use: left to itself the compiler requests
-    // each LDS fragment one MFMA ahead of its use and the wave stalls on LDS latency before most MFMAs.  Asking for
-    // the block as 24 groups of (1 MFMA, 2 LDS reads, 2 vector instructions) keeps two requests ahead: -6 % on this
-    // kernel (neighbouring group shapes are 2-10 % slower; at head_dim 64, two waves per SIMD, none changes anything).
-    if constexpr (D == 128) {
-#pragma unroll
-      for (int i = 0; i < 3 * KS; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // LDS read
-        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-      }
-    }
-    f32x16 s = c_lse, dpv = c_del;
-    // the S chain first, then the dP chain: exp2 of the finished scores runs behind the dP MFMAs
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) s = mfma32(kf[ks], qreg[ks], s);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) dpv = mfma32(vf[ks], doreg[ks], dpv);
-    bf16x8 kT[MB][2];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      kT[mb][0] = swz_frag_tr<D>(tr, mb, 2 * kb);
-      kT[mb][1] = swz_frag_tr<D>(tr, mb, 2 * kb + 1);
-    }
-    if (MASKED) {  // block touches the diagonal or the end of the keys
-      // register r holds key jb + 4hh + c_r, c_r = 8(r/4) + r%4: masked iff c_r > qlim - jb - 4hh
-      const int t = qlim - jb - 4 * hh;
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (8 * (r >> 2) + (r & 3) > t) s[r] = -INFINITY;
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r]) * dpv[r];
-    const bf16x8 ds0 = pack_c_half(s, 0), ds1 = pack_c_half(s, 1);
-    request_rowmajor(next_rm, next_kb);  // unconditional: past the last block the fragments are simply unused
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      acc[mb] = mfma32(kT[mb][0], ds0, acc[mb]);
-      acc[mb] = mfma32(kT[mb][1], ds1, acc[mb]);
-    }
-  };
-
   // ---- pipeline start-up.  Every iteration of the loop starts with its own tile AND the next one landed (the
   // second block of a tile already requests the next tile's fragments) and at most one more in flight, so tile 1,
   // requested after the row blocks had left its stage, must be complete here; the row prologue above ran in
@@ -384,41 +331,253 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     if (n_kt >= R.startup_tiles) wait_vmcnt<ring::loads_kept_before_loop(R, R.startup_tiles)>(); else wait_vmcnt<0>();
     __syncthreads();
   }
-  if (n_act > 0) request_rowmajor(rm_lane, 0);
   // leading blocks of this wave that need no mask (every key visible to every query of the wave, inside Sk)
   int n_full = p.Sk / 32;
   if (p.causal) n_full = min(n_full, (qw0 + p.q_start + 1) / 32);
   // Loop A: tiles whose two blocks need no mask; loop B: the rest (masking a fully visible block is a no-op).
   // Two loops, so that each body holds one variant of the block and the accumulators never meet at a join.
   const int n_a = PARTS == 1 ? n_full / 2 : (n_full + 1 - part) / 2;  // n_full <= n_act
-  int stage = 0, jt = 0;
-  for (; jt < n_a; ++jt) {
-    const int nstage = stage == kStages - 1 ? 0 : stage + 1;
-    const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
-    if constexpr (PARTS == 1) {
-      step(IC<0>{}, tr, 0, 64 * jt, rm, 1);
-      step(IC<0>{}, tr, 1, 64 * jt + 32, rm_lane + nstage * kStageBytes, 0);
-    } else {
-      step(IC<0>{}, tr, 0, 64 * jt + 32 * part, rm_lane + nstage * kStageBytes, 0);
+  if constexpr (PIPE) {
+    // The pipeline of the dK/dV kernel below (there: what a slot holds, and why): step n computes S^T and dP^T of block n + 1
+    // (kA matrix instructions) while the vector unit turns those of block n into dS^T, then adds block n to T^T (kB);
+    // the row-major fragments of block n + 2 come in as those of block n + 1 are used.
+    // Head_dim 128 only.  dQ, 4 x 16 / 4 heads, 4096 tokens: 437 -> 398 us (937 k -> 768 k cycles, matrix pipe 42 -> 52 % busy; a
+    // quarter of the launch is now the workgroups' first and last thousands of cycles, one workgroup a CU).  At head_dim 64 the
+    // second set of scores does not fit two workgroups per CU: 256 registers split in halves spill 95 of them.
+    constexpr int kA = 2 * KS, kB = 2 * MB;
+    auto order = [](int i) { return (i & 1) * KS + (i >> 1); };  // i-th product: k-step of S^T, or KS + that of dP^T
+    f32x16 s0, d0, s1, d1;           // scores and dP of two consecutive blocks
+    uint32_t rma[KS], tra[2 * MB];   // addresses: the next tile's row-major fragments, this tile's transposed ones
+    auto start = [&](f32x16& s, f32x16& d, int i) {  // the i-th product of a block
+      const int o = order(i), ks = o % KS;
+      if (o >= KS) ks == 0 ? mfma32_fixed_from(d, vf[ks], doreg[ks], c_del) : mfma32_fixed(d, vf[ks], doreg[ks]);
+      else ks == 0 ? mfma32_fixed_from(s, kf[ks], qreg[ks], c_lse) : mfma32_fixed(s, kf[ks], qreg[ks]);
+    };
+    auto row_frag = [&](uint32_t rm_ks, int kb, int o) { (o < KS ? kf : vf)[o % KS] = as_bf16x8(lds_read16(rm_ks + (o < KS ? 0 : Z::kTileBytes) + kb * 32 * Z::kRB)); };
+    // (s, d): block n, whose first key is jb, number kb of its tile; (sn, dn): block n + 1.  mem and alu: what else the slots
+    // hold, beside the LDS reads and beside the vector instructions
+    auto step = [&](auto masked_c, f32x16& s, f32x16& d, f32x16& sn, f32x16& dn, int kb, int jb, auto mem, auto alu) {
+      constexpr bool MASKED = decltype(masked_c)::value != 0;
+      // register r holds key jb + 4hh + c_r, c_r = 8(r/4) + r%4: masked iff c_r > qlim - jb - 4hh
+      const int t = qlim - jb - 4 * hh;
+      u32x4 dw[2];  // dS as operand, in halves of 16 keys
+      bf16x8 kT[MB][2];
+      auto v_exp = [&](int r) {
+        if (MASKED && 8 * (r >> 2) + (r & 3) > t) s[r] = -INFINITY;
+        s[r] = fast_exp2(s[r]);
+      };
+      auto v_mul = [&](int r) { s[r] *= d[r]; };
+      auto v_ds = [&](int j) { dw[j >> 2][j & 3] = pack_bf16x2(s[2 * j], s[2 * j + 1]); };
+      constexpr int kExps = 16 / kA;  // per slot
+#pragma unroll
+      for (int i = 0; i < kA; ++i) {
+        start(sn, dn, i);
+        // even slots: a transposed fragment of block n; odd ones: a row-major fragment of block n + 2, whose place is free
+        if (i & 1) row_frag(rma[order(i >> 1) % KS], kb, order(i >> 1));
+        else kT[(i >> 1) % MB][(i >> 1) / MB] = frag_tr_at<D>(tra[2 * ((i >> 1) % MB)], tra[2 * ((i >> 1) % MB) + 1], 2 * kb + (i >> 1) / MB, 0);
+        mem(i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < kExps; ++e) {
+          const int r = kExps * i + e;
+          v_exp(r);
+          if (r >= kExps) v_mul(r - kExps);
+          if (r >= kExps + 2 && (r - kExps) % 2 == 0) v_ds((r - kExps) / 2 - 1);
+        }
+        if (i == kA - 1) {
+#pragma unroll
+          for (int r = 16 - kExps; r < 16; ++r) v_mul(r);
+#pragma unroll
+          for (int j = 8 - kExps; j < 8; ++j) v_ds(j);
+        }
+        alu(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int j = 0; j < kB; ++j) {
+        mfma32_acc(acc[j % MB], kT[j % MB][j / MB], as_bf16x8(dw[j / MB]));
+        row_frag(rma[order(kA / 2 + j) % KS], kb, order(kA / 2 + j));
+        mem(kA + j);
+        __builtin_amdgcn_sched_barrier(0);
+        alu(kA + j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    static_assert(kB == kA / 2, "one row-major fragment per slot of the second half, the others in the odd ones of the first");
+    auto rm_addr = [&](uint32_t rm, int ks) { return rm ^ (uint32_t)(ks << 5); };
+    auto tr_addr = [&](uint32_t tr, int x) { return tr ^ (uint32_t)(((x >> 1) << 6) ^ (x & 1 ? Z::kHiXor : 0)); };
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) rma[ks] = rm_addr(rm_lane + kStageBytes, ks);
+#pragma unroll
+    for (int x = 0; x < 2 * MB; ++x) tra[x] = tr_addr(tr_lane, x);
+    // block 0 up to its scores, the fragments of block 1 (tiles 0 and 1 have landed)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) { mfma32_settle(qreg[ks]); mfma32_settle(doreg[ks]); }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) { row_frag(rm_addr(rm_lane, ks), 0, ks); row_frag(rm_addr(rm_lane, ks), 0, KS + ks); }
+#pragma unroll
+    for (int i = 0; i < kA; ++i) start(s0, d0, i);
+    mfma32_fixed_done(s0);
+    mfma32_fixed_done(d0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) { row_frag(rm_addr(rm_lane, ks), 1, ks); row_frag(rm_addr(rm_lane, ks), 1, KS + ks); }
+    // the tile requested in an iteration (past the last one that one again)
+    int req = min(R.startup_tiles, n_kt - 1);
+    const char* k_it = kbase + (int64_t)req * kBK * kstep;
+    const char* v_it = vbase + (int64_t)req * kBK * vstep;
+    TileLaneOff<D> lane_off = tile_lane_offsets<D>(kstep, vstep, min(p.Sk - req * kBK, kBK), src.x, src.y);
+    int stage = 0, jt = 0;
+    uint32_t req_dst = wave_dst + R.startup_tiles * kStageBytes;
+    // loads of the first and second half of a tile, in the second halves of its two steps: every kEvery slots
+    constexpr int kLoads = 2 * Z::kPasses, kEvery = 2 * kB / kLoads, kPerStep = kLoads / 2;
+    auto load = [&](int k) { issue_tile_load<D>(k, k_it, v_it, lane_off, req_dst); };
+    auto request = [&](int first) {  // outside the steps
+#pragma unroll
+      for (int k = 0; k < kPerStep; ++k) load(first + k);
+    };
+    auto end_tile = [&]() {
+      wait_vmcnt<ring::loads_kept_after_iteration(R, true)>();
+      // a bare barrier: every read of this tile has returned (the products used it), and the next tile's fragments that
+      // are still on their way come from a stage that the next iteration does not refill either
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      stage = stage == kStages - 1 ? 0 : stage + 1;
+      req_dst += kStageBytes;
+      if (req_dst >= lds0 + kStages * kStageBytes) req_dst -= kStages * kStageBytes;
+      if (req + 1 < n_kt) {
+        ++req;
+        k_it += kBK * kstep;
+        v_it += (int64_t)kBK * vstep;
+        if (p.Sk - req * kBK < kBK) lane_off = tile_lane_offsets<D>(kstep, vstep, p.Sk - req * kBK, src.x, src.y);
+      }
+    };
+    auto first_step = [&](auto masked_c) {
+      step(masked_c, s0, d0, s1, d1, 0, kBK * jt,
+           [&](int slot) { const int j = slot - kA; if (j >= 0 && j % kEvery == kEvery - 1) load(j / kEvery); }, [](int) {});
+    };
+    auto second_step = [&](auto masked_c) {
+      uint32_t rm_next = 0, tr_next = 0;
+      step(masked_c, s1, d1, s0, d0, 1, kBK * jt + 32,
+           [&](int slot) { const int j = slot - kA; if (j >= 0 && j % kEvery == kEvery - 1) load(kPerStep + j / kEvery); },
+           [&](int slot) {  // the next iteration's addresses, each behind its last use in this one
+             const int j = slot - kA;
+             if (j == 0) {
+               tr_next = tr_lane + (stage == kStages - 1 ? 0 : stage + 1) * kStageBytes;
+               rm_next = rm_lane + (stage >= kStages - 2 ? stage + 2 - kStages : stage + 2) * kStageBytes;
+             }
+             if (j >= 0) tra[j] = tr_addr(tr_next, j);
+#pragma unroll
+             for (int ks = 0; ks < KS; ++ks)
+               if (j == (ks < KS / 2 ? ks + 1 : ks < KS - 2 ? KS - 3 : ks)) rma[ks] = rm_addr(rm_next, ks);
+           });
+    };
+    for (; jt < n_a; ++jt) {
+      first_step(IC<0>{});
+      second_step(IC<0>{});
+      end_tile();
     }
-    // stage (jt+3) % 4 == (jt-1) % 4 was last read in the previous iteration: refill it, then make sure
-    // this wave's part of tile jt+2 (needed from the next iteration's prefetch on) has landed
-    if (jt + R.issue_ahead < n_kt) { issue_tile(jt + R.issue_ahead); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
-    __syncthreads();
-    stage = nstage;
-  }
-  for (; jt < n_kt; ++jt) {
-    const int nstage = stage == kStages - 1 ? 0 : stage + 1;
-    const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
-    if constexpr (PARTS == 1) {
-      if (2 * jt < n_act) step(IC<1>{}, tr, 0, 64 * jt, rm, 1);
-      if (2 * jt + 1 < n_act) step(IC<1>{}, tr, 1, 64 * jt + 32, rm_lane + nstage * kStageBytes, 0);
-    } else {
-      if (2 * jt + part < n_act) step(IC<1>{}, tr, 0, 64 * jt + 32 * part, rm_lane + nstage * kStageBytes, 0);
+    for (; 2 * jt + 1 < n_act; ++jt) {
+      first_step(IC<1>{});
+      second_step(IC<1>{});
+      end_tile();
     }
-    if (jt + R.issue_ahead < n_kt) { issue_tile(jt + R.issue_ahead); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
+    for (; jt < n_kt; ++jt) {  // tiles of which this wave needs one block, then none
+      if (2 * jt < n_act) first_step(IC<1>{});
+      else request(0);
+      request(kPerStep);
+      end_tile();
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) mfma32_acc_done(acc[mb]);
+    static_assert(R.always_requests, "no branch around the loads of an iteration");
+    wait_vmcnt<0>();  // the last tile, requested once more, has left the stages that the epilogue uses
     __syncthreads();
-    stage = nstage;
+  } else {
+    auto request_rowmajor = [&](uint32_t rm, int kb) {  // kb compile-time at every call site
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        kf[ks] = swz_frag_rm<D>(rm, kb, ks);
+        vf[ks] = swz_frag_rm<D>(rm + Z::kTileBytes, kb, ks);
+      }
+    };
+    // one 32-key block: tr = lane address inside the block's stage; `more`: a block follows, its row-major
+    // fragments start at next_rm
+    // MASKED is compile-time so that a whole block is one straight-line scheduling region
+    auto step = [&](auto masked_c, uint32_t tr, int kb, int jb, uint32_t next_rm, int next_kb) {
+      constexpr bool MASKED = decltype(masked_c)::value != 0;
+      // head_dim 128 runs one wave per SIMD with all 256 ordinary registers in use: left to itself the compiler requests
+      // each LDS fragment one MFMA ahead of its use and the wave stalls on LDS latency before most MFMAs.  Asking for
+      // the block as 24 groups of (1 MFMA, 2 LDS reads, 2 vector instructions) keeps two requests ahead: -6 % on this
+      // kernel (neighbouring group shapes are 2-10 % slower; at head_dim 64, two waves per SIMD, none changes anything).
+      if constexpr (D == 128) {
+#pragma unroll
+        for (int i = 0; i < 3 * KS; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // LDS read
+          __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
+        }
+      }
+      f32x16 s = c_lse, dpv = c_del;
+      // the S chain first, then the dP chain: exp2 of the finished scores runs behind the dP MFMAs
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) s = mfma32(kf[ks], qreg[ks], s);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) dpv = mfma32(vf[ks], doreg[ks], dpv);
+      bf16x8 kT[MB][2];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        kT[mb][0] = swz_frag_tr<D>(tr, mb, 2 * kb);
+        kT[mb][1] = swz_frag_tr<D>(tr, mb, 2 * kb + 1);
+      }
+      if (MASKED) {  // block touches the diagonal or the end of the keys
+        // register r holds key jb + 4hh + c_r, c_r = 8(r/4) + r%4: masked iff c_r > qlim - jb - 4hh
+        const int t = qlim - jb - 4 * hh;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (8 * (r >> 2) + (r & 3) > t) s[r] = -INFINITY;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r]) * dpv[r];
+      const bf16x8 ds0 = pack_c_half(s, 0), ds1 = pack_c_half(s, 1);
+      request_rowmajor(next_rm, next_kb);  // unconditional: past the last block the fragments are simply unused
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        acc[mb] = mfma32(kT[mb][0], ds0, acc[mb]);
+        acc[mb] = mfma32(kT[mb][1], ds1, acc[mb]);
+      }
+    };
+
+    if (n_act > 0) request_rowmajor(rm_lane, 0);
+    int stage = 0, jt = 0;
+    for (; jt < n_a; ++jt) {
+      const int nstage = stage == kStages - 1 ? 0 : stage + 1;
+      const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
+      if constexpr (PARTS == 1) {
+        step(IC<0>{}, tr, 0, 64 * jt, rm, 1);
+        step(IC<0>{}, tr, 1, 64 * jt + 32, rm_lane + nstage * kStageBytes, 0);
+      } else {
+        step(IC<0>{}, tr, 0, 64 * jt + 32 * part, rm_lane + nstage * kStageBytes, 0);
+      }
+      // stage (jt+3) % 4 == (jt-1) % 4 was last read in the previous iteration: refill it, then make sure
+      // this wave's part of tile jt+2 (needed from the next iteration's prefetch on) has landed
+      if (jt + R.issue_ahead < n_kt) { issue_tile(jt + R.issue_ahead); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
+      __syncthreads();
+      stage = nstage;
+    }
+    for (; jt < n_kt; ++jt) {
+      const int nstage = stage == kStages - 1 ? 0 : stage + 1;
+      const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
+      if constexpr (PARTS == 1) {
+        if (2 * jt < n_act) step(IC<1>{}, tr, 0, 64 * jt, rm, 1);
+        if (2 * jt + 1 < n_act) step(IC<1>{}, tr, 1, 64 * jt + 32, rm_lane + nstage * kStageBytes, 0);
+      } else {
+        if (2 * jt + part < n_act) step(IC<1>{}, tr, 0, 64 * jt + 32 * part, rm_lane + nstage * kStageBytes, 0);
+      }
+      if (jt + R.issue_ahead < n_kt) { issue_tile(jt + R.issue_ahead); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
+      __syncthreads();
+      stage = nstage;
+    }
   }
 
   // ---- epilogue.  First what the dK/dV kernel reads of this row: Qhat, -delta, -lse2 (and dgate).  A gate factor

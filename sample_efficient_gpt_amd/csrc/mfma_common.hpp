@@ -40,6 +40,11 @@ __device__ __forceinline__ void mfma32_acc(f32x16& acc, bf16x8 a, bf16x8 b) {
 __device__ __forceinline__ void mfma32_fixed(f32x16& acc, bf16x8 a, bf16x8 b) {
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
 }
+__device__ __forceinline__ void mfma32_fixed_from(f32x16& acc, bf16x8 a, bf16x8 b, const f32x16& c) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "a"(b), "v"(c));
+}
+// a stationary operand moved to accumulation registers, with the two wait states behind the move
+__device__ __forceinline__ void mfma32_settle(bf16x8& b) { asm volatile("s_nop 1" : "+a"(b)); }
 __device__ __forceinline__ void mfma32_fixed_done(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc)); }
 __device__ __forceinline__ void mfma32_acc_done(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc)); }
 
@@ -133,6 +138,14 @@ __device__ __forceinline__ void gload_lds16_so(const void* base_wave_uniform, ui
                :
                : "v"(lane_off), "s"(base_wave_uniform), "s"(lds_dst_wave_uniform)
                : "memory", "m0");
+}
+// ... and to a constant distance behind an LDS address
+template <int AHEAD>
+__device__ __forceinline__ void gload_lds16_so_at(const void* base_wave_uniform, uint32_t lane_off, uint32_t lds_dst_wave_uniform) {
+  asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(lane_off), "s"(base_wave_uniform), "s"(lds_dst_wave_uniform), "n"(AHEAD)
+               : "memory", "m0", "scc");
 }
 __device__ __forceinline__ void gload_lds4_so(const void* base_wave_uniform, uint32_t lane_off, uint32_t lds_dst_wave_uniform) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
@@ -491,6 +504,16 @@ __device__ __forceinline__ void issue_tile_pair(const char* src_a, const char* s
   for (int ps = 0; ps < Z::kPasses; ++ps) {
     gload_lds16_so(src_a, o.a[ps], dst + ps * 4096);
     gload_lds16_so(src_b, o.b[ps], dst + Z::kTileBytes + ps * 4096);
+  }
+}
+
+// Number k of the loads of issue_tile_pair, for a loop that spreads them: k is a constant once the loop around it is unrolled
+template <int D, int K = 0>
+__device__ __forceinline__ void issue_tile_load(int k, const char* src_a, const char* src_b, const TileLaneOff<D>& o, uint32_t dst) {
+  using Z = Swz<D>;
+  if constexpr (K < 2 * Z::kPasses) {
+    if (k == K) gload_lds16_so_at<(K >> 1) * 4096 + (K & 1) * Z::kTileBytes>(K & 1 ? src_b : src_a, K & 1 ? o.b[K >> 1] : o.a[K >> 1], dst);
+    else issue_tile_load<D, K + 1>(k, src_a, src_b, o, dst);
   }
 }
 

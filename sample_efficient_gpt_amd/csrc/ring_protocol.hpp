@@ -68,18 +68,24 @@ constexpr Protocol forward(int stages, int q_stages, int passes) {
 }
 // dQ: key tile 0 in stage 0, the q / dO / o row blocks in stages 1..3, then key tiles 1 and 2; tile 1 is a late
 // request, hence the wait before the loop.
-constexpr Protocol dq(int passes) { return Protocol{4, 2 * passes, 1, 1, 3, 3, true, false, 3, 1, 0, 0, true}; }
+constexpr Protocol requesting_always(Protocol p, bool on) {
+  p.always_requests = on;
+  return p;
+}
+constexpr Protocol dq(int passes, bool always_requests = true) {
+  return requesting_always(Protocol{4, 2 * passes, 1, 1, 3, 3, true, false, 3, 1, 0, 0, true}, always_requests);
+}
 // dQ with a rotary embedding: the table rows of the workgroup's 128 positions are row blocks too.  First phase: q,
 // cos, sin, dO in stages 0..3; second phase: key tiles 0..2 in stages 0..2 and the o block in stage 3 (everything
 // awaited: no late tiles).  The cos and sin blocks come once more behind the loop, for the epilogue.
-constexpr Protocol dq_rope(int passes) { return Protocol{4, 2 * passes, 3, 3, 1, 3, false, false, 3, 1, 4, 2, true}; }
+constexpr Protocol dq_rope(int passes, bool always_requests = true) {
+  return requesting_always(Protocol{4, 2 * passes, 3, 3, 1, 3, false, false, 3, 1, 4, 2, true}, always_requests);
+}
 // dK/dV: (Qhat, dO) tiles 0 and 1 in stages 0 and 1 with the Khat / V' row blocks in stages 2 and 3, then tile 2;
 // a tile is the two [64, D] tiles plus one row-statistics load.
 // Behind the loop: the raw k block (and, with a value residual, the raw v and v_first blocks) for the epilogue.
 constexpr Protocol dkdv(int passes, bool always_requests = true) {
-  Protocol p{4, 2 * passes + 1, 2, 2, 2, 3, false, false, 3, 1, 0, 3, false};
-  p.always_requests = always_requests;
-  return p;
+  return requesting_always(Protocol{4, 2 * passes + 1, 2, 2, 2, 3, false, false, 3, 1, 0, 3, false}, always_requests);
 }
 
 // The same kernels in 64-row workgroups whose waves split the blocks of a tile.  The forward uses the ring behind its loop for the
@@ -93,8 +99,8 @@ constexpr Protocol merging(Protocol p, int first, int stages, int scratch_stages
   return p;
 }
 constexpr Protocol forward_parts(int stages, int q_stages, int passes) { return merging(forward(stages, q_stages, passes), 0, 2); }
-constexpr Protocol dq_parts(int passes) { return merging(dq(passes), 2, 2, 2); }
-constexpr Protocol dq_rope_parts(int passes) { return merging(dq_rope(passes), 2, 2, 2, 1); }
+constexpr Protocol dq_parts(int passes) { return merging(dq(passes, false), 2, 2, 2); }
+constexpr Protocol dq_rope_parts(int passes) { return merging(dq_rope(passes, false), 2, 2, 2, 1); }
 constexpr Protocol dkdv_parts(int passes) { return merging(dkdv(passes, false), 2, 2, 0, 2); }
 
 constexpr bool well_formed(const Protocol& p) {

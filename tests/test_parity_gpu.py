@@ -497,6 +497,23 @@ def test_bf16_dkdv_pipeline_ends(gpu_device, B, H, Hkv, Sq, Sk, D, kw):
     _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, D, seed=63, outliers=(1e-6, 2.0), rope=orc.rope_tables(max(Sq, Sk), 10000.0, D), **kw)
 
 
+@pytest.mark.parametrize("use_rope", [False, True])
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,kw", [
+    (2, 66, 22, 60, 40, {"causal": False}),      # one streamed tile, its second block of eight keys
+    (2, 66, 66, 20, 129, {"q_start": 109}),      # three, the last of one key
+    (3, 46, 23, 33, 33, {}),                     # the second row wave has one row, the others none
+    (2, 33, 33, 150, 150, {}),                   # two query tiles, the second of 22 rows
+    (2, 33, 33, 256, 330, {"q_start": 74}),      # waves that need one block of their last tile, or none of it
+])
+def test_bf16_dq_pipeline_ends(gpu_device, B, H, Hkv, Sq, Sk, kw, use_rope):
+    """dQ at head_dim 128 with 128-row workgroups, whose pipeline runs two blocks ahead of itself and requests a tile in every
+    iteration, at the shortest streams and at ragged ends (outliers: as for dK/dV above)."""
+    assert B * H * (-(-Sq // 128)) > 128
+    if use_rope:
+        kw = dict(kw, rope=orc.rope_tables(max(Sq, Sk), 10000.0, 128))
+    _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, 128, seed=64, outliers=(1e-6, 2.0), **kw)
+
+
 @pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,kw,gen_kw,use_rope", [
     (1, 2, 1, 65, 65, 64, {}, {"extras": True}, True),                         # one row in the last workgroup, its second wave beyond the end
     (1, 2, 2, 31, 130, 64, {"q_start": 99}, {"extras": True}, False),          # fewer rows than one wave owns
