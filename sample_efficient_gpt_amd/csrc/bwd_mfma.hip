@@ -64,6 +64,22 @@ inline int dq_parts(const segpt_attn_params& p) {
   return wgs <= (p.D == 128 ? 128 : tiles >= kLongTiles ? 384 : 256) ? 2 : 1;
 }
 
+// Whether a launch of 128-row workgroups takes the kernel whose loop is laid out instruction by instruction (PIPE).  Its start and end
+// cost a workgroup a few hundred cycles more (a block's scores that nothing overlaps, a tile that is requested once too often).
+// head_dim 64, 18 / 6 heads, 16384 tokens in all, plain call, compiler's loop against PIPE, us: dK/dV at 256 / 512 / 768 / 999 / 1536 /
+// 3072 tokens (12 / 24 / 36 / 48 / 72 / 144 streamed tiles) 41.7 / 44.1, 59.2 / 60.5, 74.3 / 76.9, 95.5 / 92.4, 116.4 / 113.9, 214.9 / 200.3;
+// dQ at 256 / 768 / 1152 / 2048 / 3072 (4 / 12 / 18 / 32 / 48 tiles) 54.8 / 56.0, 71.5 / 71.6, 85.8 / 85.8, 125.9 / 123.7, 162.8 / 159.3, with a rotary
+// embedding 63.8 / 67.0, 79.3 / 81.5, 91.6 / 93.6, 130.9 / 129.9, 167.3 / 165.9.  head_dim 128 has one wave per SIMD and nothing else to fill
+// the matrix pipe with: always.
+inline bool dkdv_pipelined(const segpt_attn_params& p) {
+  constexpr int kTiles = 48;
+  return dkdv_parts(p) == 1 && (p.D == 128 || (int64_t)(p.H / p.Hkv) * ((p.Sq + kBK - 1) / kBK) >= kTiles);
+}
+inline bool dq_pipelined(const segpt_attn_params& p) {
+  constexpr int kTiles = 32;
+  return dq_parts(p) == 1 && (p.D == 128 || (p.Sk + kBK - 1) / kBK >= kTiles);
+}
+
 constexpr float kGateFactorFloor = 1e-30f;  // a smaller gate factor switches its row off in the dK/dV kernel
 
 constexpr int kStages = 4;  // LDS ring of streamed stages (two tiles each): tile t lives in stage t % 4
@@ -85,17 +101,18 @@ constexpr int kStages = 4;  // LDS ring of streamed stages (two tiles each): til
 //
 // PARTS: see dq_parts(); with 2 the workgroup owns 64 query rows, two waves each take one of the two 32-key blocks of
 // every tile for the same rows, and the pair adds up T^T through LDS behind the loop.
-template <int D, bool ROPE, int PARTS>
+// PIPE (PARTS == 1): see dq_pipelined().
+template <int D, bool ROPE, int PARTS, bool PIPE>
 __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel(KArgs a) {
   using Z = Swz<D>;
-  static_assert(PARTS == 1 || PARTS == 2, "a tile has two 32-key blocks");
+  static_assert(PARTS == 1 || (PARTS == 2 && !PIPE), "a tile has two 32-key blocks");
   constexpr int BQ = kBwdRows / PARTS;
   constexpr int kRowWaves = 4 / PARTS;  // waves side by side along the query rows
   constexpr int KS = D / 16;
   constexpr int MB = D / 32;
   constexpr int kStageBytes = 2 * Z::kTileBytes;
   // the pipeline's numbers: ring_protocol.hpp
-  constexpr bool PIPE = D == 128 && PARTS == 1;
+  constexpr bool AGPR = D == 128;
   constexpr ring::Protocol R = PARTS == 1 ? (ROPE ? ring::dq_rope(Z::kPasses, PIPE) : ring::dq(Z::kPasses, PIPE))
                                           : (ROPE ? ring::dq_rope_parts(Z::kPasses) : ring::dq_parts(Z::kPasses));
   static_assert(ring::well_formed(R) && R.stages == kStages && !R.issue_at_top, "tile pipeline");
@@ -341,23 +358,27 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     // The pipeline of the dK/dV kernel below (there: what a slot holds, and why): step n computes S^T and dP^T of block n + 1
     // (kA matrix instructions) while the vector unit turns those of block n into dS^T, then adds block n to T^T (kB);
     // the row-major fragments of block n + 2 come in as those of block n + 1 are used.
-    // Head_dim 128 only.  dQ, 4 x 16 / 4 heads, 4096 tokens: 437 -> 398 us (937 k -> 768 k cycles, matrix pipe 42 -> 52 % busy; a
-    // quarter of the launch is now the workgroups' first and last thousands of cycles, one workgroup a CU).  At head_dim 64 the
-    // second set of scores does not fit two workgroups per CU: 256 registers split in halves spill 95 of them.
+    // dQ, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 437 -> 398 (937 k -> 768 k cycles, matrix pipe 42 -> 52 % busy; a quarter
+    // of the launch is now the workgroups' first and last thousands of cycles, one workgroup a CU); head_dim 64, 2 x 18 / 6
+    // heads, 8192 tokens 774 k -> 712 k cycles, 57 -> 63 % busy, of which the clock takes two thirds (1.87 -> 1.75 GHz).  At head_dim 64
+    // everything is in ordinary registers (250 of 256): a kernel that uses both files gets half of each, and the ordinary
+    // half spills.
     constexpr int kA = 2 * KS, kB = 2 * MB;
     auto order = [](int i) { return (i & 1) * KS + (i >> 1); };  // i-th product: k-step of S^T, or KS + that of dP^T
     f32x16 s0, d0, s1, d1;           // scores and dP of two consecutive blocks
     uint32_t rma[KS], tra[2 * MB];   // addresses: the next tile's row-major fragments, this tile's transposed ones
     auto start = [&](f32x16& s, f32x16& d, int i) {  // the i-th product of a block
       const int o = order(i), ks = o % KS;
-      if (o >= KS) ks == 0 ? mfma32_fixed_from(d, vf[ks], doreg[ks], c_del) : mfma32_fixed(d, vf[ks], doreg[ks]);
-      else ks == 0 ? mfma32_fixed_from(s, kf[ks], qreg[ks], c_lse) : mfma32_fixed(s, kf[ks], qreg[ks]);
+      if (o >= KS) ks == 0 ? mfma32_fixed_from<AGPR>(d, vf[ks], doreg[ks], c_del) : mfma32_fixed<AGPR>(d, vf[ks], doreg[ks]);
+      else ks == 0 ? mfma32_fixed_from<AGPR>(s, kf[ks], qreg[ks], c_lse) : mfma32_fixed<AGPR>(s, kf[ks], qreg[ks]);
     };
     auto row_frag = [&](uint32_t rm_ks, int kb, int o) { (o < KS ? kf : vf)[o % KS] = as_bf16x8(lds_read16(rm_ks + (o < KS ? 0 : Z::kTileBytes) + kb * 32 * Z::kRB)); };
     // (s, d): block n, whose first key is jb, number kb of its tile; (sn, dn): block n + 1.  mem and alu: what else the slots
     // hold, beside the LDS reads and beside the vector instructions
+    // masked_c: 0 no mask, 1 masked, 2 masked and the wave's last block (no products of a next one, whose registers would be
+    // given to others while they are still on their way)
     auto step = [&](auto masked_c, f32x16& s, f32x16& d, f32x16& sn, f32x16& dn, int kb, int jb, auto mem, auto alu) {
-      constexpr bool MASKED = decltype(masked_c)::value != 0;
+      constexpr bool MASKED = decltype(masked_c)::value != 0, LAST = decltype(masked_c)::value == 2;
       // register r holds key jb + 4hh + c_r, c_r = 8(r/4) + r%4: masked iff c_r > qlim - jb - 4hh
       const int t = qlim - jb - 4 * hh;
       u32x4 dw[2];  // dS as operand, in halves of 16 keys
@@ -371,9 +392,9 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
       constexpr int kExps = 16 / kA;  // per slot
 #pragma unroll
       for (int i = 0; i < kA; ++i) {
-        start(sn, dn, i);
+        if constexpr (!LAST) start(sn, dn, i);
         // even slots: a transposed fragment of block n; odd ones: a row-major fragment of block n + 2, whose place is free
-        if (i & 1) row_frag(rma[order(i >> 1) % KS], kb, order(i >> 1));
+        if (i & 1) { if constexpr (!LAST) row_frag(rma[order(i >> 1) % KS], kb, order(i >> 1)); }
         else kT[(i >> 1) % MB][(i >> 1) / MB] = frag_tr_at<D>(tra[2 * ((i >> 1) % MB)], tra[2 * ((i >> 1) % MB) + 1], 2 * kb + (i >> 1) / MB, 0);
         mem(i);
         __builtin_amdgcn_sched_barrier(0);
@@ -395,8 +416,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
       }
 #pragma unroll
       for (int j = 0; j < kB; ++j) {
-        mfma32_acc(acc[j % MB], kT[j % MB][j / MB], as_bf16x8(dw[j / MB]));
-        row_frag(rma[order(kA / 2 + j) % KS], kb, order(kA / 2 + j));
+        mfma32_acc<AGPR>(acc[j % MB], kT[j % MB][j / MB], as_bf16x8(dw[j / MB]));
+        if constexpr (!LAST) row_frag(rma[order(kA / 2 + j) % KS], kb, order(kA / 2 + j));
         mem(kA + j);
         __builtin_amdgcn_sched_barrier(0);
         alu(kA + j);
@@ -412,7 +433,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     for (int x = 0; x < 2 * MB; ++x) tra[x] = tr_addr(tr_lane, x);
     // block 0 up to its scores, the fragments of block 1 (tiles 0 and 1 have landed)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) { mfma32_settle(qreg[ks]); mfma32_settle(doreg[ks]); }
+    for (int ks = 0; ks < KS; ++ks) { mfma32_settle<AGPR>(qreg[ks]); mfma32_settle<AGPR>(doreg[ks]); }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) { row_frag(rm_addr(rm_lane, ks), 0, ks); row_frag(rm_addr(rm_lane, ks), 0, KS + ks); }
 #pragma unroll
@@ -483,13 +504,13 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
       end_tile();
     }
     for (; jt < n_kt; ++jt) {  // tiles of which this wave needs one block, then none
-      if (2 * jt < n_act) first_step(IC<1>{});
+      if (2 * jt < n_act) first_step(IC<2>{});
       else request(0);
       request(kPerStep);
       end_tile();
     }
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) mfma32_acc_done(acc[mb]);
+    for (int mb = 0; mb < MB; ++mb) mfma32_acc_done<AGPR>(acc[mb]);
     static_assert(R.always_requests, "no branch around the loads of an iteration");
     wait_vmcnt<0>();  // the last tile, requested once more, has left the stages that the epilogue uses
     __syncthreads();
@@ -709,17 +730,17 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
 // blocks are 32 queries, and B(n) starts from the two row statistics of the block, read from LDS
 // straight into the accumulators of S and dP.  PARTS: see dkdv_parts(); with 2 a wave computes one block of every tile
 // and the two waves of a key block add up their accumulators through LDS behind the loop.
-template <int D, bool ROPE, int PARTS>
+// PIPE (PARTS == 1): see dkdv_pipelined().
+template <int D, bool ROPE, int PARTS, bool PIPE>
 __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kernel(KArgs a) {
   using Z = Swz<D>;
-  static_assert(PARTS == 1 || PARTS == 2, "a tile has two 32-query blocks");
-  constexpr bool PIPE = PARTS == 1;
+  static_assert(PARTS == 1 || (PARTS == 2 && !PIPE), "a tile has two 32-query blocks");
   constexpr int BKV = kBwdRows / PARTS;
   constexpr int kKeyWaves = 4 / PARTS;  // waves side by side along the keys
   constexpr int KS = D / 16;
   constexpr int MB = D / 32;
   constexpr int kStageBytes = 2 * Z::kTileBytes;
-  constexpr ring::Protocol R = PARTS == 1 ? ring::dkdv(Z::kPasses) : ring::dkdv_parts(Z::kPasses);  // the pipeline's numbers: ring_protocol.hpp
+  constexpr ring::Protocol R = PARTS == 1 ? ring::dkdv(Z::kPasses, PIPE) : ring::dkdv_parts(Z::kPasses);  // the pipeline's numbers: ring_protocol.hpp
   static_assert(ring::well_formed(R) && R.stages == kStages && R.row_stages == 2 && !R.wait_before_loop && !R.issue_at_top, "tile pipeline");
   static_assert(R.early_tiles >= ring::kTilesNeededAtLoopStart, "the loop is entered without a further wait");
   static_assert(R.loads_per_tile == 2 * Z::kPasses + 1, "per wave: the two tiles plus one row-statistics load");
@@ -771,13 +792,13 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   const TileLaneOff<D> full_tile = tile_lane_offsets<D>(D * 2, dstep, kBK, src.x, src.y);
   // The stream of (query tile, head) pairs is walked by running pointers kept beside the compute loop's own counters
   // (three tiles ahead of it): per tile a few scalar additions.
-  // PARTS == 1: from the last tile down, every head of the group at a tile before the next tile.  All workgroups of a
+  // PIPE: from the last tile down, every head of the group at a tile before the next tile.  All workgroups of a
   // (batch, kv head) pair start at the same tile and stay together, so that a tile comes into the XCD's L2 once for all of them.
   // Head by head and upwards from the diagonal every workgroup was somewhere else: L2 misses per launch (128-byte lines),
   // 4 x 16 / 4 heads, 4096 tokens, head_dim 128 9.8 M -> 4.0 M, 2 x 18 / 6 heads, 8192 tokens, head_dim 64 10.7 M -> 3.9 M.
-  // PARTS == 2, head by head and upwards: these launches' streams fit the L2 anyway, and in step their workgroups
+  // Without, head by head and upwards: these launches' streams are short and fit the L2 anyway, and in step their workgroups
   // only queue for the same lines (8 x 18 / 6 heads, 999 tokens: the whole step 177.3 us, in step 178.5).
-  constexpr bool kInStep = PARTS == 1;
+  constexpr bool kInStep = PIPE;
   int iss_h = 0, iss_t = 0, iss_stage = 0, issued = 0;
   const int i_first = kInStep ? (n_qt - 1) * kBK : qt_start * kBK;  // first query of the stream's first tile
   const int64_t row_first = ((int64_t)b * p.H + g * rep) * p.Sq + i_first;
@@ -875,7 +896,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   if (p.causal) t_diag = min(max((max(kw0 + 31 - p.q_start, 0) + kBK - 1) / kBK - qt_start, 0), n_vis);
   const int t_full = min(max(p.Sq / kBK - qt_start, 0), n_vis);  // tiles whose 64 queries all exist
   const int t_end = max(t_full, t_diag);
-  if constexpr (PARTS == 1) {
+  if constexpr (PIPE) {
     // A software pipeline over 32-query blocks, laid out instruction by instruction: step n computes the scores and dP of
     // block n + 1 (first half: kA matrix instructions) while the vector unit turns those of block n into P and dS, then
     // adds block n to dV and dK (second half: kB) while the row-major fragments and row statistics of block n + 2 come in.
@@ -1170,13 +1191,19 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
       for (int t = t_lo; t < t_hi; ++t, ++it) {
         const int nstage = stage == kStages - 1 ? 0 : stage + 1;
         const int i0 = (qt_start + t) * kBK;
-        const uint32_t tr = tr_lane + stage * kStageBytes;
+        const uint32_t rm = rm_lane + stage * kStageBytes, tr = tr_lane + stage * kStageBytes;
         const uint32_t st = st_lane + stage * 512;
         // on the diagonal a block whose last query still lies before this wave's first key is masked entirely:
         // it only passes the fragment request on (wave-uniform, so the barrier below is reached all the same)
-        const int ib = i0 + 32 * part;
-        if (MASK == 1 && kw0 > ib + 31 + p.q_start) request_rowmajor(rm_lane + nstage * kStageBytes, 0);
-        else step(masked_c, tr, st, 0, ib, rm_lane + nstage * kStageBytes, 0);
+        if constexpr (PARTS == 1) {
+          if (MASK == 1 && kw0 > i0 + 31 + p.q_start) request_rowmajor(rm, 1); else step(masked_c, tr, st, 0, i0, rm, 1);
+          if (MASK == 1 && kw0 > i0 + 63 + p.q_start) request_rowmajor(rm_lane + nstage * kStageBytes, 0);
+          else step(masked_c, tr, st, 1, i0 + 32, rm_lane + nstage * kStageBytes, 0);
+        } else {
+          const int ib = i0 + 32 * part;
+          if (MASK == 1 && kw0 > ib + 31 + p.q_start) request_rowmajor(rm_lane + nstage * kStageBytes, 0);
+          else step(masked_c, tr, st, 0, ib, rm_lane + nstage * kStageBytes, 0);
+        }
         if (it + R.issue_ahead < n_it) { issue_next(); wait_vmcnt<ring::loads_kept_after_iteration(R, true)>(); } else wait_vmcnt<ring::loads_kept_after_iteration(R, false)>();
         __syncthreads();
         stage = nstage;
@@ -1326,32 +1353,20 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
   }
 }
 
-template <int D>
-int launch_dkdv_t(const KArgs& a, hipStream_t st) {
-  const segpt_attn_params& p = a.p;
-  const dim3 grid((unsigned)(bf16_dkdv_grid(p) + 1));
-  if (dkdv_parts(p) == 1) {
-    if (p.rope_cos) hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, true, 1>), grid, dim3(kThreadsM), 0, st, a);
-    else hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, false, 1>), grid, dim3(kThreadsM), 0, st, a);
-  } else {
-    if (p.rope_cos) hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, true, 2>), grid, dim3(kThreadsM), 0, st, a);
-    else hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, false, 2>), grid, dim3(kThreadsM), 0, st, a);
-  }
-  return (int)hipGetLastError();
+template <int D, bool ROPE>
+void launch_dkdv_t(const KArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)(bf16_dkdv_grid(a.p) + 1));
+  if (dkdv_pipelined(a.p)) hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, ROPE, 1, true>), grid, dim3(kThreadsM), 0, st, a);
+  else if (dkdv_parts(a.p) == 2) hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, ROPE, 2, false>), grid, dim3(kThreadsM), 0, st, a);
+  else if constexpr (D == 64) hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<D, ROPE, 1, false>), grid, dim3(kThreadsM), 0, st, a);
 }
 
-template <int D>
-int launch_dq_t(const KArgs& a, hipStream_t st) {
-  const segpt_attn_params& p = a.p;
-  const dim3 grid((unsigned)bf16_dq_grid(p));
-  if (dq_parts(p) == 1) {
-    if (p.rope_cos) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, true, 1>), grid, dim3(kThreadsM), 0, st, a);
-    else hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 1>), grid, dim3(kThreadsM), 0, st, a);
-  } else {
-    if (p.rope_cos) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, true, 2>), grid, dim3(kThreadsM), 0, st, a);
-    else hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 2>), grid, dim3(kThreadsM), 0, st, a);
-  }
-  return (int)hipGetLastError();
+template <int D, bool ROPE>
+void launch_dq_t(const KArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)bf16_dq_grid(a.p));
+  if (dq_pipelined(a.p)) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, ROPE, 1, true>), grid, dim3(kThreadsM), 0, st, a);
+  else if (dq_parts(a.p) == 2) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, ROPE, 2, false>), grid, dim3(kThreadsM), 0, st, a);
+  else if constexpr (D == 64) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, ROPE, 1, false>), grid, dim3(kThreadsM), 0, st, a);
 }
 
 }  // namespace
@@ -1368,15 +1383,19 @@ int bf16_dkdv_grid(const segpt_attn_params& p) {
 }
 
 int launch_bwd_dkdv_bf16(const KArgs& a, hipStream_t st) {
-  if (a.p.D == 64) return launch_dkdv_t<64>(a, st);
-  if (a.p.D == 128) return launch_dkdv_t<128>(a, st);
-  return (int)hipErrorInvalidValue;
+  const bool rope = a.p.rope_cos != nullptr;
+  if (a.p.D == 64) rope ? launch_dkdv_t<64, true>(a, st) : launch_dkdv_t<64, false>(a, st);
+  else if (a.p.D == 128) rope ? launch_dkdv_t<128, true>(a, st) : launch_dkdv_t<128, false>(a, st);
+  else return (int)hipErrorInvalidValue;
+  return (int)hipGetLastError();
 }
 
 int launch_bwd_dq_bf16(const KArgs& a, hipStream_t st) {
-  if (a.p.D == 64) return launch_dq_t<64>(a, st);
-  if (a.p.D == 128) return launch_dq_t<128>(a, st);
-  return (int)hipErrorInvalidValue;
+  const bool rope = a.p.rope_cos != nullptr;
+  if (a.p.D == 64) rope ? launch_dq_t<64, true>(a, st) : launch_dq_t<64, false>(a, st);
+  else if (a.p.D == 128) rope ? launch_dq_t<128, true>(a, st) : launch_dq_t<128, false>(a, st);
+  else return (int)hipErrorInvalidValue;
+  return (int)hipGetLastError();
 }
 
 }  // namespace segpt

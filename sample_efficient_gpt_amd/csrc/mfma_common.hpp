@@ -34,19 +34,34 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
 // in accumulation registers (_fixed).  The compiler sees neither as a matrix instruction: what it inserts around those
 // (two wait states behind a vector instruction that wrote an operand, twelve before one that reads the result) the caller's
 // order has to provide, and behind the last one the _done form does.
+// AGPR == false: all of it in ordinary registers (a kernel of two waves per SIMD that uses both files gets half of each).
+template <bool AGPR = true>
 __device__ __forceinline__ void mfma32_acc(f32x16& acc, bf16x8 a, bf16x8 b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  if constexpr (AGPR) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
+template <bool AGPR = true>
 __device__ __forceinline__ void mfma32_fixed(f32x16& acc, bf16x8 a, bf16x8 b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
+  if constexpr (AGPR) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
+  else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
+template <bool AGPR = true>
 __device__ __forceinline__ void mfma32_fixed_from(f32x16& acc, bf16x8 a, bf16x8 b, const f32x16& c) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "a"(b), "v"(c));
+  if constexpr (AGPR) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "a"(b), "v"(c));
+  else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(c));
 }
 // a stationary operand moved to accumulation registers, with the two wait states behind the move
-__device__ __forceinline__ void mfma32_settle(bf16x8& b) { asm volatile("s_nop 1" : "+a"(b)); }
+template <bool AGPR = true>
+__device__ __forceinline__ void mfma32_settle(bf16x8& b) {
+  if constexpr (AGPR) asm volatile("s_nop 1" : "+a"(b));
+  else asm volatile("s_nop 1" : "+v"(b));
+}
 __device__ __forceinline__ void mfma32_fixed_done(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc)); }
-__device__ __forceinline__ void mfma32_acc_done(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc)); }
+template <bool AGPR = true>
+__device__ __forceinline__ void mfma32_acc_done(f32x16& acc) {
+  if constexpr (AGPR) asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc));
+  else asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc));
+}
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 

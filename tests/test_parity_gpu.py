@@ -487,8 +487,8 @@ def test_bf16_dkdv_workgroup_shapes(gpu_device, B, H, Hkv, Sq, Sk, D, kw):
     (3, 90, 90, 200, 140, {"causal": False}),   # four, and a last key tile of 12 rows
 ])
 def test_bf16_dkdv_pipeline_ends(gpu_device, B, H, Hkv, Sq, Sk, D, kw):
-    """dK/dV of launches that fill the card (128-key workgroups), whose pipeline runs two blocks ahead of itself and requests
-    a tile in every iteration, at the shortest streams and at ragged ends.
+    """dK/dV of launches that fill the card (128-key workgroups) at the shortest streams and at ragged ends; at head_dim 128 the
+    loop runs two blocks ahead of itself and requests a tile in every iteration.
     Outliers: a launch that fills the card has millions of entries, and dk of a row that few queries see is a sum of few terms
     with roundings of 2^-9 each against a result that cancels; over the 198-head case dk is 3.7e-3 from float64 in norm and
     one entry of 2.5 million is 0.043 away where the elementwise bound says 0.04 (both to all digits also with the products
@@ -512,6 +512,32 @@ def test_bf16_dq_pipeline_ends(gpu_device, B, H, Hkv, Sq, Sk, kw, use_rope):
     if use_rope:
         kw = dict(kw, rope=orc.rope_tables(max(Sq, Sk), 10000.0, 128))
     _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, 128, seed=64, outliers=(1e-6, 2.0), **kw)
+
+
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,kw,extras,use_rope", [
+    (11, 18, 6, 999, 999, {}, True, True),                   # dK/dV pipelined at its shortest stream (48 tiles), dQ not
+    (9, 12, 4, 1030, 2050, {"q_start": 1020}, False, True),  # both, queries at the end of the keys
+    (6, 18, 6, 2017, 2017, {}, True, False),                 # both, ragged
+    (5, 24, 6, 777, 2300, {"causal": False}, False, False),  # both, no mask but the ends
+])
+def test_bf16_backward_pipelines_against_single_batches(gpu_device, B, H, Hkv, Sq, Sk, kw, extras, use_rope):
+    """head_dim 64: a launch long and large enough for the backward loops that are laid out instruction by instruction, against
+    its batches one by one, whose launches take the compiler's loops.  Scores, P and dS are the same bits; dK, dV and T are
+    fp32 sums of them in another order (at most 7000 terms: 7000 x 2^-24 of their magnitudes' sum), rounded to bf16 once: equal but
+    for roundings that fall the other way, one unit in the last place (2^-7 of a value's power of two) each, and few of them."""
+    assert B * Hkv * (-(-Sk // 128)) > 512 and H // Hkv * (-(-Sq // 64)) >= 48
+    x = gen(B, H, Hkv, Sq, Sk, 64, BF16, extras=extras, seed=65)
+    if use_rope:
+        kw = dict(kw, rope=orc.rope_tables(max(Sq, Sk), 10000.0, 64))
+    got = run_gpu(x, gpu_device, **kw)
+    per_batch = [n for n in ("q", "k", "v", "d_o", "v_first", "gate_logits") if x.get(n) is not None]
+    for i in (0, B - 1):
+        one = run_gpu(dict(x, **{n: x[n][i:i + 1] for n in per_batch}), gpu_device, **kw)
+        for n in ("dq", "dk", "dv") + (("dv_first", "dgate_logits") if extras else ()):
+            a, b = got[n][i].float(), one[n][0].float()
+            scale = torch.maximum(b.abs(), b.square().mean().sqrt())
+            assert ((a - b).abs() <= 2.0 ** -7 * scale).all(), (n, float(((a - b).abs() / scale).max()))
+            assert (a - b).norm() <= 1e-3 * b.norm(), (n, float((a - b).norm() / b.norm()))
 
 
 @pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,kw,gen_kw,use_rope", [
