@@ -358,9 +358,9 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     // The pipeline of the dK/dV kernel below (there: what a slot holds, and why): step n computes S^T and dP^T of block n + 1
     // (kA matrix instructions) while the vector unit turns those of block n into dS^T, then adds block n to T^T (kB);
     // the row-major fragments of block n + 2 come in as those of block n + 1 are used.
-    // dQ, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 437 -> 398 (937 k -> 768 k cycles, matrix pipe 42 -> 52 % busy; a quarter
+    // dQ, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 435 -> 390 (939 k -> 764 k cycles, matrix pipe 42 -> 52 % busy; a quarter
     // of the launch is now the workgroups' first and last thousands of cycles, one workgroup a CU); head_dim 64, 2 x 18 / 6
-    // heads, 8192 tokens 774 k -> 712 k cycles, 57 -> 63 % busy, of which the clock takes two thirds (1.87 -> 1.75 GHz).  At head_dim 64
+    // heads, 8192 tokens 418 -> 402 (776 k -> 698 k cycles, 57 -> 64 % busy, 1.86 -> 1.74 GHz).  At head_dim 64
     // everything is in ordinary registers (250 of 256): a kernel that uses both files gets half of each, and the ordinary
     // half spills.
     constexpr int kA = 2 * KS, kB = 2 * MB;
@@ -907,8 +907,9 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
     // The accumulators and the stationary rows live in accumulation registers, scores and dP in ordinary ones; a kernel
     // of more than 256 registers gets one form for all matrix instructions from the compiler, hence the inline assembly,
     // whose wait states tests/test_mfma_hazards.py checks on the built code.
-    // dK/dV, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 515 -> 430 (matrix pipe 54 -> 72 % busy; the clock gives part of
-    // it back, 1.98 -> 1.74 GHz); head_dim 64, 2 x 18 / 6 heads, 8192 tokens 587 -> 530 (58 -> 67 %), 8 x 2048 154 -> 149.
+    // dK/dV, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 529 -> 436 (1161 k -> 745 k cycles, matrix pipe 45 -> 73 % busy; the
+    // card holds its power, so the clock gives part of it back, 2.20 -> 1.71 GHz); head_dim 64, 2 x 18 / 6 heads, 8192 tokens 572 ->
+    // 535 (54 -> 68 %), 8 x 2048 154 -> 152 (48 -> 57 %).
     constexpr int kA = 2 * KS, kB = 4 * MB;
     // i-th product of the first half: k-step of S (0 .. KS-1) or KS + that of dP.  S leads, so that the statistics from which
     // dP starts, requested last, have time.
