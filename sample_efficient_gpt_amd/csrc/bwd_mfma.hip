@@ -1026,7 +1026,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
       }
     }
     // the tile requested in an iteration: its rows' lane offsets, cut off at the last query, and where the stream goes on
-    const int q_row = src.x * D * 2, d_row = src.x * (int)dstep;
+    const uint32_t q_row = (uint32_t)src.x * D * 2, d_row = (uint32_t)src.x * dstep;
     const int64_t q_wrap = -((rep - 1) * q_head + kBK * D * 2), d_wrap = -((rep - 1) * d_head + (int64_t)kBK * dstep);
     const int s_wrap = -((rep - 1) * p.Sq + kBK);
     constexpr int kLoads = 2 * Z::kPasses;
@@ -1045,9 +1045,9 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
         int64_t q_step = 0, d_step = 0;
         int s_step = 0, left_step = 0;
         auto offset = [&](int k) {  // rows past the last query re-read it
-          const int lim = min(left_it, kBK) - 1, row = (k >> 1) * 4 * Z::kRowsPerInst;
-          if (k & 1) off = min(d_row, (lim - row) * (int)dstep) + src.y + row * (int)dstep;
-          else off = min(q_row, (lim - row) * D * 2) + src.y + row * D * 2;
+          const uint32_t last = min(left_it, kBK) - 1, row = (k >> 1) * 4 * Z::kRowsPerInst;
+          if (k & 1) off = min(d_row + row * dstep, last * dstep) + src.y;
+          else off = min(q_row + row * D * 2, last * D * 2) + src.y;
         };
         auto load = [&](int k) {
           const uint32_t dst = lds0 + iss_stage * kStageBytes + wave * 1024 + (k >> 1) * 4096;
