@@ -18,8 +18,9 @@
 //              dV'^T += dO^T . P                  dKhat^T += Qhat^T . dS        (A = transposing LDS read)
 //            epilogue: through the k normaliser, dk, dv (= c1 dV'), dv_first (= c2 dV'), (dc1, dc2) partials.
 //
-// One workgroup = 4 waves (one per SIMD); several workgroups share a CU so that the softmax-like VALU
-// phase of one overlaps the MFMA phase of another.  Streamed tiles (64 rows) are double-buffered in LDS.
+// One workgroup = 4 waves (one per SIMD); at head_dim 64 two workgroups share a CU so that the softmax-like VALU
+// phase of one overlaps the MFMA phase of another.  Streamed tiles (64 rows) travel through a ring in LDS.  Both kernels
+// have a second form of their loop (PIPE) in which a wave overlaps the two phases by itself: dkdv_pipelined(), dq_pipelined().
 #include "mfma_common.hpp"
 #include "ring_protocol.hpp"
 
@@ -527,7 +528,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     // MASKED is compile-time so that a whole block is one straight-line scheduling region
     auto step = [&](auto masked_c, uint32_t tr, int kb, int jb, uint32_t next_rm, int next_kb) {
       constexpr bool MASKED = decltype(masked_c)::value != 0;
-      // head_dim 128 runs one wave per SIMD with all 256 ordinary registers in use: left to itself the compiler requests
+      // head_dim 128 (64-row workgroups here) runs one wave per SIMD with all 256 ordinary registers in use: left to itself the compiler requests
       // each LDS fragment one MFMA ahead of its use and the wave stalls on LDS latency before most MFMAs.  Asking for
       // the block as 24 groups of (1 MFMA, 2 LDS reads, 2 vector instructions) keeps two requests ahead: -6 % on this
       // kernel (neighbouring group shapes are 2-10 % slower; at head_dim 64, two waves per SIMD, none changes anything).
@@ -1130,7 +1131,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
     auto step = [&](auto masked_c, uint32_t tr, uint32_t st, int qb, int ib, uint32_t next_rm, int next_qb) {
       constexpr int MASK = decltype(masked_c)::value;
       // head_dim 128 (one wave per SIMD, nothing else to hide the exp2 phase behind): the compiler's interleaving
-      // strategy for exp2 work between MFMA chains, measured -3 % on this kernel; at head_dim 64 it changes nothing
+      // strategy for exp2 work between MFMA chains, measured -3 % on 128-key workgroups; at head_dim 64 it changes nothing
       if constexpr (D == 128) __builtin_amdgcn_iglp_opt(3);
       // accumulators of S and dP start from -lse2 / -delta of the 16 query rows their registers map to
       f32x16 s, dpv;
