@@ -1037,24 +1037,36 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
     auto slot_load = [](int j, int first, int n) { return j >= first && (j - first) % kEvery == 0 && (j - first) / kEvery < n ? (j - first) / kEvery : -1; };
     int stage = 0, it = 0;
     iss_stage = R.startup_tiles;  // also where there are fewer tiles than that
+    uint32_t off = 0;
+    auto offset = [&](int k) {  // rows past the last query re-read it
+      const uint32_t last = min(left_it, kBK) - 1, row = (k >> 1) * 4 * Z::kRowsPerInst;
+      if (k & 1) off = min(d_row + row * dstep, last * dstep) + src.y;
+      else off = min(q_row + row * D * 2, last * D * 2) + src.y;
+    };
+    auto load = [&](int k) {
+      const uint32_t dst = lds0 + iss_stage * kStageBytes + wave * 1024 + (k >> 1) * 4096;
+      if (k & 1) gload_lds16_so(d_it, off, dst + Z::kTileBytes);
+      else gload_lds16_so(q_it, off, dst);
+    };
+    auto stat_offset = [&]() { off = (uint32_t)min(lane, left_it - 1) * 4; };
+    auto stat_load = [&]() { gload_lds4_so(s_it, off, ldl0 + (iss_stage * 128 + (wave & 1) * 64) * 4); };
+    auto end_tile = [&]() {
+      iss_stage = iss_stage == kStages - 1 ? 0 : iss_stage + 1;
+      wait_vmcnt<ring::loads_kept_after_iteration(R, true)>();
+      // a bare barrier: the reads of this tile have returned (the products above used them), and those of the next tile's
+      // first fragments, still on their way, come from a stage that the next iteration does not refill either
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
     auto run_tiles = [&](auto masked_c, int t_lo, int t_hi) {
       for (int x = (t_hi - t_lo) * rep, t = t_hi - 1, hq = 0; x > 0; --x, ++it) {
         const int nstage = stage == kStages - 1 ? 0 : stage + 1;
         const int i0 = (qt_start + t) * kBK;
-        uint32_t off = 0, tr_next = 0, tra_next[2 * MB];
+        uint32_t tr_next = 0, tra_next[2 * MB];
         bool more = false, wrap = false;
         int64_t q_step = 0, d_step = 0;
         int s_step = 0, left_step = 0;
-        auto offset = [&](int k) {  // rows past the last query re-read it
-          const uint32_t last = min(left_it, kBK) - 1, row = (k >> 1) * 4 * Z::kRowsPerInst;
-          if (k & 1) off = min(d_row + row * dstep, last * dstep) + src.y;
-          else off = min(q_row + row * D * 2, last * D * 2) + src.y;
-        };
-        auto load = [&](int k) {
-          const uint32_t dst = lds0 + iss_stage * kStageBytes + wave * 1024 + (k >> 1) * 4096;
-          if (k & 1) gload_lds16_so(d_it, off, dst + Z::kTileBytes);
-          else gload_lds16_so(q_it, off, dst);
-        };
         step(masked_c, s0, d0, s1, d1, 0, i0,
              [&](int slot) {
                const int j = slot - kA;
@@ -1082,7 +1094,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
              [&](int slot) {
                const int j = slot - kA, k = slot_load(j, kAt1, kLoads - kFirst);
                if (k >= 0) load(kFirst + k);
-               if (j == kStatAt) gload_lds4_so(s_it, off, ldl0 + (iss_stage * 128 + (wave & 1) * 64) * 4);
+               if (j == kStatAt) stat_load();
                if (j == kMoveAt) q_it += q_step;
                if (j == kMoveAt + 1) d_it += d_step;
                if (j == kMoveAt + 2) { s_it += s_step; left_it += left_step; }
@@ -1092,25 +1104,94 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
                if (j == kB / 2 - 3) tr_next = tr_lane + nstage * kStageBytes;
                if (x2 >= 0 && x2 < 2 * MB) tra_next[x2] = tr_addr(tr_next, x2);
                if (k >= 0) offset(kFirst + k);
-               if (j == kStatAt - 1) off = (uint32_t)min(lane, left_it - 1) * 4;
+               if (j == kStatAt - 1) stat_offset();
              });
-        iss_stage = iss_stage == kStages - 1 ? 0 : iss_stage + 1;
-        wait_vmcnt<ring::loads_kept_after_iteration(R, true)>();
-        // a bare barrier: the reads of this tile have returned (the products above used them), and those of the next tile's
-        // first fragments, still on their way, come from a stage that the next iteration does not refill either
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        end_tile();
         stage = nstage;
 #pragma unroll
         for (int i = 0; i < 2 * MB; ++i) tra[i] = tra_next[i];
         if (++hq == rep) { hq = 0; --t; }
       }
     };
+    // Blocks whose queries all lie before this wave's first key are left out (6 of 16 per head in a full workgroup on the diagonal), not
+    // computed and masked: 0 times a value that is not finite would reach dV and dK of keys that the query does not see.  The stream ends with
+    // them.  Of the tiles [t_none, t_half), one at most, the wave needs the second block (its scores first, then the rest: nothing overlaps),
+    // of [0, t_none) nothing: it requests its share and keeps the others company.  What the block before has computed ahead nobody reads.
+    // dK/dV, all blocks -> this, us: head_dim 64, 8 x 18 / 6 heads, 2048 tokens 157.1 -> 154.8, 24 x 16 / 4, 1024 121.1 -> 116.5, 96 x 16 / 2, 384 84.0 ->
+    // 78.2; head_dim 128 (the others' products of a workgroup that is alone on its CU set the time) 12 x 16 / 4, 2048 373.6 -> 372.7.
+    const int before = p.causal ? max(kw0 - p.q_start, 0) : 0;  // queries before the wave's first key
+    const int t_none = min(max(before / kBK - qt_start, 0), n_vis), t_half = min(max((before + 32) / kBK - qt_start, 0), n_vis);
+    auto request = [&]() {  // a tile's loads outside the slots
+#pragma unroll
+      for (int k = 0; k < kLoads; ++k) { offset(k); load(k); }
+      stat_offset();
+      stat_load();
+      if (it + R.issue_ahead + 1 < n_it) advance();
+    };
+    auto run_second_blocks = [&](int t) {
+      for (int hq = 0; hq < rep; ++hq, ++it) {  // its fragments and statistics are there, as at the start of every iteration
+        const int nstage = stage == kStages - 1 ? 0 : stage + 1;
+#pragma unroll
+        for (int i = 0; i < kA; ++i) {
+          const int o = order(i);
+          if (o < KS) mfma32_fixed(s1, qf[o], kreg[o]);
+          else mfma32_fixed(d1, df[o - KS], vreg[o - KS]);
+        }
+        request();
+        bf16x8 dT[MB][2], qT[MB][2];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            dT[mb][half] = frag_tr_at<D>(tra[2 * mb], tra[2 * mb + 1], 2 + half, Z::kTileBytes);
+            qT[mb][half] = frag_tr_at<D>(tra[2 * mb], tra[2 * mb + 1], 2 + half, 0);
+          }
+        mfma32_fixed_done(s1);
+        mfma32_fixed_done(d1);
+        const int ib = (qt_start + t) * kBK + 32, lo = key - p.q_start - ib - 4 * hh, hi = p.Sq - ib - 4 * hh;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int c = 8 * (r >> 2) + (r & 3);
+          if (c < lo || c >= hi) s1[r] = -INFINITY;
+          s1[r] = fast_exp2(s1[r]);
+          d1[r] *= s1[r];
+        }
+        bf16x8 pw[2] = {pack_c_half(s1, 0), pack_c_half(s1, 1)}, dw[2] = {pack_c_half(d1, 0), pack_c_half(d1, 1)};
+#pragma unroll
+        for (int half = 0; half < 2; ++half) { mfma32_settle<false>(pw[half]); mfma32_settle<false>(dw[half]); }
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) {
+            mfma32_acc(dvacc[mb], dT[mb][half], pw[half]);
+            mfma32_acc(dkacc[mb], qT[mb][half], dw[half]);
+          }
+        rm_next = rm_lane + nstage * kStageBytes;
+        st_next = st_lane + nstage * 512;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          qf[ks] = swz_frag_rm<D>(rm_next, 1, ks);
+          df[ks] = swz_frag_rm<D>(rm_next + Z::kTileBytes, 1, ks);
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) load_stat(s1, d1, st_next, 1, c);
+#pragma unroll
+        for (int x = 0; x < 2 * MB; ++x) tra[x] = tr_addr(tr_lane + nstage * kStageBytes, x);
+        end_tile();
+        stage = nstage;
+      }
+    };
+    const int t_inside = min(t_diag, t_full);
     run_tiles(IC<2>{}, t_end, n_vis);
     run_tiles(IC<0>{}, t_diag, t_end);
-    run_tiles(IC<2>{}, min(t_diag, t_full), t_diag);
-    run_tiles(IC<1>{}, 0, min(t_diag, t_full));
+    run_tiles(IC<2>{}, max(t_half, t_inside), t_diag);
+    run_tiles(IC<1>{}, t_half, t_inside);
+    if (t_half > t_none) run_second_blocks(t_none);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // fragments requested for a block that is left out: no product waits for them
+    for (int x = t_none * rep; x > 0; --x, ++it) {
+      request();
+      end_tile();
+    }
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) { mfma32_acc_done(dvacc[mb]); mfma32_acc_done(dkacc[mb]); }
     static_assert(R.always_requests, "no branch around the loads of an iteration");

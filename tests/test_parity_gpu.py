@@ -540,6 +540,36 @@ def test_bf16_backward_pipelines_against_single_batches(gpu_device, B, H, Hkv, S
             assert (a - b).norm() <= 1e-3 * b.norm(), (n, float((a - b).norm() / b.norm()))
 
 
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,q_start", [
+    (11, 18, 6, 999, 999, 64, 0),        # launches that take the laid-out dK/dV loop
+    (9, 12, 4, 1030, 2050, 64, 1020),    # ... the diagonal off the tiles' edges
+    (9, 8, 4, 1000, 1000, 128, 0),
+    (8, 8, 4, 500, 1100, 128, 600),
+    (4, 18, 6, 999, 999, 64, 0),         # ... and the compiler's
+])
+def test_bf16_non_finite_rows_stay_with_the_keys_they_see(gpu_device, B, H, Hkv, Sq, Sk, D, q_start):
+    """One query row of every batch with a gradient or a query that is not finite: dk and dv of the keys behind the 32-key block in
+    which the row's 32-query block ends are the same bits as without it, as are the other heads' and dq's other rows."""
+    x = gen(B, H, Hkv, Sq, Sk, D, BF16, seed=66)
+    bad = {n: x[n].clone() for n in ("q", "d_o")}
+    rows = [(5, 40, 70, 100, 127, 128, 300, 400)[b % 8] for b in range(B)]
+    for b, i in enumerate(rows):
+        if b % 2: bad["q"][b, b % H, i] = math.nan
+        else: bad["d_o"][b, b % H, i] = math.inf
+    ref, got = (run_gpu(t, gpu_device, q_start=q_start) for t in (x, dict(x, **bad)))
+    for b, i in enumerate(rows):
+        h, g = b % H, b % H // (H // Hkv)
+        first = 32 * ((i // 32 * 32 + 31 + q_start) // 32) + 32  # first key that must not notice
+        for n in ("dk", "dv"):
+            assert not got[n][b, g, : i + q_start + 1].float().isfinite().any(-1).any(), (n, b)
+            assert torch.equal(got[n][b, g, first:], ref[n][b, g, first:]), (n, b, i)
+            others = [o for o in range(Hkv) if o != g]
+            assert torch.equal(got[n][b, others], ref[n][b, others]), (n, b)
+        keep = torch.ones(H, Sq, dtype=torch.bool)
+        keep[h, i] = False
+        assert torch.equal(got["dq"][b][keep], ref["dq"][b][keep]), b
+
+
 @pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,kw,gen_kw,use_rope", [
     (1, 2, 1, 65, 65, 64, {}, {"extras": True}, True),                         # one row in the last workgroup, its second wave beyond the end
     (1, 2, 2, 31, 130, 64, {"q_start": 99}, {"extras": True}, False),          # fewer rows than one wave owns
