@@ -139,14 +139,15 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     if (tid < D) a.dg_part[(int64_t)blockIdx.x * D + tid] = 0.f;
     return;
   }
-  const int b = wg.b, g = wg.g, h = wg.g * rep + wg.hh;
-  const int q0 = wg.tile * BQ;
+  const int b = __builtin_amdgcn_readfirstlane(wg.b), g = __builtin_amdgcn_readfirstlane(wg.g);  // divided in vector registers
+  const int h = __builtin_amdgcn_readfirstlane(wg.g * rep + wg.hh);
+  const int q0 = __builtin_amdgcn_readfirstlane(wg.tile) * BQ;
   const int row_wave = PARTS == 1 ? wave : wave % kRowWaves, part = PARTS == 1 ? 0 : wave / kRowWaves;
   const int qw0 = q0 + row_wave * 32;
   const int row = qw0 + ln;
   const bool live = row < p.Sq;
   const int row_c = live ? row : p.Sq - 1;  // padding lanes recompute the last row and store nothing
-  const int64_t ridx = ((int64_t)b * p.H + h) * p.Sq + row_c;
+  const int64_t head_row = ((int64_t)b * p.H + h) * p.Sq;  // scalar: what the epilogue needs of it costs no vector registers over the loop
 
   int kend = p.Sk;
   if (p.causal) kend = min(p.Sk, q0 + BQ + p.q_start);
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     if constexpr (ROPE) issue_rope_rows(kCosRows, kSinRows);
   }
   if constexpr (!ROPE) issue_o_rows();
-  const float lse_row = p.lse[ridx];
+  const float lse_row = (p.lse + head_row)[row_c];
   // the conditional reads last: the compiler waits for every outstanding load where their branches join
   float gate_z = 0.f;
   if (p.gate.ptr)
@@ -362,7 +363,7 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     // dQ, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 435 -> 390 (939 k -> 764 k cycles, matrix pipe 42 -> 52 % busy; a quarter
     // of the launch is now the workgroups' first and last thousands of cycles, one workgroup a CU); head_dim 64, 2 x 18 / 6
     // heads, 8192 tokens 418 -> 402 (776 k -> 698 k cycles, 57 -> 64 % busy, 1.86 -> 1.74 GHz).  At head_dim 64
-    // everything is in ordinary registers (250 of 256): a kernel that uses both files gets half of each, and the ordinary
+    // everything is in ordinary registers (248 of 256, 255 with a rotary embedding): a kernel that uses both files gets half of each, and the ordinary
     // half spills.
     constexpr int kA = 2 * KS, kB = 2 * MB;
     auto order = [](int i) { return (i & 1) * KS + (i >> 1); };  // i-th product: k-step of S^T, or KS + that of dP^T
@@ -648,8 +649,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     if (live) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        *reinterpret_cast<bf16x8*>(a.qhat + ridx * D + 16 * ks + 8 * hh) = qreg[ks];
-        if (a.do_eff) *reinterpret_cast<bf16x8*>(reinterpret_cast<uint16_t*>(a.do_eff) + ridx * D + 16 * ks + 8 * hh) = doreg[ks];
+        *reinterpret_cast<bf16x8*>(a.qhat + head_row * D + (int64_t)row_c * D + 16 * ks + 8 * hh) = qreg[ks];
+        if (a.do_eff) *reinterpret_cast<bf16x8*>(reinterpret_cast<uint16_t*>(a.do_eff) + head_row * D + (int64_t)row_c * D + 16 * ks + 8 * hh) = doreg[ks];
       }
       if (hh == 0) {
         float stat_d = -delta, stat_l = nlse2;
@@ -658,8 +659,8 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
           stat_l = on ? nlse2 + __log2f(gfac) : -INFINITY;
           stat_d = on ? -delta / gfac : 0.f;
         }
-        a.delta[ridx] = stat_d;
-        a.nlse2[ridx] = stat_l;
+        (a.delta + head_row)[row_c] = stat_d;
+        (a.nlse2 + head_row)[row_c] = stat_l;
         if (p.gate.ptr)
           reinterpret_cast<uint16_t*>(p.dgate.ptr)[(int64_t)b * p.dgate.stride_b + (int64_t)row * p.dgate.stride_s + (int64_t)h * p.dgate.stride_h] = f32_to_bf16(dgate_row);
       }

@@ -136,19 +136,38 @@ def test_the_checker_sees_what_it_is_for(wrong, right):
     assert not violations(right)
 
 
-def test_built_kernels_keep_the_wait_states(tmp_path):
+def _code_objects(tmp_path):
+    """The library's device code, one file per source, and the path of the LLVM tools."""
     objdump = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
     if not os.path.exists(objdump) or not os.path.exists(LIB):
         pytest.skip("no llvm-objdump, or the library is not built")
     so = shutil.copy(LIB, tmp_path / "lib.so")  # the code objects are written beside the file
     subprocess.run([objdump, "--offloading", str(so)], check=True, stdout=subprocess.DEVNULL, cwd=tmp_path)
-    objects = [f for f in os.listdir(tmp_path) if f.endswith("gfx950")]
+    objects = [str(tmp_path / f) for f in os.listdir(tmp_path) if f.endswith("gfx950")]
     assert objects
+    return objects, os.path.dirname(objdump)
+
+
+def test_built_kernels_keep_the_wait_states(tmp_path):
+    objects, tools = _code_objects(tmp_path)
     n_mfma = 0
     for f in objects:
-        out = subprocess.run([objdump, "-d", "--mcpu=gfx950", "--no-show-raw-insn", str(tmp_path / f)], check=True, capture_output=True, text=True).stdout
+        out = subprocess.run([os.path.join(tools, "llvm-objdump"), "-d", "--mcpu=gfx950", "--no-show-raw-insn", f], check=True, capture_output=True, text=True).stdout
         lines = out.splitlines()
         n_mfma += sum("v_mfma" in l for l in lines)
         found = violations(lines)
         assert not found, (f, len(found), found[:4])
     assert n_mfma > 0
+
+
+def test_bf16_backward_kernels_keep_everything_in_registers(tmp_path):
+    """The bf16 backward loops count their vector-memory operations and are laid out for the registers there are: no scratch."""
+    objects, tools = _code_objects(tmp_path)
+    seen = {}
+    for f in objects:
+        notes = subprocess.run([os.path.join(tools, "llvm-readelf"), "--notes", f], check=True, capture_output=True, text=True).stdout
+        for kernel in notes.split("  - .agpr_count:")[1:]:
+            name = re.search(r"\.name:\s+(\S+)", kernel)[1]
+            if re.search(r"bwd_(dq|dkdv)_bf16_kernel", name):
+                seen[name] = [int(re.search(key + r":\s+(\d+)", kernel)[1]) for key in (r"\.vgpr_spill_count", r"\.private_segment_fixed_size")]
+    assert len(seen) >= 16 and all(v == [0, 0] for v in seen.values()), {n: v for n, v in seen.items() if v != [0, 0]}
