@@ -59,32 +59,33 @@ constexpr int loads_kept_after_iteration(const Protocol& p, bool requested_a_til
   return requested_a_tile || p.always_requests ? p.keep_tiles * p.loads_per_tile : 0;
 }
 
-// ---- the kernels' protocols.  passes = wave-wide 16-byte loads per wave and [64, D] tile (2 at both head dims).
+// ---- the kernels' protocols.  passes = wave-wide 16-byte loads per wave and [64, D] tile (2 at head_dim 64, 4 at 128).
 // Forward: `stages` and the rows of the query block (q_stages stages of 128 rows, the LAST stages of the ring) depend
 // on the shape; the tile of iteration jt + stages - 1 is requested at the top of iteration jt.
 constexpr Protocol forward(int stages, int q_stages, int passes) {
   return Protocol{stages, 2 * passes, stages - (q_stages > 1 ? q_stages : 1), stages - q_stages, q_stages, stages - 1,
                   false, true, stages - 1, stages - 3};
 }
-// dQ: key tile 0 in stage 0, the q / dO / o row blocks in stages 1..3, then key tiles 1 and 2; tile 1 is a late
-// request, hence the wait before the loop.
+// The backward's 128-row workgroups: always_requests where the loop is laid out by hand, not in the compiler's.
 constexpr Protocol requesting_always(Protocol p, bool on) {
   p.always_requests = on;
   return p;
 }
-constexpr Protocol dq(int passes, bool always_requests = true) {
+// dQ: key tile 0 in stage 0, the q / dO / o row blocks in stages 1..3, then key tiles 1 and 2; tile 1 is a late
+// request, hence the wait before the loop.
+constexpr Protocol dq(int passes, bool always_requests) {
   return requesting_always(Protocol{4, 2 * passes, 1, 1, 3, 3, true, false, 3, 1, 0, 0, true}, always_requests);
 }
 // dQ with a rotary embedding: the table rows of the workgroup's 128 positions are row blocks too.  First phase: q,
 // cos, sin, dO in stages 0..3; second phase: key tiles 0..2 in stages 0..2 and the o block in stage 3 (everything
 // awaited: no late tiles).  The cos and sin blocks come once more behind the loop, for the epilogue.
-constexpr Protocol dq_rope(int passes, bool always_requests = true) {
+constexpr Protocol dq_rope(int passes, bool always_requests) {
   return requesting_always(Protocol{4, 2 * passes, 3, 3, 1, 3, false, false, 3, 1, 4, 2, true}, always_requests);
 }
 // dK/dV: (Qhat, dO) tiles 0 and 1 in stages 0 and 1 with the Khat / V' row blocks in stages 2 and 3, then tile 2;
 // a tile is the two [64, D] tiles plus one row-statistics load.
 // Behind the loop: the raw k block (and, with a value residual, the raw v and v_first blocks) for the epilogue.
-constexpr Protocol dkdv(int passes, bool always_requests = true) {
+constexpr Protocol dkdv(int passes, bool always_requests) {
   return requesting_always(Protocol{4, 2 * passes + 1, 2, 2, 2, 3, false, false, 3, 1, 0, 3, false}, always_requests);
 }
 

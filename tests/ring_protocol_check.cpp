@@ -11,7 +11,8 @@
 //     were retired by a wait in an epoch < e (every wave waited for its own quarter before a barrier that the reader
 //     has passed);
 //   - a request that refills a stage in epoch e is safe iff the last read of the stage's previous content happened
-//     in an epoch < e (a barrier separates the slowest reader from the first new byte) and that content had landed.
+//     in an epoch < e (a barrier separates the slowest reader from the first new byte) and that content had landed; content
+//     that nobody read must have been retired in an epoch < e (every wave's part of it).
 // Exit code 0 and "ok" per line when everything holds; the deliberately broken protocols at the end must each be
 // reported as a violation, or the program fails: a checker that cannot see the known bug proves nothing.
 #include <cstdio>
@@ -113,6 +114,10 @@ std::string replay(const Protocol& p, const std::vector<Op>& ops) {
         if (s.ever) {
           if (s.loads_pending > 0) {
             snprintf(buf, sizeof buf, "op %zu: stage %d refilled with content %d while content %d is still in flight", i, o.stage, o.content, s.content);
+            return buf;
+          }
+          if (s.last_read_epoch < 0 && s.retired_epoch >= epoch) {  // never read: nothing else says that the other waves' parts have landed
+            snprintf(buf, sizeof buf, "op %zu: stage %d refilled with content %d in the epoch of this wave's wait for content %d (no barrier in between)", i, o.stage, o.content, s.content);
             return buf;
           }
           if (s.last_read_epoch >= epoch) {
@@ -248,9 +253,12 @@ int main() {
     const Named shipped[] = {
         {"forward, 32 rows per wave (3 stages; head_dim 64 up to 2048 keys, head_dim 128)", forward(3, 1, passes)},
         {"forward, 64 rows per wave (4 stages; head_dim 64 beyond 2048 keys)", forward(4, 2, passes)},
-        {"dQ", dq(passes)},
-        {"dQ with a rotary embedding (two start-up phases, table rows once more behind the loop)", dq_rope(passes)},
-        {"dK/dV (k, v, v_first rows behind the loop; a key tile may see no query at all)", dkdv(passes)},
+        {"dQ", dq(passes, false)},
+        {"dQ with a rotary embedding (two start-up phases, table rows once more behind the loop)", dq_rope(passes, false)},
+        {"dK/dV (k, v, v_first rows behind the loop; a key tile may see no query at all)", dkdv(passes, false)},
+        {"dQ requesting a tile in every iteration", dq(passes, true)},
+        {"dQ with a rotary embedding requesting a tile in every iteration", dq_rope(passes, true)},
+        {"dK/dV requesting a tile in every iteration", dkdv(passes, true)},
     };
     for (const Named& k : shipped) {
       const bool can_be_empty = k.p.loads_per_tile == 2 * passes + 1;  // dK/dV: key tiles beyond every query
@@ -295,18 +303,23 @@ int main() {
 
   // ---- protocols that are wrong on purpose: each must be caught
   struct Broken { const char* name; Protocol p; };
-  Protocol dq_no_wait = dq(passes);
-  dq_no_wait.wait_before_loop = false;  // the start-up that shipped once: tile 1, a late request, not awaited before iteration 0
-  Protocol dq_keep2 = dq(passes);
-  dq_keep2.keep_tiles = 2;              // the iteration's wait leaves the tile in flight that the next iteration prefetches from
-  Protocol dkdv_ahead4 = dkdv(passes);
-  dkdv_ahead4.issue_ahead = 4;          // refills the stage the iteration has just read, before the barrier
+  Protocol dq_no_wait[2], dq_keep2[2], dkdv_ahead4[2];
+  for (const bool always : {false, true}) {
+    dq_no_wait[always] = dq_keep2[always] = dq(passes, always);
+    dkdv_ahead4[always] = dkdv(passes, always);
+    dq_no_wait[always].wait_before_loop = false;  // the start-up that shipped once: tile 1, a late request, not awaited before iteration 0
+    dq_keep2[always].keep_tiles = 2;              // the iteration's wait leaves the tile in flight that the next iteration prefetches from
+    dkdv_ahead4[always].issue_ahead = 4;          // refills the stage the iteration has just read, before the barrier
+  }
   Protocol fwd_early_into_rows = forward(4, 2, passes);
   fwd_early_into_rows.early_tiles = 3;  // an early tile lands in a stage the query rows borrow
   const Broken broken[] = {
-      {"dQ without the wait before the loop", dq_no_wait},
-      {"dQ leaving two tiles in flight per iteration", dq_keep2},
-      {"dK/dV requesting four tiles ahead in a ring of four", dkdv_ahead4},
+      {"dQ without the wait before the loop", dq_no_wait[0]},
+      {"dQ leaving two tiles in flight per iteration", dq_keep2[0]},
+      {"dK/dV requesting four tiles ahead in a ring of four", dkdv_ahead4[0]},
+      {"dQ, always requesting, without the wait before the loop", dq_no_wait[1]},
+      {"dQ, always requesting, leaving two tiles in flight per iteration", dq_keep2[1]},
+      {"dK/dV, always requesting, four tiles ahead in a ring of four", dkdv_ahead4[1]},
       {"forward with an early tile in a borrowed stage", fwd_early_into_rows},
   };
   for (const Broken& k : broken) {
@@ -314,9 +327,9 @@ int main() {
     printf("%-93s %s\n", k.name, v.empty() ? "NOT CAUGHT" : ("caught: " + v).c_str());
     failures += v.empty();
   }
-  {  // a vmcnt unit larger than what a wave really issues per tile (say the statistics load was dropped from the
-     // kernel but not from the count): the iteration's wait then leaves part of the next tile in flight
-    const Protocol p = dkdv(passes);
+  for (const bool always : {false, true}) {  // a vmcnt unit larger than what a wave really issues per tile (say the statistics
+     // load was dropped from the kernel but not from the count): the iteration's wait then leaves part of the next tile in flight
+    const Protocol p = dkdv(passes, always);
     std::vector<Op> ops = wave_program(p, 12, 2 * p.loads_per_tile);
     for (Op& o : ops)
       if (o.kind == REQUEST && o.content >= 0) o.n = p.loads_per_tile - 1;
@@ -336,7 +349,12 @@ int main() {
     return ops;
   };
   struct BrokenOps { const char* name; Protocol p; std::vector<Op> ops; };
-  const Protocol dr = dq_rope(passes), dk = dkdv(passes);
+  const Protocol dr = dq_rope(passes, false), dk = dkdv(passes, false), da = dq(passes, true), ka = dkdv(passes, true);
+  const int iterations = 12;
+  // an iteration that requested nothing waits as if it had: the tail of the loop reads tiles that are still in flight
+  std::vector<Op> keeping = wave_program(dk, iterations, 2 * dk.loads_per_tile);
+  for (size_t i = keeping.size(), left = (size_t)dk.issue_ahead; i-- > 0 && left > 0;)
+    if (keeping[i].kind == WAIT) { keeping[i].n = dk.keep_tiles * dk.loads_per_tile; --left; }
   const BrokenOps broken_ops[] = {
       {"dK/dV reading its epilogue row blocks without the wait behind their requests", dk,
        drop(wave_program(dk, 12, 2 * dk.loads_per_tile, 3), WAIT, 0)},
@@ -346,6 +364,15 @@ int main() {
        drop_nth(wave_program(dr, 12, 2 * dr.loads_per_tile, 2), BARRIER, 1)},
       {"dQ (rotary) writing the epilogue's scratch over the ring without a barrier behind the table-row reads", dr,
        drop(wave_program(dr, 12, 2 * dr.loads_per_tile, 2), BARRIER, 0)},
+      {"dK/dV ending iterations that requested nothing with the wait of those that did", dk, keeping},
+      {"dQ, always requesting, writing scratch data over a tile in flight: no wait behind the loop", da,
+       drop(wave_program(da, iterations, 2 * da.loads_per_tile), WAIT, 0)},
+      {"dQ, always requesting, writing scratch data over another wave's part of a tile: no barrier behind the wait", da,
+       drop(wave_program(da, iterations, 2 * da.loads_per_tile), BARRIER, 0)},
+      {"dK/dV, always requesting, row blocks over a tile in flight: no wait behind the loop", ka,
+       drop(wave_program(ka, iterations, 2 * ka.loads_per_tile, 3), WAIT, 1)},
+      {"dK/dV, always requesting, row blocks over another wave's part of a tile: no barrier behind the wait", ka,
+       drop(wave_program(ka, iterations, 2 * ka.loads_per_tile, 3), BARRIER, 1)},
   };
   for (const BrokenOps& k : broken_ops) {
     const std::string v = replay(k.p, k.ops);

@@ -36,12 +36,12 @@ def test_shipped_protocols_hold_and_broken_ones_are_caught(checker):
     assert proc.returncode == 0, out
     lines = out.strip().splitlines()
     ok = [l for l in lines if l.rstrip().endswith(" ok")]
-    # five pipelines (forward 2 shapes, dQ, dQ with rotary tables, dK/dV) and four of 64-row workgroups at both head dims;
-    # decode with and without staged tables and a value residual at both
-    assert len(ok) == 10 + 8 + 8, out
+    # eight pipelines (forward 2 shapes; dQ, dQ with rotary tables and dK/dV, each with and without a request in every iteration) and four
+    # of 64-row workgroups at both head dims; decode with and without staged tables and a value residual at both
+    assert len(ok) == 16 + 8 + 8, out
     assert "VIOLATION" not in out and "NOT CAUGHT" not in out, out
     caught = [l for l in lines if "caught:" in l]
-    assert len(caught) == 9 + 3 + 5, out
+    assert len(caught) == 7 + 2 + 9 + 3 + 5, out
     # the start-up bug that once shipped must be reported as exactly what it was
     bug = next(l for l in caught if l.startswith("dQ without the wait before the loop"))
     assert "read of content 1" in bug and "before it has landed" in bug, bug
