@@ -488,13 +488,23 @@ def test_bf16_dkdv_workgroup_shapes(gpu_device, B, H, Hkv, Sq, Sk, D, kw):
 ])
 def test_bf16_dkdv_pipeline_ends(gpu_device, B, H, Hkv, Sq, Sk, D, kw):
     """dK/dV of launches that fill the card (128-key workgroups) at the shortest streams and at ragged ends; at head_dim 128 the
-    loop runs two blocks ahead of itself and requests a tile in every iteration.
+    loop runs two blocks ahead of itself and requests a tile in every iteration (at head_dim 64 it takes longer streams: the next test).
     Outliers: a launch that fills the card has millions of entries, and dk of a row that few queries see is a sum of few terms
     with roundings of 2^-9 each against a result that cancels; over the 198-head case dk is 3.7e-3 from float64 in norm and
     one entry of 2.5 million is 0.043 away where the elementwise bound says 0.04 (both to all digits also with the products
     in the order of tiles, head by head).  One in a million may be up to twice the bound away."""
     assert B * Hkv * (-(-Sk // 128)) > 256
     _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, D, seed=63, outliers=(1e-6, 2.0), rope=orc.rope_tables(max(Sq, Sk), 10000.0, D), **kw)
+
+
+def test_bf16_dkdv_pipeline_ends_many_heads_a_group(gpu_device):
+    """The same at head_dim 64, whose laid-out loop takes streams of 48 tiles and more: one tile of every head, its second block of one
+    query; a second key tile of one row (outliers: as above).  More such ends stand with the single batches below: where 24
+    heads of a group add up, the bf16 roundings of P and dS (2^-9 each, some thousand of them) pass the elementwise
+    bound against float64 in either form of the loop."""
+    B, H, Hkv, Sq, Sk = 3, 86 * 48, 86, 33, 129
+    assert B * Hkv * (-(-Sk // 128)) > 512 and H // Hkv * (-(-Sq // 64)) >= 48
+    _case(gpu_device, BF16, B, H, Hkv, Sq, Sk, 64, seed=67, outliers=(1e-6, 2.0), rope=orc.rope_tables(max(Sq, Sk), 10000.0, 64), q_start=96)
 
 
 @pytest.mark.parametrize("use_rope", [False, True])
@@ -519,6 +529,8 @@ def test_bf16_dq_pipeline_ends(gpu_device, B, H, Hkv, Sq, Sk, kw, use_rope):
     (9, 12, 4, 1030, 2050, {"q_start": 1020}, False, True),  # both, queries at the end of the keys
     (6, 18, 6, 2017, 2017, {}, True, False),                 # both, ragged
     (5, 24, 6, 777, 2300, {"causal": False}, False, False),  # both, no mask but the ends
+    (4, 24 * 43, 43, 66, 257, {}, False, True),              # dK/dV: 24 short heads, the last tile of two queries; the third key tile sees no query
+    (3, 48 * 58, 58, 60, 300, {"q_start": 240}, True, True), # 48 heads of one tile; a third key tile that only sees its last block
 ])
 def test_bf16_backward_pipelines_against_single_batches(gpu_device, B, H, Hkv, Sq, Sk, kw, extras, use_rope):
     """head_dim 64: a launch long and large enough for the backward loops that are laid out instruction by instruction, against
@@ -538,6 +550,67 @@ def test_bf16_backward_pipelines_against_single_batches(gpu_device, B, H, Hkv, S
             scale = torch.maximum(b.abs(), b.square().mean().sqrt())
             assert ((a - b).abs() <= 2.0 ** -7 * scale).all(), (n, float(((a - b).abs() / scale).max()))
             assert (a - b).norm() <= 1e-3 * b.norm(), (n, float((a - b).norm() / b.norm()))
+
+
+@pytest.mark.parametrize("option", ["gated copy", "rows switched off", "no norm"])
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,q_start", [(9, 12, 4, 1030, 2050, 64, 1020), (9, 8, 4, 1000, 1000, 128, 0)])
+def test_bf16_backward_pipelines_options_against_single_batches(gpu_device, B, H, Hkv, Sq, Sk, D, q_start, option):
+    """The laid-out loops on what else they stream: a copy of the gradient that the dQ kernel writes (gate scale not positive), rows whose
+    gate factor vanishes (their -lse is -inf), scores of any size (no normaliser).  Against single batches, with the bounds
+    of the test above."""
+    assert B * Hkv * (-(-Sk // 128)) > 512 // (D // 64) and B * H * (-(-Sq // 128)) > 384
+    x = gen(B, H, Hkv, Sq, Sk, D, BF16, extras=option != "no norm", seed=68)
+    kw = {"q_start": q_start, "rope": orc.rope_tables(Sk, 10000.0, D)}
+    if option == "gated copy": kw["gate_scale"] = -1.5
+    if option == "rows switched off": x["gate_logits"][:, ::3] = -200.0
+    if option == "no norm": kw["qk_norm"] = False
+    got = run_gpu(x, gpu_device, **kw)
+    per_batch = [n for n in ("q", "k", "v", "d_o", "v_first", "gate_logits") if x.get(n) is not None]
+    for i in (0, B - 1):
+        one = run_gpu(dict(x, **{n: x[n][i:i + 1] for n in per_batch}), gpu_device, **kw)
+        for n in ("dq", "dk", "dv") + (("dv_first", "dgate_logits") if "gate_logits" in per_batch else ()):
+            a, b = got[n][i].float(), one[n][0].float()
+            scale = torch.maximum(b.abs(), b.square().mean().sqrt())
+            assert ((a - b).abs() <= 2.0 ** -7 * scale).all(), (n, float(((a - b).abs() / scale).max()))
+            assert (a - b).norm() <= 1e-3 * b.norm(), (n, float((a - b).norm() / b.norm()))
+
+
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,q_start,gate_scale,layout", [
+    (9, 12, 4, 1030, 2050, 64, 1020, None, "b seq head d"),  # dQ and dK/dV
+    (9, 12, 4, 1030, 2050, 64, 1020, -1.5, "b seq head d"),  # ... which streams a copy of the gradient
+    (43, 96, 6, 190, 190, 64, 0, None, "b seq head d"),      # dK/dV, short heads
+    (43, 96, 6, 190, 190, 64, 0, None, "rows far apart"),
+    (30, 8, 4, 300, 300, 128, 0, None, "b seq head d"),
+    (30, 8, 4, 300, 300, 128, 0, None, "rows far apart"),
+    (30, 8, 4, 300, 300, 128, 0, -1.5, "rows far apart"),
+])
+def test_bf16_backward_pipelines_with_strided_operands(gpu_device, B, H, Hkv, Sq, Sk, D, q_start, gate_scale, layout):
+    """The laid-out loops walk the heads and tiles of a gradient, and the tiles of v, that have strides of their own: the same bits
+    as with contiguous ones.  Far apart: the largest row stride that is accepted (3 to 5 GB an operand)."""
+    assert B * Hkv * (-(-Sk // 128)) > 512 // (D // 64) and (D == 128 or H // Hkv * (-(-Sq // 64)) >= 48)
+    far = 2**23 - 8
+    x = gen(B, H, Hkv, Sq, Sk, D, BF16, extras=gate_scale is not None, seed=69)
+    x = {n: t.to(gpu_device) for n, t in x.items() if t is not None}
+    kw = {"q_start": q_start}
+    if gate_scale is not None:
+        kw.update(gate_scale=gate_scale, gate_logits=x["gate_logits"])
+
+    def placed(t):
+        b, h, s, d = t.shape
+        if layout == "b seq head d":
+            return t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
+        out = torch.empty(s * far, dtype=t.dtype, device=t.device).as_strided((b, h, s, d), (h * d, d, far, 1))
+        return out.copy_(t)
+
+    def grads(place):
+        q, k = x["q"].clone().requires_grad_(), x["k"].clone().requires_grad_()
+        v = place(x["v"]).requires_grad_()
+        y = qknorm_attention(q, k, v, x["g_q"], x["g_k"], **kw)
+        return torch.autograd.grad(y, [q, k, v], place(x["d_o"]))
+
+    for n, a, b in zip(("dq", "dk", "dv"), grads(placed), grads(lambda t: t)):
+        assert torch.equal(a, b), n
+    torch.cuda.empty_cache()
 
 
 @pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,q_start", [
@@ -2127,7 +2200,7 @@ def _sweep_cases(n, seed):
 @pytest.mark.parametrize("case", _sweep_cases(48, seed=2024), ids=lambda c: f"sweep{c[0]}")
 def test_seeded_sweep(gpu_device, case):
     """Ragged lengths around every tile size, caches of odd lengths, GQA ratios, every optional operand, both
-    dtypes, forward-only (decode kernels where the shape allows) and forward + backward.  Here (and only here)
+    dtypes, forward-only (decode kernels where the shape allows) and forward + backward.  Here
     one element in 10^4 of a tensor may exceed the tolerance, by at most a factor 2: with gate_scale 2, a value
     residual and head_dim 128 the dS entries of the first rows reach +-10 and a couple of dk entries of the
     first keys collect rounding errors of 4e-2 (the fp32 kernels agree with the oracle to 6e-6 on that case)."""
