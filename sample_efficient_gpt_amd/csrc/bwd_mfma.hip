@@ -67,11 +67,16 @@ inline int dq_parts(const segpt_attn_params& p) {
 
 // Whether a launch of 128-row workgroups takes the kernel whose loop is laid out instruction by instruction (PIPE).  Its start and end
 // cost a workgroup a few hundred cycles more (a block's scores that nothing overlaps, a tile that is requested once too often).
-// head_dim 64, 18 / 6 heads, 16384 tokens in all, plain call, compiler's loop against PIPE, us: dK/dV at 256 / 512 / 768 / 999 / 1536 /
-// 3072 tokens (12 / 24 / 36 / 48 / 72 / 144 streamed tiles) 41.7 / 44.1, 59.2 / 60.5, 74.3 / 76.9, 95.5 / 92.4, 116.4 / 113.9, 214.9 / 200.3;
-// dQ at 256 / 768 / 1152 / 2048 / 3072 (4 / 12 / 18 / 32 / 48 tiles) 54.8 / 56.0, 71.5 / 71.6, 85.8 / 85.8, 125.9 / 123.7, 162.8 / 159.3, with a rotary
-// embedding 63.8 / 67.0, 79.3 / 81.5, 91.6 / 93.6, 130.9 / 129.9, 167.3 / 165.9.  head_dim 128 has one wave per SIMD and nothing else to fill
-// the matrix pipe with: always.
+// head_dim 64, us, compiler's loop / PIPE, causal plain calls.  dK/dV, 18 / 6 heads, 16384 tokens in all: at 256 / 512 / 768 / 999 / 1536 / 3072 tokens
+// (12 / 24 / 36 / 48 / 72 / 144 streamed tiles) 42.1 / 42.1, 61.0 / 56.4, 75.3 / 75.7, 96.2 / 93.2, 121.8 / 115.2, 239.2 / 207.8; other heads at 48 tiles:
+// 8 / 8, 5 x 3072 110.7 / 103.1, 16 / 4, 32 x 768 95.1 / 94.4 (not causal 164.4 / 148.3), 16 / 2, 96 x 384 83.7 / 79.6.  dQ, 18 / 6 heads: at 256 / 768 / 1152 /
+// 2048 / 3072 (4 / 12 / 18 / 32 / 48 tiles) 55.0 / 55.6, 73.0 / 70.4, 89.6 / 87.6, 138.6 / 128.8, 180.6 / 167.6, with a rotary embedding 59.9 / 61.2,
+// 81.4 / 79.2, 97.7 / 94.2, 143.9 / 135.2, 184.4 / 173.8; 8 / 8, 8 x 2048 65.6 / 62.7 (not causal 109.6 / 103.8).  The lines were drawn when dK/dV still
+// computed masked blocks; below them PIPE now wins at some shapes (dK/dV 16 / 4, 64 x 384 65.6 / 61.1, 8 / 8, 16 x 1024 50.1 / 47.3) and loses or
+// is even at others (above; dQ 16 / 2, 192 x 192 117.9 / 122.9).
+// head_dim 128 has one wave per SIMD and nothing else to fill the matrix pipe with: always.  dQ and dK/dV, 16 / 4 heads: 96 x 256 201.6 / 199.1 and 117.6 /
+// 112.1 (not causal 216.4 / 220.3 and 162.9 / 142.9), 24 x 1024 298.9 / 282.1 and 258.8 / 204.9, 12 x 2048 430.1 / 402.9 and 477.2 / 372.7; 8 / 8, 48 x 256
+// 57.1 / 54.3 and 52.2 / 52.0, 6 x 2048 113.2 / 101.7 and 139.0 / 113.5.
 inline bool dkdv_pipelined(const segpt_attn_params& p) {
   constexpr int kTiles = 48;
   return dkdv_parts(p) == 1 && (p.D == 128 || (int64_t)(p.H / p.Hkv) * ((p.Sq + kBK - 1) / kBK) >= kTiles);
@@ -360,9 +365,9 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dq_bf16_kernel
     // The pipeline of the dK/dV kernel below (there: what a slot holds, and why): step n computes S^T and dP^T of block n + 1
     // (kA matrix instructions) while the vector unit turns those of block n into dS^T, then adds block n to T^T (kB);
     // the row-major fragments of block n + 2 come in as those of block n + 1 are used.
-    // dQ, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 435 -> 390 (939 k -> 764 k cycles, matrix pipe 42 -> 52 % busy; a quarter
+    // dQ, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 452 -> 406 (942 k -> 770 k cycles, matrix pipe 42 -> 52 % busy; a quarter
     // of the launch is now the workgroups' first and last thousands of cycles, one workgroup a CU); head_dim 64, 2 x 18 / 6
-    // heads, 8192 tokens 418 -> 402 (776 k -> 698 k cycles, 57 -> 64 % busy, 1.86 -> 1.74 GHz).  At head_dim 64
+    // heads, 8192 tokens 437 -> 421 (775 k -> 692 k cycles, 57 -> 64 % busy, 1.78 -> 1.65 GHz).  At head_dim 64
     // everything is in ordinary registers (248 of 256, 255 with a rotary embedding): a kernel that uses both files gets half of each, and the ordinary
     // half spills.
     constexpr int kA = 2 * KS, kB = 2 * MB;
@@ -909,9 +914,9 @@ __global__ __launch_bounds__(kThreadsM, D == 64 ? 2 : 1) void bwd_dkdv_bf16_kern
     // The accumulators and the stationary rows live in accumulation registers, scores and dP in ordinary ones; a kernel
     // of more than 256 registers gets one form for all matrix instructions from the compiler, hence the inline assembly,
     // whose wait states tests/test_mfma_hazards.py checks on the built code.
-    // dK/dV, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 529 -> 436 (1161 k -> 745 k cycles, matrix pipe 45 -> 73 % busy; the
-    // card holds its power, so the clock gives part of it back, 2.20 -> 1.71 GHz); head_dim 64, 2 x 18 / 6 heads, 8192 tokens 572 ->
-    // 535 (54 -> 68 %), 8 x 2048 154 -> 152 (48 -> 57 %).
+    // dK/dV, us: head_dim 128, 4 x 16 / 4 heads, 4096 tokens 543 -> 451 (1159 k -> 741 k cycles, matrix pipe 46 -> 71 % busy; the
+    // card holds its power, so the clock gives part of it back, 2.13 -> 1.64 GHz); head_dim 64, 2 x 18 / 6 heads, 8192 tokens 599 ->
+    // 556 (54 -> 67 %), 8 x 2048 161 -> 156 (48 -> 55 %).
     constexpr int kA = 2 * KS, kB = 4 * MB;
     // i-th product of the first half: k-step of S (0 .. KS-1) or KS + that of dP.  S leads, so that the statistics from which
     // dP starts, requested last, have time.
